@@ -5,11 +5,21 @@
 //   lse[i]  = ln sum_j exp(z[i,j]);   out_i = sum_j exp(z[i,j] - lse[i]) v_j
 // with the query head h reading kv head h / (H / Hkv).
 //
-// Work decomposition (one workgroup = 8 waves = 512 threads per CU, two waves per SIMD; 4-wave
-// workgroups, two per CU, when the grid is too small for 8-wave ones):
+// Work decomposition (one workgroup = 8 waves = 512 threads per CU, two waves per SIMD, or 4-wave
+// workgroups, two per CU):
 //   * a workgroup owns one KV head and HP query heads of its GQA group (HP = 2 when the group
-//     size is even) over NW * 32/HP consecutive query positions; every K/V tile it streams
+//     size is even) over (NW / KS) * 32/HP consecutive query positions; every K/V tile it streams
 //     through LDS serves all HP heads;
+//   * its waves form KS key groups of NW / KS column waves.  KS = 1 on large grids.  Where a launch
+//     has too few query tiles to fill the CUs, or one round of causal tiles leaves most of the chip
+//     waiting for the longest, KS = 2 or 4 shortens every workgroup and makes more of them: each step
+//     then brings 128 keys, group g takes its 64 (KS = 2) or 32 (KS = 4) of them, and the groups'
+//     running max, row sum and O are merged through LDS at the end.  What bounds it there: with half
+//     or a quarter of the query positions per workgroup each LDS DMA byte serves half or a quarter of
+//     the MFMAs (a step of the same MFMA work takes 1.06x the time at KS = 2, 1.4x at KS = 4), so the
+//     launch takes the form that a cost estimate from both effects picks (launch_cost).  Measured
+//     (16 / 8 heads, causal, with bias; before: 4-wave workgroups with the key split below): 1024
+//     rows 22.6 -> 16.0 us, 2048 40.5 -> 32.9, 2320 44.7 -> 39.2, 4096 88.5 -> 76.6;
 //   * each wave owns 32 MFMA columns in two blocks of 16: 32 consecutive query positions of one
 //     head (half the waves take each head of a pair), so a wave reads one head's key bias per
 //     tile; the KV sequence is streamed in 64-key tiles by LDS DMA (buffer_load ...
@@ -42,19 +52,19 @@ namespace tg {
 namespace {
 
 constexpr int kD = 128;        // head dim
-constexpr int kBN = 64;        // keys per tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-// A wave's 32 MFMA columns are 32 consecutive query positions of one head; a workgroup of NW waves
-// covers NW * 32/HP positions of its HP heads.  NW = 8 (two waves per SIMD, one workgroup per CU)
-// unless the grid would then be too small to fill the chip, where NW = 4 (two workgroups per CU)
-// halves the query tile.
-template <int HP> constexpr int qpw() { return 32 / HP; }
-template <int NW, int HP> constexpr int bm() { return NW * qpw<HP>(); }
+// A wave's 32 MFMA columns are 32 consecutive query positions of one head; a workgroup of NW waves in
+// KS key groups covers (NW / KS) * 32/HP positions of its HP heads.  NW = 8: two waves per SIMD, one
+// workgroup per CU; NW = 4 (KS = 1 only): two workgroups per CU.
+template <int NW, int KS> constexpr int col_waves() { return NW / KS; }
+template <int CW, int HP> constexpr int bm() { return CW * 32 / HP; }
 constexpr int kQW = 32;   // query positions per wave
+// Keys per wave and step, and per workgroup and step (one ring slot)
+template <int KS> constexpr int wave_keys() { return KS == 4 ? 32 : 64; }
+template <int KS> constexpr int step_keys() { return KS * wave_keys<KS>(); }
 
 constexpr int kKRowBytes = kD * 2;      // one K or V row in LDS (256 B, 16 chunks of 16 B)
-constexpr int kKTileBytes = kBN * kKRowBytes;
 constexpr int kStages = 2;              // K/V/bias ring: tile t resident, tile t+1 in flight
 
 struct FwdArgs {
@@ -117,28 +127,32 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) {
   return d;
 }
 
-// Wave w owns head wave_head(w) of the workgroup's HP heads (waves 0 .. NW/2-1 the first of a pair,
-// the others the second) at positions wave_pos(w) .. +31 of the workgroup's query tile; its column
-// block cb (0, 1) is positions 16 cb .. 16 cb + 15 of those, lane l holding column l%16 of each.
-// One head per wave means one bias row per wave.
-template <int NW, int HP> __device__ __forceinline__ int wave_head(int w) { return HP == 2 ? w / (NW / 2) : 0; }
-template <int NW, int HP> __device__ __forceinline__ int wave_pos(int w) { return kQW * (HP == 2 ? w % (NW / 2) : w); }
+// Column wave w (of the CW in a key group) owns head wave_head(w) of the workgroup's HP heads (column
+// waves 0 .. CW/2-1 the first of a pair, the others the second) at positions wave_pos(w) .. +31 of
+// the workgroup's query tile; its column block cb (0, 1) is positions 16 cb .. 16 cb + 15 of those,
+// lane l holding column l%16 of each.  One head per wave means one bias row per wave.
+template <int CW, int HP> __device__ __forceinline__ int wave_head(int w) { return HP == 2 ? w / (CW / 2) : 0; }
+template <int CW, int HP> __device__ __forceinline__ int wave_pos(int w) { return kQW * (HP == 2 ? w % (CW / 2) : w); }
 __device__ __forceinline__ int col_query(int cb, int c16) { return 16 * cb + c16; }
 
-template <int NW, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
+template <int NW, int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a) {
   constexpr int kWaves = NW;
-  constexpr int BM = bm<NW, HP>();
+  constexpr int CW = col_waves<NW, KS>();
+  constexpr int BM = bm<CW, HP>();
+  constexpr int KN = wave_keys<KS>(), SK = step_keys<KS>();
+  constexpr int KB = KN / 16, ST = KN / 32;   // 16-key blocks and 32-key steps of a wave's keys
+  constexpr int kKTileBytes = SK * kKRowBytes;
   // One __shared__ object per ring slot: the compiler separates LDS-DMA writes from LDS reads only
   // across distinct objects, so the DMA of tile t+1 does not hold up the reads of tile t.
   static_assert(kStages == 2, "two named LDS objects per operand");
   __shared__ __attribute__((aligned(1024))) char ks0[kKTileBytes], ks1[kKTileBytes];
   __shared__ __attribute__((aligned(1024))) char vs0[kKTileBytes], vs1[kKTileBytes];
   // bias rows padded by 4 floats so that the two heads' rows fall on different banks
-  __shared__ __attribute__((aligned(256))) float bs0[HP][kBN + 4], bs1[HP][kBN + 4];
+  __shared__ __attribute__((aligned(256))) float bs0[HP][SK + 4], bs1[HP][SK + 4];
   auto kslot = [&](auto b) -> char * { if constexpr (decltype(b)::value == 0) return ks0; else return ks1; };
   auto vslot = [&](auto b) -> char * { if constexpr (decltype(b)::value == 0) return vs0; else return vs1; };
-  auto bslot = [&](auto b) -> float (*)[kBN + 4] {
+  auto bslot = [&](auto b) -> float (*)[SK + 4] {
     if constexpr (decltype(b)::value == 0) return bs0; else return bs1;
   };
 
@@ -206,17 +220,22 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   const uint32_t vspan = sk > 0 ? (uint32_t)(((int64_t)(sk - 1) * a.v_rs + kD) * 2) : 0u;
   const brsrc_t krs = make_rsrc(kbase, kspan);
   const brsrc_t vrs = make_rsrc(vbase, vspan);
-  // the bias row of head h0 + w is loaded by wave w < HP, through a descriptor of exactly its sk
-  // columns: columns past the sequence's keys read as 0 (whatever the table holds there)
-  const int bwave = __builtin_amdgcn_readfirstlane(wave < HP ? wave : 0);
+  // the step's bias values of head h0 + w / BP are loaded by wave w < HP BP, 64 each, through a
+  // descriptor of exactly its sk columns: columns past the sequence's keys read as 0 (whatever the
+  // table holds there)
+  constexpr int BP = SK / 64;
+  const int bwave = __builtin_amdgcn_readfirstlane(wave < HP * BP ? wave : 0);
   const float *bbase =
-      HAS_BIAS ? a.bias + (int64_t)b * a.bias_bs + (int64_t)(h0 + bwave) * a.bias_hs : nullptr;
+      HAS_BIAS ? a.bias + (int64_t)b * a.bias_bs + (int64_t)(h0 + bwave / BP) * a.bias_hs : nullptr;
   const brsrc_t brs = make_rsrc(bbase, (HAS_BIAS && sk > 0) ? (uint32_t)sk * 4u : 0u);
 
   // ---- this wave's head and queries, and its Q fragments (B operand of S^T = K Q^T, 32 d per
   // k-step) ----
-  const int hw = wave_head<NW, HP>(wave);
-  const int qw0 = q0 + wave_pos<NW, HP>(wave);
+  // wave w: column wave w % CW of key group w / CW
+  const int cw = KS == 1 ? wave : wave % CW;
+  const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave / CW);
+  const int hw = wave_head<CW, HP>(cw);
+  const int qw0 = q0 + wave_pos<CW, HP>(cw);
   int qrow[2];
   bool qvalid[2];
 #pragma unroll
@@ -236,7 +255,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
 
   int kv_end = sk;
   if constexpr (CAUSAL) kv_end = min(sk, q0 + BM + off);
-  const int n_tiles = kv_end > 0 ? (kv_end + kBN - 1) / kBN : 0;
+  const int n_tiles = kv_end > 0 ? (kv_end + SK - 1) / SK : 0;
   // key tiles [t_lo, t_hi) of this workgroup (a split tile's chunk covers its share of them)
   int t_lo = 0, t_hi = n_tiles;
   if (chunk >= 0) {
@@ -245,7 +264,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   }
 
   // ---- per-lane DMA source offsets (bytes within a tile; + tile * 64 rows per tile) ----
-  // A 16 KB tile is 16 wave-loads of 1 KB; wave w issues loads w, w + kWaves, ...
+  // A tile of SK rows is SK/4 wave-loads of 1 KB; wave w issues loads w, w + kWaves, ...
   constexpr int kLoads = kKTileBytes / 1024 / kWaves;
   uint32_t koff[kLoads], voff[kLoads];
 #pragma unroll
@@ -259,8 +278,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     voff[it] = (uint32_t)(vkey * a.v_rs * 2 + vc * 16);
   }
   auto issue_tile = [&](int tile, auto buf_c) {
-    const uint32_t kb0 = (uint32_t)((int64_t)tile * kBN * a.k_rs * 2);
-    const uint32_t vb0 = (uint32_t)((int64_t)tile * kBN * a.v_rs * 2);
+    const uint32_t kb0 = (uint32_t)((int64_t)tile * SK * a.k_rs * 2);
+    const uint32_t vb0 = (uint32_t)((int64_t)tile * SK * a.v_rs * 2);
     char *kd = kslot(buf_c), *vd = vslot(buf_c);
     // the LDS destination goes to M0: with the wave index in a scalar register it is scalar
     // arithmetic instead of a per-lane add and a readfirstlane per DMA (+0.5 % at 32k)
@@ -271,8 +290,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
       dma16(vrs, vd + (wv + it * kWaves) * 1024, vb0 + voff[it]);
     }
     if constexpr (HAS_BIAS) {
-      if (wave < HP)
-        dma4(brs, &bslot(buf_c)[wave][0], (uint32_t)((tile * kBN + lane) * 4));
+      if (wave < HP * BP)
+        dma4(brs, &bslot(buf_c)[wave / BP][64 * (wave % BP)], (uint32_t)((tile * SK + 64 * (wave % BP) + lane) * 4));
     }
   };
 
@@ -312,48 +331,50 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   // and tile t+1 is issued into it while tile t is computed.
   auto tile_step = [&](int t, auto buf_c) {
     constexpr int BUF = decltype(buf_c)::value;
-    const int n0 = t * kBN;
+    const int n0 = t * SK + KN * kg;   // this wave's first key of the step
     wait_vm<0>();
     ring_barrier();
     if (t + 1 < t_hi) issue_tile(t + 1, std::integral_constant<int, 1 - BUF>());
     if (!wave_has_rows || (CAUSAL && n0 > qw_hi + off)) return;
 
-    // ---- S^T = K Q^T + bias: 2 column blocks x 4 key blocks x 4 d-steps.  The accumulators start
+    // ---- S^T = K Q^T + bias: 2 column blocks x KB key blocks x 4 d-steps.  The accumulators start
     // from the bias of their keys (raw-score units), so the bias add costs no VALU work. ----
-    f32x4 sacc[2][4];
+    f32x4 sacc[2][KB];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < KB; ++kb) {
       if constexpr (HAS_BIAS) {
         // both column blocks are the wave's head: one read of its 16 keys' bias serves both
-        sacc[0][kb] = *reinterpret_cast<const f32x4 *>(&bslot(buf_c)[hw][32 * (kb >> 1) + 8 * G + 4 * (kb & 1)]);
+        sacc[0][kb] =
+            *reinterpret_cast<const f32x4 *>(&bslot(buf_c)[hw][KN * kg + 32 * (kb >> 1) + 8 * G + 4 * (kb & 1)]);
       } else {
         sacc[0][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
       sacc[1][kb] = sacc[0][kb];
     }
-    // all 16 K fragments of the tile are read before the first MFMA, so LDS latency is paid once
-    bf16x8 kfr[4][4];
+    // all K fragments of the wave's keys are read before the first MFMA, so LDS latency is paid once
+    bf16x8 kfr[KB][4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
         const int lr = 16 * kb + c16;
-        kfr[kb][ks] = lds_load16(kslot(buf_c), lr * kKRowBytes + ((uint32_t)((4 * ks + G) ^ c16) << 4));
+        kfr[kb][ks] = lds_load16(kslot(buf_c) + KN * kg * kKRowBytes,
+                                 lr * kKRowBytes + ((uint32_t)((4 * ks + G) ^ c16) << 4));
       }
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) sacc[cb][kb] = mfma16(kfr[kb][ks], qf[cb][ks], sacc[cb][kb]);
       }
     }
 
-    // ---- online softmax: lane holds 16 keys of one column per block; the other 48 keys of that
+    // ---- online softmax: lane holds KN/4 keys of one column per block; the other keys of that
     // column sit in lanes l^16, l^32, l^48 ----
-    const bool need_mask = (n0 + kBN > sk) || (CAUSAL && n0 + kBN - 1 > qw0 + off);
+    const bool need_mask = (n0 + KN > sk) || (CAUSAL && n0 + KN - 1 > qw0 + off);
     if (need_mask) {
       // key > lim -> -inf by adding 0 or -inf, selected by the sign of lim - key (an arithmetic
       // shift the compiler cannot turn back into per-element compares, whose 64-bit results would
@@ -363,7 +384,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
         int lim = sk - 1;
         if constexpr (CAUSAL) lim = min(lim, qrow[cb] + off);
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
+        for (int kb = 0; kb < KB; ++kb) {
           const int rel = lim - (n0 + 32 * (kb >> 1) + 8 * G + 4 * (kb & 1));
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -380,9 +401,13 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     for (int cb = 0; cb < 2; ++cb) {
       const f32x4 *s = sacc[cb];
       const float m0 = vmax3(s[0][0], s[0][1], s[0][2]), m1 = vmax3(s[0][3], s[1][0], s[1][1]);
-      const float m2 = vmax3(s[1][2], s[1][3], s[2][0]), m3 = vmax3(s[2][1], s[2][2], s[2][3]);
-      const float m4 = vmax3(s[3][0], s[3][1], s[3][2]);
-      mt[cb] = vmax3(vmax3(m0, m1, m2), vmax3(m3, m4, s[3][3]), m0);
+      if constexpr (KB == 4) {
+        const float m2 = vmax3(s[1][2], s[1][3], s[2][0]), m3 = vmax3(s[2][1], s[2][2], s[2][3]);
+        const float m4 = vmax3(s[3][0], s[3][1], s[3][2]);
+        mt[cb] = vmax3(vmax3(m0, m1, m2), vmax3(m3, m4, s[3][3]), m0);
+      } else {
+        mt[cb] = vmax3(vmax3(s[1][2], s[1][3], m0), m1, m0);
+      }
     }
     // Both column blocks' maxima over the four lane groups in three permlane swaps:
     // swap16(cb0, cb1) + max leaves cb0's pair maxima (groups 0|1, 2|3) in groups 0 and 2 and cb1's
@@ -415,11 +440,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
       }
     }
     // P rounded to bf16 pairs (the B operand of P V and of the row-sum product)
-    uint32_t pk[2][4][2];
+    uint32_t pk[2][KB][2];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
           const float p0 = fast_exp2(fmaf(sacc[cb][kb][i], a.scale_log2, mneg[cb]));
@@ -429,9 +454,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
       }
     }
 
-    // ---- O^T += V^T P^T: 2 key steps x 8 d-blocks x 2 column blocks ----
+    // ---- O^T += V^T P^T: ST key steps x 8 d-blocks x 2 column blocks ----
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
+    for (int st = 0; st < ST; ++st) {
       bf16x8 pb[2];
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) {
@@ -443,8 +468,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
       const uint32_t krow = (uint32_t)(32 * st * kKRowBytes);
 #pragma unroll
       for (int dblk = 0; dblk < 8; ++dblk) {
-        const s16x4 lo = lds_read_tr16(vslot(buf_c) + krow + vch[dblk]);
-        const s16x4 hi = lds_read_tr16(vslot(buf_c) + krow + 4 * kKRowBytes + vch[dblk]);
+        const char *vbuf = vslot(buf_c) + KN * kg * kKRowBytes;
+        const s16x4 lo = lds_read_tr16(vbuf + krow + vch[dblk]);
+        const s16x4 hi = lds_read_tr16(vbuf + krow + 4 * kKRowBytes + vch[dblk]);
         const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) oacc[cb][dblk] = mfma16(vf, pb[cb], oacc[cb][dblk]);
@@ -459,6 +485,70 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   }
   if (t < t_hi) tile_step(t, std::integral_constant<int, 0>());
 
+  // ---- merge of the KS key groups (KS > 1): a column's max over the groups, every group's row sum
+  // and O rescaled to it (weight 0 where a group saw no key), then group g adds up d-blocks DB g ..
+  // DB g + DB-1 of all groups in group order, through the K / V ring, which no wave reads any more.
+  // Group kg's waves are left with the final m, l and those d-blocks in oacc[cb][0 .. DB-1]. ----
+  constexpr int DB = 8 / KS;
+  if constexpr (KS > 1) {
+    constexpr int kSlot = 64 * 16;                                 // one f32x4 per lane
+    static_assert((KS - 1) * CW * 2 * DB * kSlot <= kKTileBytes, "a group's pieces fit one ring slot");
+    __shared__ __attribute__((aligned(16))) float2 ml_s[KS][CW][2][16];
+    if (G == 0) {
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) ml_s[kg][cw][cb][c16] = float2{mrun[cb], lacc[cb][0]};
+    }
+    __syncthreads();   // also: every wave is done with the ring
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      float2 g[KS];
+      float m = -INFINITY, l = 0.f;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        g[i] = ml_s[i][cw][cb][c16];
+        m = fmaxf(m, g[i].x);
+      }
+      const float mz = m == -INFINITY ? 0.f : m;   // no key in any group: every weight is 2^-inf = 0
+#pragma unroll
+      for (int i = 0; i < KS; ++i) l += g[i].y * fast_exp2(g[i].x - mz);
+      const float w = fast_exp2(mrun[cb] - mz);
+      mrun[cb] = m;
+      lacc[cb][0] = l;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) oacc[cb][d] *= w;
+    }
+    auto dst = [&](int g) -> char * { return g == 0 ? ks0 : g == 1 ? vs0 : g == 2 ? ks1 : vs1; };
+#pragma unroll
+    for (int g = 0; g < KS; ++g) {
+      if (g == kg) continue;
+      char *p = dst(g) + ((kg - (kg > g ? 1 : 0)) * CW + cw) * 2 * DB * kSlot + lane * 16;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int d = 0; d < DB; ++d) *reinterpret_cast<f32x4 *>(p + (cb * DB + d) * kSlot) = oacc[cb][g * DB + d];
+    }
+    // this group's own d-blocks to the front
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        f32x4 own = oacc[cb][d];
+#pragma unroll
+        for (int g = 1; g < KS; ++g) own = kg == g ? oacc[cb][g * DB + d] : own;
+        oacc[cb][d] = own;
+      }
+    __syncthreads();
+    const char *src = kg == 0 ? ks0 : kg == 1 ? vs0 : kg == 2 ? ks1 : vs1;
+#pragma unroll
+    for (int i = 0; i < KS - 1; ++i)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+          oacc[cb][d] += *reinterpret_cast<const f32x4 *>(src + ((i * CW + cw) * 2 * DB + cb * DB + d) * kSlot + lane * 16);
+  }
+  const int db0 = DB * kg;   // first d-block held
+
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) ----
   float l[2], inv[2];
 #pragma unroll
@@ -467,27 +557,30 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     inv[cb] = l[cb] > 0.f ? 1.f / l[cb] : 0.f;
   }
   if (chunk >= 0) {
-    // partial result of this key chunk: O / l as bf16 (piece j = 4 cb + p holds d-blocks 2p and
-    // 2p+1 of column block cb; each piece a coalesced 1 KB wave store) and, per column block,
-    // (running max in log2 units, row sum l)
-    const int64_t pw = (hunit * a.ns + chunk) * kWaves + wave;
+    // partial result of this key chunk: O / l as bf16 (piece 4 cb + p holds d-blocks 2p and 2p+1 of
+    // column block cb; each piece a coalesced 1 KB wave store) and, per column block, (running max
+    // in log2 units, row sum l)
+    const int64_t pw = (hunit * a.ns + chunk) * CW + cw;
     u32x4 *po = reinterpret_cast<u32x4 *>(a.ws_o) + pw * (8 * 64) + lane;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int cb = j >> 2, p = j & 3;
-      const f32x4 &o0 = oacc[cb][2 * p], &o1 = oacc[cb][2 * p + 1];
-      const float s = inv[cb];
-      const u32x4 w = {pack_bf16x2(o0[0] * s, o0[1] * s), pack_bf16x2(o0[2] * s, o0[3] * s),
-                       pack_bf16x2(o1[0] * s, o1[1] * s), pack_bf16x2(o1[2] * s, o1[3] * s)};
-      po[j * 64] = w;
-    }
-    float2 *pml = reinterpret_cast<float2 *>(a.ws_ml) + pw * 128 + lane;
+    for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      float2 ml;
-      ml.x = mrun[cb];
-      ml.y = l[cb];
-      pml[cb * 64] = ml;
+      for (int p = 0; p < DB / 2; ++p) {
+        const f32x4 &o0 = oacc[cb][2 * p], &o1 = oacc[cb][2 * p + 1];
+        const float s = inv[cb];
+        const u32x4 w = {pack_bf16x2(o0[0] * s, o0[1] * s), pack_bf16x2(o0[2] * s, o0[3] * s),
+                         pack_bf16x2(o1[0] * s, o1[1] * s), pack_bf16x2(o1[2] * s, o1[3] * s)};
+        po[(4 * cb + db0 / 2 + p) * 64] = w;
+      }
+    if (kg == 0) {
+      float2 *pml = reinterpret_cast<float2 *>(a.ws_ml) + pw * 128 + lane;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        float2 ml;
+        ml.x = mrun[cb];
+        ml.y = l[cb];
+        pml[cb * 64] = ml;
+      }
     }
     return;
   }
@@ -498,12 +591,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     bf16_t *orow = obase + (int64_t)qrow[cb] * a.o_rs + (int64_t)hl * a.o_hs;
     const float s = inv[cb];
 #pragma unroll
-    for (int dblk = 0; dblk < 8; ++dblk) {
-      const f32x4 &o = oacc[cb][dblk];
+    for (int d = 0; d < DB; ++d) {
+      const f32x4 &o = oacc[cb][d];
       const u32x2 w = {pack_bf16x2(o[0] * s, o[1] * s), pack_bf16x2(o[2] * s, o[3] * s)};
-      *reinterpret_cast<u32x2 *>(orow + 16 * dblk + 4 * G) = w;
+      *reinterpret_cast<u32x2 *>(orow + 16 * (db0 + d) + 4 * G) = w;
     }
-    if (G == 0) {
+    if (G == 0 && kg == 0) {
       const float lse = l[cb] > 0.f ? (mrun[cb] + __log2f(l[cb])) * kLn2 : INFINITY;
       const int hh = h0 + hl;
       if constexpr (VARLEN)
@@ -523,21 +616,21 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
 // m = max m_c, w_c = l_c 2^(m_c - m), O = sum w_c O_c / sum w_c, lse = (m + log2 sum w_c) ln 2.
 // Chunks that saw no key (l_c = 0) weigh nothing.
 constexpr int kCombineMaxGroups = 8;
-template <int NW, int HP, bool VARLEN>
+template <int CW, int HP, bool VARLEN>
 __global__ __launch_bounds__(512) void keybias_fwd_combine_kernel(FwdArgs a, int CG) {
-  constexpr int BM = bm<NW, HP>();
+  constexpr int BM = bm<CW, HP>();
   // (m, wsum, acc[8]) of groups 1..CG-1 of each piece: PP * (CG - 1) < 8 slots
   __shared__ float part[kCombineMaxGroups - 1][10][64];
   const int PP = 8 / CG;                                   // pieces per workgroup
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int cg = wv % CG, pj = wv / CG;
   const int j = (int)(blockIdx.x % CG) * PP + pj;          // piece
-  const int wave = (int)((blockIdx.x / CG) % NW);          // forward wave whose columns these are
-  const int64_t hunit = (blockIdx.x / CG) / NW;
+  const int wave = (int)((blockIdx.x / CG) % CW);          // forward wave whose columns these are
+  const int64_t hunit = (blockIdx.x / CG) / CW;
   float (*mypart)[10][64] = part + pj * (CG - 1);
   const int c16 = lane & 15, G = lane >> 4;
   const int cb = j >> 2, p = j & 3;                        // column block, d-block pair of the piece
-  const int hl = wave_head<NW, HP>(wave);
+  const int hl = wave_head<CW, HP>(wave);
   const int per_q = a.hkv * (a.group / HP);
   const int x = (int)(hunit % per_q), r2 = (int)(hunit / per_q);
   const int kh = x % a.hkv, hg = x / a.hkv;
@@ -551,21 +644,21 @@ __global__ __launch_bounds__(512) void keybias_fwd_combine_kernel(FwdArgs a, int
     row0 = s0;
     sq = min(s1 - s0, a.sq);
   }
-  const int qw0 = qt * BM + wave_pos<NW, HP>(wave);
+  const int qw0 = qt * BM + wave_pos<CW, HP>(wave);
   if (qw0 >= sq) return;   // workgroup-uniform: the forward computed nothing for these rows
   const int qrow = qw0 + col_query(cb, c16);
   const bool valid = qrow < sq;
 
   const float2 *ml = reinterpret_cast<const float2 *>(a.ws_ml);
   const u32x4 *po = reinterpret_cast<const u32x4 *>(a.ws_o);
-  const int64_t pw0 = hunit * a.ns * NW + wave;   // chunk c: pw0 + c * NW
+  const int64_t pw0 = hunit * a.ns * CW + wave;   // chunk c: pw0 + c * CW
   // fold this group's chunks, the weights relative to the largest m seen so far
   float mmax = -INFINITY, wsum = 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (valid) {
 #pragma unroll 4
     for (int c = cg; c < a.ns; c += CG) {
-      const int64_t pw = pw0 + (int64_t)c * NW;
+      const int64_t pw = pw0 + (int64_t)c * CW;
       const float2 mc = ml[pw * 128 + cb * 64 + lane];
       const u32x4 pv = po[pw * (8 * 64) + j * 64 + lane];
       if (!(mc.y > 0.f)) continue;
@@ -623,29 +716,34 @@ __global__ __launch_bounds__(512) void keybias_fwd_combine_kernel(FwdArgs a, int
   }
 }
 
-template <int NW, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
+template <int NW, int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
 void launch_fwd(const FwdArgs &a, int nblocks, hipStream_t stream) {
-  hipLaunchKernelGGL((keybias_fwd_kernel<NW, HP, CAUSAL, HAS_BIAS, VARLEN>), dim3(nblocks), dim3(64 * NW), 0,
+  constexpr int CW = col_waves<NW, KS>();
+  hipLaunchKernelGGL((keybias_fwd_kernel<NW, KS, HP, CAUSAL, HAS_BIAS, VARLEN>), dim3(nblocks), dim3(64 * NW), 0,
                      stream, a);
   if (a.heavy_blocks > 0) {
     // chunk groups: up to 8, and at least two chunks per group; CG workgroups of 512 threads per
-    // (split tile, forward wave)
+    // (split tile, column wave)
     int cgroups = 1;
     while (cgroups < kCombineMaxGroups && 2 * cgroups * 2 <= a.ns) cgroups *= 2;
-    const int64_t blocks = a.heavy_blocks / a.ns * NW * cgroups;
-    hipLaunchKernelGGL((keybias_fwd_combine_kernel<NW, HP, VARLEN>), dim3((unsigned)blocks), dim3(512), 0, stream, a,
+    const int64_t blocks = a.heavy_blocks / a.ns * CW * cgroups;
+    hipLaunchKernelGGL((keybias_fwd_combine_kernel<CW, HP, VARLEN>), dim3((unsigned)blocks), dim3(512), 0, stream, a,
                        cgroups);
   }
 }
 
 template <bool VARLEN>
-void dispatch_fwd(const FwdArgs &a, int nw, int hp, bool causal, bool has_bias, int nblocks, hipStream_t s) {
+void dispatch_fwd(const FwdArgs &a, int nw, int ks, int hp, bool causal, bool has_bias, int nblocks, hipStream_t s) {
 #define TG_FWD_CASE(HPV, C, B)                                              \
   if (hp == HPV && causal == C && has_bias == B) {                          \
-    if (nw == 8)                                                            \
-      launch_fwd<8, HPV, C, B, VARLEN>(a, nblocks, s);                      \
-    else                                                                    \
-      launch_fwd<4, HPV, C, B, VARLEN>(a, nblocks, s);                      \
+    if (nw == 4)                                                            \
+      launch_fwd<4, 1, HPV, C, B, VARLEN>(a, nblocks, s);                   \
+    else if (ks == 1)                                                       \
+      launch_fwd<8, 1, HPV, C, B, VARLEN>(a, nblocks, s);                   \
+    if constexpr (!VARLEN) {                                                \
+      if (ks == 2) launch_fwd<8, 2, HPV, C, B, false>(a, nblocks, s);       \
+      if (ks == 4) launch_fwd<8, 4, HPV, C, B, false>(a, nblocks, s);       \
+    }                                                                       \
     return;                                                                 \
   }
   TG_FWD_CASE(2, true, true)
@@ -661,48 +759,50 @@ void dispatch_fwd(const FwdArgs &a, int nw, int hp, bool causal, bool has_bias, 
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Waves per workgroup and query tiles for a launch over `rows` query positions x `units` (sequence,
-// head group) pairs: 8-wave workgroups when that still gives at least two per CU, else 4-wave ones.
-void pick_tiling(int hp, int rows, int64_t units, int &nw, int &n_qtiles) {
-  const int bm8 = hp == 2 ? bm<8, 2>() : bm<8, 1>();
-  const int bm4 = hp == 2 ? bm<4, 2>() : bm<4, 1>();
-  const int64_t t8 = (rows + bm8 - 1) / bm8;
-  nw = t8 * units >= 2 * (int64_t)device_cus() ? 8 : 4;
-  n_qtiles = nw == 8 ? (int)t8 : (rows + bm4 - 1) / bm4;
-}
+// The four forms of the kernel: waves per workgroup and key groups.  A CU holds one workgroup of eight
+// waves or two of four.
+struct Form {
+  int nw, ks;
+  float group, solo, full, combine;   // see launch_cost
+};
 
-// Key-range split plan.  A grid that leaves at least a quarter of the resident-workgroup slots
-// empty from the start (Phase 2 at small K, a few rows over a long cache, single-row decode) is
-// bound by its longest tiles while the chip idles: the tiles whose key range exceeds 1/ns of the
-// longest are split into ns chunks of consecutive key tiles (ns from the free slots, at least 4
-// key tiles per chunk), merged by the combine kernel.  A grid that fills the slots (a 4k prompt)
-// is not split: measured, the split's partial traffic and second launch cost more there than the
-// causal tail it removes.  Returns ns = 1 when nothing is split.
+// Query tiles and key steps of a launch in one form (causal limits included).
+struct Tiles {
+  int bm, step, n_qtiles, sq, sk;
+  bool causal;
+  Tiles(const Form &f, int hp, int sq_, int sk_, bool causal_)
+      : bm(f.nw / f.ks * 32 / hp), step(f.ks == 1 ? 64 : 128), n_qtiles((sq_ + bm - 1) / bm), sq(sq_), sk(sk_),
+        causal(causal_) {}
+  int steps(int qt) const {
+    int64_t kv_end = sk;
+    if (causal) kv_end = std::min<int64_t>(sk, (int64_t)(qt + 1) * bm + sk - sq);
+    return kv_end > 0 ? (int)((kv_end + step - 1) / step) : 0;
+  }
+};
+
+// Key-range split plan of a launch.  A grid that leaves at least a quarter of the resident-workgroup
+// slots empty from the start (a few rows over a long cache, single-row decode) is bound by its
+// longest tiles while the chip idles: the tiles whose key range exceeds 1/ns of the longest are split
+// into ns chunks of consecutive key steps (ns from the free slots), merged by the combine kernel.
+// Returns ns = 1 when nothing is split.
 struct SplitPlan {
   int ns = 1, n_heavy = 0;
   int64_t heavy_units = 0, bytes = 0;
 };
 constexpr int64_t kPartialBytesPerLane = 8 * 16 + 2 * 8;   // O / l as 64 bf16, then (m, l) per column block
-SplitPlan plan_split(int nw, int hp, int n_qtiles, int64_t units, int sq, int sk, bool causal) {
+SplitPlan plan_split(const Form &f, const Tiles &t, int64_t units) {
   SplitPlan p;
-  const int bmq = nw == 8 ? (hp == 2 ? bm<8, 2>() : bm<8, 1>()) : (hp == 2 ? bm<4, 2>() : bm<4, 1>());
-  const int64_t slots = (int64_t)device_cus() * (8 / nw);
-  const int64_t nblocks = (int64_t)n_qtiles * units;
-  if (nblocks <= 0 || 4 * nblocks > 3 * slots || sk <= 0) return p;
-  const int off = sk - sq;
-  auto tiles = [&](int qt) -> int {
-    int kv_end = sk;
-    if (causal) kv_end = std::min<int64_t>(sk, (int64_t)(qt + 1) * bmq + off);
-    return kv_end > 0 ? (kv_end + kBN - 1) / kBN : 0;
-  };
-  const int tmax = tiles(n_qtiles - 1);
+  const int64_t slots = (int64_t)device_cus() * (8 / f.nw);
+  const int64_t nblocks = (int64_t)t.n_qtiles * units;
+  if (nblocks <= 0 || 4 * nblocks > 3 * slots || t.sk <= 0) return p;
+  const int tmax = t.steps(t.n_qtiles - 1);
   int ns = (int)std::min<int64_t>(32, std::max<int64_t>(2, slots / nblocks));
-  // at least 4 key tiles per chunk; 2 for a few query rows (a decode step), whose chunks are short
-  // enough that the tile count, not the merge, sets their time (decode at 2.3k keys: -2 %)
-  ns = std::min(ns, tmax / (sq <= 16 ? 2 : 4));
+  // at least 256 keys per chunk; 128 for a few query rows (a decode step), whose chunks are short
+  // enough that the step count, not the merge, sets their time (decode at 2.3k keys: -2 %)
+  ns = std::min(ns, tmax / ((t.sq <= 16 ? 128 : 256) / t.step));
   if (ns < 2) return p;
   int n_heavy = 0;
-  for (int qt = n_qtiles - 1; qt >= 0 && (int64_t)tiles(qt) * ns > tmax; --qt) ++n_heavy;
+  for (int qt = t.n_qtiles - 1; qt >= 0 && (int64_t)t.steps(qt) * ns > tmax; --qt) ++n_heavy;
   // The split grid (nblocks + heavy_units * (ns - 1) workgroups) must fit the resident slots: past
   // that, extra chunks only queue behind the others.  ns <= slots / nblocks already ensures it
   // unless ns was raised to 2 for a grid of more than half the slots; then only the heaviest tiles
@@ -713,19 +813,97 @@ SplitPlan plan_split(int nw, int hp, int n_qtiles, int64_t units, int sq, int sk
   p.ns = ns;
   p.n_heavy = n_heavy;
   p.heavy_units = (int64_t)n_heavy * units;
-  p.bytes = p.heavy_units * ns * nw * 64 * kPartialBytesPerLane;
+  p.bytes = p.heavy_units * ns * (f.nw / f.ks) * 64 * kPartialBytesPerLane;
   return p;
 }
 
-// Apply a plan to the launch arguments (no split if the workspace is missing or too small).
-// Returns the grid size.
-int64_t apply_split(FwdArgs &a, SplitPlan p, int nw, int64_t units, void *workspace, int64_t workspace_bytes) {
-  if (p.ns < 2 || workspace == nullptr || workspace_bytes < p.bytes) p = SplitPlan{};
+// Estimated time of a launch, in microseconds.  Workgroups are issued heaviest first to `slots`
+// places, so the launch takes at least its heaviest workgroup, its work over the places plus one start
+// per round, and k + 1 times the (k slots + 1)-th heaviest workgroup.  A workgroup takes `group`
+// (start, first loads, merge of the key groups, stores) plus `full` per key step while the chip is
+// full and `solo` while the longest workgroups run on alone; `combine` is the split's second launch.
+// The constants are fitted to launches of 1 to 16384 rows (8 to 16 heads, batches of 1 to 8) timed in
+// each form; the form they pick is within 5 % of the fastest at all of those, and where the forms
+// differ most: 4 waves / 8 waves / 8 waves with 2 / with 4 key groups take, at 1024 rows 22.6 / 25.0 /
+// 20.8 / 16.0 us, at 2048 40.5 / 40.2 / 36.6 / 32.9, at 4096 88.9 / 107.4 / 76.6 / 98.4, at 6001 142 /
+// 158 / 160 / 194, at 8192 266 / 239 / 268 / 339 (16 / 8 heads, causal, with bias).
+constexpr Form kForms[] = {{8, 1, 3.5f, 1.6f, 1.77f, 6.f},
+                           {4, 1, 2.4f, 1.3f, 1.95f, 6.f},
+                           {8, 2, 4.0f, 1.75f, 1.88f, 10.f},
+                           {8, 4, 4.2f, 1.2f, 1.25f, 6.f}};
+float launch_cost(const Form &f, const Tiles &t, int64_t units, const SplitPlan &p) {
+  const int64_t slots = (int64_t)device_cus() * (8 / f.nw), nblocks = t.n_qtiles * units;
+  const int longest = t.steps(t.n_qtiles - 1);
+  if (p.ns > 1) {   // one round; two workgroups of four waves share each CU throughout
+    const int chunk = (longest + p.ns - 1) / p.ns;
+    const int light = p.n_heavy < t.n_qtiles ? t.steps(t.n_qtiles - 1 - p.n_heavy) : 0;
+    return (f.nw == 4 ? f.full : f.solo) * std::max(chunk, light) + f.group + f.combine;
+  }
+  int64_t total = 0;
+  for (int qt = 0; qt < t.n_qtiles; ++qt) total += t.steps(qt);
+  const int64_t rounds = (nblocks + slots - 1) / slots;
+  float cost = std::max(f.solo * longest + f.group, f.full * total * units / slots + rounds * f.group);
+  for (int64_t k = 1; k < rounds; ++k)
+    cost = std::max(cost, (k + 1) * (f.solo * t.steps(t.n_qtiles - 1 - (int)(k * slots / units)) + f.group));
+  return cost;
+}
+
+struct FwdPlan {
+  int nw = 8, ks = 1, n_qtiles = 0;
+  SplitPlan split;
+};
+
+// A dense launch's form and split: the cheapest of the four forms, each with and without its split
+// where it has one and the workspace holds it.  key_groups: whether ks > 1 may be taken (its last
+// step's LDS DMA offsets reach up to 127 rows past sk and must not wrap at 4 GiB).
+FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, int64_t workspace_bytes, bool key_groups) {
+  FwdPlan best;
+  float best_cost = INFINITY;
+  for (const Form &f : kForms) {
+    if (f.ks > 1 && !key_groups) continue;
+    const Tiles t(f, hp, sq, sk, causal);
+    const SplitPlan s = plan_split(f, t, units);
+    for (int with = s.ns > 1 && s.bytes <= workspace_bytes ? 1 : 0; with >= 0; --with) {
+      const SplitPlan p = with ? s : SplitPlan{};
+      const float cost = launch_cost(f, t, units, p);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best.nw = f.nw;
+        best.ks = f.ks;
+        best.n_qtiles = t.n_qtiles;
+        best.split = p;
+      }
+    }
+  }
+  return best;
+}
+
+// A varlen launch (prefill and decode over packed rows): 8-wave workgroups when the grid gives at
+// least two per CU, else 4-wave ones with the split.  The lengths behind max_seqlen are not known
+// here, and key groups would change the order in which a column's keys are summed: of a whole gated
+// prefill at 2320 kept rows they took 0.5 % off the time and moved the logits by 2.6 %, the noise
+// of 26 bf16 layers rounded otherwise, so packed launches keep one key group.
+FwdPlan plan_varlen(int hp, int max_sq, int max_sk, int64_t units, bool causal, int64_t workspace_bytes) {
+  FwdPlan plan;
+  const Tiles wide(kForms[0], hp, max_sq, max_sk, causal), narrow(kForms[1], hp, max_sq, max_sk, causal);
+  const bool w = wide.n_qtiles * units >= 2 * (int64_t)device_cus();
+  plan.nw = w ? 8 : 4;
+  plan.n_qtiles = w ? wide.n_qtiles : narrow.n_qtiles;
+  plan.split = plan_split(kForms[w ? 0 : 1], w ? wide : narrow, units);
+  if (plan.split.bytes > workspace_bytes) plan.split = SplitPlan{};
+  return plan;
+}
+
+// Put a plan into the launch arguments.  Returns the grid size.
+int64_t apply_plan(FwdArgs &a, const FwdPlan &f, int64_t units, void *workspace) {
+  const SplitPlan &p = f.split;
+  a.n_qtiles = f.n_qtiles;
   a.ns = p.ns;
   a.n_heavy = p.n_heavy;
   a.heavy_blocks = p.heavy_units * p.ns;
   a.ws_o = static_cast<bf16_t *>(workspace);
-  a.ws_ml = workspace ? reinterpret_cast<float *>(static_cast<char *>(workspace) + p.heavy_units * p.ns * nw * 64 * 128)
+  a.ws_ml = workspace ? reinterpret_cast<float *>(static_cast<char *>(workspace) +
+                                                  p.heavy_units * p.ns * (f.nw / f.ks) * 64 * 128)
                       : nullptr;
   return a.heavy_blocks + (int64_t)(a.n_qtiles - a.n_heavy) * units;
 }
@@ -795,28 +973,30 @@ int keybias_fwd_dense(const void *q, const void *k, const void *v, const float *
   a.h = num_heads; a.hkv = num_heads_k; a.group = num_heads / num_heads_k;
   a.scale_log2 = softmax_scale * kLog2e;
   const int hp = (a.group % 2 == 0) ? 2 : 1;
-  int nw = 8;
   const int64_t units = (int64_t)batch * (num_heads / hp);
-  pick_tiling(hp, seqlen_q, units, nw, a.n_qtiles);
   TG_CHECK(workspace == nullptr || aligned16(workspace), "workspace must be 16-byte aligned");
-  const int64_t nblocks = apply_split(a, plan_split(nw, hp, a.n_qtiles, units, seqlen_q, seqlen_k, causal != 0), nw,
-                                      units, workspace, workspace_bytes);
+  const FwdPlan plan = plan_dense(hp, seqlen_q, seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0,
+                                span_ok(seqlen_k + 128ll, k_row_stride) && span_ok(seqlen_k + 128ll, v_row_stride));
+  const int64_t nblocks = apply_plan(a, plan, units, workspace);
   TG_CHECK(nblocks < (1ll << 31), "grid too large");
-  dispatch_fwd<false>(a, nw, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
+  dispatch_fwd<false>(a, plan.nw, plan.ks, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
   TG_HIP_CHECK(hipPeekAtLastError());
   return 0;
 }
 
-int64_t fwd_workspace_size(int32_t units_batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads,
+// Workspace of a dense launch (the largest split that any form of it has) or of a varlen one.
+int64_t fwd_workspace_size(bool varlen, int32_t units_batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads,
                            int32_t num_heads_k, int32_t causal) {
   if (units_batch <= 0 || seqlen_q <= 0 || seqlen_k <= 0 || num_heads <= 0 || num_heads_k <= 0 ||
       num_heads % num_heads_k != 0)
     return 0;
   const int hp = ((num_heads / num_heads_k) % 2 == 0) ? 2 : 1;
   const int64_t units = (int64_t)units_batch * (num_heads / hp);
-  int nw = 8, nq = 0;
-  pick_tiling(hp, seqlen_q, units, nw, nq);
-  return plan_split(nw, hp, nq, units, seqlen_q, seqlen_k, causal != 0).bytes;
+  if (varlen) return plan_varlen(hp, seqlen_q, seqlen_k, units, causal != 0, INT64_MAX).split.bytes;
+  int64_t bytes = 0;
+  for (const Form &f : kForms)
+    bytes = std::max(bytes, plan_split(f, Tiles(f, hp, seqlen_q, seqlen_k, causal != 0), units).bytes);
+  return bytes;
 }
 
 // Device scratch of tg_keybias_fwd_noalloc: the key-range split's partial results.  plan_split
@@ -875,7 +1055,7 @@ extern "C" int tg_keybias_fwd_noalloc(const void *q, const void *k, const void *
                                       int64_t bias_batch_stride, int64_t bias_head_stride, float softmax_scale,
                                       int32_t causal, hipStream_t stream) {
   clear_error();
-  const int64_t need = fwd_workspace_size(batch, seqlen_q, seqlen_k, num_heads, num_heads_k, causal);
+  const int64_t need = fwd_workspace_size(false, batch, seqlen_q, seqlen_k, num_heads, num_heads_k, causal);
   TG_CHECK(need <= kScratchBytes,
            "tg_keybias_fwd_noalloc: this launch's key-range split needs %lld bytes of scratch, above the "
            "library's static %lld; call tg_keybias_fwd with a workspace instead",
@@ -936,15 +1116,12 @@ int keybias_fwd_varlen(const void *q, const void *k, const void *v, const float 
   a.h = num_heads; a.hkv = num_heads_k; a.group = num_heads / num_heads_k;
   a.scale_log2 = softmax_scale * kLog2e;
   const int hp = (a.group % 2 == 0) ? 2 : 1;
-  int nw = 8;
   const int64_t units = (int64_t)num_seqs * (num_heads / hp);
-  pick_tiling(hp, max_seqlen_q, units, nw, a.n_qtiles);
   TG_CHECK(workspace == nullptr || aligned16(workspace), "workspace must be 16-byte aligned");
-  const int64_t nblocks = apply_split(
-      a, plan_split(nw, hp, a.n_qtiles, units, max_seqlen_q, max_seqlen_k, causal != 0), nw, units, workspace,
-      workspace_bytes);
+  const FwdPlan plan = plan_varlen(hp, max_seqlen_q, max_seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0);
+  const int64_t nblocks = apply_plan(a, plan, units, workspace);
   TG_CHECK(nblocks < (1ll << 31), "grid too large");
-  dispatch_fwd<true>(a, nw, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
+  dispatch_fwd<true>(a, plan.nw, plan.ks, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
   TG_HIP_CHECK(hipPeekAtLastError());
   return 0;
 }
@@ -990,15 +1167,15 @@ extern "C" int tg_keybias_varlen_kv_fwd(const void *q, const void *k, const void
 extern "C" int64_t tg_keybias_varlen_kv_fwd_workspace_size(int32_t num_seqs, int32_t max_seqlen_q,
                                                             int32_t max_seqlen_k, int32_t num_heads,
                                                             int32_t num_heads_k, int32_t causal) {
-  return fwd_workspace_size(num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_heads_k, causal);
+  return fwd_workspace_size(true, num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_heads_k, causal);
 }
 
 extern "C" int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
                                                   int32_t num_heads, int32_t num_heads_k, int32_t causal) {
-  return fwd_workspace_size(batch, seqlen_q, seqlen_k, num_heads, num_heads_k, causal);
+  return fwd_workspace_size(false, batch, seqlen_q, seqlen_k, num_heads, num_heads_k, causal);
 }
 
 extern "C" int64_t tg_keybias_varlen_fwd_workspace_size(int32_t num_seqs, int32_t max_seqlen, int32_t num_heads,
                                                          int32_t num_heads_k, int32_t causal) {
-  return fwd_workspace_size(num_seqs, max_seqlen, max_seqlen, num_heads, num_heads_k, causal);
+  return fwd_workspace_size(true, num_seqs, max_seqlen, max_seqlen, num_heads, num_heads_k, causal);
 }
