@@ -65,3 +65,62 @@ def test_forward_forms(cuda, B, Sq, Sk, H, Hkv, causal, has_bias):
     assert torch.equal(torch.isfinite(lse), seen)
     assert_close("out", to_np(out), ro.cpu().numpy())
     assert_close("lse", to_np(lse[seen]), rl[seen].cpu().numpy())
+
+
+def _grads(q, k, v, bias, dout, scale):
+    """Causal gradients of one sequence in float64: dq, dk, dv, dbias_raw."""
+    n, H, _ = q.shape
+    g = H // k.shape[1]
+    q, k, v, bias, dout = (t.double() for t in (q, k, v, bias, dout))
+    dq, dk, dv, db = (torch.zeros_like(t) for t in (q, k, v, bias))
+    hidden = torch.ones(n, n, dtype=torch.bool, device=q.device).triu(1)
+    for h in range(H):
+        kh, vh = k[:, h // g], v[:, h // g]
+        p = torch.softmax((scale * (q[:, h] @ kh.t() + bias[h])).masked_fill(hidden, float("-inf")), -1)
+        dp = dout[:, h] @ vh.t()
+        ds = p * (dp - (p * dp).sum(-1, keepdim=True))
+        dq[:, h] = scale * (ds @ kh)
+        dk[:, h // g] += scale * (ds.t() @ q[:, h])
+        dv[:, h // g] += p.t() @ dout[:, h]
+        db[h] = scale * ds.sum(0)
+    return dq, dk, dv, db
+
+
+RAGGED = {
+    "nine": [0, 1, 63, 64, 65, 300, 0, 129, 700],
+    "equal": [512, 512, 512],
+    "sixty_four": [17 * (i % 7) for i in range(64)],
+    "sixty_five": [40 + (i % 3) for i in range(65)],
+}
+
+
+@pytest.mark.parametrize("name", list(RAGGED))
+@pytest.mark.parametrize("H,Hkv", [(4, 2), (3, 3)])
+def test_varlen_tile_order(cuda, name, H, Hkv):
+    """Packed sequences through the varlen launches' level order (up to 64 sequences; 65 take the
+    sequence-major order), with empty sequences and a max_seqlen longer than any."""
+    from tests.attn_util import assert_close_grad
+    from tokengate_amd.fa2bias.keybias import ext
+    lens = RAGGED[name]
+    total, mx, scale = sum(lens), max(lens) + 75, 128 ** -0.5
+    g = torch.Generator(device=cuda).manual_seed(total + H)
+    q, k, v, dout = (torch.randn(total, h, 128, generator=g, device=cuda).to(torch.bfloat16) for h in (H, Hkv, Hkv, H))
+    bias = (torch.randn(len(lens), H, mx, generator=g, device=cuda) / scale).contiguous()
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=cuda)
+    out, lse, _, _ = ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, bias, mx, mx, 0.0, scale, False, True,
+                                      -1, -1, 0.0, False, None)
+    dq, dk, dv, _, db = ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, bias, mx, mx, 0.0, scale,
+                                         False, True, -1, -1, 0.0, False, None, None)
+    r0 = 0
+    for b, n in enumerate(lens):
+        s = slice(r0, r0 + n)
+        r0 += n
+        assert not db[b, :, n:].any()
+        if n == 0:
+            continue
+        ro, rl = _reference(q[None, s], k[None, s], v[None, s], bias[None, b, :, :n], scale, True)
+        assert_close(f"out {b}", to_np(out[s]), ro[0].cpu().numpy())
+        assert_close(f"lse {b}", to_np(lse[:, s]), rl[0].cpu().numpy())
+        for what, got, ref in zip(("dq", "dk", "dv", "db"), (dq[s], dk[s], dv[s], db[b, :, :n]),
+                                  _grads(q[s], k[s], v[s], bias[b, :, :n], dout[s], scale)):
+            assert_close_grad(f"{what} {b}", to_np(got), ref.cpu().numpy())

@@ -43,6 +43,7 @@ struct BwdArgs {
   int64_t lse_total;       // varlen: lse / softmax_d are (H, total)
   int batch, sq, sk, h, hkv, group;
   int n_tiles;             // grid decomposition (q tiles for dQ, key tiles for dK/dV; set per launch)
+  int level_order;         // varlen: level order (varlen_level_order)
   float scale, scale_log2;
 };
 
@@ -172,9 +173,17 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   const int per_q = a.hkv * hgroups;
   const int x = blockIdx.x % per_q, rest = blockIdx.x / per_q;
   const int kh = x % a.hkv, hg = x / a.hkv;
-  // varlen: sequence-major (resident workgroups share one sequence's K/V in L2 / MALL)
-  const int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
-  const int qt = a.n_tiles - 1 - (VARLEN ? rest % a.n_tiles : rest / a.batch);
+  // varlen: level order, or sequence-major (resident workgroups share one sequence's K/V in L2 / MALL)
+  int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
+  int qt = a.n_tiles - 1 - (VARLEN ? rest % a.n_tiles : rest / a.batch);
+  if constexpr (VARLEN) {
+    if (a.level_order) {
+      const LevelTile lt = level_tile<BM>(a.cu_seqlens, a.batch, a.sq, rest, lane);
+      if (lt.seq < 0) return;
+      b = lt.seq;
+      qt = lt.level;
+    }
+  }
   const Seq sq_ = seq_of<VARLEN>(a, b);
   const int sq = sq_.sq, sk = sq_.sk;
   const int64_t row0 = sq_.row0;
@@ -456,8 +465,16 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kh = blockIdx.x % a.hkv;
   const int rest = blockIdx.x / a.hkv;
-  const int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
-  const int kt = VARLEN ? rest % a.n_tiles : rest / a.batch;
+  int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
+  int kt = VARLEN ? rest % a.n_tiles : rest / a.batch;
+  if constexpr (VARLEN) {
+    if (a.level_order) {   // a key tile's causal work is the query tiles after it
+      const LevelTile lt = level_tile<kKBlock>(a.cu_seqlens, a.batch, a.sq, rest, lane);
+      if (lt.seq < 0) return;
+      b = lt.seq;
+      kt = lt.n_tiles - 1 - lt.level;
+    }
+  }
   const Seq sq_ = seq_of<VARLEN>(a, b);
   const int sq = sq_.sq, sk = sq_.sk;
   const int64_t row0 = sq_.row0;
@@ -696,7 +713,9 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, hi
   const int hp = (a.group % 2 == 0) ? 2 : 1;
   const int bmq = hp == 2 ? dq_bm<2>() : dq_bm<1>();
   a.n_tiles = (a.sq + bmq - 1) / bmq;
-  const unsigned nq = (unsigned)((int64_t)a.n_tiles * a.batch * (a.h / hp));
+  a.level_order = VARLEN && varlen_level_order(a.batch, a.lse_total, a.hkv);
+  const unsigned nq = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, bmq) : (int64_t)a.n_tiles * a.batch) *
+                                 (a.h / hp));
 #define TG_DQ(HPV, C, B)                                                                               \
   if (hp == HPV && causal == C && has_bias == B)                                                       \
     hipLaunchKernelGGL((bwd_dq_kernel<HPV, C, B, VARLEN>), dim3(nq), dim3(kQThreads), 0, st, a);
@@ -705,7 +724,8 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, hi
 #undef TG_DQ
   const int nkt = (a.sk + kKBlock - 1) / kKBlock;
   a.n_tiles = nkt;
-  const unsigned nk = (unsigned)((int64_t)nkt * a.batch * a.hkv);
+  const unsigned nk = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, kKBlock) : (int64_t)nkt * a.batch) *
+                                 a.hkv);
 #define TG_DKV(C, B)                                                                                   \
   if (causal == C && has_bias == B)                                                                    \
     hipLaunchKernelGGL((bwd_dkdv16_kernel<C, B, VARLEN>), dim3(nk), dim3(kK16Threads), 0, st, a);

@@ -84,6 +84,7 @@ struct FwdArgs {
   int sq, sk;                  // dense lengths (varlen: per sequence, read from cu_seqlens)
   int h, hkv, group;
   int n_qtiles;
+  int level_order;             // varlen: unsplit launches in level order (varlen_level_order)
   float scale_log2;            // softmax_scale * log2(e)
   // Key-range split of the heaviest query tiles (small grids): the n_heavy heaviest query tiles
   // of every (sequence, head group) are each processed by ns workgroups over consecutive key
@@ -169,7 +170,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   const int x = bid % per_q;
   const int kh = x % a.hkv;
   const int hg = x / a.hkv;
-  // Dense: heaviest q tile of every batch row first.  Varlen: sequence-major (all tiles of
+  // Dense: heaviest q tile of every batch row first.  Varlen: the same over the tiles that exist
+  // (level order), or, for batches whose K/V outgrow the last-level cache, sequence-major (all tiles of
   // sequence b before sequence b+1, heaviest first within it), so the workgroups resident at one
   // time share one sequence's K/V in L2 / MALL instead of streaming every sequence's K/V at once.
   // A split launch lists the chunks of the n_heavy heaviest tiles first, then the other tiles.
@@ -188,7 +190,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     b = VARLEN ? r2 / n_light : r2 % a.batch;
     rank = a.n_heavy + (VARLEN ? r2 % n_light : r2 / a.batch);
   }
-  const int qt = a.n_qtiles - 1 - rank;
+  int qt = a.n_qtiles - 1 - rank;
+  if constexpr (VARLEN) {
+    if (a.level_order) {
+      const LevelTile lt = level_tile<BM>(a.cu_seqlens, a.batch, a.sq, bid / per_q, lane);
+      if (lt.seq < 0) return;   // workgroup-uniform: past the last tile
+      b = lt.seq;
+      qt = lt.level;
+    }
+  }
 
   int sq = a.sq, sk = a.sk;
   int64_t row0 = 0, krow0 = 0;
@@ -1119,7 +1129,10 @@ int keybias_fwd_varlen(const void *q, const void *k, const void *v, const float 
   const int64_t units = (int64_t)num_seqs * (num_heads / hp);
   TG_CHECK(workspace == nullptr || aligned16(workspace), "workspace must be 16-byte aligned");
   const FwdPlan plan = plan_varlen(hp, max_seqlen_q, max_seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0);
-  const int64_t nblocks = apply_plan(a, plan, units, workspace);
+  int64_t nblocks = apply_plan(a, plan, units, workspace);
+  a.level_order = a.n_heavy == 0 && a.n_qtiles > 1 &&
+                  varlen_level_order(num_seqs, cu_k != nullptr ? (int64_t)num_seqs * max_seqlen_k : total_q, num_heads_k);
+  if (a.level_order) nblocks = level_tiles(num_seqs, total_q, plan.nw * 32 / hp) * (num_heads / hp);
   TG_CHECK(nblocks < (1ll << 31), "grid too large");
   dispatch_fwd<true>(a, plan.nw, plan.ks, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
   TG_HIP_CHECK(hipPeekAtLastError());

@@ -157,6 +157,40 @@ __device__ __forceinline__ void wait_vm_outstanding(int n) {
 #undef TG_VMCNT
 }
 
+// Level order of the tiles of n <= 64 packed sequences: the longest sequence's last tile first, then
+// level by level down, at each level (tile index) one tile of every sequence that has it, longest
+// first.  Only tiles that exist are counted: workgroups are handed to an XCD's shader engines in strict
+// rotation, so workgroups that leave at once between those that stay would unbalance the engines (six
+// packed sequences of 260 to 4021 tokens, forward, profiled: sequence-major 185 us, heaviest first with
+// the shorter sequences' missing tiles in between 205, in level order 178).  Tile i of the order, for every lane of the wave alike; seq < 0 past the end.
+struct LevelTile {
+  int seq, level, n_tiles;   // n_tiles: of that sequence
+};
+template <int ROWS>
+__device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int max_len, int i, int lane) {
+  const int len = lane < n ? max(0, min(cu[lane + 1] - cu[lane], max_len)) : 0;
+  const int nt = (len + ROWS - 1) / ROWS;
+  int rank = 0;   // by tiles, ties by index
+  for (int j = 0; j < n; ++j) {
+    const int tj = __builtin_amdgcn_readlane(nt, j);
+    rank += (tj > nt || (tj == nt && j < lane)) ? 1 : 0;
+  }
+  rank = lane < n ? rank : 64;
+  auto lane_of = [&](int r) { return (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == r)); };
+  int hi = __builtin_amdgcn_readlane(nt, lane_of(0));
+  for (int m = 1; m <= n; ++m) {   // levels that exactly m sequences have
+    const int lo = m < n ? __builtin_amdgcn_readlane(nt, lane_of(m)) : 0;
+    const int c = (hi - lo) * m;
+    if (i < c) {
+      const int seq = lane_of(i % m);
+      return LevelTile{seq, hi - 1 - i / m, __builtin_amdgcn_readlane(nt, seq)};
+    }
+    i -= c;
+    hi = lo;
+  }
+  return LevelTile{-1, 0, 0};
+}
+
 // Index of this wave in its workgroup, held in a scalar register.  The compiler cannot prove that
 // threadIdx.x / 64 is the same in every lane of a wave, so without this every condition derived
 // from the wave index (tile skips, mask checks) is compiled as exec-masked per-lane code that
@@ -184,6 +218,17 @@ __device__ __forceinline__ float sum_bf16x2(uint32_t pair, float acc) {
 __device__ __forceinline__ float bf16_to_f32(bf16_t x) {
   return __builtin_bit_cast(float, (uint32_t)x << 16);
 }
+
+// Whether a varlen attention launch takes its tiles in level order, which packs the CUs best but streams
+// every sequence's K/V at once: with up to 64 sequences (one wave orders them) and K/V of at most half
+// the 256 MB last-level cache.  Six packed sequences of 260 to 4021 tokens (48 MB): forward +
+// backward 761 -> 674 us against sequence-major, four of 2048 forward 106 -> 74; eight prompts of 16k to
+// 128k (2.9 GB) ran at 682 TFLOP/s heaviest first and 996 sequence-major.
+inline bool varlen_level_order(int num_seqs, int64_t key_rows, int num_heads_k) {
+  return num_seqs > 1 && num_seqs <= 64 && key_rows * num_heads_k * 512 <= (128ll << 20);
+}
+// At most this many tiles of `rows` rows exist among total_rows rows of num_seqs sequences.
+inline int64_t level_tiles(int num_seqs, int64_t total_rows, int rows) { return total_rows / rows + num_seqs; }
 
 // Compute units of the current device (cached per device id).
 inline int device_cus() {
