@@ -67,23 +67,66 @@ def test_forward_forms(cuda, B, Sq, Sk, H, Hkv, causal, has_bias):
     assert_close("lse", to_np(lse[seen]), rl[seen].cpu().numpy())
 
 
-def _grads(q, k, v, bias, dout, scale):
-    """Causal gradients of one sequence in float64: dq, dk, dv, dbias_raw."""
-    n, H, _ = q.shape
+def _grads(q, k, v, bias, dout, scale, causal=True):
+    """Gradients of one sequence in float64: dq, dk, dv, dbias_raw (None without a bias)."""
+    (n, H, _), m = q.shape, k.shape[0]
     g = H // k.shape[1]
-    q, k, v, bias, dout = (t.double() for t in (q, k, v, bias, dout))
-    dq, dk, dv, db = (torch.zeros_like(t) for t in (q, k, v, bias))
-    hidden = torch.ones(n, n, dtype=torch.bool, device=q.device).triu(1)
+    q, k, v, dout = (t.double() for t in (q, k, v, dout))
+    dq, dk, dv = (torch.zeros_like(t) for t in (q, k, v))
+    db = None if bias is None else torch.zeros_like(bias, dtype=torch.float64)
+    hidden = torch.ones(n, m, dtype=torch.bool, device=q.device).triu(1 + m - n)
     for h in range(H):
         kh, vh = k[:, h // g], v[:, h // g]
-        p = torch.softmax((scale * (q[:, h] @ kh.t() + bias[h])).masked_fill(hidden, float("-inf")), -1)
+        z = q[:, h] @ kh.t() * scale
+        if bias is not None:
+            z = z + bias[h].double() * scale
+        p = torch.softmax(z.masked_fill(hidden, float("-inf")) if causal else z, -1)
         dp = dout[:, h] @ vh.t()
         ds = p * (dp - (p * dp).sum(-1, keepdim=True))
         dq[:, h] = scale * (ds @ kh)
         dk[:, h // g] += scale * (ds.t() @ q[:, h])
         dv[:, h // g] += p.t() @ dout[:, h]
-        db[h] = scale * ds.sum(0)
+        if bias is not None:
+            db[h] = scale * ds.sum(0)
     return dq, dk, dv, db
+
+
+BWD_SHAPES = [
+    # B, Sq, Sk, H, Hkv, causal, bias
+    (1, 1, 1, 16, 8, True, True), (1, 31, 31, 16, 8, True, True), (1, 33, 33, 2, 2, True, False),
+    (1, 129, 129, 16, 8, True, True), (2, 517, 517, 16, 8, True, True), (1, 161, 417, 16, 8, True, True),
+    (1, 300, 140, 6, 2, False, True), (1, 777, 777, 8, 8, False, False), (1, 1025, 1025, 6, 2, True, True),
+    (1, 2049, 2049, 8, 2, True, True), (3, 1000, 1000, 4, 4, True, True), (1, 3073, 3073, 16, 8, True, True),
+]
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,has_bias", BWD_SHAPES,
+                         ids=[f"{s[1]}x{s[2]}h{s[3]}b{s[0]}" for s in BWD_SHAPES])
+def test_backward_forms(cuda, B, Sq, Sk, H, Hkv, causal, has_bias):
+    """The backward's groups (two or four per workgroup, summed through LDS) and its own D = rowsum(dO * O),
+    into buffers full of NaN, twice with the same bits."""
+    from tests.attn_util import assert_close_grad
+    from tokengate_amd.fa2bias.keybias import ext
+    g = torch.Generator(device=cuda).manual_seed(Sq + 3 * Sk + H)
+    q, k, v, dout = (torch.randn(B, s, h, 128, generator=g, device=cuda).to(torch.bfloat16)
+                     for s, h in ((Sq, H), (Sk, Hkv), (Sk, Hkv), (Sq, H)))
+    scale = 128 ** -0.5
+    bias = torch.randn(B, H, Sk, generator=g, device=cuda) / scale if has_bias else None
+    out, lse, _, _ = ext().fwd(q, k, v, None, bias, 0.0, scale, causal, -1, -1, 0.0, False, None)
+    got = []
+    for _ in range(2):
+        bufs = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        got.append(ext().bwd(dout, q, k, v, out, lse, *bufs, bias, 0.0, scale, causal, -1, -1, 0.0, False, None, None))
+    for x, y in zip(*got):
+        assert x is None or torch.equal(x, y)
+    dq, dk, dv, sd, db = got[0]
+    d_ref = (dout.double() * out.double()).sum(-1).transpose(1, 2)
+    assert float((sd - d_ref).abs().max()) <= 1e-4      # 128 products of bf16 values summed in fp32
+    for b in range(B):
+        ref = _grads(q[b], k[b], v[b], None if bias is None else bias[b], dout[b], scale, causal)
+        for what, x, r in zip(("dq", "dk", "dv", "db"), (dq[b], dk[b], dv[b], None if db is None else db[b]), ref):
+            if r is not None:
+                assert_close_grad(f"{what} {b}", to_np(x), r.cpu().numpy())
 
 
 RAGGED = {

@@ -5,19 +5,27 @@
 //   dQ = scale dS K,  dK = scale sum_{h in group} dS^T Q,  dV = sum_{h in group} P^T dO,
 //   dbias_raw[b,h,j] = scale * sum_i dS[i,j]   (the gradient with respect to bias_raw).
 //
-// Three launches, no atomics (every output element is written exactly once, so results are
-// deterministic, unlike the reference's atomicAdd dBias, keybias.patch:267):
-//   1. preprocess: D = rowsum(dO * O) (returned as softmax_d, like FA2);
+// No atomics (every output element is written exactly once, so results are deterministic, unlike the
+// reference's atomicAdd dBias, keybias.patch:267):
+//   1. packed rows only: D = rowsum(dO * O) (returned as softmax_d, like FA2); a dense launch forms D in
+//      the dQ kernel, which reads dO anyway;
 //   2. dQ kernel, query-parallel (same 8-wave / 32-column structure as the forward): per 64-key
 //      tile recompute S^T = K Q^T and dP^T = V dO^T, form dS^T, accumulate dQ^T += K^T dS^T;
 //   3. dK/dV/dBias kernel, key-parallel: each wave owns 16 keys (K^T and V^T resident in
 //      registers) of one KV head and loops over every query head of its GQA group and every
 //      32-query tile: S = Q K^T, dP = dO V^T, P, dS, dV^T += dO^T P, dK^T += Q^T dS, and the dBias
 //      column sums stay in registers (one scalar per lane per head).
+// Where a launch has too few 128-row tiles to fill the CUs, or one round of causal tiles waits for the
+// longest, a workgroup's eight waves split the other axis as well: two or four groups share 64 or 32
+// query positions (dQ) or keys (dK/dV), each takes its part of every step, and their sums meet in LDS at
+// the end.  What it costs: each LDS DMA byte then serves half or a quarter of the MFMAs; the forms and
+// what they measured stand at kDqForms below.  One 2048-row sequence, 16 / 8 heads: backward 198 -> 105
+// us; 4096 rows 383 -> 274; 5000 rows, 8 / 2 heads: 729 -> 315.
 // Both kernels run on v_mfma_f32_16x16x32_bf16.  Tiles that are read both row-major (MFMA A
 // operand) and transposed (ds_read_b64_tr_b16) use a chunk swizzle chosen so that both access
 // patterns are bank-conflict free (dq_kswz() for the dQ kernel's K tile, k16_swz() for the dK/dV
 // kernel's Q / dO tiles).
+#include <algorithm>
 #include <type_traits>
 
 #include "tg_common.h"
@@ -65,27 +73,16 @@ __device__ __forceinline__ Seq seq_of(const BwdArgs &a, int b) {
   return s;
 }
 
-// ---- 1. D = rowsum(dO * O): 16 lanes per (row, head) ----------------------------------------
-template <bool VARLEN>
+// ---- 1. D = rowsum(dO * O) of packed rows: 16 lanes per (row, head) --------------------------
 __global__ __launch_bounds__(256) void bwd_preprocess_kernel(BwdArgs a, int64_t nrows) {
-  const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;   // (b, i, h) flattened
+  const int64_t r = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;   // (packed row i, h) flattened
   const int sub = threadIdx.x & 15;
   float acc = 0.f;
-  int64_t b = 0, i = 0, hh = 0;
-  bool valid = r < nrows;
+  const bool valid = r < nrows;
+  const int64_t hh = r % a.h, i = r / a.h;
   if (valid) {
-    hh = r % a.h;
-    const int64_t bi = r / a.h;
-    if constexpr (VARLEN) {
-      i = bi;   // packed row
-    } else {
-      b = bi / a.sq;
-      i = bi % a.sq;
-    }
-    const bf16_t *o = a.o + b * a.o_bs + i * a.o_rs + hh * a.o_hs + 8 * sub;
-    const bf16_t *d = a.dout + b * a.do_bs + i * a.do_rs + hh * a.do_hs + 8 * sub;
-    const u32x4 ov = *reinterpret_cast<const u32x4 *>(o);
-    const u32x4 dv = *reinterpret_cast<const u32x4 *>(d);
+    const u32x4 ov = *reinterpret_cast<const u32x4 *>(a.o + i * a.o_rs + hh * a.o_hs + 8 * sub);
+    const u32x4 dv = *reinterpret_cast<const u32x4 *>(a.dout + i * a.do_rs + hh * a.do_hs + 8 * sub);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       acc += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
@@ -96,20 +93,17 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(BwdArgs a, int64_t 
   acc += __shfl_xor(acc, 2);
   acc += __shfl_xor(acc, 4);
   acc += __shfl_xor(acc, 8);
-  if (valid && sub == 0) {
-    if constexpr (VARLEN)
-      a.softmax_d[hh * a.lse_total + i] = acc;
-    else
-      a.softmax_d[(b * a.h + hh) * a.sq + i] = acc;
-  }
+  if (valid && sub == 0) a.softmax_d[hh * a.lse_total + i] = acc;
 }
 
 // ---- 2. dQ kernel ------------------------------------------------------------------------
+// The eight waves form KS key groups of 8 / KS column waves, as in the forward: group g takes its wave_keys
+// of each step's keys, and the groups' dQ are added through LDS at the end.
 constexpr int kQWaves = 8;
 constexpr int kQThreads = 64 * kQWaves;
-constexpr int kBN = 64;                 // keys per tile
-constexpr int kTileBytes = kBN * kRow;  // 16 KiB
-template <int HP> constexpr int dq_bm() { return kQWaves * (32 / HP); }
+template <int KS> constexpr int dq_wave_keys() { return KS == 4 ? 32 : 64; }
+template <int KS> constexpr int dq_step() { return KS * dq_wave_keys<KS>(); }
+constexpr int dq_bm(int ks, int hp) { return kQWaves / ks * 32 / hp; }
 
 // dQ kernel tile layouts (16x16x32 MFMAs).  LDS row lr of a 64-key tile holds key dq_perm(lr):
 // within each 32-key step, S^T block kb' row m carries key 8(m/4) + 4kb' + m%4, so that lane group
@@ -157,15 +151,19 @@ __device__ __forceinline__ void dma_asm(const RawRsrc &rs, const void *lds_wave_
                  :: "s"(m0), "v"(voff), "s"(r) : "memory", "m0");
 }
 
-template <int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
+template <int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
 __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   constexpr int QW = 32;   // query positions per wave (all of one head)
-  constexpr int BM = dq_bm<HP>();
+  constexpr int CW = kQWaves / KS;
+  constexpr int BM = dq_bm(KS, HP);
+  constexpr int KN = dq_wave_keys<KS>(), SK = dq_step<KS>();
+  constexpr int KB = KN / 16, ST = KN / 32;   // 16-key blocks and 32-key steps of a wave's keys
+  constexpr int kTileBytes = SK * kRow;
   // K: rows in dq_perm order, chunk ^ dq_kswz(row) (read row-major and transposed);
   // V: rows in dq_perm order, chunk ^ (row % 16) (read row-major only)
   __shared__ __attribute__((aligned(1024))) char ks[2][kTileBytes];
   __shared__ __attribute__((aligned(1024))) char vs[2][kTileBytes];
-  __shared__ __attribute__((aligned(256))) float bs[2][HP][kBN + 4];
+  __shared__ __attribute__((aligned(256))) float bs[2][HP][SK + 4];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63;
   const int c16 = lane & 15, G = lane >> 4;
@@ -204,11 +202,12 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   const RawRsrc brs =
       raw_rsrc(bbase, (HAS_BIAS && sk > 0) ? (uint32_t)(((int64_t)(HP - 1) * a.bias_hs + sk) * 4) : 0u);
 
-  // this wave's 32 columns: 32 query positions of one head (HP = 2: waves 0-3 the first head of the
-  // pair, 4-7 the second), block cb (0, 1) = positions 16 cb .. 16 cb + 15, lane l holding column
+  // this wave's 32 columns: 32 query positions of one head (HP = 2: the first half of a group's column
+  // waves the first head of the pair, the others the second), block cb (0, 1) = positions 16 cb .. 16 cb + 15, lane l holding column
   // l % 16 of each block; one head per wave means one bias row per wave
-  const int hw = HP == 2 ? wave / (kQWaves / 2) : 0;
-  const int qw0 = q0 + QW * (HP == 2 ? wave % (kQWaves / 2) : wave);
+  const int cw = KS == 1 ? wave : wave % CW, kg = KS == 1 ? 0 : wave / CW;
+  const int hw = HP == 2 ? cw / (CW / 2) : 0;
+  const int qw0 = q0 + QW * (HP == 2 ? cw % (CW / 2) : cw);
   int qrow[2], hh[2];
   bool qvalid[2];
 #pragma unroll
@@ -237,41 +236,67 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
       const int64_t li = VARLEN ? (int64_t)hh[cb] * a.lse_total + row0 + qrow[cb]
                                 : ((int64_t)b * a.h + hh[cb]) * sq + qrow[cb];
       lse2[cb] = a.lse[li] * kLog2e;
-      dsum[cb] = a.softmax_d[li];
+      if constexpr (VARLEN) dsum[cb] = a.softmax_d[li];
+    }
+  }
+  // D = rowsum(dO * O) of this workgroup's rows (dense: every row belongs to one workgroup, which also
+  // writes it for the dK/dV kernel; varlen rows outside every sequence have none, so there the
+  // preprocess kernel forms it)
+  if constexpr (!VARLEN) {
+    const int64_t ob = (int64_t)b * a.o_bs;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      float d = 0.f;
+#pragma unroll
+      for (int ks4 = 0; ks4 < 4; ++ks4) {
+        const u32x4 ov = gload16(a.o + ob + (int64_t)qrow[cb] * a.o_rs + (int64_t)hh[cb] * a.o_hs + 32 * ks4 + 8 * G,
+                                 qvalid[cb]);
+        const u32x4 dv = __builtin_bit_cast(u32x4, df[cb][ks4]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          d += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
+          d += bf16_to_f32((bf16_t)(ov[w] >> 16)) * bf16_to_f32((bf16_t)(dv[w] >> 16));
+        }
+      }
+      dsum[cb] = quad_sum(d);
+      if (qvalid[cb] && G == 0 && kg == 0) a.softmax_d[((int64_t)b * a.h + hh[cb]) * sq + qrow[cb]] = dsum[cb];
     }
   }
 
   const f32x4 nd4[2] = {f32x4{-dsum[0], -dsum[0], -dsum[0], -dsum[0]}, f32x4{-dsum[1], -dsum[1], -dsum[1], -dsum[1]}};
   int kv_end = sk;
   if constexpr (CAUSAL) kv_end = min(sk, q0 + BM + off);
-  const int n_tiles = kv_end > 0 ? (kv_end + kBN - 1) / kBN : 0;
+  const int n_tiles = kv_end > 0 ? (kv_end + SK - 1) / SK : 0;
 
-  uint32_t koff[2], voff[2];
+  constexpr int kLoads = kTileBytes / 1024 / kQWaves;          // 1 KB DMA per wave and operand
+  uint32_t koff[kLoads], voff[kLoads];
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int lr = (wave * 2 + it) * 4 + (lane >> 4);          // LDS row written by this lane
+  for (int it = 0; it < kLoads; ++it) {
+    const int lr = (wave * kLoads + it) * 4 + (lane >> 4);     // LDS row written by this lane
     const int key = dq_perm(lr);
     koff[it] = (uint32_t)(key * a.k_rs * 2 + (((lane & 15) ^ dq_kswz(lr)) << 4));
     voff[it] = (uint32_t)(key * a.v_rs * 2 + (((lane & 15) ^ (lr & 15)) << 4));
   }
   auto issue_tile = [&](int tile, int buf) {
-    const uint32_t kb0 = (uint32_t)((int64_t)tile * kBN * a.k_rs * 2);
-    const uint32_t vb0 = (uint32_t)((int64_t)tile * kBN * a.v_rs * 2);
+    const uint32_t kb0 = (uint32_t)((int64_t)tile * SK * a.k_rs * 2);
+    const uint32_t vb0 = (uint32_t)((int64_t)tile * SK * a.v_rs * 2);
     // with the bias: the DMA from inline assembly (see dma_asm); without, the builtin (that variant
     // has fewer registers to spare: the assembly form spills 13 VGPRs against 7, 3 % slower)
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
+    for (int it = 0; it < kLoads; ++it) {
       if constexpr (HAS_BIAS) {
-        dma_asm<16>(krs, ks[buf] + (wave * 2 + it) * 1024, kb0 + koff[it]);
-        dma_asm<16>(vrs, vs[buf] + (wave * 2 + it) * 1024, vb0 + voff[it]);
+        dma_asm<16>(krs, ks[buf] + (wave * kLoads + it) * 1024, kb0 + koff[it]);
+        dma_asm<16>(vrs, vs[buf] + (wave * kLoads + it) * 1024, vb0 + voff[it]);
       } else {
-        dma16(krs_b, ks[buf] + (wave * 2 + it) * 1024, kb0 + koff[it]);
-        dma16(vrs_b, vs[buf] + (wave * 2 + it) * 1024, vb0 + voff[it]);
+        dma16(krs_b, ks[buf] + (wave * kLoads + it) * 1024, kb0 + koff[it]);
+        dma16(vrs_b, vs[buf] + (wave * kLoads + it) * 1024, vb0 + voff[it]);
       }
     }
     if constexpr (HAS_BIAS) {
-      if (wave < HP)
-        dma_asm<4>(brs, &bs[buf][wave][0], (uint32_t)(((int64_t)wave * a.bias_hs + tile * kBN + lane) * 4));
+      constexpr int BP = SK / 64;   // 64 bias values per DMA
+      if (wave < HP * BP)
+        dma_asm<4>(brs, &bs[buf][wave / BP][64 * (wave % BP)],
+                   (uint32_t)(((int64_t)(wave / BP) * a.bias_hs + tile * SK + 64 * (wave % BP) + lane) * 4));
     }
   };
 
@@ -313,19 +338,20 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   if (n_tiles > 0) issue_tile(0, 0);
   for (int t = 0; t < n_tiles; ++t) {
     const int buf = t & 1;
-    const int n0 = t * kBN;
+    const int n0 = t * SK + KN * kg;   // this wave's first key of the step
+    const char *const kt_ = ks[buf] + KN * kg * kRow, *const vt_ = vs[buf] + KN * kg * kRow;
     wait_all_mem();
     __syncthreads();
     if (t + 1 < n_tiles) issue_tile(t + 1, buf ^ 1);
     if (!wave_has_rows || (CAUSAL && n0 > qw_hi + off)) continue;
 
-    // S^T = K Q^T (+ bias, as the accumulators' start) and dP^T = V dO^T: 2 column blocks x 4 key
+    // S^T = K Q^T (+ bias, as the accumulators' start) and dP^T = V dO^T: 2 column blocks x KB key
     // blocks x 4 d-steps each
-    f32x4 sacc[2][4], pacc[2][4];
+    f32x4 sacc[2][KB], pacc[2][KB];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < KB; ++kb) {
       if constexpr (HAS_BIAS)   // both column blocks are the wave's head: one read serves both
-        sacc[0][kb] = *reinterpret_cast<const f32x4 *>(&bs[buf][hw][32 * (kb >> 1) + 8 * G + 4 * (kb & 1)]);
+        sacc[0][kb] = *reinterpret_cast<const f32x4 *>(&bs[buf][hw][KN * kg + 32 * (kb >> 1) + 8 * G + 4 * (kb & 1)]);
       else
         sacc[0][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
       sacc[1][kb] = sacc[0][kb];
@@ -334,14 +360,14 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
     }
     // keys past the end or in the causal future start from -inf (one uniform branch, before the
     // MFMAs), so that P = exp2(-inf) = +0 below needs no per-element test
-    const bool need_mask = (n0 + kBN > sk) || (CAUSAL && n0 + kBN - 1 > qw0 + off);
+    const bool need_mask = (n0 + KN > sk) || (CAUSAL && n0 + KN - 1 > qw0 + off);
     if (need_mask) {
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) {
         int lim = sk - 1;
         if constexpr (CAUSAL) lim = min(lim, qrow[cb] + off);
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
+        for (int kb = 0; kb < KB; ++kb) {
           const int rel = lim - (n0 + 32 * (kb >> 1) + 8 * G + 4 * (kb & 1));
 #pragma unroll
           for (int i = 0; i < 4; ++i) sacc[cb][kb][i] = rel - i < 0 ? -__builtin_inff() : sacc[cb][kb][i];
@@ -350,20 +376,20 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
     }
 #pragma unroll
     for (int ks4 = 0; ks4 < 4; ++ks4) {
-      bf16x8 kf[4], vf[4];
+      bf16x8 kf[KB], vf[KB];
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
         if constexpr (HAS_BIAS) {
-          kf[kb] = lds_load16(ks[buf] + 16 * kb * kRow, lpk[ks4]);
-          vf[kb] = lds_load16(vs[buf] + 16 * kb * kRow, lpv[ks4]);
+          kf[kb] = lds_load16(kt_ + 16 * kb * kRow, lpk[ks4]);
+          vf[kb] = lds_load16(vt_ + 16 * kb * kRow, lpv[ks4]);
         } else {
           const int lr = 16 * kb + c16;
-          kf[kb] = lds_load16(ks[buf], lr * kRow + ((((uint32_t)(4 * ks4 + G)) ^ dq_kswz(lr)) << 4));
-          vf[kb] = lds_load16(vs[buf], lr * kRow + ((uint32_t)((4 * ks4 + G) ^ c16) << 4));
+          kf[kb] = lds_load16(kt_, lr * kRow + ((((uint32_t)(4 * ks4 + G)) ^ dq_kswz(lr)) << 4));
+          vf[kb] = lds_load16(vt_, lr * kRow + ((uint32_t)((4 * ks4 + G) ^ c16) << 4));
         }
       }
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
           sacc[cb][kb] = mfma16(kf[kb], qf[cb][ks4], sacc[cb][kb]);
@@ -375,11 +401,11 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
     // scheduling fences keep the three phases apart (hoisting across them raises the register
     // pressure past the file)
     __builtin_amdgcn_sched_barrier(0);
-    uint32_t dsk[2][4][2];
+    uint32_t dsk[2][KB][2];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
         float ds[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -391,9 +417,9 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    // dQ^T += K^T dS^T: 2 key steps x 8 d-blocks x 2 column blocks
+    // dQ^T += K^T dS^T: ST key steps x 8 d-blocks x 2 column blocks
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
+    for (int st = 0; st < ST; ++st) {
       bf16x8 bop[2];
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) {
@@ -402,13 +428,19 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
       }
 #pragma unroll
       for (int dblk = 0; dblk < 8; ++dblk) {
-        const s16x4 lo = lds_read_tr16(ks[buf] + 32 * st * kRow + ktr[dblk]);
-        const s16x4 hi = lds_read_tr16(ks[buf] + (32 * st + 16) * kRow + ktr[dblk]);
+        const s16x4 lo = lds_read_tr16(kt_ + 32 * st * kRow + ktr[dblk]);
+        const s16x4 hi = lds_read_tr16(kt_ + (32 * st + 16) * kRow + ktr[dblk]);
         const bf16x8 aop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) dqacc[cb][dblk] = mfma16(aop, bop[cb], dqacc[cb][dblk]);
       }
     }
+  }
+  constexpr int DB = 8 / KS;   // d-blocks DB kg .. DB kg + DB-1 of all groups' sums
+  if constexpr (KS > 1) {
+    static_assert(merge_bytes<KS, CW>() <= kTileBytes, "a group's pieces fit one ring slot");
+    __syncthreads();
+    merge_groups<KS, CW>(dqacc, kg, cw, lane, ks[0], ks[1], vs[0], vs[1]);
   }
 #pragma unroll
   for (int cb = 0; cb < 2; ++cb) {
@@ -416,18 +448,19 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
     bf16_t *row = a.dq + (VARLEN ? row0 * a.dq_rs : (int64_t)b * a.dq_bs) + (int64_t)qrow[cb] * a.dq_rs +
                   (int64_t)hh[cb] * a.dq_hs;
 #pragma unroll
-    for (int dblk = 0; dblk < 8; ++dblk) {
-      const f32x4 &o = dqacc[cb][dblk];
+    for (int d = 0; d < DB; ++d) {
+      const f32x4 &o = dqacc[cb][d];
       const u32x2 w = {pack_bf16x2(o[0] * a.scale, o[1] * a.scale), pack_bf16x2(o[2] * a.scale, o[3] * a.scale)};
-      *reinterpret_cast<u32x2 *>(row + 16 * dblk + 4 * G) = w;
+      *reinterpret_cast<u32x2 *>(row + 16 * (DB * kg + d) + 4 * G) = w;
     }
   }
 }
 
 // ---- 3. dK / dV / dBias kernel -----------------------------------------------------------
-constexpr int kKBlock = 128;            // keys per workgroup
-constexpr int kQT = 32;                 // queries per tile
-constexpr int kQSub = 2;                // query tiles per LDS ring slot (per workgroup barrier)
+constexpr int dkv_keys(int kq) { return 128 / kq; }   // keys per workgroup
+constexpr int kQT = 32;                               // queries per tile
+// query tiles per LDS ring slot (per workgroup barrier)
+template <int KQ> constexpr int dkv_sub() { return KQ == 1 ? 2 : 4; }
 constexpr int kQTileBytes = kQT * kRow; // 8 KiB
 
 // Eight waves; each owns 16 keys of one KV head and loops over every query head of its GQA group
@@ -448,10 +481,14 @@ __device__ __forceinline__ uint32_t k16_swz(int row) {
 }
 constexpr int kK16Waves = 8;
 constexpr int kK16Threads = 64 * kK16Waves;
-static_assert(16 * kK16Waves == kKBlock, "eight waves of 16 keys");
+static_assert(16 * kK16Waves == dkv_keys(1), "eight waves of 16 keys");
 
-template <bool CAUSAL, bool HAS_BIAS, bool VARLEN>
+// The eight waves form KQ query groups of 8 / KQ key waves (16 keys each): group g takes every KQ-th
+// query tile of a slot, and the groups' dK, dV and dBias are added through LDS.
+template <int KQ, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
 __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
+  constexpr int KW = kK16Waves / KQ;
+  constexpr int kKBlock = dkv_keys(KQ), kQSub = dkv_sub<KQ>();
   // each ring slot holds kQSub query tiles of kQT rows: one barrier per kQSub tiles
   __shared__ __attribute__((aligned(1024))) char qs0[kQSub * kQTileBytes], qs1[kQSub * kQTileBytes];
   __shared__ __attribute__((aligned(1024))) char dos0[kQSub * kQTileBytes], dos1[kQSub * kQTileBytes];
@@ -461,8 +498,11 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   auto doslot = [&](auto b) -> char * { if constexpr (decltype(b)::value == 0) return dos0; else return dos1; };
   auto lslot = [&](auto b) -> float * { if constexpr (decltype(b)::value == 0) return ls0; else return ls1; };
   auto dslot = [&](auto b) -> float * { if constexpr (decltype(b)::value == 0) return dsh0; else return dsh1; };
+  // KQ > 1: the groups' dBias sums of one head, two heads in turn
+  __shared__ float dbs[2][KQ > 1 && HAS_BIAS ? KQ : 1][kKBlock];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int kw = KQ == 1 ? wave : wave % KW, qg = KQ == 1 ? 0 : wave / KW;
   const int kh = blockIdx.x % a.hkv;
   const int rest = blockIdx.x / a.hkv;
   int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
@@ -481,7 +521,7 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   const int n0 = kt * kKBlock;
   if (n0 >= sk) return;
   const int off = sk - sq;
-  const int kw0 = n0 + 16 * wave;
+  const int kw0 = n0 + 16 * kw;
   const int key = kw0 + l16;             // this lane's key (MFMA column)
   const bool kvalid = key < sk;
   const bool wave_has_keys = kw0 < sk;
@@ -498,6 +538,7 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   int m_start = 0;
   if constexpr (CAUSAL) m_start = max(0, n0 - off) / kQT * kQT;
   constexpr int kQSlot = kQSub * kQT;   // query rows per ring slot
+  constexpr int kLD = kQSlot / 64;      // waves that bring a slot's lse (and as many its D)
   const int n_qt = sq > m_start ? (sq - m_start + kQSlot - 1) / kQSlot : 0;
 
   // LDS DMA: wave w fills rows 4w .. 4w+3 of the Q and dO tiles (one 1 KB load each)
@@ -515,11 +556,23 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   const int tk = l16 >> 2, tm = l16 & 3;
   const int trow0 = 8 * g + tk, trow1 = trow0 + 4;
 
-  f32x4 dkacc[8], dvacc[8];
+  f32x4 acc[2][8];
+  f32x4 (&dkacc)[8] = acc[0], (&dvacc)[8] = acc[1];
 #pragma unroll
   for (int d = 0; d < 8; ++d)
 #pragma unroll
     for (int v = 0; v < 4; ++v) { dkacc[d][v] = 0.f; dvacc[d][v] = 0.f; }
+  // group 0 writes the dBias that the groups left for head hi
+  auto store_dbias = [&](int hi) {
+    if constexpr (HAS_BIAS && KQ > 1) {
+      if (qg == 0 && g == 0 && kvalid) {
+        float tot = 0.f;
+#pragma unroll
+        for (int i = 0; i < KQ; ++i) tot += dbs[hi & 1][i][16 * kw + l16];
+        a.dbias[(int64_t)b * a.dbias_bs + (int64_t)(kh * a.group + hi) * a.dbias_hs + key] = tot * a.scale;
+      }
+    }
+  };
 
   for (int hi = 0; hi < a.group; ++hi) {
     const int hh = kh * a.group + hi;
@@ -545,7 +598,6 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
               (uint32_t)((int64_t)(m0 + sub * kQT) * a.do_rs * 2) + dooff);
       }
       // lse / D of the slot: 64 rows per 4-byte DMA, waves 0 .. kLD-1 and kLD .. 2 kLD-1
-      constexpr int kLD = kQSub * kQT / 64;
       static_assert(kLD * 64 == kQSub * kQT && 2 * kLD <= kK16Waves, "lse / D rows in 64-row DMAs");
       if (wave < kLD) dma4(lrs, lslot(buf_c) + 64 * wave, (uint32_t)(m0 + 64 * wave + lane) * 4);
       else if (wave < 2 * kLD) dma4(drs, dslot(buf_c) + 64 * (wave - kLD), (uint32_t)(m0 + 64 * (wave - kLD) + lane) * 4);
@@ -555,21 +607,21 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
       constexpr int BUF = decltype(buf_c)::value;
       const int m00 = m_start + t * kQSlot;
       wait_vm<0>();
-      // the slot's LSE rows (DMA'd by wave 0, now complete) to log2 units and its D rows (wave 1)
+      // the slot's LSE rows (DMA'd by these waves, now complete) to log2 units and its D rows
       // negated, once for every wave; the barrier below orders these writes before the other
       // waves' reads
-      static_assert(kQSub * kQT == 64, "waves 0 and 1 DMA every LSE / D row of a slot");
-      if (wave == 0) {
-        float *lw = lslot(buf_c) + lane;
+      if (wave < kLD) {
+        float *lw = lslot(buf_c) + 64 * wave + lane;
         *lw = *lw * kLog2e;
-      } else if (wave == 1) {
-        float *dw = dslot(buf_c) + lane;
+      } else if (wave < 2 * kLD) {
+        float *dw = dslot(buf_c) + 64 * (wave - kLD) + lane;
         *dw = -*dw;
       }
       ring_barrier();
       if (t + 1 < n_qt) issue_tile(m00 + kQSlot, std::integral_constant<int, 1 - BUF>());
 #pragma unroll
-      for (int sub = 0; sub < kQSub; ++sub) {
+      for (int s_ = 0; s_ < kQSub / KQ; ++s_) {
+      const int sub = KQ * s_ + qg;
       const int m0 = m00 + sub * kQT;
       if (!wave_has_keys || m0 >= sq || (CAUSAL && m0 + kQT - 1 + off < kw0)) continue;
       char *const qsl = qslot(buf_c) + sub * kQTileBytes;
@@ -673,6 +725,7 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
       }   // sub-tiles
     };
     ring_barrier();   // previous head's last tile fully consumed before its slots are reused
+    if (hi > 0) store_dbias(hi - 1);
     if (n_qt > 0) issue_tile(m_start, std::integral_constant<int, 0>());
     {
       int t = 0;
@@ -685,16 +738,25 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
     if constexpr (HAS_BIAS) {
       float tot = dbacc + __shfl_xor(dbacc, 16);
       tot += __shfl_xor(tot, 32);
-      if (g == 0 && kvalid)
+      if (KQ > 1) {
+        if (g == 0) dbs[hi & 1][qg][16 * kw + l16] = tot;
+      } else if (g == 0 && kvalid)
         a.dbias[(int64_t)b * a.dbias_bs + (int64_t)hh * a.dbias_hs + key] = tot * a.scale;
     }
+  }
+  constexpr int DB = 8 / KQ;   // d-blocks DB qg .. DB qg + DB-1 of all groups' sums
+  if constexpr (KQ > 1) {
+    static_assert(merge_bytes<KQ, KW>() <= kQSub * kQTileBytes, "a group's pieces fit one ring slot");
+    __syncthreads();
+    store_dbias(a.group - 1);
+    merge_groups<KQ, KW>(acc, qg, kw, lane, qs0, qs1, dos0, dos1);
   }
   if (kvalid) {
     bf16_t *krow = a.dk + (VARLEN ? row0 * a.dk_rs : (int64_t)b * a.dk_bs) + (int64_t)key * a.dk_rs + (int64_t)kh * a.dk_hs;
     bf16_t *vrow = a.dv + (VARLEN ? row0 * a.dv_rs : (int64_t)b * a.dv_bs) + (int64_t)key * a.dv_rs + (int64_t)kh * a.dv_hs;
 #pragma unroll
-    for (int dblk = 0; dblk < 8; ++dblk) {
-      const int d = 16 * dblk + 4 * g;   // accumulator value i is d + i
+    for (int dblk = 0; dblk < DB; ++dblk) {
+      const int d = 16 * (DB * qg + dblk) + 4 * g;   // accumulator value i is d + i
       const u32x2 wk = {pack_bf16x2(dkacc[dblk][0] * a.scale, dkacc[dblk][1] * a.scale),
                         pack_bf16x2(dkacc[dblk][2] * a.scale, dkacc[dblk][3] * a.scale)};
       const u32x2 wv = {pack_bf16x2(dvacc[dblk][0], dvacc[dblk][1]), pack_bf16x2(dvacc[dblk][2], dvacc[dblk][3])};
@@ -705,31 +767,103 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
 }
 
 // ---- host dispatch ---------------------------------------------------------------------------
+// Groups per workgroup (KS of the dQ kernel, KQ of the dK/dV kernel): the form with the least
+// grid_cost.  A step is 64 keys (dQ) or queries of one head (dK/dV) with one group and 128 with more;
+// its cost and a workgroup's are fitted to launches of 128 to 8192 rows timed in each form, and the form
+// they pick is the fastest, or within 6 % of it, at every one.  Where the forms differ most (16 / 8 heads,
+// causal, with bias, us with 1 / 2 / 4 groups): dQ at 1024 rows 45 / 31 / 23, 2048 81 / 52 / 46, 4096
+// 152 / 108 / 140, 8192 356 / 378 / 460; dK/dV 64 / 44 / 29, 122 / 82 / 62, 239 / 172 / 205, 569 / 639 / 740,
+// and at 5000 rows of 8 / 2 heads 547 / 345 / 212.
+struct GroupForm {
+  int groups;
+  float wg, solo, full;
+};
+constexpr GroupForm kDqForms[] = {{1, 8.f, 2.2f, 2.55f}, {2, 8.f, 2.45f, 2.75f}, {4, 8.f, 1.65f, 1.7f}};
+constexpr GroupForm kDkvForms[] = {{1, 6.f, 1.82f, 2.05f}, {2, 6.f, 2.45f, 2.45f}, {4, 6.f, 1.5f, 1.45f}};
+template <typename Cost>
+int cheapest(const GroupForm (&forms)[3], Cost cost) {
+  int best = 1;
+  float c0 = cost(forms[0]);
+  for (int i = 1; i < 3; ++i) {
+    const float c = cost(forms[i]);
+    if (c < c0) { c0 = c; best = forms[i].groups; }
+  }
+  return best;
+}
+// The r-th heaviest tile's level (tiles before it in dQ's order of work, after it in dK/dV's) among the
+// launch's sequences: dense, n tiles of each; packed, one sequence of n tiles and the others of `rest` on
+// average (their lengths are on the device).
+struct Levels {
+  int n, rest, others;
+  int count() const { return n + rest * others; }
+  int level(int r) const { return r < n - rest ? n - 1 - r : rest - 1 - (r - (n - rest)) / (1 + others); }
+};
+Levels levels_of(const BwdArgs &a, bool varlen, int len, int tile) {
+  Levels v{(len + tile - 1) / tile, 0, 0};
+  if (varlen && a.batch > 1) {
+    v.others = a.batch - 1;
+    v.rest = (int)std::min<int64_t>(v.n, std::max<int64_t>(0, (a.lse_total - len) / v.others) / tile);
+  }
+  return v;
+}
+int dq_groups(const BwdArgs &a, int hp, bool causal, bool varlen) {
+  return cheapest(kDqForms, [&](const GroupForm &f) {
+    const int bm = dq_bm(f.groups, hp), step = f.groups == 1 ? 64 : 128;
+    const Levels v = levels_of(a, varlen, a.sq, bm);
+    return grid_cost(v.count(), (int64_t)(varlen ? 1 : a.batch) * (a.h / hp), device_cus(), f.wg, f.solo, f.full, [&](int r) {
+      const int64_t end = causal ? std::min<int64_t>(a.sk, (int64_t)(v.level(r) + 1) * bm + a.sk - a.sq) : a.sk;
+      return end > 0 ? (int)((end + step - 1) / step) : 0;
+    });
+  });
+}
+int dkv_groups(const BwdArgs &a, bool causal, bool varlen) {
+  return cheapest(kDkvForms, [&](const GroupForm &f) {
+    const int keys = dkv_keys(f.groups), slot = f.groups == 1 ? 64 : 128;
+    const Levels v = levels_of(a, varlen, a.sk, keys);
+    return grid_cost(v.count(), (int64_t)(varlen ? 1 : a.batch) * a.hkv, device_cus(), f.wg, f.solo, f.full, [&](int r) {
+      // queries from the tile's first key on
+      const int64_t start = causal ? std::max<int64_t>(0, (int64_t)(v.n - 1 - v.level(r)) * keys - (a.sk - a.sq)) : 0;
+      return start < a.sq ? a.group * (int)((a.sq - start + slot - 1) / slot) : 0;
+    });
+  });
+}
+
+// groups: whether more than one group may be taken (the last step's LDS DMA offsets then reach up to
+// 127 rows past the end and must not wrap at 4 GiB)
 template <bool VARLEN>
-void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, hipStream_t st) {
+void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bool groups, hipStream_t st) {
   BwdArgs a = a0;
-  hipLaunchKernelGGL(bwd_preprocess_kernel<VARLEN>, dim3((unsigned)((nrows * 16 + 255) / 256)), dim3(256), 0, st,
-                     a, nrows);
+  if constexpr (VARLEN)
+    hipLaunchKernelGGL(bwd_preprocess_kernel, dim3((unsigned)((nrows * 16 + 255) / 256)), dim3(256), 0, st, a, nrows);
   const int hp = (a.group % 2 == 0) ? 2 : 1;
-  const int bmq = hp == 2 ? dq_bm<2>() : dq_bm<1>();
-  a.n_tiles = (a.sq + bmq - 1) / bmq;
+  // a batch that runs sequence-major fills the chip with one group
   a.level_order = VARLEN && varlen_level_order(a.batch, a.lse_total, a.hkv);
+  if (VARLEN && a.batch > 1 && !a.level_order) groups = false;
+  const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
+  const int bmq = dq_bm(ks, hp);
+  a.n_tiles = (a.sq + bmq - 1) / bmq;
   const unsigned nq = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, bmq) : (int64_t)a.n_tiles * a.batch) *
                                  (a.h / hp));
-#define TG_DQ(HPV, C, B)                                                                               \
-  if (hp == HPV && causal == C && has_bias == B)                                                       \
-    hipLaunchKernelGGL((bwd_dq_kernel<HPV, C, B, VARLEN>), dim3(nq), dim3(kQThreads), 0, st, a);
-  TG_DQ(2, true, true) TG_DQ(2, true, false) TG_DQ(2, false, true) TG_DQ(2, false, false)
-  TG_DQ(1, true, true) TG_DQ(1, true, false) TG_DQ(1, false, true) TG_DQ(1, false, false)
+#define TG_DQ(K, HPV, C, B)                                                                            \
+  if (ks == K && hp == HPV && causal == C && has_bias == B)                                            \
+    hipLaunchKernelGGL((bwd_dq_kernel<K, HPV, C, B, VARLEN>), dim3(nq), dim3(kQThreads), 0, st, a);
+#define TG_DQ_ALL(K)                                                                                   \
+  TG_DQ(K, 2, true, true) TG_DQ(K, 2, true, false) TG_DQ(K, 2, false, true) TG_DQ(K, 2, false, false)  \
+  TG_DQ(K, 1, true, true) TG_DQ(K, 1, true, false) TG_DQ(K, 1, false, true) TG_DQ(K, 1, false, false)
+  TG_DQ_ALL(1) TG_DQ_ALL(2) TG_DQ_ALL(4)
+#undef TG_DQ_ALL
 #undef TG_DQ
-  const int nkt = (a.sk + kKBlock - 1) / kKBlock;
-  a.n_tiles = nkt;
-  const unsigned nk = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, kKBlock) : (int64_t)nkt * a.batch) *
+  const int kq = groups ? dkv_groups(a, causal, VARLEN) : 1;
+  const int keys = dkv_keys(kq);
+  a.n_tiles = (a.sk + keys - 1) / keys;
+  const unsigned nk = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, keys) : (int64_t)a.n_tiles * a.batch) *
                                  a.hkv);
-#define TG_DKV(C, B)                                                                                   \
-  if (causal == C && has_bias == B)                                                                    \
-    hipLaunchKernelGGL((bwd_dkdv16_kernel<C, B, VARLEN>), dim3(nk), dim3(kK16Threads), 0, st, a);
-  TG_DKV(true, true) TG_DKV(true, false) TG_DKV(false, true) TG_DKV(false, false)
+#define TG_DKV(K, C, B)                                                                                \
+  if (kq == K && causal == C && has_bias == B)                                                         \
+    hipLaunchKernelGGL((bwd_dkdv16_kernel<K, C, B, VARLEN>), dim3(nk), dim3(kK16Threads), 0, st, a);
+#define TG_DKV_ALL(K) TG_DKV(K, true, true) TG_DKV(K, true, false) TG_DKV(K, false, true) TG_DKV(K, false, false)
+  TG_DKV_ALL(1) TG_DKV_ALL(2) TG_DKV_ALL(4)
+#undef TG_DKV_ALL
 #undef TG_DKV
 }
 
@@ -807,7 +941,10 @@ extern "C" int tg_keybias_bwd(const void *dout, const void *q, const void *k, co
   a.h = num_heads; a.hkv = num_heads_k; a.group = num_heads / num_heads_k;
   a.scale = softmax_scale;
   a.scale_log2 = softmax_scale * kLog2e;
-  launch_bwd<false>(a, causal != 0, bias_raw != nullptr, (int64_t)batch * seqlen_q * num_heads, stream);
+  launch_bwd<false>(a, causal != 0, bias_raw != nullptr, (int64_t)batch * seqlen_q * num_heads,
+                    span_ok(seqlen_k + 128ll, a.k_rs) && span_ok(seqlen_k + 128ll, a.v_rs) &&
+                        span_ok(seqlen_q + 128ll, a.q_rs) && span_ok(seqlen_q + 128ll, a.do_rs),
+                    stream);
   TG_HIP_CHECK(hipPeekAtLastError());
   return 0;
 }
@@ -855,7 +992,10 @@ extern "C" int tg_keybias_varlen_bwd(const void *dout, const void *q, const void
   a.h = num_heads; a.hkv = num_heads_k; a.group = num_heads / num_heads_k;
   a.scale = softmax_scale;
   a.scale_log2 = softmax_scale * kLog2e;
-  launch_bwd<true>(a, causal != 0, bias_raw != nullptr, (int64_t)total * num_heads, stream);
+  launch_bwd<true>(a, causal != 0, bias_raw != nullptr, (int64_t)total * num_heads,
+                   span_ok(total + 128ll, a.k_rs) && span_ok(total + 128ll, a.v_rs) && span_ok(total + 128ll, a.q_rs) &&
+                       span_ok(total + 128ll, a.do_rs),
+                   stream);
   TG_HIP_CHECK(hipPeekAtLastError());
   return 0;
 }

@@ -501,8 +501,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   // Group kg's waves are left with the final m, l and those d-blocks in oacc[cb][0 .. DB-1]. ----
   constexpr int DB = 8 / KS;
   if constexpr (KS > 1) {
-    constexpr int kSlot = 64 * 16;                                 // one f32x4 per lane
-    static_assert((KS - 1) * CW * 2 * DB * kSlot <= kKTileBytes, "a group's pieces fit one ring slot");
+    static_assert(merge_bytes<KS, CW>() <= kKTileBytes, "a group's pieces fit one ring slot");
     __shared__ __attribute__((aligned(16))) float2 ml_s[KS][CW][2][16];
     if (G == 0) {
 #pragma unroll
@@ -527,35 +526,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
 #pragma unroll
       for (int d = 0; d < 8; ++d) oacc[cb][d] *= w;
     }
-    auto dst = [&](int g) -> char * { return g == 0 ? ks0 : g == 1 ? vs0 : g == 2 ? ks1 : vs1; };
-#pragma unroll
-    for (int g = 0; g < KS; ++g) {
-      if (g == kg) continue;
-      char *p = dst(g) + ((kg - (kg > g ? 1 : 0)) * CW + cw) * 2 * DB * kSlot + lane * 16;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-        for (int d = 0; d < DB; ++d) *reinterpret_cast<f32x4 *>(p + (cb * DB + d) * kSlot) = oacc[cb][g * DB + d];
-    }
-    // this group's own d-blocks to the front
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int d = 0; d < DB; ++d) {
-        f32x4 own = oacc[cb][d];
-#pragma unroll
-        for (int g = 1; g < KS; ++g) own = kg == g ? oacc[cb][g * DB + d] : own;
-        oacc[cb][d] = own;
-      }
-    __syncthreads();
-    const char *src = kg == 0 ? ks0 : kg == 1 ? vs0 : kg == 2 ? ks1 : vs1;
-#pragma unroll
-    for (int i = 0; i < KS - 1; ++i)
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-        for (int d = 0; d < DB; ++d)
-          oacc[cb][d] += *reinterpret_cast<const f32x4 *>(src + ((i * CW + cw) * 2 * DB + cb * DB + d) * kSlot + lane * 16);
+    merge_groups<KS, CW>(oacc, kg, cw, lane, ks0, vs0, ks1, vs1);
   }
   const int db0 = DB * kg;   // first d-block held
 
@@ -827,35 +798,25 @@ SplitPlan plan_split(const Form &f, const Tiles &t, int64_t units) {
   return p;
 }
 
-// Estimated time of a launch, in microseconds.  Workgroups are issued heaviest first to `slots`
-// places, so the launch takes at least its heaviest workgroup, its work over the places plus one start
-// per round, and k + 1 times the (k slots + 1)-th heaviest workgroup.  A workgroup takes `group`
-// (start, first loads, merge of the key groups, stores) plus `full` per key step while the chip is
-// full and `solo` while the longest workgroups run on alone; `combine` is the split's second launch.
-// The constants are fitted to launches of 1 to 16384 rows (8 to 16 heads, batches of 1 to 8) timed in
-// each form; the form they pick is within 5 % of the fastest at all of those, and where the forms
-// differ most: 4 waves / 8 waves / 8 waves with 2 / with 4 key groups take, at 1024 rows 22.6 / 25.0 /
-// 20.8 / 16.0 us, at 2048 40.5 / 40.2 / 36.6 / 32.9, at 4096 88.9 / 107.4 / 76.6 / 98.4, at 6001 142 /
-// 158 / 160 / 194, at 8192 266 / 239 / 268 / 339 (16 / 8 heads, causal, with bias).
+// Estimated time of a launch, in microseconds: grid_cost with the form's workgroup cost (start, first
+// loads, merge of the key groups, stores) and its costs per key step; `combine` is the split's second
+// launch.  The constants are fitted to launches of 1 to 16384 rows (8 to 16 heads, batches of 1 to 8)
+// timed in each form; the form they pick is within 5 % of the fastest at all of those, and where the
+// forms differ most: 4 waves / 8 waves / 8 waves with 2 / with 4 key groups take, at 1024 rows 22.6 /
+// 25.0 / 20.8 / 16.0 us, at 2048 40.5 / 40.2 / 36.6 / 32.9, at 4096 88.9 / 107.4 / 76.6 / 98.4, at 6001
+// 142 / 158 / 160 / 194, at 8192 266 / 239 / 268 / 339 (16 / 8 heads, causal, with bias).
 constexpr Form kForms[] = {{8, 1, 3.5f, 1.6f, 1.77f, 6.f},
                            {4, 1, 2.4f, 1.3f, 1.95f, 6.f},
                            {8, 2, 4.0f, 1.75f, 1.88f, 10.f},
                            {8, 4, 4.2f, 1.2f, 1.25f, 6.f}};
 float launch_cost(const Form &f, const Tiles &t, int64_t units, const SplitPlan &p) {
-  const int64_t slots = (int64_t)device_cus() * (8 / f.nw), nblocks = t.n_qtiles * units;
-  const int longest = t.steps(t.n_qtiles - 1);
   if (p.ns > 1) {   // one round; two workgroups of four waves share each CU throughout
-    const int chunk = (longest + p.ns - 1) / p.ns;
+    const int chunk = (t.steps(t.n_qtiles - 1) + p.ns - 1) / p.ns;
     const int light = p.n_heavy < t.n_qtiles ? t.steps(t.n_qtiles - 1 - p.n_heavy) : 0;
     return (f.nw == 4 ? f.full : f.solo) * std::max(chunk, light) + f.group + f.combine;
   }
-  int64_t total = 0;
-  for (int qt = 0; qt < t.n_qtiles; ++qt) total += t.steps(qt);
-  const int64_t rounds = (nblocks + slots - 1) / slots;
-  float cost = std::max(f.solo * longest + f.group, f.full * total * units / slots + rounds * f.group);
-  for (int64_t k = 1; k < rounds; ++k)
-    cost = std::max(cost, (k + 1) * (f.solo * t.steps(t.n_qtiles - 1 - (int)(k * slots / units)) + f.group));
-  return cost;
+  return grid_cost(t.n_qtiles, units, (int64_t)device_cus() * (8 / f.nw), f.group, f.solo, f.full,
+                   [&](int r) { return t.steps(t.n_qtiles - 1 - r); });
 }
 
 struct FwdPlan {

@@ -142,6 +142,59 @@ __device__ __forceinline__ void ring_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
+// Sum of 2 x 8 accumulators over the GR groups of CW waves of a workgroup, through LDS: group g adds up
+// accumulators acc[.][DB g .. DB g + DB-1] (DB = 8 / GR) of all groups and is left with them in
+// acc[.][0 .. DB-1].  d0 .. d3: GR LDS areas of merge_bytes() that no wave uses any more (the caller has
+// synchronised the workgroup).
+template <int GR, int CW> constexpr int merge_bytes() { return (GR - 1) * CW * 2 * (8 / GR) * 1024; }
+template <int GR, int CW>
+__device__ __forceinline__ void merge_groups(f32x4 (&acc)[2][8], int grp, int cw, int lane, char *d0, char *d1, char *d2,
+                                             char *d3) {
+  typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+  typedef __attribute__((address_space(3))) char lds_char;
+  constexpr int DB = 8 / GR;
+  // (selects of values: a branch on the group, or a conditional between two elements of acc, which is a
+  // conditional between their addresses, leaves acc in scratch memory)
+  auto piece = [&](int r, int d, int g) {
+    f32x4 v = acc[r][d];
+#pragma unroll
+    for (int i = 1; i < GR; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = acc[r][i * DB + d][e], y = v[e];
+        v[e] = g == i ? x : y;
+      }
+    return v;
+  };
+  auto area = [&](int g) { return (lds_char *)(g == 0 ? d0 : g == 1 ? d1 : g == 2 ? d2 : d3); };
+  f32x4 own[2][DB];
+#pragma unroll
+  for (int j = 0; j < GR; ++j) {
+    const int g = (grp + j) & (GR - 1);   // the pieces of group g; a group's area holds its peers in turn
+    lds_char *p = area(g) + ((GR - 1 - j) * CW + cw) * 2 * DB * 1024 + lane * 16;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const f32x4 v = piece(r, d, g);
+        if (j == 0) own[r][d] = v;
+        else *reinterpret_cast<lds_f32x4 *>(p + (r * DB + d) * 1024) = v;
+      }
+  }
+  __syncthreads();
+  lds_char *src = area(grp);
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      f32x4 v = own[r][d];
+#pragma unroll
+      for (int i = 0; i < GR - 1; ++i)   // the groups after this one, in turn
+        v += *reinterpret_cast<lds_f32x4 *>(src + ((i * CW + cw) * 2 * DB + r * DB + d) * 1024 + lane * 16);
+      acc[r][d] = v;
+    }
+}
+
 // Wait until at most n (0..63) vector-memory operations of this wave are outstanding (vmcnt: low
 // four bits in [3:0], high two in [15:14]), leaving the LDS and export counters unconstrained.
 __device__ __forceinline__ void wait_vm_outstanding(int n) {
@@ -217,6 +270,26 @@ __device__ __forceinline__ float sum_bf16x2(uint32_t pair, float acc) {
 
 __device__ __forceinline__ float bf16_to_f32(bf16_t x) {
   return __builtin_bit_cast(float, (uint32_t)x << 16);
+}
+
+// Estimated time, in microseconds, of a launch of `units` times n workgroups issued heaviest first to
+// `slots` places; steps(r) is the work of the r-th heaviest.  A workgroup takes `wg` plus `full` per step
+// while the chip is full and `solo` while the longest run on alone, so the launch takes at least its
+// heaviest workgroup, its work over the places plus one start per round, and k + 1 times the
+// (k slots + 1)-th heaviest workgroup.
+template <typename F>
+float grid_cost(int n, int64_t units, int64_t slots, float wg, float solo, float full, F steps) {
+  int64_t total = 0;
+  for (int r = 0; r < n; ++r) total += steps(r);
+  const int64_t rounds = (n * units + slots - 1) / slots;
+  const float even = full * total * units / slots + rounds * wg;
+  float cost = solo * steps(0) + wg;
+  cost = cost < even ? even : cost;
+  for (int64_t k = 1; k < rounds; ++k) {
+    const float c = (k + 1) * (solo * steps((int)(k * slots / units)) + wg);
+    cost = cost < c ? c : cost;
+  }
+  return cost;
 }
 
 // Whether a varlen attention launch takes its tiles in level order, which packs the CUs best but streams
