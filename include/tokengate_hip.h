@@ -361,6 +361,15 @@ int tg_linear_rows_norm(const void *h, int64_t h_row_stride, const void *residua
                         int32_t n_rows, const void *weight, int64_t n_out, int32_t dim, void *out,
                         int64_t out_row_stride, int32_t out_fp32, hipStream_t stream);
 
+/* tg_linear_rows_norm of a fused gate|up projection with the SwiGLU product formed on the way out:
+ * weight (2 * inter, dim) bf16 = [gate_proj; up_proj], out (n_rows, inter) = bf16(silu(g) * u) of the
+ * bf16 projections g and u, as tg_linear_rows_norm followed by tg_silu_mul computes it —
+ * post_attention_layernorm and the first half of Qwen3MLP in the decode step (gate_decode.py:210-226). */
+int tg_linear_rows_norm_act(const void *h, int64_t h_row_stride, const void *residual, int64_t residual_row_stride,
+                            void *residual_out, int64_t residual_out_row_stride, const void *norm_weight, float eps,
+                            int32_t n_rows, const void *weight, int64_t inter, int32_t dim, void *out,
+                            int64_t out_row_stride, hipStream_t stream);
+
 /* tg_linear_rows of the SwiGLU product: x = bf16(silu(g) * u) of the gate/up rows [g | u] (inter
  * values each), as tg_silu_mul computes it — Qwen3MLP's down_proj(act_fn(gate_proj(x)) *
  * up_proj(x)) in the decode step (gate_decode.py:210-226). */

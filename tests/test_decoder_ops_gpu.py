@@ -223,6 +223,31 @@ def test_linear_rows_swiglu_long_rows(cuda, rows, n_out, inter):
     assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("rows,inter,dim", [(1, 6144, 2048), (8, 6144, 2048), (2, 1027, 512), (3, 5, 2560), (7, 40000, 2048)])
+def test_linear_rows_norm_act(cuda, rows, inter, dim):
+    """The gate|up projection with the SwiGLU product formed on the way out equals the norm-fused
+    projection followed by silu_mul bit for bit (the SwiGLU kernel reads rows of whole 16-byte
+    pieces: odd inner sizes are compared with the product in torch, one bf16 unit apart at most); up to
+    65536 weight rows and beyond, a last workgroup with fewer rows, residual write-back, strided out."""
+    from tokengate_amd import decoder as dec
+    g = torch.Generator(device=cuda).manual_seed(rows * 5 + inter)
+    h, res = (_bf(torch.randn(rows, dim, generator=g, device=cuda)) for _ in range(2))
+    nw = _bf(1.0 + 0.1 * torch.randn(dim, generator=g, device=cuda))
+    w = _bf(torch.randn(2 * inter, dim, generator=g, device=cuda) * dim ** -0.5)
+    ro, ro2 = torch.empty_like(h), torch.empty_like(h)
+    buf = torch.zeros(rows, inter + 24, dtype=torch.bfloat16, device=cuda)
+    got = dec.linear_rows_norm_act(h, nw, 1e-6, w, residual=res, residual_out=ro, out=buf[:, :inter])
+    gu = dec.linear_rows_norm(h, nw, 1e-6, w, residual=res, residual_out=ro2)
+    torch.cuda.synchronize()
+    assert torch.equal(ro, ro2) and bool((buf[:, inter:] == 0).all())
+    if inter % 8 == 0:
+        assert torch.equal(got, dec.silu_mul(gu))
+    else:
+        f = gu.double()
+        ref = torch.nn.functional.silu(f[:, :inter]) * f[:, inter:]
+        assert bool(((got.double() - ref).abs() <= torch.finfo(torch.bfloat16).eps * ref.abs() + 1e-12).all())
+
+
 @pytest.mark.parametrize("rows,V", [(1, 151936), (3, 1001), (8, 151936)])
 def test_argmax_rows(cuda, rows, V):
     """tg_argmax_rows against torch.argmax: bf16-valued logits (ties at the top are common), a

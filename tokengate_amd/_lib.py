@@ -55,6 +55,7 @@ SIGNATURES = {
     "tg_lm_head": [vp, i64, i32, vp, i64, i32, vp, i64, vp],
     "tg_linear_rows": [vp, i64, i32, vp, i64, i32, vp, i64, vp],
     "tg_linear_rows_norm": [vp, i64, vp, i64, vp, i64, vp, f32, i32, vp, i64, i32, vp, i64, i32, vp],
+    "tg_linear_rows_norm_act": [vp, i64, vp, i64, vp, i64, vp, f32, i32, vp, i64, i32, vp, i64, vp],
     "tg_linear_rows_swiglu": [vp, i64, i32, i32, vp, i64, vp, i64, vp],
     "tg_argmax_rows": [vp, i64, i32, i64, vp, vp],
 }

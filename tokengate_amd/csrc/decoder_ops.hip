@@ -3,9 +3,9 @@
 //   * per-head q/k RMSNorm + rotary embedding at each token's own position, writing q in place
 //     and k / v into the layer's KV cache rows,
 //   * SiLU(gate) * up of the fused gate/up projection;
-//   * for the few rows of a decode step: the projections as HBM-bound GEMVs (a row form for rows
-//     of up to 2048 inputs, a split-K form for longer ones), optionally with the RMSNorm or the
-//     SwiGLU product folded into their input, and the greedy argmax over the logits.
+//   * for the few rows of a decode step: the projections on the matrix cores, streaming the weight
+//     once, optionally with the RMSNorm or the SwiGLU product folded into their input, or the SwiGLU
+//     product into their output, and the greedy argmax over the logits.
 // The prefill's projections (many rows) are plain GEMMs and stay on hipBLASLt.
 #include <type_traits>
 
@@ -216,15 +216,14 @@ __global__ __launch_bounds__(256) void branch_readout_kernel(const bf16_t *__res
 // ---- Linear layer on a few rows: y[b, v] = bf16(sum_d x[b, d] * w[v, d]) ------------------------
 // F.linear on bf16 tensors for the rows of a decode step (1..8): the vocab projection of the rows
 // that produce the next token (written as fp32, .float() of the bf16 result) and the decoder
-// layers' projections (written as bf16).  HBM-bound on the (n_out, dim) weight: each wave owns 4
-// consecutive output rows and issues the 16-byte loads of up to four 512-element column chunks
-// of them (16 KB per wave) before their bf16 pair dot products, so that enough of the weight is
-// in flight to cover HBM latency even for a 2048 x 2048 matrix; the NR input rows come from L2.
+// layers' projections (written as bf16).  HBM-bound on the (n_out, dim) weight.
 // The input x can be formed on the fly from the previous kernel's output, removing a launch:
 //   kPreNorm:   x = bf16(w_n * s / sqrt(mean(s^2) + eps)) with s = bf16(h + res) (res optional),
 //               exactly the RMSNorm kernel's arithmetic and summation order; block 0 writes
 //               res_out = s (a buffer other than res: every block reads res);
-//   kPreSwiGLU: x = bf16(silu(g) * u) of the gate/up rows [g | u], as the silu_mul kernel.
+//   kPreSwiGLU: x = bf16(silu(g) * u) of the gate/up rows [g | u], as the silu_mul kernel;
+// and of a gate|up projection the SwiGLU product can be formed on the way out (ACT), each workgroup
+// owning the gate and the up rows of its outputs.
 constexpr int kLmMaxRows = 8;
 constexpr int kPrePlain = 0, kPreNorm = 1, kPreSwiGLU = 2;
 struct LinIn {
@@ -238,19 +237,31 @@ struct LinIn {
   float eps;
   int inter;                // swiglu: offset of u within a row (= dim)
 };
-template <int NR, int PRE>
-__device__ __forceinline__ u32x4 lin_input(const LinIn &in, int b, int c, const float (&rinv)[NR]) {
+__device__ __forceinline__ u32x4 swiglu8(u32x4 gv, u32x4 uv) {
+  float g[8], u[8], y[8];
+  unpack8(gv, g);
+  unpack8(uv, u);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = g[e] / (1.f + __expf(-g[e])) * u[e];
+  return pack8(y);
+}
+__device__ __forceinline__ u32x4 norm8(u32x4 sv, u32x4 nwv, float rinv) {
+  float v[8], wf[8], y[8];
+  unpack8(sv, v);
+  unpack8(nwv, wf);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = wf[e] * (v[e] * rinv);
+  return pack8(y);
+}
+// Eight inputs of input row b from column c on (rinv: the row's normaliser, norm stage only)
+template <int PRE>
+__device__ __forceinline__ u32x4 lin_input(const LinIn &in, int b, int c, float rinv) {
   if constexpr (PRE == kPrePlain) {
     return ld16(in.x + b * in.x_rs + c);
   } else if constexpr (PRE == kPreSwiGLU) {
-    float g[8], u[8], y[8];
-    unpack8(ld16(in.x + b * in.x_rs + c), g);
-    unpack8(ld16(in.x + b * in.x_rs + in.inter + c), u);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = g[e] / (1.f + __expf(-g[e])) * u[e];
-    return pack8(y);
+    return swiglu8(ld16(in.x + b * in.x_rs + c), ld16(in.x + b * in.x_rs + in.inter + c));
   } else {
-    float v[8], wf[8], y[8];
+    float v[8];
     unpack8(ld16(in.x + b * in.x_rs + c), v);
     if (in.res) {
       float r[8];
@@ -258,301 +269,239 @@ __device__ __forceinline__ u32x4 lin_input(const LinIn &in, int b, int c, const 
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
     }
-    unpack8(ld16(in.nw + c), wf);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = wf[e] * (v[e] * rinv[b]);
-    return pack8(y);
+    return norm8(pack8(v), ld16(in.nw + c), rinv);   // (v is exact in bf16)
   }
 }
-// NCH consecutive 512-column chunks of a wave's 4 output rows: every weight load first
-// (lin_load), then the bf16 pair dot products against the NR input rows (lin_dot).
-template <int NCH>
-__device__ __forceinline__ void lin_load(const bf16_t *const (&wr)[4], int cg, u32x4 (&wv)[NCH][4]) {
-#pragma unroll
-  for (int ch = 0; ch < NCH; ++ch)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) wv[ch][r] = ld16(wr[r] + cg + 512 * ch);
-}
-// xs: the NR input rows formed once per workgroup in LDS (norm / SwiGLU stages), row stride
-// kLinXsRow; NULL for the plain stage, whose rows are read from global memory (L2).
-constexpr int kLinXsRow = 2048;
-template <int NCH, int NR, int PRE>
-__device__ __forceinline__ void lin_dot(const LinIn &in, const bf16_t *xs, const u32x4 (&wv)[NCH][4], int cg,
-                                        int lane, float (&acc)[4][NR]) {
-#pragma unroll
-  for (int ch = 0; ch < NCH; ++ch) {
-    const int c = cg + 512 * ch + 8 * lane;
-#pragma unroll
-    for (int b = 0; b < NR; ++b) {
-      const u32x4 xv = PRE == kPrePlain ? ld16(in.x + b * in.x_rs + c)
-                                        : *reinterpret_cast<const u32x4 *>(xs + b * kLinXsRow + c);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t wd = wv[ch][r][e], xd = xv[e];   // scalar copies: see u32_as_f32
-          acc[r][b] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wd), __builtin_bit_cast(bf16x2, xd),
-                                                      acc[r][b], false);
-        }
-    }
-  }
-}
-// Rows of at most 2048 inputs (longer ones take the split-K form below).  The norm / SwiGLU
-// input stage is formed once per workgroup into LDS: with the norm, wave w computes the sum of
-// squares of input rows w, w + 4, ... (in the RMSNorm kernel's order), then the 256 threads
-// write the normalised (or SwiGLU) rows; every wave's dot products read them from LDS.
-template <int NR, typename OutT, int PRE>
-__global__ __launch_bounds__(256) void linear_rows_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t vocab,
-                                                          int dim, OutT *__restrict__ out, int64_t out_rs) {
-  constexpr bool kStage = PRE != kPrePlain;
-  __shared__ __attribute__((aligned(16))) bf16_t xs[kStage ? NR * kLinXsRow : 8];
-  __shared__ float rinv_s[NR];
+// A workgroup (8 waves) owns RB blocks of 8 output rows; wave w takes the 64-column pieces w, w + 8,
+// w + 16, ... of the inner dimension, so that every request of a wave is 8 whole 128-byte lines and,
+// with all of a wave's pieces requested before the first product (NK of them, when dim = 512 NK), the
+// workgroup's whole slice of the weight is in flight at once.  One MFMA (16x16x32) takes a piece of a
+// block: rows 0..7 of its A operand are the block's weights at the piece's first 32 columns and rows
+// 8..15 the same output rows at the other 32; the columns of B are the (up to 8) input rows in the
+// same two halves.  The diagonal quarters of the result hold the two halves' sums, the other two are
+// not used.  Each input element is read once per workgroup, by the one lane that feeds it to the
+// matrix core.  The dot products used to run on the VALU, each wave reading all input rows for 4
+// output rows: twice the weight's bytes at 8 rows.  Before -> now, weights from HBM, at 1 / 8 rows
+// (us): 4096 x 2048 with the norm 6.9 / 14.5 -> 5.3 / 7.0, 2048 x 2048 4.3 / 8.3 -> 3.9 / 4.4,
+// 12288 x 2048 with the norm 12.4 / 28.6 -> 11.8 / 13.4 (with the SwiGLU product on the way out 11.0 /
+// 13.6), 2048 x 6144 6.3 / 12.1 -> 6.6 / 8.2, 151936 x 2048 with the norm 109 / 250 -> 104 / 112 (6.0 /
+// 5.6 TB/s).  WALK: fewer workgroups than blocks, which walk them with the next blocks' weights in flight
+// (only where a launch has that many: the second set of weight registers costs a 2048 x 6144 launch of
+// one block per workgroup 6.6 -> 7.6 us).
+template <int RB, int NK, typename OutT, int PRE, bool ACT, bool WALK>
+__global__ __launch_bounds__(512) void linear_rows_mfma_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
+                                                               int dim, int nr, OutT *__restrict__ out,
+                                                               int64_t out_rs) {
+  constexpr int kWaves = 8, NKR = NK > 0 ? NK : 1;
+  constexpr bool kStage = PRE == kPreNorm && NK == 4;   // dim = 2048
+  constexpr bool kStageAct = PRE == kPreSwiGLU && NK > 0;   // each wave forms its own pieces, in LDS
+  constexpr int kXsRow = kStageAct ? 64 * NK + 8 : 2048 + 8;   // padded: 8 rows' 16-byte reads on different banks
+  __shared__ __attribute__((aligned(16))) bf16_t xs[kStage ? 8 * kXsRow : kStageAct ? kWaves * 8 * kXsRow : 8];
+  __shared__ __attribute__((aligned(16))) float part2[WALK ? 2 : 1][kWaves][RB][2][64];
+  __shared__ float rinv_s[8];
   const int lane = threadIdx.x & 63, wv = wave_id();
-  const int64_t v0 = ((int64_t)blockIdx.x * 4 + wv) * 4;
-  // rows past the end read the last row (in bounds; their sums are not stored); a wave whose rows
-  // are all past the end still takes part in the workgroup's barriers
-  const bf16_t *wr[4];
+  const int c = lane & 7, G = lane >> 4;
+  const int xr = min(c, nr - 1);                         // input rows past nr repeat the last (not stored)
+  const int kl = 64 * wv + 32 * ((lane >> 3) & 1) + 8 * G;
+  constexpr int OB = ACT ? RB / 2 : RB;                  // blocks of stored rows
+  const bf16_t *wr[RB];
+  auto rows_from = [&](int64_t v0) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) wr[r] = w + min(v0 + r, vocab - 1) * dim + 8 * lane;
-  const int groups = dim / 8;   // NR * groups <= 256 * NR: thread t owns chunks t + 256 i, i < NR
-  // The norm stage's inputs are requested first, then the first 2048 columns of the weight:
-  // loads complete in issue order, so the stage can run while the weight bytes stream in.
-  constexpr int kIn = PRE == kPreNorm ? NR : 1;
-  u32x4 xin[kIn], rin[kIn], nwv[kIn];
-  if constexpr (PRE == kPreNorm) {
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int idx = threadIdx.x + 256 * i;
-      if (idx < NR * groups) {
-        const int b = idx / groups, c = 8 * (idx - b * groups);
-        nwv[i] = ld16(in.nw + c);
-        xin[i] = ld16(in.x + b * in.x_rs + c);
-        if (in.res) rin[i] = ld16(in.res + b * in.res_rs + c);
-      }
+    for (int rb = 0; rb < RB; ++rb) {
+      // rows past the end read the last row (in bounds; not stored)
+      const int64_t v = min(v0 + 8 * (rb % OB) + c, n_out - 1);
+      wr[rb] = w + (v + (rb / OB) * n_out) * dim + kl;
     }
-  }
-  u32x4 wfirst[4][4];
-  const bool first = dim >= 2048;
-  if (first) lin_load<4>(wr, 0, wfirst);
-  if constexpr (kStage) {
-    if constexpr (PRE == kPreNorm) {
-      // One read of the input rows: s = bf16(h + res) (exact in bf16) goes to LDS (block 0 also
-      // writes res_out) and the norm weight of the thread's chunks to registers.  The sums of
-      // squares then come from LDS in the RMSNorm kernel's order (lane l sums its chunks l,
-      // l + 64, ... element by element, then the wave butterfly), and each thread scales its own
-      // chunks in place: the same arithmetic as lin_input, one global round trip fewer.
-      const bool writer = blockIdx.x == 0 && in.res_out != nullptr;
+  };
+  const int64_t step = (int64_t)gridDim.x * (8 * OB);
+  int64_t v0 = (int64_t)blockIdx.x * (8 * OB);
+  rows_from(v0);
+  // inputs are requested before the weights: loads complete in issue order, so the input stage runs
+  // while the weight bytes stream in
+  u32x4 xin[NKR], rin[NKR], nwv[NKR], wf[NKR][RB];
+  u32x4 sx[kStage ? 4 : 1], sr[kStage ? 4 : 1];
+  if constexpr (NK > 0) {
+    if constexpr (PRE == kPrePlain) {
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int idx = threadIdx.x + 256 * i;
-        if (idx < NR * groups) {
-          const int b = idx / groups, c = 8 * (idx - b * groups);
+      for (int s = 0; s < NK; ++s) xin[s] = ld16(in.x + xr * in.x_rs + kl + 512 * s);
+    } else if constexpr (kStageAct) {
+      // the wave's 8 NK chunks of every row, once each (NK rounds at 8 rows)
+#pragma unroll
+      for (int s = 0; s < NK; ++s) {
+        const int idx = lane + 64 * s, b = idx / (8 * NK), j = idx % (8 * NK);
+        if (b < nr) {
+          const bf16_t *p = in.x + b * in.x_rs + 64 * wv + 512 * (j >> 3) + 8 * (j & 7);
+          xin[s] = ld16(p);
+          rin[s] = ld16(p + in.inter);
+        }
+      }
+    } else if constexpr (kStage) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int idx = threadIdx.x + 512 * i, b = idx >> 8, ch = 8 * (idx & 255);
+        if (b < nr) {
+          sx[i] = ld16(in.x + b * in.x_rs + ch);
+          if (in.res) sr[i] = ld16(in.res + b * in.res_rs + ch);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < NK; ++s) nwv[s] = ld16(in.nw + kl + 512 * s);
+    }
+#pragma unroll
+    for (int s = 0; s < NK; ++s)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) wf[s][rb] = ld16(wr[rb] + 512 * s);
+  }
+  float rinv = 0.f;
+  if constexpr (PRE == kPreNorm) {
+    const bool writer = blockIdx.x == 0 && in.res_out != nullptr;
+    if constexpr (kStage) {
+      // s = bf16(h + res) to LDS (block 0 also writes res_out), then wave b sums row b's squares in
+      // the RMSNorm kernel's order (lane l its chunks l, l + 64, ..., then the wave butterfly)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int idx = threadIdx.x + 512 * i, b = idx >> 8, ch = 8 * (idx & 255);
+        if (b < nr) {
           float v[8];
-          unpack8(xin[i], v);
+          unpack8(sx[i], v);
           if (in.res) {
             float r[8];
-            unpack8(rin[i], r);
+            unpack8(sr[i], r);
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
           }
           const u32x4 pv = pack8(v);
-          if (writer) st16(in.res_out + b * in.ro_rs + c, pv);
-          *reinterpret_cast<u32x4 *>(xs + b * kLinXsRow + c) = pv;
+          if (writer) st16(in.res_out + b * in.ro_rs + ch, pv);
+          *reinterpret_cast<u32x4 *>(xs + b * kXsRow + ch) = pv;
         }
       }
       __syncthreads();
-      for (int b = wv; b < NR; b += 4) {
+      if (wv < nr) {
         float ss = 0.f;
-        for (int c = 8 * lane; c < dim; c += 512) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
           float v[8];
-          unpack8(*reinterpret_cast<const u32x4 *>(xs + b * kLinXsRow + c), v);
+          unpack8(*reinterpret_cast<const u32x4 *>(xs + wv * kXsRow + 8 * lane + 512 * i), v);
 #pragma unroll
           for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
         }
         ss = wave_sum(ss);
-        if (lane == 0) rinv_s[b] = rsqrtf(ss / (float)dim + in.eps);
+        if (lane == 0) rinv_s[wv] = rsqrtf(ss / (float)dim + in.eps);
       }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int idx = threadIdx.x + 256 * i;
-        if (idx < NR * groups) {
-          const int b = idx / groups, c = 8 * (idx - b * groups);
-          float v[8], wf[8], y[8];
-          unpack8(*reinterpret_cast<const u32x4 *>(xs + b * kLinXsRow + c), v);
-          unpack8(nwv[i], wf);
-          const float ri = rinv_s[b];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) y[e] = wf[e] * (v[e] * ri);
-          *reinterpret_cast<u32x4 *>(xs + b * kLinXsRow + c) = pack8(y);
-        }
-      }
-    } else {
-      const float rinv[NR] = {};
-      for (int idx = threadIdx.x; idx < NR * groups; idx += 256) {
-        const int b = idx / groups, c = 8 * (idx - b * groups);
-        *reinterpret_cast<u32x4 *>(xs + b * kLinXsRow + c) = lin_input<NR, PRE>(in, b, c, rinv);
-      }
-    }
-    __syncthreads();
-  }
-  float acc[4][NR];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int b = 0; b < NR; ++b) acc[r][b] = 0.f;
-  int cg = 0;
-  if (first) {
-    lin_dot<4, NR, PRE>(in, xs, wfirst, 0, lane, acc);
-    cg = 2048;
-  }
-  for (; cg + 2048 <= dim; cg += 2048) {
-    u32x4 wv_[4][4];
-    lin_load<4>(wr, cg, wv_);
-    lin_dot<4, NR, PRE>(in, xs, wv_, cg, lane, acc);
-  }
-  if (dim - cg >= 1024) {
-    u32x4 wv_[2][4];
-    lin_load<2>(wr, cg, wv_);
-    lin_dot<2, NR, PRE>(in, xs, wv_, cg, lane, acc);
-    cg += 1024;
-  }
-  if (dim - cg >= 512) {
-    u32x4 wv_[1][4];
-    lin_load<1>(wr, cg, wv_);
-    lin_dot<1, NR, PRE>(in, xs, wv_, cg, lane, acc);
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int b = 0; b < NR; ++b) acc[r][b] = wave_sum(acc[r][b]);
-  if (lane == 0) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (v0 + r < vocab)
-#pragma unroll
-        for (int b = 0; b < NR; ++b) {
-          const __bf16 y = (__bf16)acc[r][b];
-          if constexpr (std::is_same<OutT, float>::value)
-            out[b * out_rs + v0 + r] = (float)y;
-          else
-            out[b * out_rs + v0 + r] = __builtin_bit_cast(bf16_t, y);
-        }
-  }
-}
-
-// Split-K form for dim > 2048 (the down projection, 6144 inputs): the kernel above walks a long
-// row in 2048-column steps, one HBM round trip each, over only n_out / 16 workgroups.  Here a
-// workgroup (4 waves) owns 4 output rows and wave wv takes the 512-column chunks wv, wv + 4,
-// wv + 8, ... of them, so the four waves split the dot products 4 ways.  When dim is 2048 * NJ
-// (NJ = 3: 6144) every wave has exactly NJ chunks and requests all of them (NJ x 4 rows x 16 B
-// per lane) before anything else, so a workgroup's whole 4-row slice of the weight is in flight
-// at once; other multiples of 512 take them one at a time (NJ = 0).
-template <int NCH>
-__device__ __forceinline__ void lin_load_sk(const bf16_t *const (&wr)[4], int c0, u32x4 (&wv_)[NCH][4]) {
-#pragma unroll
-  for (int j = 0; j < NCH; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) wv_[j][r] = ld16(wr[r] + c0 + 2048 * j);
-}
-template <int NCH, int NR, int PRE>
-__device__ __forceinline__ void lin_dot_sk(const LinIn &in, const u32x4 (&wv_)[NCH][4], int c0, int lane,
-                                        const float (&rinv)[NR], float (&acc)[4][NR]) {
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int c = c0 + 2048 * j + 8 * lane;
-#pragma unroll
-    for (int b = 0; b < NR; ++b) {
-      const u32x4 xv = lin_input<NR, PRE>(in, b, c, rinv);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t wd = wv_[j][r][e], xd = xv[e];   // scalar copies: see u32_as_f32
-          acc[r][b] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wd), __builtin_bit_cast(bf16x2, xd),
-                                                      acc[r][b], false);
-        }
-    }
-  }
-}
-// One workgroup (4 waves) per 4 output rows; per wave the bf16 pair dot products of its chunks,
-// a wave butterfly per (row, input row), then the four waves' partial sums added in wave order
-// through LDS.
-template <int NR, typename OutT, int PRE, int NJ>
-__global__ __launch_bounds__(256) void linear_rows_splitk_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t vocab,
-                                                          int dim, OutT *__restrict__ out, int64_t out_rs) {
-  __shared__ float part[4][4][NR];
-  const int lane = threadIdx.x & 63, wv = wave_id();
-  const int64_t v0 = (int64_t)blockIdx.x * 4;
-  // rows past the end read the last row (in bounds; their sums are not stored)
-  const bf16_t *wr[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) wr[r] = w + min(v0 + r, vocab - 1) * dim + 8 * lane;
-  // the wave's chunks of the weight are requested before the input is formed
-  u32x4 wfirst[NJ > 0 ? NJ : 1][4];
-  if constexpr (NJ > 0) lin_load_sk<NJ>(wr, 512 * wv, wfirst);
-  float rinv[NR];
-  if constexpr (PRE == kPreNorm) {
-    // sum of squares in the RMSNorm kernel's order: lane l sums its chunks l, l + 64, ... element
-    // by element, then the wave butterfly
-    const bool writer = blockIdx.x == 0 && wv == 0 && in.res_out != nullptr;
-#pragma unroll
-    for (int b = 0; b < NR; ++b) {
+    } else if (wv < nr) {
       float ss = 0.f;
-      for (int c = 8 * lane; c < dim; c += 512) {
+      for (int ch = 8 * lane; ch < dim; ch += 512) {
         float v[8];
-        unpack8(ld16(in.x + b * in.x_rs + c), v);
+        unpack8(ld16(in.x + wv * in.x_rs + ch), v);
         if (in.res) {
           float r[8];
-          unpack8(ld16(in.res + b * in.res_rs + c), r);
+          unpack8(ld16(in.res + wv * in.res_rs + ch), r);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
         }
-        if (writer) st16(in.res_out + b * in.ro_rs + c, pack8(v));
+        if (writer) st16(in.res_out + wv * in.ro_rs + ch, pack8(v));
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
       }
       ss = wave_sum(ss);
-      rinv[b] = rsqrtf(ss / (float)dim + in.eps);
+      if (lane == 0) rinv_s[wv] = rsqrtf(ss / (float)dim + in.eps);
     }
+    __syncthreads();
+    rinv = rinv_s[xr];
   }
-  float acc[4][NR];
+  if constexpr (kStageAct) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int b = 0; b < NR; ++b) acc[r][b] = 0.f;
-  if constexpr (NJ > 0) {
-    lin_dot_sk<NJ, NR, PRE>(in, wfirst, 512 * wv, lane, rinv, acc);
-  } else {
-    for (int c0 = 512 * wv; c0 < dim; c0 += 2048) {
-      u32x4 wv_[1][4];
-      lin_load_sk<1>(wr, c0, wv_);
-      lin_dot_sk<1, NR, PRE>(in, wv_, c0, lane, rinv, acc);
+    for (int s = 0; s < NK; ++s) {
+      const int idx = lane + 64 * s, b = idx / (8 * NK), j = idx % (8 * NK);
+      if (b < nr) *reinterpret_cast<u32x4 *>(xs + (8 * wv + b) * kXsRow + 8 * j) = swiglu8(xin[s], rin[s]);
     }
+    // only this wave reads its part: its LDS operations complete in order
   }
+  u32x4 xf[NKR];
+  if constexpr (NK > 0) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int b = 0; b < NR; ++b) acc[r][b] = wave_sum(acc[r][b]);
-  if (lane == 0) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int b = 0; b < NR; ++b) part[wv][r][b] = acc[r][b];
-  }
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (t < 4 * NR) {
-    const int r = t / NR, b = t % NR;
-    if (v0 + r < vocab) {
-      const float sum = ((part[0][r][b] + part[1][r][b]) + part[2][r][b]) + part[3][r][b];
-      const __bf16 y = (__bf16)sum;
-      if constexpr (std::is_same<OutT, float>::value)
-        out[b * out_rs + v0 + r] = (float)y;
+    for (int s = 0; s < NK; ++s) {
+      if constexpr (PRE == kPrePlain)
+        xf[s] = xin[s];
+      else if constexpr (kStageAct)
+        xf[s] = *reinterpret_cast<const u32x4 *>(xs + (8 * wv + xr) * kXsRow + 64 * s + (kl - 64 * wv));
+      else if constexpr (kStage)
+        xf[s] = norm8(*reinterpret_cast<const u32x4 *>(xs + xr * kXsRow + kl + 512 * s), nwv[s], rinv);
       else
-        out[b * out_rs + v0 + r] = __builtin_bit_cast(bf16_t, y);
+        xf[s] = lin_input<PRE>(in, xr, kl + 512 * s, rinv);
     }
   }
+  int buf = 0;
+  do {
+    f32x4 acc[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (NK > 0) {
+      // the next blocks' weights are requested before these are used
+      u32x4 wn[WALK ? NK : 1][RB];
+      if (WALK && v0 + step < n_out) {
+        rows_from(v0 + step);
+#pragma unroll
+        for (int s = 0; s < NK; ++s)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) wn[s][rb] = ld16(wr[rb] + 512 * s);
+      }
+#pragma unroll
+      for (int s = 0; s < NK; ++s)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb] = mfma16(__builtin_bit_cast(bf16x8, wf[s][rb]), __builtin_bit_cast(bf16x8, xf[s]), acc[rb]);
+      if constexpr (WALK)
+#pragma unroll
+        for (int s = 0; s < NK; ++s)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) wf[s][rb] = wn[s][rb];
+    } else {
+      for (int k = 0; k < dim; k += 512) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) wf[0][rb] = ld16(wr[rb] + k);
+        const u32x4 x = lin_input<PRE>(in, xr, kl + k, rinv);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb] = mfma16(__builtin_bit_cast(bf16x8, wf[0][rb]), __builtin_bit_cast(bf16x8, x), acc[rb]);
+      }
+    }
+    // lane l holds rows 4 (G % 2) .. + 3 of column half G / 2 for input row c where its own column is
+    // of that half
+    float (*part)[RB][2][64] = part2[WALK ? buf : 0];
+    if (((lane >> 3) & 1) == (G >> 1)) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) *reinterpret_cast<f32x4 *>(&part[wv][rb][G >> 1][8 * c + 4 * (G & 1)]) = acc[rb];
+    }
+    // one barrier per round: the sums of a round are read while the next round writes the other buffer.
+    // Not __syncthreads(), which would wait for the weights in flight.
+    ring_barrier();
+    const int t = threadIdx.x;
+    if (t < 64 * OB) {
+      const int ob = t >> 6, e = t & 63, b = e >> 3, r = e & 7;
+      auto total = [&](int rb) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) sum += part[i][rb][0][e] + part[i][rb][1][e];
+        return sum;
+      };
+      const int64_t v = v0 + 8 * ob + r;
+      if (b < nr && v < n_out) {
+        if constexpr (ACT) {
+          const float g = (float)(__bf16)total(ob), u = (float)(__bf16)total(OB + ob);
+          out[b * out_rs + v] = __builtin_bit_cast(bf16_t, (__bf16)(g / (1.f + __expf(-g)) * u));
+        } else {
+          const __bf16 y = (__bf16)total(ob);
+          if constexpr (std::is_same<OutT, float>::value)
+            out[b * out_rs + v] = (float)y;
+          else
+            out[b * out_rs + v] = __builtin_bit_cast(bf16_t, y);
+        }
+      }
+    }
+    v0 += step;
+    buf ^= 1;
+  } while (WALK && v0 < n_out);
 }
 
 // ---- Greedy token: the index of each row's largest logit -----------------------------------------
@@ -741,26 +690,63 @@ extern "C" int tg_gate_branch_readout(const void *gate_up, int64_t gate_up_row_s
 namespace tg {
 namespace {
 
-template <typename OutT, int PRE>
+template <int RB, int NK, typename OutT, int PRE, bool ACT>
+void launch_linear_rows_form(const LinIn &in, int32_t n_rows, const bf16_t *w, int64_t n_out, int32_t dim, OutT *out,
+                             int64_t out_row_stride, int64_t max_grid, hipStream_t stream) {
+  const int64_t rows = ACT ? 4 * RB : 8 * RB;
+  const int64_t blocks = (n_out + rows - 1) / rows;
+  if constexpr (NK == 4 && RB >= 2) {
+    if (blocks > max_grid) {
+      hipLaunchKernelGGL((linear_rows_mfma_kernel<RB, NK, OutT, PRE, ACT, true>), dim3((unsigned)max_grid), dim3(512), 0,
+                         stream, in, w, n_out, dim, n_rows, out, out_row_stride);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((linear_rows_mfma_kernel<RB, NK, OutT, PRE, ACT, false>), dim3((unsigned)blocks), dim3(512), 0,
+                     stream, in, w, n_out, dim, n_rows, out, out_row_stride);
+}
+// n_out: stored outputs (ACT: weight holds 2 n_out rows, [gate; up]).
+// Blocks of 8 weight rows per workgroup (RB) and workgroups, us at 1 / 8 input rows:
+//   * 2048 rows fill the CUs with one block each (2048 x 2048: RB 1 / 2 / 4 3.9 / 4.7 / 6.3 and 4.4 / 5.4 / 6.9;
+//     2048 x 6144: 6.6 / 9.0 / 16.1 and 8.2 / 10.8 / 17.6);
+//   * up to 65536 rows two blocks spread the input stage over more weight bytes, except at 4096 rows and
+//     up to two input rows (RB 1 / 2: 5.3 / 5.6 and 7.7 / 7.0); two workgroups per CU that walk the
+//     blocks, the next block's weights in flight, beat one workgroup per block (12288 rows with the
+//     SwiGLU product: 11.0 against 12.2, 13.6 against 14.5);
+//   * beyond (the LM head) the blocks' own workgroups keep more bytes in flight: plain input RB 1 / 2 /
+//     4 99.8 / 104.2 / 105.5 and 145 / 112 / 119; with the norm in every workgroup 143 / 104 / 114 and
+//     172 / 133 / 126, four blocks walked by four workgroups per CU 108 and 112.
+template <typename OutT, int PRE, bool ACT = false>
 int launch_linear_rows(const LinIn &in, int32_t n_rows, const void *weight, int64_t n_out, int32_t dim, OutT *out,
                        int64_t out_row_stride, hipStream_t stream) {
-  const int64_t blocks = (n_out + 15) / 16;
-  const bf16_t *wp = static_cast<const bf16_t *>(weight);
-  const int64_t sk_blocks = (n_out + 3) / 4;
-#define TG_LR(NR)                                                                                          \
-  if (n_rows == NR) {                                                                                      \
-    if (dim <= 2048)                                                                                       \
-      hipLaunchKernelGGL((linear_rows_kernel<NR, OutT, PRE>), dim3((unsigned)blocks), dim3(256), 0, stream, in, wp, \
-                         n_out, dim, out, out_row_stride);                                                 \
-    else if (dim == 6144)                                                                                  \
-      hipLaunchKernelGGL((linear_rows_splitk_kernel<NR, OutT, PRE, 3>), dim3((unsigned)sk_blocks), dim3(256), 0,  \
-                         stream, in, wp, n_out, dim, out, out_row_stride);                                 \
-    else                                                                                                   \
-      hipLaunchKernelGGL((linear_rows_splitk_kernel<NR, OutT, PRE, 0>), dim3((unsigned)sk_blocks), dim3(256), 0,  \
-                         stream, in, wp, n_out, dim, out, out_row_stride);                                 \
+  const bf16_t *w = static_cast<const bf16_t *>(weight);
+  const int64_t w_rows = ACT ? 2 * n_out : n_out;
+  const int64_t cus = device_cus();
+  int rb = 1;
+  int64_t max_grid = INT32_MAX;
+  if (w_rows >= 65536) {
+    rb = PRE == kPreNorm ? (n_rows == 1 ? 2 : 4) : (n_rows <= 2 ? 1 : 2);
+    if (rb == 4) max_grid = 4 * cus;
+  } else if (w_rows > 4096 || (w_rows == 4096 && n_rows > 2)) {
+    rb = 2;
+    max_grid = 2 * cus;
   }
-  TG_LR(1) TG_LR(2) TG_LR(3) TG_LR(4) TG_LR(5) TG_LR(6) TG_LR(7) TG_LR(8)
-#undef TG_LR
+  if (ACT) rb = std::max(rb, 2);
+  if (dim > 2048) rb = ACT ? 2 : 1;
+  auto form = [&](auto rb_c) {
+    constexpr int RB = decltype(rb_c)::value;
+    if (dim == 2048)
+      launch_linear_rows_form<RB, 4, OutT, PRE, ACT>(in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
+    else if (RB == 1 && PRE != kPreNorm && dim == 6144)
+      launch_linear_rows_form<RB, RB == 1 && PRE != kPreNorm ? 12 : 0, OutT, PRE, ACT>(
+          in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
+    else
+      launch_linear_rows_form<RB, 0, OutT, PRE, ACT>(in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
+  };
+  if constexpr (!ACT)
+    if (rb == 1) form(std::integral_constant<int, 1>());
+  if (rb == 2) form(std::integral_constant<int, 2>());
+  if (rb == 4) form(std::integral_constant<int, 4>());
   TG_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -772,7 +758,7 @@ int check_linear_rows(const char *what, const void *x, int64_t x_row_stride, int
   TG_CHECK(n_out > 0 && x_row_stride % 8 == 0 && x_row_stride >= dim && out_row_stride >= n_out,
            "%s: bad output size or row strides", what);
   TG_CHECK(aligned16(x) && aligned16(weight), "%s: x and weight must be 16-byte aligned", what);
-  TG_CHECK((n_out + 15) / 16 < (1ll << 31), "%s: too many output features", what);
+  TG_CHECK((n_out + 3) / 4 < (1ll << 31), "%s: too many output features", what);
   return 0;
 }
 
@@ -803,6 +789,31 @@ extern "C" int tg_linear_rows(const void *x, int64_t x_row_stride, int32_t n_row
                                                out_row_stride, stream);
 }
 
+namespace tg {
+namespace {
+int norm_input(const char *what, const void *h, int64_t h_row_stride, const void *residual, int64_t residual_row_stride,
+               void *residual_out, int64_t residual_out_row_stride, const void *norm_weight, float eps, int32_t dim,
+               LinIn *in) {
+  TG_CHECK(norm_weight && aligned16(norm_weight), "%s: norm weight must be non-null and 16-byte aligned", what);
+  TG_CHECK(!residual || (aligned16(residual) && residual_row_stride % 8 == 0 && residual_row_stride >= dim),
+           "%s: bad residual", what);
+  TG_CHECK(!residual_out || (aligned16(residual_out) && residual_out_row_stride % 8 == 0 &&
+                             residual_out_row_stride >= dim && residual_out != residual),
+           "%s: bad residual_out (it must not be the residual input)", what);
+  TG_CHECK(eps >= 0.f, "%s: eps must be non-negative", what);
+  in->x = static_cast<const bf16_t *>(h);
+  in->x_rs = h_row_stride;
+  in->res = static_cast<const bf16_t *>(residual);
+  in->res_rs = residual_row_stride;
+  in->res_out = static_cast<bf16_t *>(residual_out);
+  in->ro_rs = residual_out_row_stride;
+  in->nw = static_cast<const bf16_t *>(norm_weight);
+  in->eps = eps;
+  return 0;
+}
+}  // namespace
+}  // namespace tg
+
 extern "C" int tg_linear_rows_norm(const void *h, int64_t h_row_stride, const void *residual,
                                    int64_t residual_row_stride, void *residual_out, int64_t residual_out_row_stride,
                                    const void *norm_weight, float eps, int32_t n_rows, const void *weight,
@@ -811,27 +822,32 @@ extern "C" int tg_linear_rows_norm(const void *h, int64_t h_row_stride, const vo
   clear_error();
   if (int e = check_linear_rows("linear_rows_norm", h, h_row_stride, n_rows, weight, n_out, dim, out, out_row_stride))
     return e;
-  TG_CHECK(norm_weight && aligned16(norm_weight), "linear_rows_norm: norm weight must be non-null and 16-byte aligned");
-  TG_CHECK(!residual || (aligned16(residual) && residual_row_stride % 8 == 0 && residual_row_stride >= dim),
-           "linear_rows_norm: bad residual");
-  TG_CHECK(!residual_out || (aligned16(residual_out) && residual_out_row_stride % 8 == 0 &&
-                             residual_out_row_stride >= dim && residual_out != residual),
-           "linear_rows_norm: bad residual_out (it must not be the residual input)");
-  TG_CHECK(eps >= 0.f, "linear_rows_norm: eps must be non-negative");
   LinIn in{};
-  in.x = static_cast<const bf16_t *>(h);
-  in.x_rs = h_row_stride;
-  in.res = static_cast<const bf16_t *>(residual);
-  in.res_rs = residual_row_stride;
-  in.res_out = static_cast<bf16_t *>(residual_out);
-  in.ro_rs = residual_out_row_stride;
-  in.nw = static_cast<const bf16_t *>(norm_weight);
-  in.eps = eps;
+  if (int e = norm_input("linear_rows_norm", h, h_row_stride, residual, residual_row_stride, residual_out,
+                         residual_out_row_stride, norm_weight, eps, dim, &in))
+    return e;
   if (out_fp32)
     return launch_linear_rows<float, kPreNorm>(in, n_rows, weight, n_out, dim, static_cast<float *>(out),
                                                out_row_stride, stream);
   return launch_linear_rows<bf16_t, kPreNorm>(in, n_rows, weight, n_out, dim, static_cast<bf16_t *>(out),
                                               out_row_stride, stream);
+}
+
+extern "C" int tg_linear_rows_norm_act(const void *h, int64_t h_row_stride, const void *residual,
+                                       int64_t residual_row_stride, void *residual_out,
+                                       int64_t residual_out_row_stride, const void *norm_weight, float eps,
+                                       int32_t n_rows, const void *weight, int64_t inter, int32_t dim, void *out,
+                                       int64_t out_row_stride, hipStream_t stream) {
+  clear_error();
+  if (int e = check_linear_rows("linear_rows_norm_act", h, h_row_stride, n_rows, weight, inter, dim, out,
+                                out_row_stride))
+    return e;
+  LinIn in{};
+  if (int e = norm_input("linear_rows_norm_act", h, h_row_stride, residual, residual_row_stride, residual_out,
+                         residual_out_row_stride, norm_weight, eps, dim, &in))
+    return e;
+  return launch_linear_rows<bf16_t, kPreNorm, true>(in, n_rows, weight, inter, dim, static_cast<bf16_t *>(out),
+                                                    out_row_stride, stream);
 }
 
 extern "C" int tg_linear_rows_swiglu(const void *gate_up, int64_t gate_up_row_stride, int32_t n_rows, int32_t inter,

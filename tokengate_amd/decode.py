@@ -27,7 +27,7 @@ from typing import List, Optional
 import torch
 
 from tokengate_amd.decoder import (CacheGap, DecoderWeights, LayerKV, argmax_rows, h2d, linear_rows, linear_rows_norm,
-                                   linear_rows_swiglu, logits_last, qk_norm_rope, rmsnorm, silu_mul,
+                                   linear_rows_norm_act, logits_last, qk_norm_rope, rmsnorm, silu_mul,
                                    varlen_kv_attention)
 from tokengate_amd.gate import ScoringHead
 from tokengate_amd.prefill import PrefillResult
@@ -56,7 +56,7 @@ def _relayout(kv: LayerKV, cu: List[int], gap: int) -> LayerKV:
 
 class DecodeState:
     # most rows per step for which the norms and the SwiGLU product are folded into the projections
-    max_fused_rows = 2
+    max_fused_rows = 8
 
     def __init__(self, wts: DecoderWeights, head: ScoringHead, gate_layer: int, pf: PrefillResult,
                  max_new_tokens: int, prune_below_gate: bool = False, graph: bool = False, fused: bool = True):
@@ -156,8 +156,8 @@ class DecodeState:
             r_dec = (torch.log(m) / torch.log(p)).clamp(max=1.0)
         scale = 1.0 / math.sqrt(s.head_dim)
         if fused:
-            # each norm is folded into the projection after it, and the SwiGLU product into the down
-            # projection; the residual stream alternates between two buffers (a fused norm reads one
+            # each norm is folded into the projection after it, and the SwiGLU product into the
+            # gate|up projection; the residual stream alternates between two buffers (a fused norm reads one
             # and writes the other)
             rbuf = [torch.empty_like(x), torch.empty_like(x)]
             cur = 0
@@ -183,9 +183,9 @@ class DecodeState:
                                 self.bias[j] if g else None, out=att, lse=lse)
             linear_rows(att.view(B, -1), lw.w_o, out=hid)
             if fused:
-                gu = linear_rows_norm(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur], residual_out=rbuf[1 - cur])
+                act = linear_rows_norm_act(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur], residual_out=rbuf[1 - cur])
                 cur = 1 - cur
-                linear_rows_swiglu(gu, lw.w_down, out=hid)
+                linear_rows(act, lw.w_down, out=hid)
             else:
                 rmsnorm(hid, lw.ln2, s.rms_eps, residual=res, residual_out=res, out=normed)
                 act = silu_mul(linear_rows(normed, lw.w_gu))

@@ -452,6 +452,26 @@ def linear_rows_norm(h: torch.Tensor, norm_w: torch.Tensor, eps: float, weight: 
     return out
 
 
+def linear_rows_norm_act(h: torch.Tensor, norm_w: torch.Tensor, eps: float, weight: torch.Tensor,
+                         residual: Optional[torch.Tensor] = None, residual_out: Optional[torch.Tensor] = None,
+                         out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """silu(g) * u of F.linear(RMSNorm(h + residual), weight) = [g | u] for up to 8 rows in one launch
+    (tg_linear_rows_norm_act); residual_out as in linear_rows_norm."""
+    n, d = h.shape
+    inter = weight.shape[0] // 2
+    if not (1 <= n <= 8 and d % 512 == 0 and _rows_ok(h, residual, residual_out) and weight.stride(1) == 1
+            and weight.stride(0) == d and weight.shape[0] == 2 * inter):
+        raise RuntimeError("linear_rows_norm_act: 1..8 contiguous 16-byte aligned rows, dim a multiple of 512, "
+                           "an even number of weight rows")
+    out = torch.empty(n, inter, dtype=torch.bfloat16, device=h.device) if out is None else out
+    _lib.call("tg_linear_rows_norm_act", h.data_ptr(), h.stride(0),
+              residual.data_ptr() if residual is not None else None, residual.stride(0) if residual is not None else 0,
+              residual_out.data_ptr() if residual_out is not None else None,
+              residual_out.stride(0) if residual_out is not None else 0,
+              norm_w.data_ptr(), float(eps), n, weight.data_ptr(), inter, d, out.data_ptr(), out.stride(0), _stream(h))
+    return out
+
+
 def linear_rows_swiglu(gate_up: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear(silu(g) * u, weight) of gate/up rows [g | u] for up to 8 rows in one launch."""
     n, two_i = gate_up.shape
