@@ -376,6 +376,33 @@ int tg_linear_rows_norm_act(const void *h, int64_t h_row_stride, const void *res
 int tg_linear_rows_swiglu(const void *gate_up, int64_t gate_up_row_stride, int32_t n_rows, int32_t inter,
                           const void *weight, int64_t n_out, void *out, int64_t out_row_stride, hipStream_t stream);
 
+/* What the layers of one decode step share, for num_seqs sequences at positions[b] (head_dim 128): the
+ * rotary table rope[b][64][2] = (cos, sin)(positions[b] * inv_freq), kv_used[i * num_seqs + b] += 1 for the
+ * n_used cache groups, and, with slots, slots[b] += 1 and the new token's scaled-softmax ratio
+ * ratio[b] = min(1, ln max(2, slots[b]) / ln max(2, positions[b] + 1)) (FormDecodeState.step,
+ * qwen3_flex_attention.py:1090-1101); positions[b] += 1 last. */
+int tg_decode_begin(int64_t *positions, int32_t num_seqs, const float *inv_freq, float *rope, int32_t *kv_used,
+                    int32_t n_used, float *slots, float *ratio, hipStream_t stream);
+
+/* Attention of one decode step, one query row per sequence, from the raw q|k|v projection rows to the
+ * attention output in one launch: q/k RMSNorm, rotary embedding (rope: tg_decode_begin's table) and query
+ * scale as tg_qk_norm_rope (same roundings); the new k / v rows written to cache row kv_start[b] + kv_used[b] - 1; then every
+ * head over the cache rows kv_start[b] .. kv_start[b] + kv_used[b] - 1 (the new row included), logits
+ * softmax_scale * (q . k_j + bias_raw[b, h, j]), fp32 weights.  kv_used[b] is at least 1 and at most
+ * max_seqlen_k (FormDecodeState.step, qwen3_flex_attention.py:1017-1117).
+ * out: bf16 rows (num_heads * 128).  workspace: tg_decode_attention_workspace_size bytes, zeroed once
+ * when it is allocated; every launch leaves the words it counts in at zero, so launches of one stream
+ * share it (launches that may overlap need one each). */
+int64_t tg_decode_attention_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_heads_k,
+                                           int32_t max_seqlen_k);
+int tg_decode_attention(const void *qkv, int64_t qkv_row_stride, const float *rope, int32_t num_seqs,
+                        int32_t num_heads, int32_t num_heads_k, int32_t head_dim, const void *q_norm_weight,
+                        const void *k_norm_weight, float eps, const float *q_head_scale, const float *q_row_scale,
+                        void *k_cache, int64_t k_row_stride, void *v_cache, int64_t v_row_stride,
+                        const int32_t *kv_start, const int32_t *kv_used, int32_t max_seqlen_k, const float *bias_raw, int64_t bias_seq_stride,
+                        int64_t bias_head_stride, float softmax_scale, void *out, int64_t out_row_stride,
+                        void *workspace, int64_t workspace_bytes, hipStream_t stream);
+
 /* Greedy next token: out[b] = argmax_v x[b, v] (int64) with torch.argmax's rules (a NaN wins, ties
  * go to the lower index) — the reference's logits.argmax(-1) of the first-token and decode steps
  * (gate_forward.py:1559-1562, gate_decode.py:227).  One launch and no memory clears, so a decode

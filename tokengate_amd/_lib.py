@@ -57,11 +57,15 @@ SIGNATURES = {
     "tg_linear_rows_norm": [vp, i64, vp, i64, vp, i64, vp, f32, i32, vp, i64, i32, vp, i64, i32, vp],
     "tg_linear_rows_norm_act": [vp, i64, vp, i64, vp, i64, vp, f32, i32, vp, i64, i32, vp, i64, vp],
     "tg_linear_rows_swiglu": [vp, i64, i32, i32, vp, i64, vp, i64, vp],
+    "tg_decode_begin": [vp, i32, vp, vp, vp, i32, vp, vp, vp],
+    "tg_decode_attention": [vp, i64, vp, i32, i32, i32, i32, vp, vp, f32, vp, vp, vp, i64, vp, i64, vp, vp, i32,
+                            vp, i64, i64, f32, vp, i64, vp, i64, vp],
+    "tg_decode_attention_workspace_size": [i32, i32, i32, i32],
     "tg_argmax_rows": [vp, i64, i32, i64, vp, vp],
 }
 RESTYPES = {"tg_last_error": C.c_char_p, "tg_keybias_fwd_workspace_size": C.c_int64,
             "tg_keybias_varlen_fwd_workspace_size": C.c_int64, "tg_keybias_varlen_kv_fwd_workspace_size": C.c_int64,
-            "tg_gate_select_pack_workspace_size": C.c_int64}
+            "tg_decode_attention_workspace_size": C.c_int64, "tg_gate_select_pack_workspace_size": C.c_int64}
 
 
 def lib_path(site: str = None) -> str:

@@ -867,7 +867,6 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
 #undef TG_DKV
 }
 
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 bool strides_ok(std::initializer_list<int64_t> s) {
   for (int64_t x : s)
     if (x % 8 != 0) return false;

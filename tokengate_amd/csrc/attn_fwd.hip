@@ -96,6 +96,26 @@ struct FwdArgs {
   float *ws_ml;                // [heavy unit][chunk][wave][column block][64 lanes] x (m, l)
 };
 
+// A decode step's launch (one query row per sequence): q and the new key come from the raw q|k|v
+// projection rows, and the chunks of a split are merged by the workgroup that arrives last.
+struct DecArgs {
+  const bf16_t *qkv;           // rows of h + 2 hkv heads, one per sequence
+  int64_t qkv_rs;
+  const float2 *rope;          // (nseq, 64) (cos, sin) of every sequence's position
+  const bf16_t *qw, *kw;       // q/k norm weights
+  float eps;
+  const float *q_head_scale, *q_row_scale;
+  bf16_t *k_cache, *v_cache;   // = FwdArgs' k, v
+  uint32_t *counters;          // per (sequence, head group): chunks arrived; zero between launches
+  uint64_t *ml;                // [unit][chunk][head]: running max (log2 units) and row sum
+  uint64_t *po;                // [unit][chunk][head][16 pieces of 8 bf16]: O / l, 32 words
+};
+struct NoDec {};
+template <typename T>
+__device__ __forceinline__ void st_agent(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 // LDS row lr of a 64-key tile holds key kperm(lr): within each 32-key step, S^T block kb' (rows
 // 16kb' .. 16kb'+15) row m carries key 8(m/4) + 4kb' + m%4, so that lane group G of the two S^T
 // accumulators of a step holds keys 8G .. 8G+7 of the step — exactly the k range of the B operand
@@ -103,6 +123,10 @@ struct FwdArgs {
 __device__ __forceinline__ int kperm(int lr) {
   const int m = lr & 15;
   return 32 * (lr >> 5) + 8 * (m >> 2) + 4 * ((lr >> 4) & 1) + (m & 3);
+}
+
+__device__ __forceinline__ int kperm_inv(int key) {
+  return 32 * (key >> 5) + 16 * ((key >> 2) & 1) + 4 * ((key >> 3) & 3) + (key & 3);
 }
 
 // Lazy rescaling threshold (log2 units): the running max used for exp2 is raised only when a tile
@@ -136,8 +160,60 @@ template <int CW, int HP> __device__ __forceinline__ int wave_head(int w) { retu
 template <int CW, int HP> __device__ __forceinline__ int wave_pos(int w) { return kQW * (HP == 2 ? w % (CW / 2) : w); }
 __device__ __forceinline__ int col_query(int cb, int c16) { return 16 * cb + c16; }
 
-template <int NW, int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a) {
+// Merge of key chunks.  With chunk c's running max m_c (log2 units), row sum l_c and normalised partial
+// O_c: m = max m_c, w_c = l_c 2^(m_c - m), O = sum w_c O_c / sum w_c, lse = (m + log2 sum w_c) ln 2.
+// Chunks that saw no key (l_c = 0) weigh nothing.  One thread holds 8 O values; up to kCombineMaxGroups
+// groups of threads fold every so many-th chunk each, then their results in turn (merge_fold).
+constexpr int kCombineMaxGroups = 8;
+struct Fold {
+  float mmax = -INFINITY, wsum = 0.f;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+};
+__device__ __forceinline__ void fold_chunk(Fold &f, float2 mc, u32x4 pv) {
+  if (!(mc.y > 0.f)) return;
+  if (mc.x > f.mmax) {
+    const float sc = fast_exp2(f.mmax - mc.x);   // 0 while nothing has been added yet
+    f.wsum *= sc;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f.acc[i] *= sc;
+    f.mmax = mc.x;
+  }
+  const float w = mc.y * fast_exp2(mc.x - f.mmax);
+  f.wsum += w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    f.acc[2 * e] += w * __builtin_bit_cast(float, pv[e] << 16);
+    f.acc[2 * e + 1] += w * __builtin_bit_cast(float, pv[e] & 0xffff0000u);
+  }
+}
+// p: another group's (mmax, wsum, acc), `stride` floats apart
+__device__ __forceinline__ void merge_fold(Fold &f, const float *p, int stride) {
+  const float m2 = p[0], w2 = p[stride];
+  if (!(w2 > 0.f)) return;
+  const float mn = fmaxf(f.mmax, m2);
+  const float s1 = fast_exp2(f.mmax - mn), s2 = fast_exp2(m2 - mn);   // s1 = 0 if mmax = -inf
+  f.wsum = f.wsum * s1 + w2 * s2;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f.acc[i] = f.acc[i] * s1 + p[(2 + i) * stride] * s2;
+  f.mmax = mn;
+}
+__device__ __forceinline__ void store_fold(const Fold &f, float *p, int stride) {
+  p[0] = f.mmax;
+  p[stride] = f.wsum;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p[(2 + i) * stride] = f.acc[i];
+}
+// chunk groups of a split into ns chunks: up to 8, and at least two chunks per group
+__host__ __device__ __forceinline__ int combine_groups(int ns) {
+  int n = 1;
+  while (n < kCombineMaxGroups && 2 * n * 2 <= ns) n *= 2;
+  return n;
+}
+
+template <int NW, int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN, bool DEC = false>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
+                                                                      std::conditional_t<DEC, DecArgs, NoDec> dec) {
+  static_assert(!DEC || (VARLEN && NW == 4 && KS == 1), "the decode step's form");
   constexpr int kWaves = NW;
   constexpr int CW = col_waves<NW, KS>();
   constexpr int BM = bm<CW, HP>();
@@ -202,7 +278,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
 
   int sq = a.sq, sk = a.sk;
   int64_t row0 = 0, krow0 = 0;
-  if constexpr (VARLEN) {
+  if constexpr (DEC) {
+    row0 = b;
+    sq = 1;
+    krow0 = a.cu_k[b];
+    sk = max(0, min(a.used_k[b], a.sk));
+  } else if constexpr (VARLEN) {
     const int s0 = a.cu_seqlens[b], s1 = a.cu_seqlens[b + 1];
     row0 = s0;
     sq = min(s1 - s0, a.sq);   // rows past max_seqlen are outside the bias row: not computed
@@ -256,12 +337,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   const bool wave_has_rows = qw0 < sq;
   const int qw_hi = min(qw0 + kQW, sq) - 1;
   bf16x8 qf[2][4];
+  if constexpr (!DEC) {
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb)
+    for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      qf[cb][ks] = __builtin_bit_cast(
-          bf16x8, gload16(qbase + (int64_t)qrow[cb] * a.q_rs + (int64_t)hw * a.q_hs + 32 * ks + 8 * G, qvalid[cb]));
+      for (int ks = 0; ks < 4; ++ks)
+        qf[cb][ks] = __builtin_bit_cast(
+            bf16x8, gload16(qbase + (int64_t)qrow[cb] * a.q_rs + (int64_t)hw * a.q_hs + 32 * ks + 8 * G, qvalid[cb]));
+  }
 
   int kv_end = sk;
   if constexpr (CAUSAL) kv_end = min(sk, q0 + BM + off);
@@ -271,6 +354,33 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
   if (chunk >= 0) {
     t_lo = (int)((int64_t)n_tiles * chunk / a.ns);
     t_hi = (int)((int64_t)n_tiles * (chunk + 1) / a.ns);
+  }
+  // decode: a chunk without a tile has nothing to add (the first one stands in where there is no key)
+  const int n_parts = max(1, min(n_tiles, a.ns));   // chunks with a tile
+  if constexpr (DEC) {
+    if (chunk >= 0 && t_lo == t_hi && (n_tiles > 0 || chunk > 0)) return;   // workgroup-uniform
+  }
+  // decode: 16 threads per row, HP query rows, then the new k and v rows (the last tile's workgroup)
+  [[maybe_unused]] const int drow = tid >> 4, dj = tid & 15;
+  [[maybe_unused]] const bool has_new = t_hi == n_tiles && n_tiles > 0;
+  [[maybe_unused]] const bool dwork = DEC && (drow < HP || (has_new && drow < HP + 2));
+  [[maybe_unused]] u32x4 draw = {0u, 0u, 0u, 0u}, dnw = draw;
+  [[maybe_unused]] f32x4 dcs[4];
+  [[maybe_unused]] float dscale = 1.f;
+  if constexpr (DEC) {   // requested before the first tile: loads complete in issue order
+    if (dwork) {
+      const int head = drow < HP ? h0 + drow : drow == HP ? a.h + kh : a.h + a.hkv + kh;
+      draw = ld16(dec.qkv + b * dec.qkv_rs + (int64_t)head * kHeadDim + 8 * dj);
+      if (drow <= HP) {
+        dnw = ld16((drow < HP ? dec.qw : dec.kw) + 8 * dj);
+        const f32x4 *rp = reinterpret_cast<const f32x4 *>(dec.rope + b * (kHeadDim / 2) + 8 * (dj & 7));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dcs[i] = rp[i];
+      }
+      if (drow < HP)
+        dscale = (float)(__bf16)((dec.q_head_scale ? dec.q_head_scale[h0 + drow] : 1.f) *
+                                 (dec.q_row_scale ? dec.q_row_scale[b] : 1.f));
+    }
   }
 
   // ---- per-lane DMA source offsets (bytes within a tile; + tile * 64 rows per tile) ----
@@ -344,6 +454,18 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     const int n0 = t * SK + KN * kg;   // this wave's first key of the step
     wait_vm<0>();
     ring_barrier();
+    if constexpr (DEC) {
+      if (t == n_tiles - 1) {   // the new key's rows replace what the cache held there
+        const int key = (sk - 1) & 63;
+        if (drow == HP) {
+          const int lr = kperm_inv(key);
+          *reinterpret_cast<u32x4 *>(kslot(buf_c) + lr * kKRowBytes + 16 * (dj ^ (lr & 15))) = draw;
+        } else if (drow == HP + 1) {
+          *reinterpret_cast<u32x4 *>(vslot(buf_c) + key * kKRowBytes + 16 * (dj ^ vswz(key))) = draw;
+        }
+        ring_barrier();
+      }
+    }
     if (t + 1 < t_hi) issue_tile(t + 1, std::integral_constant<int, 1 - BUF>());
     if (!wave_has_rows || (CAUSAL && n0 > qw_hi + off)) return;
 
@@ -488,6 +610,38 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     }
   };
   if (t_lo < t_hi) issue_tile(t_lo, std::integral_constant<int, 0>());
+  if constexpr (DEC) {
+    __shared__ __attribute__((aligned(16))) bf16_t qs[HP][kHeadDim];
+    if (dwork && drow <= HP) {
+      float x[8], wf[8], y[8], cs[8][2];
+      unpack8(draw, x);
+      unpack8(dnw, wf);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        cs[e][0] = dcs[e >> 1][2 * (e & 1)];
+        cs[e][1] = dcs[e >> 1][2 * (e & 1) + 1];
+      }
+      norm_rope8(x, wf, dec.eps, cs, dj, dscale, y);
+      draw = pack8(y);
+      if (drow < HP) *reinterpret_cast<u32x4 *>(&qs[drow][8 * dj]) = draw;
+    }
+    // the new rows go to the cache, from one of the head groups that read this KV head
+    if (dwork && drow >= HP && hg == 0 && a.used_k[b] <= a.sk) {
+      const int64_t crow = krow0 + sk - 1;
+      bf16_t *dst = drow == HP ? dec.k_cache + crow * a.k_rs + (int64_t)kh * a.k_hs
+                               : dec.v_cache + crow * a.v_rs + (int64_t)kh * a.v_hs;
+      st16(dst + 8 * dj, draw);
+    }
+    ring_barrier();
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(&qs[hw][32 * ks + 8 * G]);
+        qf[cb][ks] = __builtin_bit_cast(bf16x8, qvalid[cb] ? v : zero);
+      }
+  }
   int t = t_lo;
   for (; t + 1 < t_hi; t += 2) {
     tile_step(t, std::integral_constant<int, 0>());
@@ -537,7 +691,77 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
     l[cb] = lacc[cb][0];
     inv[cb] = l[cb] > 0.f ? 1.f / l[cb] : 0.f;
   }
-  if (chunk >= 0) {
+  if constexpr (DEC) {
+    if (chunk >= 0) {
+      // The partial result of this chunk (column 0 of the first wave of each head), written and read with
+      // agent-scope accesses: those write through and read past the XCD's L2, where a release would have
+      // to write all of that L2 back.  The last workgroup to arrive merges them in the order and with the
+      // arithmetic of the combine kernel, whoever it is, and leaves the counter at zero.
+      const int64_t unit = hunit;
+      if (wave_has_rows && c16 == 0) {
+        const int64_t at = (unit * a.ns + chunk) * HP + hw;
+        uint64_t *po = dec.po + at * 32;
+        const float s = inv[0];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const f32x4 &o0 = oacc[0][2 * p], &o1 = oacc[0][2 * p + 1];
+          const u32x2 w0 = {pack_bf16x2(o0[0] * s, o0[1] * s), pack_bf16x2(o0[2] * s, o0[3] * s)};
+          const u32x2 w1 = {pack_bf16x2(o1[0] * s, o1[1] * s), pack_bf16x2(o1[2] * s, o1[3] * s)};
+          st_agent(po + 2 * (4 * p + G), __builtin_bit_cast(uint64_t, w0));
+          st_agent(po + 2 * (4 * p + G) + 1, __builtin_bit_cast(uint64_t, w1));
+        }
+        if (G == 0) {
+          const float2 ml = {mrun[0], l[0]};
+          st_agent(dec.ml + at, __builtin_bit_cast(uint64_t, ml));
+        }
+      }
+      __shared__ int last_s;
+      wait_all_mem();   // this wave's stores are done
+      __syncthreads();
+      if (tid == 0)
+        last_s = __hip_atomic_fetch_add(dec.counters + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 (uint32_t)n_parts - 1u;
+      __syncthreads();
+      if (!last_s) return;
+      if (tid == 0) st_agent(dec.counters + unit, 0u);
+      constexpr int kItems = HP * 16;   // a head's pieces of 8 O values
+      __shared__ float part[kCombineMaxGroups - 1][10][kItems];
+      const int CG = combine_groups(a.ns), item = tid % kItems, cg = tid / kItems, hl = item >> 4, piece = item & 15;
+      Fold f;
+      if (cg < CG) {
+        constexpr int kR = 4;   // chunks in flight
+        for (int c0 = cg; c0 < a.ns; c0 += kR * CG) {
+          uint64_t ml[kR], w0[kR], w1[kR];
+#pragma unroll
+          for (int r = 0; r < kR; ++r) {
+            const int c = c0 + r * CG;
+            const bool there = c < a.ns && (int)((int64_t)n_tiles * c / a.ns) < (int)((int64_t)n_tiles * (c + 1) / a.ns);
+            const int64_t at = (unit * a.ns + c) * HP + hl;
+            ml[r] = there ? ld_agent(dec.ml + at) : 0u;
+            w0[r] = there ? ld_agent(dec.po + at * 32 + 2 * piece) : 0u;
+            w1[r] = there ? ld_agent(dec.po + at * 32 + 2 * piece + 1) : 0u;
+          }
+#pragma unroll
+          for (int r = 0; r < kR; ++r) {
+            const u32x2 a0 = __builtin_bit_cast(u32x2, w0[r]), a1 = __builtin_bit_cast(u32x2, w1[r]);
+            fold_chunk(f, __builtin_bit_cast(float2, ml[r]), u32x4{a0[0], a0[1], a1[0], a1[1]});
+          }
+        }
+        if (cg > 0) store_fold(f, &part[cg - 1][0][item], kItems);
+      }
+      __syncthreads();
+      if (cg > 0) return;
+      for (int q = 0; q < CG - 1; ++q) merge_fold(f, &part[q][0][item], kItems);
+      const float s = f.wsum > 0.f ? 1.f / f.wsum : 0.f;
+      bf16_t *orow = obase + (int64_t)hl * a.o_hs;
+      const int d0 = 32 * (piece >> 2) + 4 * (piece & 3);
+      const u32x2 y0 = {pack_bf16x2(f.acc[0] * s, f.acc[1] * s), pack_bf16x2(f.acc[2] * s, f.acc[3] * s)};
+      const u32x2 y1 = {pack_bf16x2(f.acc[4] * s, f.acc[5] * s), pack_bf16x2(f.acc[6] * s, f.acc[7] * s)};
+      *reinterpret_cast<u32x2 *>(orow + d0) = y0;
+      *reinterpret_cast<u32x2 *>(orow + d0 + 16) = y1;
+      return;
+    }
+  } else if (chunk >= 0) {
     // partial result of this key chunk: O / l as bf16 (piece 4 cb + p holds d-blocks 2p and 2p+1 of
     // column block cb; each piece a coalesced 1 KB wave store) and, per column block, (running max
     // in log2 units, row sum l)
@@ -577,7 +801,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
       const u32x2 w = {pack_bf16x2(o[0] * s, o[1] * s), pack_bf16x2(o[2] * s, o[3] * s)};
       *reinterpret_cast<u32x2 *>(orow + 16 * (db0 + d) + 4 * G) = w;
     }
-    if (G == 0 && kg == 0) {
+    if (!DEC && G == 0 && kg == 0) {
       const float lse = l[cb] > 0.f ? (mrun[cb] + __log2f(l[cb])) * kLn2 : INFINITY;
       const int hh = h0 + hl;
       if constexpr (VARLEN)
@@ -593,10 +817,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a)
 // tile; per piece, thread (group cg, lane) folds chunks cg, cg + CG, ... of its column and group 0
 // merges the CG partial results through LDS, so that a long chunk list (a decode row over a long
 // cache) is walked CG ways in parallel.
-// With chunk c's running max m_c (log2 units), row sum l_c and normalised partial O_c:
-// m = max m_c, w_c = l_c 2^(m_c - m), O = sum w_c O_c / sum w_c, lse = (m + log2 sum w_c) ln 2.
-// Chunks that saw no key (l_c = 0) weigh nothing.
-constexpr int kCombineMaxGroups = 8;
 template <int CW, int HP, bool VARLEN>
 __global__ __launch_bounds__(512) void keybias_fwd_combine_kernel(FwdArgs a, int CG) {
   constexpr int BM = bm<CW, HP>();
@@ -634,49 +854,22 @@ __global__ __launch_bounds__(512) void keybias_fwd_combine_kernel(FwdArgs a, int
   const u32x4 *po = reinterpret_cast<const u32x4 *>(a.ws_o);
   const int64_t pw0 = hunit * a.ns * CW + wave;   // chunk c: pw0 + c * CW
   // fold this group's chunks, the weights relative to the largest m seen so far
-  float mmax = -INFINITY, wsum = 0.f;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  Fold f;
   if (valid) {
 #pragma unroll 4
     for (int c = cg; c < a.ns; c += CG) {
       const int64_t pw = pw0 + (int64_t)c * CW;
       const float2 mc = ml[pw * 128 + cb * 64 + lane];
       const u32x4 pv = po[pw * (8 * 64) + j * 64 + lane];
-      if (!(mc.y > 0.f)) continue;
-      if (mc.x > mmax) {
-        const float sc = fast_exp2(mmax - mc.x);   // 0 while nothing has been added yet
-        wsum *= sc;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] *= sc;
-        mmax = mc.x;
-      }
-      const float w = mc.y * fast_exp2(mc.x - mmax);
-      wsum += w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[2 * e] += w * __builtin_bit_cast(float, pv[e] << 16);
-        acc[2 * e + 1] += w * __builtin_bit_cast(float, pv[e] & 0xffff0000u);
-      }
+      fold_chunk(f, mc, pv);
     }
   }
-  if (cg > 0) {
-    mypart[cg - 1][0][lane] = mmax;
-    mypart[cg - 1][1][lane] = wsum;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) mypart[cg - 1][2 + i][lane] = acc[i];
-  }
+  if (cg > 0) store_fold(f, &mypart[cg - 1][0][lane], 64);
   __syncthreads();
   if (cg > 0 || !valid) return;
-  for (int q = 0; q < CG - 1; ++q) {
-    const float m2 = mypart[q][0][lane], w2 = mypart[q][1][lane];
-    if (!(w2 > 0.f)) continue;
-    const float mn = fmaxf(mmax, m2);
-    const float s1 = fast_exp2(mmax - mn), s2 = fast_exp2(m2 - mn);   // s1 = 0 if mmax = -inf
-    wsum = wsum * s1 + w2 * s2;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = acc[i] * s1 + mypart[q][2 + i][lane] * s2;
-    mmax = mn;
-  }
+  for (int q = 0; q < CG - 1; ++q) merge_fold(f, &mypart[q][0][lane], 64);
+  const float wsum = f.wsum, mmax = f.mmax;
+  const float (&acc)[8] = f.acc;
   const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
   const int h0 = kh * a.group + hg * HP;
   bf16_t *orow = a.o + (VARLEN ? row0 * a.o_rs : (int64_t)b * a.o_bs) + (int64_t)qrow * a.o_rs +
@@ -701,12 +894,9 @@ template <int NW, int KS, int HP, bool CAUSAL, bool HAS_BIAS, bool VARLEN>
 void launch_fwd(const FwdArgs &a, int nblocks, hipStream_t stream) {
   constexpr int CW = col_waves<NW, KS>();
   hipLaunchKernelGGL((keybias_fwd_kernel<NW, KS, HP, CAUSAL, HAS_BIAS, VARLEN>), dim3(nblocks), dim3(64 * NW), 0,
-                     stream, a);
+                     stream, a, NoDec{});
   if (a.heavy_blocks > 0) {
-    // chunk groups: up to 8, and at least two chunks per group; CG workgroups of 512 threads per
-    // (split tile, column wave)
-    int cgroups = 1;
-    while (cgroups < kCombineMaxGroups && 2 * cgroups * 2 <= a.ns) cgroups *= 2;
+    const int cgroups = combine_groups(a.ns);   // workgroups of 512 threads per (split tile, column wave)
     const int64_t blocks = a.heavy_blocks / a.ns * CW * cgroups;
     hipLaunchKernelGGL((keybias_fwd_combine_kernel<CW, HP, VARLEN>), dim3((unsigned)blocks), dim3(512), 0, stream, a,
                        cgroups);
@@ -737,8 +927,6 @@ void dispatch_fwd(const FwdArgs &a, int nw, int ks, int hp, bool causal, bool ha
   TG_FWD_CASE(1, false, false)
 #undef TG_FWD_CASE
 }
-
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // The four forms of the kernel: waves per workgroup and key groups.  A CU holds one workgroup of eight
 // waves or two of four.
@@ -1152,4 +1340,113 @@ extern "C" int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q
 extern "C" int64_t tg_keybias_varlen_fwd_workspace_size(int32_t num_seqs, int32_t max_seqlen, int32_t num_heads,
                                                          int32_t num_heads_k, int32_t causal) {
   return fwd_workspace_size(true, num_seqs, max_seqlen, max_seqlen, num_heads, num_heads_k, causal);
+}
+
+namespace tg {
+namespace {
+// A decode step's split: the varlen launch's of one query row per sequence in four-wave workgroups.
+struct DecLayout {
+  int hp;
+  int64_t units, ml, po, bytes;   // byte offsets; the counters come first
+  FwdPlan plan;
+};
+DecLayout decode_layout(int64_t num_seqs, int num_heads, int num_heads_k, int max_k) {
+  DecLayout w{};
+  w.hp = (num_heads / num_heads_k) % 2 == 0 ? 2 : 1;
+  w.units = num_seqs * (num_heads / w.hp);
+  const Tiles t(kForms[1], w.hp, 1, max_k, true);
+  w.plan.nw = 4;
+  w.plan.n_qtiles = 1;
+  w.plan.split = plan_split(kForms[1], t, w.units);
+  const int64_t parts = w.plan.split.heavy_units * w.plan.split.ns * w.hp;
+  w.ml = (w.units * 4 + 255) / 256 * 256;
+  w.po = w.ml + (parts * 8 + 255) / 256 * 256;
+  w.bytes = w.plan.split.ns > 1 ? w.po + parts * 256 : 0;
+  return w;
+}
+}  // namespace
+}  // namespace tg
+
+extern "C" int64_t tg_decode_attention_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_heads_k,
+                                                       int32_t max_seqlen_k) {
+  if (num_seqs <= 0 || num_heads <= 0 || num_heads_k <= 0 || num_heads % num_heads_k != 0 || max_seqlen_k <= 0) return 0;
+  return decode_layout(num_seqs, num_heads, num_heads_k, max_seqlen_k).bytes;
+}
+
+extern "C" int tg_decode_attention(const void *qkv, int64_t qkv_row_stride, const float *rope, int32_t num_seqs,
+                                   int32_t num_heads, int32_t num_heads_k, int32_t head_dim, const void *q_norm_weight,
+                                   const void *k_norm_weight, float eps, const float *q_head_scale,
+                                   const float *q_row_scale, void *k_cache, int64_t k_row_stride, void *v_cache, int64_t v_row_stride, const int32_t *kv_start,
+                                   const int32_t *kv_used, int32_t max_seqlen_k, const float *bias_raw,
+                                   int64_t bias_seq_stride, int64_t bias_head_stride, float softmax_scale, void *out,
+                                   int64_t out_row_stride, void *workspace, int64_t workspace_bytes,
+                                   hipStream_t stream) {
+  clear_error();
+  TG_CHECK(qkv && rope && q_norm_weight && k_norm_weight && k_cache && v_cache && kv_start && kv_used &&
+               out,
+           "decode_attention: null pointer");
+  TG_CHECK(head_dim == kD, "decode_attention: head_dim must be 128");
+  TG_CHECK(num_heads > 0 && num_heads_k > 0 && num_heads <= 256 && num_heads % num_heads_k == 0,
+           "decode_attention: heads must be in 1..256 and a multiple of the KV heads");
+  TG_CHECK(num_seqs >= 0 && max_seqlen_k >= 0, "decode_attention: negative size");
+  TG_CHECK(qkv_row_stride % 8 == 0 && k_row_stride % 8 == 0 && v_row_stride % 8 == 0 &&
+               qkv_row_stride >= (int64_t)(num_heads + 2 * num_heads_k) * kHeadDim &&
+               k_row_stride >= (int64_t)num_heads_k * kHeadDim && v_row_stride >= (int64_t)num_heads_k * kHeadDim &&
+               out_row_stride >= (int64_t)num_heads * kHeadDim,
+           "decode_attention: row strides must be multiples of 8 elements that hold every head");
+  TG_CHECK(aligned16(qkv) && aligned16(k_cache) && aligned16(v_cache) && aligned16(q_norm_weight) &&
+               aligned16(k_norm_weight) && aligned16(rope) && aligned16(workspace),
+           "decode_attention: pointers must be 16-byte aligned");
+  TG_CHECK(softmax_scale > 0.f, "decode_attention: softmax_scale must be positive");
+  if (num_seqs == 0) return 0;
+  TG_CHECK(span_ok(max_seqlen_k, k_row_stride) && span_ok(max_seqlen_k, v_row_stride) &&
+               (bias_raw == nullptr || span_ok(max_seqlen_k + bias_head_stride, 2)),
+           "decode_attention: the k/v/bias rows of one sequence must span less than 4 GiB");
+  const DecLayout w = decode_layout(num_seqs, num_heads, num_heads_k, max_seqlen_k);
+  TG_CHECK(w.bytes == 0 || (workspace != nullptr && workspace_bytes >= w.bytes),
+           "decode_attention: needs a workspace of %lld bytes (got %lld)", (long long)w.bytes, (long long)workspace_bytes);
+  FwdArgs a{};
+  a.k = static_cast<const bf16_t *>(k_cache);
+  a.v = static_cast<const bf16_t *>(v_cache);
+  a.bias = bias_raw;
+  a.o = static_cast<bf16_t *>(out);
+  a.cu_k = kv_start;
+  a.used_k = kv_used;
+  a.k_rs = k_row_stride; a.k_hs = kD;
+  a.v_rs = v_row_stride; a.v_hs = kD;
+  a.o_rs = out_row_stride; a.o_hs = kD;
+  a.bias_bs = bias_seq_stride; a.bias_hs = bias_head_stride;
+  a.batch = num_seqs; a.sq = 1; a.sk = max_seqlen_k;
+  a.h = num_heads; a.hkv = num_heads_k; a.group = num_heads / num_heads_k;
+  a.scale_log2 = softmax_scale * kLog2e;
+  const int64_t nblocks = apply_plan(a, w.plan, w.units, nullptr);
+  TG_CHECK(nblocks < (1ll << 31), "decode_attention: too many sequences");
+  DecArgs d{};
+  d.qkv = static_cast<const bf16_t *>(qkv);
+  d.qkv_rs = qkv_row_stride;
+  d.rope = reinterpret_cast<const float2 *>(rope);
+  d.qw = static_cast<const bf16_t *>(q_norm_weight);
+  d.kw = static_cast<const bf16_t *>(k_norm_weight);
+  d.eps = eps;
+  d.q_head_scale = q_head_scale;
+  d.q_row_scale = q_row_scale;
+  d.k_cache = static_cast<bf16_t *>(k_cache);
+  d.v_cache = static_cast<bf16_t *>(v_cache);
+  if (w.bytes > 0) {
+    char *ws = static_cast<char *>(workspace);
+    d.counters = reinterpret_cast<uint32_t *>(ws);
+    d.ml = reinterpret_cast<uint64_t *>(ws + w.ml);
+    d.po = reinterpret_cast<uint64_t *>(ws + w.po);
+  }
+  const dim3 grid((unsigned)nblocks), block(256);
+  if (w.hp == 2 && bias_raw)
+    hipLaunchKernelGGL((keybias_fwd_kernel<4, 1, 2, true, true, true, true>), grid, block, 0, stream, a, d);
+  else if (w.hp == 2)
+    hipLaunchKernelGGL((keybias_fwd_kernel<4, 1, 2, true, false, true, true>), grid, block, 0, stream, a, d);
+  else if (bias_raw)
+    hipLaunchKernelGGL((keybias_fwd_kernel<4, 1, 1, true, true, true, true>), grid, block, 0, stream, a, d);
+  else
+    hipLaunchKernelGGL((keybias_fwd_kernel<4, 1, 1, true, false, true, true>), grid, block, 0, stream, a, d);
+  TG_HIP_CHECK(hipGetLastError());
+  return 0;
 }

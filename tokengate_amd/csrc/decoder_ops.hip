@@ -5,7 +5,8 @@
 //   * SiLU(gate) * up of the fused gate/up projection;
 //   * for the few rows of a decode step: the projections on the matrix cores, streaming the weight
 //     once, optionally with the RMSNorm or the SwiGLU product folded into their input, or the SwiGLU
-//     product into their output, and the greedy argmax over the logits.
+//     product into their output; the counters and rotary table that its layers share; and the greedy
+//     argmax over the logits.
 // The prefill's projections (many rows) are plain GEMMs and stay on hipBLASLt.
 #include <type_traits>
 
@@ -14,28 +15,6 @@
 
 namespace tg {
 namespace {
-
-__device__ __forceinline__ void unpack8(u32x4 v, float (&f)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = __builtin_bit_cast(float, v[i] << 16);
-    f[2 * i + 1] = __builtin_bit_cast(float, v[i] & 0xffff0000u);
-  }
-}
-__device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
-  u32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = pack_bf16x2(f[2 * i], f[2 * i + 1]);
-  return v;
-}
-__device__ __forceinline__ u32x4 ld16(const bf16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
-__device__ __forceinline__ void st16(bf16_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
-
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) x += __shfl_xor(x, m);
-  return x;
-}
 
 // ---- residual add + RMSNorm: one wave per row, CPL chunks of 8 elements per lane ----------------
 // s = residual ? bf16(x + residual) : x;  residual_out = s;  out = bf16(w * s / sqrt(mean(s^2) + eps))
@@ -86,7 +65,6 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const bf16_t *x, int64_t x
 // 16-lane group takes one 128-element head row at a time (lane j holds elements 8j..8j+7, the
 // rotate-half partner 8j+-64 sits in lane j^8).
 constexpr int kRopeTok = 2;
-constexpr int kHeadDim = 128;
 
 __global__ __launch_bounds__(256) void qk_rope_kernel(const bf16_t *qkv, int64_t qkv_rs,
                                                       const int64_t *__restrict__ pos, int64_t T, int H,
@@ -131,17 +109,6 @@ __global__ __launch_bounds__(256) void qk_rope_kernel(const bf16_t *qkv, int64_t
     float x[8], wf[8];
     unpack8(raw, x);
     unpack8(ld16((is_q ? qw : kw) + 8 * j), wf);
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-    ss += __shfl_xor(ss, 1);
-    ss += __shfl_xor(ss, 2);
-    ss += __shfl_xor(ss, 4);
-    ss += __shfl_xor(ss, 8);
-    const float rinv = rsqrtf(ss * (1.f / kHeadDim) + eps);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = wf[e] * (x[e] * rinv);
-    const float sgn = j < 8 ? -1.f : 1.f;
     // Query multiplier s = bf16(head * row), applied to the bf16-rounded rotated query with one
     // more bf16 rounding: the reference scales its bf16 query states in bf16 (q * s_eff,
     // qwen3_flex_attention.py:442-451, :400).  With no multiplier s = 1 and the second rounding
@@ -150,12 +117,7 @@ __global__ __launch_bounds__(256) void qk_rope_kernel(const bf16_t *qkv, int64_t
                                             (q_row_scale ? q_row_scale[t] : 1.f))
                           : 1.f;
     float y[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float p = __shfl_xor(x[e], 8);
-      const int fi = (8 * j + e) & 63;
-      y[e] = hs * (float)(__bf16)(x[e] * cs[tt][fi][0] + sgn * p * cs[tt][fi][1]);
-    }
+    norm_rope8(x, wf, eps, cs[tt] + 8 * (j & 7), j, hs, y);
     bf16_t *dst = is_q ? q_out + t * q_rs + (int64_t)rr * kHeadDim
                        : k_out + crow * k_rs + (int64_t)(rr - H) * kHeadDim;
     st16(dst + 8 * j, pack8(y));
@@ -504,6 +466,29 @@ __global__ __launch_bounds__(512) void linear_rows_mfma_kernel(LinIn in, const b
   } while (WALK && v0 < n_out);
 }
 
+// ---- start of a decode step -----------------------------------------------------------------------
+// What the layers of a step share, one workgroup per sequence: the position's rotary table (angle =
+// position * inv_freq in fp32, accurate sincosf: tg_qk_norm_rope's, which forms it in every launch), the
+// caches' used counts (+ 1, the new row), the new token's scaled-softmax ratio
+// min(1, ln max(2, slots) / ln max(2, position + 1)), then position (+ 1).
+__global__ __launch_bounds__(64) void decode_begin_kernel(int64_t *pos, const float *__restrict__ inv_freq, float2 *rope,
+                                                          int32_t *used, int n_used, float *slots, float *ratio) {
+  const int b = blockIdx.x, nseq = gridDim.x, t = threadIdx.x;
+  const int64_t p = pos[b];   // one wave: read before lane 0 raises it
+  float s, c;
+  sincosf((float)p * inv_freq[t], &s, &c);
+  rope[b * (kHeadDim / 2) + t] = float2{c, s};
+  for (int i = t; i < n_used; i += 64) used[i * nseq + b] += 1;
+  if (t == 0) {
+    if (slots) {
+      const float m = slots[b] + 1.f;
+      slots[b] = m;
+      ratio[b] = fminf(1.f, logf(fmaxf(m, 2.f)) / logf(fmaxf((float)p + 1.f, 2.f)));
+    }
+    pos[b] = p + 1;
+  }
+}
+
 // ---- Greedy token: the index of each row's largest logit -----------------------------------------
 // torch.argmax semantics: a NaN beats every number, and equal values go to the lower index.  One
 // 1024-thread workgroup per row: each thread scans its strided 16-byte pieces, then the (value,
@@ -561,8 +546,6 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float *__restri
     out[blockIdx.x] = bi;
   }
 }
-
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
 }  // namespace tg
@@ -875,6 +858,19 @@ extern "C" int tg_argmax_rows(const float *x, int64_t x_row_stride, int32_t n_ro
   TG_CHECK(aligned16(x), "argmax_rows: x must be 16-byte aligned");
   if (n_rows == 0) return 0;
   hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)n_rows), dim3(1024), 0, stream, x, x_row_stride, n_cols, out);
+  TG_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int tg_decode_begin(int64_t *positions, int32_t num_seqs, const float *inv_freq, float *rope,
+                               int32_t *kv_used, int32_t n_used, float *slots, float *ratio, hipStream_t stream) {
+  clear_error();
+  TG_CHECK(positions && inv_freq && rope && (kv_used || n_used == 0) && (ratio || !slots), "decode_begin: null pointer");
+  TG_CHECK(num_seqs >= 0 && n_used >= 0, "decode_begin: negative size");
+  TG_CHECK(aligned16(rope), "decode_begin: rope must be 16-byte aligned");
+  if (num_seqs == 0) return 0;
+  hipLaunchKernelGGL(decode_begin_kernel, dim3((unsigned)num_seqs), dim3(64), 0, stream, positions, inv_freq,
+                     reinterpret_cast<float2 *>(rope), kv_used, n_used, slots, ratio);
   TG_HIP_CHECK(hipGetLastError());
   return 0;
 }

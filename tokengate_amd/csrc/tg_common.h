@@ -272,6 +272,57 @@ __device__ __forceinline__ float bf16_to_f32(bf16_t x) {
   return __builtin_bit_cast(float, (uint32_t)x << 16);
 }
 
+// ---- rows of bf16 in 16-byte pieces -------------------------------------------------------------
+__device__ __forceinline__ void unpack8(u32x4 v, float (&f)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = __builtin_bit_cast(float, v[i] << 16);
+    f[2 * i + 1] = __builtin_bit_cast(float, v[i] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
+  u32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = pack_bf16x2(f[2 * i], f[2 * i + 1]);
+  return v;
+}
+__device__ __forceinline__ u32x4 ld16(const bf16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+__device__ __forceinline__ void st16(bf16_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
+
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) x += __shfl_xor(x, m);
+  return x;
+}
+
+
+// RMSNorm and rotary embedding of one 128-element head row held by 16 lanes: lane j has elements 8j ..
+// 8j+7 in x and their norm weights in wf, the rotate-half partner 8j+-64 sits in lane j^8; cs[e] is
+// (cos, sin) of frequency (8j + e) % 64.  y = hs * bf16(rotated), rounded by the caller.  The fused
+// multiply-adds are written out, so that every kernel that rotates a row gets the same bits.
+constexpr int kHeadDim = 128;
+__device__ __forceinline__ void norm_rope8(float (&x)[8], const float (&wf)[8], float eps,
+                                           const float (*cs)[2], int j, float hs, float (&y)[8]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+  ss += __shfl_xor(ss, 1);
+  ss += __shfl_xor(ss, 2);
+  ss += __shfl_xor(ss, 4);
+  ss += __shfl_xor(ss, 8);
+  const float rinv = rsqrtf(ss * (1.f / kHeadDim) + eps);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = wf[e] * (x[e] * rinv);
+  const float sgn = j < 8 ? -1.f : 1.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float p = __shfl_xor(x[e], 8);
+    y[e] = hs * (float)(__bf16)fmaf(x[e], cs[e][0], sgn * p * cs[e][1]);
+  }
+}
+
+inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // Estimated time, in microseconds, of a launch of `units` times n workgroups issued heaviest first to
 // `slots` places; steps(r) is the work of the r-th heaviest.  A workgroup takes `wg` plus `full` per step
 // while the chip is full and `solo` while the longest run on alone, so the launch takes at least its

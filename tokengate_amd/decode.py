@@ -10,13 +10,12 @@ produced EOS, and answers are cut at the first EOS (gate_decode.py:241-257).
 
 Cache layout: the prefill run with decode_headroom >= the steps to come leaves every layer's
 cache with that many free rows after each sequence (decoder.CacheGap), and the decode appends in
-place: each step's new K/V rows are written by the q/k-norm + RoPE kernel straight into row
-seg[b] + used[b] of each sequence's segment, and each layer's attention is ONE varlen launch
-(tg_keybias_varlen_kv_fwd) with one query row per sequence over its segment's used rows.  A
+place: each layer's q/k norm, RoPE, cache append (row seg[b] + used[b] of each sequence's segment)
+and attention over its segment's used rows are ONE launch (tg_decode_attention).  A
 prefill without enough headroom is re-laid out once (one copy per layer) into that layout.
 The per-step counters live on the device, so nothing in a step synchronises with the host, and
 every step launches the same kernels with the same arguments: with graph=True the second and
-later steps replay one captured HIP graph of the whole step (about 250 launches), whose inputs
+later steps replay one captured HIP graph of the whole step (about 150 launches), whose inputs
 and outputs are static device buffers; the first step runs eagerly and warms every kernel and
 library handle the capture records.
 """
@@ -26,9 +25,9 @@ from typing import List, Optional
 
 import torch
 
-from tokengate_amd.decoder import (CacheGap, DecoderWeights, LayerKV, argmax_rows, h2d, linear_rows, linear_rows_norm,
-                                   linear_rows_norm_act, logits_last, qk_norm_rope, rmsnorm, silu_mul,
-                                   varlen_kv_attention)
+from tokengate_amd.decoder import (CacheGap, DecoderWeights, LayerKV, argmax_rows, decode_attention,
+                                   decode_attention_workspace, decode_begin, h2d, linear_rows, linear_rows_norm,
+                                   linear_rows_norm_act, logits_last, rmsnorm, silu_mul)
 from tokengate_amd.gate import ScoringHead
 from tokengate_amd.prefill import PrefillResult
 
@@ -102,11 +101,11 @@ class DecodeState:
         last = torch.tensor([pf.cu_kept[b + 1] - 1 for b in range(B)], dtype=torch.int64)
         self.next_pos = pf.kept_positions.index_select(0, h2d(last, dev)) + 1
         self.ssmax = pf.kept_ratio is not None
-        self.n_kept_f = h2d(torch.tensor([float(x) for x in pf.n_kept], dtype=torch.float32), dev)
-        self.cu_q = torch.arange(B + 1, dtype=torch.int32, device=dev)
+        # cache slots of the Phase-2 layers, the new token's included once a step has begun
+        self.slots = h2d(torch.tensor([float(x) for x in pf.n_kept], dtype=torch.float32), dev) if self.ssmax else None
+        self.att_ws = decode_attention_workspace(B, shape, max(self.cap_k), dev)
         self.rows_b = torch.arange(B, device=dev)
         self.steps = 0
-        self.step_f = torch.zeros((), dtype=torch.float32, device=dev)   # steps taken, on the device
         self.max_new_tokens = max_new_tokens
         self.use_graph = graph
         self.fused = fused
@@ -146,14 +145,9 @@ class DecodeState:
         hid = torch.empty_like(x)
         qkv = torch.empty(B, s.qkv_dim, dtype=x.dtype, device=dev)
         att = torch.empty(B, s.n_heads, s.head_dim, dtype=x.dtype, device=dev)
-        lse = torch.empty(s.n_heads, B, dtype=torch.float32, device=dev)
-        rows = self.seg_dev + self.used          # the new token's cache row in each group, (2, B)
-        self.used += 1
-        r_dec = None
-        if self.ssmax:   # the new token's own ratio: slot n_kept + 1 + step at position next_pos
-            m = (self.n_kept_f + 1.0 + self.step_f).clamp(min=2.0)
-            p = (self.next_pos.to(torch.float32) + 1.0).clamp(min=2.0)
-            r_dec = (torch.log(m) / torch.log(p)).clamp(max=1.0)
+        # the rotary table of the new token's position, its cache rows and its own scaled-softmax ratio
+        # (slot n_kept + 1 + step at position next_pos); all counters are raised
+        rope, r_dec = decode_begin(self.next_pos, w.inv_freq, self.used, self.slots)
         scale = 1.0 / math.sqrt(s.head_dim)
         if fused:
             # each norm is folded into the projection after it, and the SwiGLU product into the
@@ -176,11 +170,10 @@ class DecodeState:
             if not fused:
                 linear_rows(normed, lw.w_qkv, out=qkv)
             kv = self.kv[l]
-            q = qk_norm_rope(qkv, self.next_pos, lw, s, w.inv_freq, kv.k, kv.v,
+            decode_attention(qkv, rope, lw, s, kv.k, kv.v, self.seg_dev[g], self.used[g],
+                             self.cap_k[g], scale, self.att_ws, self.bias[j] if g else None,
                              self.qscale[j] if (g and self.qscale is not None) else None,
-                             r_dec if (r_dec is not None and g) else None, kv_rows=rows[g])
-            varlen_kv_attention(q, kv.k, kv.v, self.cu_q, self.seg_dev[g], self.used[g], 1, self.cap_k[g], scale,
-                                self.bias[j] if g else None, out=att, lse=lse)
+                             r_dec if (r_dec is not None and g) else None, out=att)
             linear_rows(att.view(B, -1), lw.w_o, out=hid)
             if fused:
                 act = linear_rows_norm_act(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur], residual_out=rbuf[1 - cur])
@@ -190,8 +183,6 @@ class DecodeState:
                 rmsnorm(hid, lw.ln2, s.rms_eps, residual=res, residual_out=res, out=normed)
                 act = silu_mul(linear_rows(normed, lw.w_gu))
                 linear_rows(act, lw.w_down, out=hid)
-        self.next_pos += 1
-        self.step_f += 1.0
         if fused:   # every row produces a token: the final norm folds into the LM head
             logits = linear_rows_norm(hid, w.final_norm, s.rms_eps, w.lm_head, residual=rbuf[cur], out_fp32=True)
         else:

@@ -222,6 +222,71 @@ def varlen_kv_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_q:
     return out
 
 
+def decode_attention_workspace(n_seqs: int, shape: DecoderShape, max_k: int, device) -> torch.Tensor:
+    """Zeroed workspace for decode_attention calls of up to max_k keys (its counters stay zero between calls)."""
+    n = int(_lib.load().tg_decode_attention_workspace_size(n_seqs, shape.n_heads, shape.n_kv_heads, int(max_k)))
+    return torch.zeros(max(n, 16), dtype=torch.uint8, device=device)
+
+
+def decode_begin(positions: torch.Tensor, inv_freq: torch.Tensor, kv_used: Optional[torch.Tensor] = None,
+                 slots: Optional[torch.Tensor] = None):
+    """Starts a decode step at positions (B,) int64, which it raises by one (tg_decode_begin): returns
+    the rotary table (B, 64, 2) fp32 for decode_attention and, with slots (B,) fp32 (raised by one), the
+    new token's scaled-softmax ratio (B,), else None; kv_used (groups, B) int32 is raised by one."""
+    B = positions.numel()
+    if positions.dtype != torch.int64 or not positions.is_contiguous() or inv_freq.numel() != 64 \
+            or inv_freq.dtype != torch.float32:
+        raise RuntimeError("decode_begin: positions must be contiguous int64, inv_freq 64 fp32 frequencies")
+    if kv_used is not None and (kv_used.dtype != torch.int32 or not kv_used.is_contiguous() or kv_used.shape[-1] != B):
+        raise RuntimeError("decode_begin: kv_used must be contiguous int32 (groups, B)")
+    if slots is not None and (slots.dtype != torch.float32 or not slots.is_contiguous() or slots.numel() != B):
+        raise RuntimeError("decode_begin: slots must be contiguous fp32 (B,)")
+    rope = torch.empty(B, 64, 2, dtype=torch.float32, device=positions.device)
+    ratio = torch.empty(B, dtype=torch.float32, device=positions.device) if slots is not None else None
+    _lib.call("tg_decode_begin", positions.data_ptr(), B, inv_freq.data_ptr(), rope.data_ptr(),
+              kv_used.data_ptr() if kv_used is not None else None, kv_used.numel() // B if kv_used is not None and B else 0,
+              slots.data_ptr() if slots is not None else None, ratio.data_ptr() if ratio is not None else None,
+              _stream(positions))
+    return rope, ratio
+
+
+def decode_attention(qkv: torch.Tensor, rope: torch.Tensor, lw: LayerWeights, shape: DecoderShape, k: torch.Tensor, v: torch.Tensor, kv_start: torch.Tensor,
+                     kv_used: torch.Tensor, max_k: int, scale: float, workspace: torch.Tensor,
+                     bias_raw: Optional[torch.Tensor] = None, q_head_scale: Optional[torch.Tensor] = None,
+                     q_row_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """qk_norm_rope and varlen_kv_attention of one row per sequence in one launch (tg_decode_attention), at
+    the positions of decode_begin's rotary table:
+    the new key of sequence b goes to cache row kv_start[b] + kv_used[b] - 1 and its query attends over
+    rows kv_start[b] .. kv_start[b] + kv_used[b] - 1; bias_raw (nseq, H, >= max_k) as varlen_kv_attention."""
+    B = qkv.shape[0]
+    H, Hkv, D = shape.n_heads, shape.n_kv_heads, shape.head_dim
+    out = torch.empty(B, H, D, dtype=qkv.dtype, device=qkv.device) if out is None else out
+    if rope.dtype != torch.float32 or rope.numel() != B * D or not rope.is_contiguous():
+        raise RuntimeError("decode_attention: rope must be contiguous fp32 (B, 64, 2)")
+    for t in (kv_start, kv_used):
+        if t.dtype != torch.int32 or not t.is_contiguous() or t.numel() < B:
+            raise RuntimeError("decode_attention: kv_start and kv_used must be contiguous int32, an entry per sequence")
+    for t in (k, v):
+        if t.stride(-1) != 1 or t.stride(-2) != D:
+            raise RuntimeError("decode_attention: cache rows must hold the heads back to back")
+    if out.stride(-1) != 1 or out.stride(-2) != D or qkv.stride(1) != 1:
+        raise RuntimeError("decode_attention: qkv and out rows must be contiguous")
+    if q_row_scale is not None and (q_row_scale.dtype != torch.float32 or q_row_scale.numel() < B):
+        raise RuntimeError("decode_attention: q_row_scale must be fp32 with one entry per sequence")
+    if bias_raw is not None and (bias_raw.dtype != torch.float32 or bias_raw.stride(-1) != 1
+                                 or bias_raw.shape[-1] < max_k):
+        raise RuntimeError("decode_attention: bias must be fp32 with a contiguous key axis of >= max_k")
+    _lib.call("tg_decode_attention", qkv.data_ptr(), qkv.stride(0), rope.data_ptr(), B, H, Hkv, D,
+              lw.q_norm.data_ptr(), lw.k_norm.data_ptr(), float(shape.rms_eps),
+              q_head_scale.data_ptr() if q_head_scale is not None else None,
+              q_row_scale.data_ptr() if q_row_scale is not None else None,
+              k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), kv_start.data_ptr(), kv_used.data_ptr(), int(max_k),
+              bias_raw.data_ptr() if bias_raw is not None else None,
+              bias_raw.stride(0) if bias_raw is not None else 0, bias_raw.stride(1) if bias_raw is not None else 0,
+              float(scale), out.data_ptr(), out.stride(0), workspace.data_ptr(), workspace.numel(), _stream(qkv))
+    return out
+
+
 # ---- layer runner ------------------------------------------------------------------------------
 
 @dataclass
