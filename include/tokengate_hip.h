@@ -363,7 +363,7 @@ int tg_linear_rows_norm(const void *h, int64_t h_row_stride, const void *residua
 
 /* tg_linear_rows_norm of a fused gate|up projection with the SwiGLU product formed on the way out:
  * weight (2 * inter, dim) bf16 = [gate_proj; up_proj], out (n_rows, inter) = bf16(silu(g) * u) of the
- * bf16 projections g and u, as tg_linear_rows_norm followed by tg_silu_mul computes it —
+ * bf16 projections g and u, as tg_linear_rows_norm followed by tg_silu_mul computes it (dim <= 2048) —
  * post_attention_layernorm and the first half of Qwen3MLP in the decode step (gate_decode.py:210-226). */
 int tg_linear_rows_norm_act(const void *h, int64_t h_row_stride, const void *residual, int64_t residual_row_stride,
                             void *residual_out, int64_t residual_out_row_stride, const void *norm_weight, float eps,

@@ -223,7 +223,7 @@ def test_linear_rows_swiglu_long_rows(cuda, rows, n_out, inter):
     assert torch.equal(got, ref)
 
 
-@pytest.mark.parametrize("rows,inter,dim", [(1, 6144, 2048), (8, 6144, 2048), (2, 1027, 512), (3, 5, 2560), (7, 40000, 2048)])
+@pytest.mark.parametrize("rows,inter,dim", [(1, 6144, 2048), (8, 6144, 2048), (2, 1027, 512), (3, 5, 1536), (7, 40000, 2048)])
 def test_linear_rows_norm_act(cuda, rows, inter, dim):
     """The gate|up projection with the SwiGLU product formed on the way out equals the norm-fused
     projection followed by silu_mul bit for bit (the SwiGLU kernel reads rows of whole 16-byte
@@ -246,6 +246,8 @@ def test_linear_rows_norm_act(cuda, rows, inter, dim):
         f = gu.double()
         ref = torch.nn.functional.silu(f[:, :inter]) * f[:, inter:]
         assert bool(((got.double() - ref).abs() <= torch.finfo(torch.bfloat16).eps * ref.abs() + 1e-12).all())
+    with pytest.raises(RuntimeError, match="2048"):
+        dec.linear_rows_norm_act(torch.zeros(1, 2560, dtype=torch.bfloat16, device=cuda), nw, 1e-6, w.new_zeros(8, 2560))
 
 
 @pytest.mark.parametrize("rows,V", [(1, 151936), (3, 1001), (8, 151936)])

@@ -3,10 +3,10 @@
 //   * per-head q/k RMSNorm + rotary embedding at each token's own position, writing q in place
 //     and k / v into the layer's KV cache rows,
 //   * SiLU(gate) * up of the fused gate/up projection;
-//   * for the few rows of a decode step: the projections on the matrix cores, streaming the weight
-//     once, optionally with the RMSNorm or the SwiGLU product folded into their input, or the SwiGLU
-//     product into their output; the counters and rotary table that its layers share; and the greedy
-//     argmax over the logits.
+//   * for the few rows of a decode step: the projections, HBM-bound on the weight (a row form for rows of
+//     up to 2048 inputs, a split-K form for longer ones), optionally with the RMSNorm or the SwiGLU
+//     product folded into their input, or the SwiGLU product into their output; the counters and
+//     rotary table that its layers share; and the greedy argmax over the logits.
 // The prefill's projections (many rows) are plain GEMMs and stay on hipBLASLt.
 #include <type_traits>
 
@@ -234,236 +234,291 @@ __device__ __forceinline__ u32x4 lin_input(const LinIn &in, int b, int c, float 
     return norm8(pack8(v), ld16(in.nw + c), rinv);   // (v is exact in bf16)
   }
 }
-// A workgroup (8 waves) owns RB blocks of 8 output rows; wave w takes the 64-column pieces w, w + 8,
-// w + 16, ... of the inner dimension, so that every request of a wave is 8 whole 128-byte lines and,
-// with all of a wave's pieces requested before the first product (NK of them, when dim = 512 NK), the
-// workgroup's whole slice of the weight is in flight at once.  One MFMA (16x16x32) takes a piece of a
-// block: rows 0..7 of its A operand are the block's weights at the piece's first 32 columns and rows
-// 8..15 the same output rows at the other 32; the columns of B are the (up to 8) input rows in the
-// same two halves.  The diagonal quarters of the result hold the two halves' sums, the other two are
-// not used.  Each input element is read once per workgroup, by the one lane that feeds it to the
-// matrix core.  The dot products used to run on the VALU, each wave reading all input rows for 4
-// output rows: twice the weight's bytes at 8 rows.  Before -> now, weights from HBM, at 1 / 8 rows
-// (us): 4096 x 2048 with the norm 6.9 / 14.5 -> 5.3 / 7.0, 2048 x 2048 4.3 / 8.3 -> 3.9 / 4.4,
-// 12288 x 2048 with the norm 12.4 / 28.6 -> 11.8 / 13.4 (with the SwiGLU product on the way out 11.0 /
-// 13.6), 2048 x 6144 6.3 / 12.1 -> 6.6 / 8.2, 151936 x 2048 with the norm 109 / 250 -> 104 / 112 (6.0 /
-// 5.6 TB/s).  WALK: fewer workgroups than blocks, which walk them with the next blocks' weights in flight
-// (only where a launch has that many: the second set of weight registers costs a 2048 x 6144 launch of
-// one block per workgroup 6.6 -> 7.6 us).
-template <int RB, int NK, typename OutT, int PRE, bool ACT, bool WALK>
-__global__ __launch_bounds__(512) void linear_rows_mfma_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
-                                                               int dim, int nr, OutT *__restrict__ out,
-                                                               int64_t out_rs) {
-  constexpr int kWaves = 8, NKR = NK > 0 ? NK : 1;
-  constexpr bool kStage = PRE == kPreNorm && NK == 4;   // dim = 2048
-  constexpr bool kStageAct = PRE == kPreSwiGLU && NK > 0;   // each wave forms its own pieces, in LDS
-  constexpr int kXsRow = kStageAct ? 64 * NK + 8 : 2048 + 8;   // padded: 8 rows' 16-byte reads on different banks
-  __shared__ __attribute__((aligned(16))) bf16_t xs[kStage ? 8 * kXsRow : kStageAct ? kWaves * 8 * kXsRow : 8];
-  __shared__ __attribute__((aligned(16))) float part2[WALK ? 2 : 1][kWaves][RB][2][64];
+// The order of every sum is fixed: lane l of a wave takes columns 8 l .. 8 l + 7 of each 512-column chunk,
+// chunk by chunk, as bf16 pair dot products, and the 64 lanes are added as a butterfly.  (Other orders,
+// the matrix cores' among them, flip about 1 in 5000 of the rounded outputs, which 28 layers of bf16 turn
+// into 3 % of the logits.)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+// Butterfly sum over the 64 lanes (x += x[l ^ 1], ^ 2, ^ 4, ... ^ 32) without the LDS crossbar: pairs
+// inside a quad, then mirrored halves of 8 and 16 lanes (whose quads / octets already agree), then the
+// row swaps.  Same additions, so the same bits as wave_sum.
+__device__ __forceinline__ float wave_sum_dpp(float x) {
+  x += dpp<0xB1>(x);    // quad_perm 1 0 3 2
+  x += dpp<0x4E>(x);    // quad_perm 2 3 0 1
+  x += dpp<0x141>(x);   // row_half_mirror
+  x += dpp<0x140>(x);   // row_mirror
+  {
+    const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+                                                     false, false);
+    const uint32_t lo = sw[0], hi = sw[1];
+    x = u32_as_f32(lo) + u32_as_f32(hi);
+  }
+  const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+                                                   false, false);
+  const uint32_t lo = sw[0], hi = sw[1];
+  return u32_as_f32(lo) + u32_as_f32(hi);
+}
+// acc[r][b] += the 8 columns of weight row r times those of input row b
+template <int RW>
+__device__ __forceinline__ void lin_dot8(const u32x4 (&wv)[RW], u32x4 xv, float (&acc)[RW]) {
+#pragma unroll
+  for (int r = 0; r < RW; ++r)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t wd = wv[r][e], xd = xv[e];   // scalar copies: see u32_as_f32
+      acc[r] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wd), __builtin_bit_cast(bf16x2, xd), acc[r],
+                                               false);
+    }
+}
+template <typename OutT>
+__device__ __forceinline__ void lin_store(OutT *p, float sum) {
+  const __bf16 y = (__bf16)sum;
+  if constexpr (std::is_same<OutT, float>::value) *p = (float)y;
+  else *p = __builtin_bit_cast(bf16_t, y);
+}
+// Rows of at most 2048 inputs (512 NC; NC = 0: any multiple of 512).  A workgroup of 8 waves, each wave
+// RW weight rows (ACT: RW / 2 outputs, their gate and up rows) per round.  The NR input rows are formed
+// once per workgroup in LDS, requested before the weights (loads complete in issue order, so the stage
+// runs while the weights stream in).  Before, workgroups of 16 rows formed them (or every wave read them
+// for 4 rows: twice the weight's bytes at 8 input rows) and each of the 4 NR sums took six steps through
+// the LDS crossbar.  Before -> now, weights from HBM, at 1 / 8 input rows (us): 4096 x 2048 with the norm
+// 6.9 / 14.5 -> 4.9 / 8.4, 2048 x 2048 4.3 / 8.3 -> 3.3 / 4.6, 12288 x 2048 with the norm 12.4 / 28.6 ->
+// 10.6 / 14.5 (and with the SwiGLU product 10.4 / 14.1), 151936 x 2048 with the norm 109 / 250 -> 104 /
+// 123 (6.0 / 5.1 TB/s).  WALK: fewer workgroups than blocks, which walk them with the
+// next round's weights in flight, so that the input stage is paid once for more of the weight.
+template <int NR, int RW, int NC, typename OutT, int PRE, bool ACT, bool WALK>
+__global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
+                                                          int dim, OutT *__restrict__ out, int64_t out_rs) {
+  static_assert(!WALK || NC > 0, "the next round's weights are held in registers");
+  constexpr int kXsRow = 2048, OW = ACT ? RW / 2 : RW, NCR = NC > 0 ? NC : 1, kIn = (NR + 1) / 2;
+  __shared__ __attribute__((aligned(16))) bf16_t xs[NR * kXsRow];
   __shared__ float rinv_s[8];
   const int lane = threadIdx.x & 63, wv = wave_id();
-  const int c = lane & 7, G = lane >> 4;
-  const int xr = min(c, nr - 1);                         // input rows past nr repeat the last (not stored)
-  const int kl = 64 * wv + 32 * ((lane >> 3) & 1) + 8 * G;
-  constexpr int OB = ACT ? RB / 2 : RB;                  // blocks of stored rows
-  const bf16_t *wr[RB];
-  auto rows_from = [&](int64_t v0) {
+  const int groups = NC > 0 ? 64 * NC : dim / 8;   // 16-byte pieces of a row
+  u32x4 xin[kIn], rin[kIn], nwv[kIn];
+  int row[kIn], col[kIn];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      // rows past the end read the last row (in bounds; not stored)
-      const int64_t v = min(v0 + 8 * (rb % OB) + c, n_out - 1);
-      wr[rb] = w + (v + (rb / OB) * n_out) * dim + kl;
-    }
-  };
-  const int64_t step = (int64_t)gridDim.x * (8 * OB);
-  int64_t v0 = (int64_t)blockIdx.x * (8 * OB);
-  rows_from(v0);
-  // inputs are requested before the weights: loads complete in issue order, so the input stage runs
-  // while the weight bytes stream in
-  u32x4 xin[NKR], rin[NKR], nwv[NKR], wf[NKR][RB];
-  u32x4 sx[kStage ? 4 : 1], sr[kStage ? 4 : 1];
-  if constexpr (NK > 0) {
-    if constexpr (PRE == kPrePlain) {
-#pragma unroll
-      for (int s = 0; s < NK; ++s) xin[s] = ld16(in.x + xr * in.x_rs + kl + 512 * s);
-    } else if constexpr (kStageAct) {
-      // the wave's 8 NK chunks of every row, once each (NK rounds at 8 rows)
-#pragma unroll
-      for (int s = 0; s < NK; ++s) {
-        const int idx = lane + 64 * s, b = idx / (8 * NK), j = idx % (8 * NK);
-        if (b < nr) {
-          const bf16_t *p = in.x + b * in.x_rs + 64 * wv + 512 * (j >> 3) + 8 * (j & 7);
-          xin[s] = ld16(p);
-          rin[s] = ld16(p + in.inter);
-        }
+  for (int i = 0; i < kIn; ++i) {
+    const int idx = threadIdx.x + 512 * i;
+    row[i] = idx / groups;
+    col[i] = 8 * (idx - row[i] * groups);
+    if (row[i] < NR) {
+      xin[i] = ld16(in.x + row[i] * in.x_rs + col[i]);
+      if constexpr (PRE == kPreNorm) {
+        if (in.res) rin[i] = ld16(in.res + row[i] * in.res_rs + col[i]);
+        nwv[i] = ld16(in.nw + col[i]);
+      } else if constexpr (PRE == kPreSwiGLU) {
+        rin[i] = ld16(in.x + row[i] * in.x_rs + in.inter + col[i]);
       }
-    } else if constexpr (kStage) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = threadIdx.x + 512 * i, b = idx >> 8, ch = 8 * (idx & 255);
-        if (b < nr) {
-          sx[i] = ld16(in.x + b * in.x_rs + ch);
-          if (in.res) sr[i] = ld16(in.res + b * in.res_rs + ch);
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < NK; ++s) nwv[s] = ld16(in.nw + kl + 512 * s);
     }
-#pragma unroll
-    for (int s = 0; s < NK; ++s)
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) wf[s][rb] = ld16(wr[rb] + 512 * s);
   }
-  float rinv = 0.f;
+  const int64_t step = (int64_t)gridDim.x * (8 * OW);
+  int64_t v0 = ((int64_t)blockIdx.x * 8 + wv) * OW;
+  const bf16_t *wr[RW];
+  auto rows_from = [&](int64_t v) {   // rows past the end read the last row (in bounds; not stored)
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+      wr[r] = w + (min(v + r % OW, n_out - 1) + (r / OW) * n_out) * dim + 8 * lane;
+  };
+  auto load = [&](u32x4 (&wf)[RW], int ch) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) wf[r] = ld16(wr[r] + 512 * ch);
+  };
+  rows_from(v0);
+  u32x4 wf[NCR][RW];
+  if constexpr (NC > 0)
+#pragma unroll
+    for (int ch = 0; ch < NC; ++ch) load(wf[ch], ch);
+  // ---- input stage ----
   if constexpr (PRE == kPreNorm) {
+    // s = bf16(h + res) to LDS (block 0 also writes res_out), wave b the sum of row b's squares in the
+    // RMSNorm kernel's order (lane l its pieces l, l + 64, ... element by element, then the butterfly),
+    // then every thread scales its own pieces in place
     const bool writer = blockIdx.x == 0 && in.res_out != nullptr;
-    if constexpr (kStage) {
-      // s = bf16(h + res) to LDS (block 0 also writes res_out), then wave b sums row b's squares in
-      // the RMSNorm kernel's order (lane l its chunks l, l + 64, ..., then the wave butterfly)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int idx = threadIdx.x + 512 * i, b = idx >> 8, ch = 8 * (idx & 255);
-        if (b < nr) {
-          float v[8];
-          unpack8(sx[i], v);
-          if (in.res) {
-            float r[8];
-            unpack8(sr[i], r);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
-          }
-          const u32x4 pv = pack8(v);
-          if (writer) st16(in.res_out + b * in.ro_rs + ch, pv);
-          *reinterpret_cast<u32x4 *>(xs + b * kXsRow + ch) = pv;
-        }
-      }
-      __syncthreads();
-      if (wv < nr) {
-        float ss = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float v[8];
-          unpack8(*reinterpret_cast<const u32x4 *>(xs + wv * kXsRow + 8 * lane + 512 * i), v);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-        }
-        ss = wave_sum(ss);
-        if (lane == 0) rinv_s[wv] = rsqrtf(ss / (float)dim + in.eps);
-      }
-    } else if (wv < nr) {
-      float ss = 0.f;
-      for (int ch = 8 * lane; ch < dim; ch += 512) {
+    for (int i = 0; i < kIn; ++i)
+      if (row[i] < NR) {
         float v[8];
-        unpack8(ld16(in.x + wv * in.x_rs + ch), v);
+        unpack8(xin[i], v);
         if (in.res) {
           float r[8];
-          unpack8(ld16(in.res + wv * in.res_rs + ch), r);
+          unpack8(rin[i], r);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
         }
-        if (writer) st16(in.res_out + wv * in.ro_rs + ch, pack8(v));
+        xin[i] = pack8(v);
+        if (writer) st16(in.res_out + row[i] * in.ro_rs + col[i], xin[i]);
+        *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = xin[i];
+      }
+    ring_barrier();
+    if (wv < NR) {
+      float ss = 0.f;
+      for (int c = 8 * lane; c < dim; c += 512) {
+        float v[8];
+        unpack8(*reinterpret_cast<const u32x4 *>(xs + wv * kXsRow + c), v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
       }
-      ss = wave_sum(ss);
+      ss = wave_sum_dpp(ss);
       if (lane == 0) rinv_s[wv] = rsqrtf(ss / (float)dim + in.eps);
     }
-    __syncthreads();
-    rinv = rinv_s[xr];
-  }
-  if constexpr (kStageAct) {
+    ring_barrier();
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const int idx = lane + 64 * s, b = idx / (8 * NK), j = idx % (8 * NK);
-      if (b < nr) *reinterpret_cast<u32x4 *>(xs + (8 * wv + b) * kXsRow + 8 * j) = swiglu8(xin[s], rin[s]);
-    }
-    // only this wave reads its part: its LDS operations complete in order
-  }
-  u32x4 xf[NKR];
-  if constexpr (NK > 0) {
+    for (int i = 0; i < kIn; ++i)
+      if (row[i] < NR) *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = norm8(xin[i], nwv[i], rinv_s[row[i]]);
+  } else {
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      if constexpr (PRE == kPrePlain)
-        xf[s] = xin[s];
-      else if constexpr (kStageAct)
-        xf[s] = *reinterpret_cast<const u32x4 *>(xs + (8 * wv + xr) * kXsRow + 64 * s + (kl - 64 * wv));
-      else if constexpr (kStage)
-        xf[s] = norm8(*reinterpret_cast<const u32x4 *>(xs + xr * kXsRow + kl + 512 * s), nwv[s], rinv);
-      else
-        xf[s] = lin_input<PRE>(in, xr, kl + 512 * s, rinv);
-    }
+    for (int i = 0; i < kIn; ++i)
+      if (row[i] < NR)
+        *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = PRE == kPreSwiGLU ? swiglu8(xin[i], rin[i]) : xin[i];
   }
-  int buf = 0;
+  ring_barrier();
+  // ---- rounds ----
+  auto xrow = [&](int b, int ch) { return *reinterpret_cast<const u32x4 *>(xs + b * kXsRow + 512 * ch + 8 * lane); };
   do {
-    f32x4 acc[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (NK > 0) {
-      // the next blocks' weights are requested before these are used
-      u32x4 wn[WALK ? NK : 1][RB];
+    if (!WALK && v0 >= n_out) return;   // (no barrier follows)
+    float acc[NR][RW] = {};
+    if constexpr (NC > 0) {
+      u32x4 wn[WALK ? NC : 1][RW];
       if (WALK && v0 + step < n_out) {
         rows_from(v0 + step);
 #pragma unroll
-        for (int s = 0; s < NK; ++s)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) wn[s][rb] = ld16(wr[rb] + 512 * s);
+        for (int ch = 0; ch < NC; ++ch) load(wn[ch], ch);
       }
 #pragma unroll
-      for (int s = 0; s < NK; ++s)
+      for (int ch = 0; ch < NC; ++ch)
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-          acc[rb] = mfma16(__builtin_bit_cast(bf16x8, wf[s][rb]), __builtin_bit_cast(bf16x8, xf[s]), acc[rb]);
+        for (int b = 0; b < NR; ++b) lin_dot8(wf[ch], xrow(b, ch), acc[b]);
       if constexpr (WALK)
 #pragma unroll
-        for (int s = 0; s < NK; ++s)
+        for (int ch = 0; ch < NC; ++ch)
 #pragma unroll
-          for (int rb = 0; rb < RB; ++rb) wf[s][rb] = wn[s][rb];
+          for (int r = 0; r < RW; ++r) wf[ch][r] = wn[ch][r];
     } else {
-      for (int k = 0; k < dim; k += 512) {
+      for (int ch = 0; 512 * ch < dim; ++ch) {
+        load(wf[0], ch);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) wf[0][rb] = ld16(wr[rb] + k);
-        const u32x4 x = lin_input<PRE>(in, xr, kl + k, rinv);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-          acc[rb] = mfma16(__builtin_bit_cast(bf16x8, wf[0][rb]), __builtin_bit_cast(bf16x8, x), acc[rb]);
+        for (int b = 0; b < NR; ++b) lin_dot8(wf[0], xrow(b, ch), acc[b]);
       }
     }
-    // lane l holds rows 4 (G % 2) .. + 3 of column half G / 2 for input row c where its own column is
-    // of that half
-    float (*part)[RB][2][64] = part2[WALK ? buf : 0];
-    if (((lane >> 3) & 1) == (G >> 1)) {
+    // lane b OW + o stores output o of input row b
+    float mine = 0.f, up = 0.f;
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) *reinterpret_cast<f32x4 *>(&part[wv][rb][G >> 1][8 * c + 4 * (G & 1)]) = acc[rb];
-    }
-    // one barrier per round: the sums of a round are read while the next round writes the other buffer.
-    // Not __syncthreads(), which would wait for the weights in flight.
-    ring_barrier();
-    const int t = threadIdx.x;
-    if (t < 64 * OB) {
-      const int ob = t >> 6, e = t & 63, b = e >> 3, r = e & 7;
-      auto total = [&](int rb) {
-        float sum = 0.f;
+    for (int b = 0; b < NR; ++b)
 #pragma unroll
-        for (int i = 0; i < kWaves; ++i) sum += part[i][rb][0][e] + part[i][rb][1][e];
-        return sum;
-      };
-      const int64_t v = v0 + 8 * ob + r;
-      if (b < nr && v < n_out) {
+      for (int o = 0; o < OW; ++o) {
+        const float t = wave_sum_dpp(acc[b][o]);
+        mine = lane == b * OW + o ? t : mine;
         if constexpr (ACT) {
-          const float g = (float)(__bf16)total(ob), u = (float)(__bf16)total(OB + ob);
-          out[b * out_rs + v] = __builtin_bit_cast(bf16_t, (__bf16)(g / (1.f + __expf(-g)) * u));
-        } else {
-          const __bf16 y = (__bf16)total(ob);
-          if constexpr (std::is_same<OutT, float>::value)
-            out[b * out_rs + v] = (float)y;
-          else
-            out[b * out_rs + v] = __builtin_bit_cast(bf16_t, y);
+          const float u = wave_sum_dpp(acc[b][OW + o]);
+          up = lane == b * OW + o ? u : up;
         }
       }
+    const int64_t v = v0 + lane % OW;
+    if (lane < NR * OW && v < n_out) {
+      if constexpr (ACT) {
+        const float g = (float)(__bf16)mine, u = (float)(__bf16)up;
+        mine = g / (1.f + __expf(-g)) * u;
+      }
+      lin_store(out + (lane / OW) * out_rs + v, mine);
     }
     v0 += step;
-    buf ^= 1;
   } while (WALK && v0 < n_out);
+}
+
+// Rows of more than 2048 inputs (the down projection, 6144): four waves per 4 weight rows, wave wv the
+// 512-column chunks wv, wv + 4, wv + 8, ... of them, their partial sums added in wave order through LDS.
+// When dim is 2048 * NJ (NJ = 3: 6144) a wave's inputs and then all its weights are requested at once;
+// other multiples of 512 go chunk by chunk (NJ = 0).  2048 x 6144 at 1 / 8 input rows: 6.3 / 12.1 -> 6.1 /
+// 9.7 us (the weights used to come first, so that the inputs' way was paid after theirs).
+template <int NR, typename OutT, int PRE, int NJ>
+__global__ __launch_bounds__(256) void linear_rows_splitk_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
+                                                                 int dim, OutT *__restrict__ out, int64_t out_rs) {
+  constexpr int R = 4, NJR = NJ > 0 ? NJ : 1;
+  constexpr bool kAhead = NJ > 0 && (PRE == kPrePlain || (PRE == kPreSwiGLU && NR <= 2));
+  __shared__ float part[4][NR][R];
+  const int lane = threadIdx.x & 63, wv = wave_id();
+  const int64_t v0 = (int64_t)blockIdx.x * R;
+  // rows past the end read the last row (in bounds; not stored)
+  const bf16_t *wr[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) wr[r] = w + min(v0 + r, n_out - 1) * dim + 512 * wv + 8 * lane;
+  u32x4 xf[kAhead ? NJ : 1][NR], uf[kAhead && PRE == kPreSwiGLU ? NJ : 1][NR], wf[NJR][R];
+  if constexpr (kAhead)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int b = 0; b < NR; ++b) {
+        const bf16_t *p = in.x + b * in.x_rs + 512 * wv + 8 * lane + 2048 * j;
+        xf[j][b] = ld16(p);
+        if constexpr (PRE == kPreSwiGLU) uf[j][b] = ld16(p + in.inter);
+      }
+  if constexpr (NJ > 0)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < R; ++r) wf[j][r] = ld16(wr[r] + 2048 * j);
+  float rinv[NR] = {};
+  if constexpr (PRE == kPreNorm) {
+    // sum of squares in the RMSNorm kernel's order
+    const bool writer = blockIdx.x == 0 && wv == 0 && in.res_out != nullptr;
+#pragma unroll
+    for (int b = 0; b < NR; ++b) {
+      float ss = 0.f;
+      for (int c = 8 * lane; c < dim; c += 512) {
+        float v[8];
+        unpack8(ld16(in.x + b * in.x_rs + c), v);
+        if (in.res) {
+          float r[8];
+          unpack8(ld16(in.res + b * in.res_rs + c), r);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
+        }
+        if (writer) st16(in.res_out + b * in.ro_rs + c, pack8(v));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+      }
+      rinv[b] = rsqrtf(wave_sum_dpp(ss) / (float)dim + in.eps);
+    }
+  }
+  float acc[NR][R] = {};
+  if constexpr (NJ > 0) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int b = 0; b < NR; ++b) {
+        u32x4 x;
+        if constexpr (!kAhead) x = lin_input<PRE>(in, b, 512 * wv + 8 * lane + 2048 * j, rinv[b]);
+        else if constexpr (PRE == kPreSwiGLU) x = swiglu8(xf[j][b], uf[j][b]);
+        else x = xf[j][b];
+        lin_dot8(wf[j], x, acc[b]);
+      }
+  } else {
+    for (int c = 512 * wv; c < dim; c += 2048) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) wf[0][r] = ld16(wr[r] + c - 512 * wv);
+#pragma unroll
+      for (int b = 0; b < NR; ++b) lin_dot8(wf[0], lin_input<PRE>(in, b, c + 8 * lane, rinv[b]), acc[b]);
+    }
+  }
+  float mine = 0.f;
+#pragma unroll
+  for (int b = 0; b < NR; ++b)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float t = wave_sum_dpp(acc[b][r]);
+      mine = lane == R * b + r ? t : mine;
+    }
+  if (lane < R * NR) part[wv][lane / R][lane % R] = mine;
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < R * NR && v0 + t % R < n_out) {
+    const int b = t / R, r = t % R;
+    lin_store(out + b * out_rs + v0 + r, ((part[0][b][r] + part[1][b][r]) + part[2][b][r]) + part[3][b][r]);
+  }
 }
 
 // ---- start of a decode step -----------------------------------------------------------------------
@@ -673,63 +728,60 @@ extern "C" int tg_gate_branch_readout(const void *gate_up, int64_t gate_up_row_s
 namespace tg {
 namespace {
 
-template <int RB, int NK, typename OutT, int PRE, bool ACT>
-void launch_linear_rows_form(const LinIn &in, int32_t n_rows, const bf16_t *w, int64_t n_out, int32_t dim, OutT *out,
-                             int64_t out_row_stride, int64_t max_grid, hipStream_t stream) {
-  const int64_t rows = ACT ? 4 * RB : 8 * RB;
-  const int64_t blocks = (n_out + rows - 1) / rows;
-  if constexpr (NK == 4 && RB >= 2) {
-    if (blocks > max_grid) {
-      hipLaunchKernelGGL((linear_rows_mfma_kernel<RB, NK, OutT, PRE, ACT, true>), dim3((unsigned)max_grid), dim3(512), 0,
-                         stream, in, w, n_out, dim, n_rows, out, out_row_stride);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((linear_rows_mfma_kernel<RB, NK, OutT, PRE, ACT, false>), dim3((unsigned)blocks), dim3(512), 0,
-                     stream, in, w, n_out, dim, n_rows, out, out_row_stride);
-}
 // n_out: stored outputs (ACT: weight holds 2 n_out rows, [gate; up]).
-// Blocks of 8 weight rows per workgroup (RB) and workgroups, us at 1 / 8 input rows:
-//   * 2048 rows fill the CUs with one block each (2048 x 2048: RB 1 / 2 / 4 3.9 / 4.7 / 6.3 and 4.4 / 5.4 / 6.9;
-//     2048 x 6144: 6.6 / 9.0 / 16.1 and 8.2 / 10.8 / 17.6);
-//   * up to 65536 rows two blocks spread the input stage over more weight bytes, except at 4096 rows and
-//     up to two input rows (RB 1 / 2: 5.3 / 5.6 and 7.7 / 7.0); two workgroups per CU that walk the
-//     blocks, the next block's weights in flight, beat one workgroup per block (12288 rows with the
-//     SwiGLU product: 11.0 against 12.2, 13.6 against 14.5);
-//   * beyond (the LM head) the blocks' own workgroups keep more bytes in flight: plain input RB 1 / 2 /
-//     4 99.8 / 104.2 / 105.5 and 145 / 112 / 119; with the norm in every workgroup 143 / 104 / 114 and
-//     172 / 133 / 126, four blocks walked by four workgroups per CU 108 and 112.
+// Weight rows per wave and round (RW) and workgroups, us at 1 / 8 input rows, weights from HBM:
+//   * under 4096 weight rows one each, for enough workgroups (2048 x 2048: RW 1 / 2 / 4 3.3 / 3.6 / 4.7 and
+//     4.6 / 5.7 / 8.2);
+//   * from 65536 (the LM head) four, half as many workgroups that form the input (151936 rows with the
+//     norm: RW 2 / 4 110 / 104 and 143 / 123; walked, RW 2, 112 and 123);
+//   * between them two (4096 rows with the norm: RW 1 / 2 / 4 5.0 / 4.9 / 5.5 and 8.9 / 8.4 / 10.8); with two
+//     blocks per CU and more, one workgroup per CU walks them (12288 rows with norm and SwiGLU: 10.4
+//     against 10.3 and 14.1 against 16.9; two workgroups per CU 10.5 and 17.5).
+template <int NR, typename OutT, int PRE, bool ACT>
+void launch_linear_rows_nr(const LinIn &in, const bf16_t *w, int64_t n_out, int32_t dim, OutT *out, int64_t out_row_stride,
+                           hipStream_t stream) {
+  if (!ACT && dim > 2048) {
+    // (4 weight rows per workgroup; 2 / 8 took 5.9 / 6.3 us against 6.1 at one row, 10.5 / 11.8 against
+    // 9.7 at eight)
+    constexpr int NJ = PRE != kPreNorm ? 3 : 0;
+    const dim3 grid((unsigned)((n_out + 3) / 4)), block(256);
+    if (dim == 2048 * NJ)
+      hipLaunchKernelGGL((linear_rows_splitk_kernel<NR, OutT, PRE, NJ>), grid, block, 0, stream, in, w, n_out, dim, out,
+                         out_row_stride);
+    else
+      hipLaunchKernelGGL((linear_rows_splitk_kernel<NR, OutT, PRE, 0>), grid, block, 0, stream, in, w, n_out, dim, out,
+                         out_row_stride);
+    return;
+  }
+  auto launch = [&](auto rw_c, auto nc_c, auto walk_c, int64_t grid) {
+    constexpr int RW = decltype(rw_c)::value, NC = decltype(nc_c)::value;
+    hipLaunchKernelGGL((linear_rows_kernel<NR, RW, NC, OutT, PRE, ACT, decltype(walk_c)::value>), dim3((unsigned)grid),
+                       dim3(512), 0, stream, in, w, n_out, dim, out, out_row_stride);
+  };
+  auto with_rows = [&](auto rw_c) {
+    constexpr int RW = decltype(rw_c)::value, rows = ACT ? 4 * RW : 8 * RW;
+    typedef std::integral_constant<int, 4> C4;
+    typedef std::integral_constant<int, 0> C0;
+    const int64_t blocks = (n_out + rows - 1) / rows, cus = device_cus();
+    if (dim != 2048) return launch(rw_c, C0(), std::false_type(), blocks);
+    if constexpr (RW == 2)
+      if (blocks >= 2 * cus) return launch(rw_c, C4(), std::true_type(), cus);
+    launch(rw_c, C4(), std::false_type(), blocks);
+  };
+  const int64_t w_rows = ACT ? 2 * n_out : n_out;
+  if constexpr (!ACT)
+    if (w_rows < 4096) return with_rows(std::integral_constant<int, 1>());
+  if (w_rows < 65536) return with_rows(std::integral_constant<int, 2>());
+  with_rows(std::integral_constant<int, 4>());
+}
 template <typename OutT, int PRE, bool ACT = false>
 int launch_linear_rows(const LinIn &in, int32_t n_rows, const void *weight, int64_t n_out, int32_t dim, OutT *out,
                        int64_t out_row_stride, hipStream_t stream) {
   const bf16_t *w = static_cast<const bf16_t *>(weight);
-  const int64_t w_rows = ACT ? 2 * n_out : n_out;
-  const int64_t cus = device_cus();
-  int rb = 1;
-  int64_t max_grid = INT32_MAX;
-  if (w_rows >= 65536) {
-    rb = PRE == kPreNorm ? (n_rows == 1 ? 2 : 4) : (n_rows <= 2 ? 1 : 2);
-    if (rb == 4) max_grid = 4 * cus;
-  } else if (w_rows > 4096 || (w_rows == 4096 && n_rows > 2)) {
-    rb = 2;
-    max_grid = 2 * cus;
-  }
-  if (ACT) rb = std::max(rb, 2);
-  if (dim > 2048) rb = ACT ? 2 : 1;
-  auto form = [&](auto rb_c) {
-    constexpr int RB = decltype(rb_c)::value;
-    if (dim == 2048)
-      launch_linear_rows_form<RB, 4, OutT, PRE, ACT>(in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
-    else if (RB == 1 && PRE != kPreNorm && dim == 6144)
-      launch_linear_rows_form<RB, RB == 1 && PRE != kPreNorm ? 12 : 0, OutT, PRE, ACT>(
-          in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
-    else
-      launch_linear_rows_form<RB, 0, OutT, PRE, ACT>(in, n_rows, w, n_out, dim, out, out_row_stride, max_grid, stream);
-  };
-  if constexpr (!ACT)
-    if (rb == 1) form(std::integral_constant<int, 1>());
-  if (rb == 2) form(std::integral_constant<int, 2>());
-  if (rb == 4) form(std::integral_constant<int, 4>());
+#define TG_LR(NR) \
+  case NR: launch_linear_rows_nr<NR, OutT, PRE, ACT>(in, w, n_out, dim, out, out_row_stride, stream); break;
+  switch (n_rows) { TG_LR(1) TG_LR(2) TG_LR(3) TG_LR(4) TG_LR(5) TG_LR(6) TG_LR(7) TG_LR(8) }
+#undef TG_LR
   TG_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -825,6 +877,7 @@ extern "C" int tg_linear_rows_norm_act(const void *h, int64_t h_row_stride, cons
   if (int e = check_linear_rows("linear_rows_norm_act", h, h_row_stride, n_rows, weight, inter, dim, out,
                                 out_row_stride))
     return e;
+  TG_CHECK(dim <= 2048, "linear_rows_norm_act: dim must be at most 2048 (got %d)", dim);
   LinIn in{};
   if (int e = norm_input("linear_rows_norm_act", h, h_row_stride, residual, residual_row_stride, residual_out,
                          residual_out_row_stride, norm_weight, eps, dim, &in))

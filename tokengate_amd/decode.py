@@ -27,7 +27,7 @@ import torch
 
 from tokengate_amd.decoder import (CacheGap, DecoderWeights, LayerKV, argmax_rows, decode_attention,
                                    decode_attention_workspace, decode_begin, h2d, linear_rows, linear_rows_norm,
-                                   linear_rows_norm_act, logits_last, rmsnorm, silu_mul)
+                                   linear_rows_norm_act, linear_rows_swiglu, logits_last, rmsnorm, silu_mul)
 from tokengate_amd.gate import ScoringHead
 from tokengate_amd.prefill import PrefillResult
 
@@ -54,8 +54,9 @@ def _relayout(kv: LayerKV, cu: List[int], gap: int) -> LayerKV:
 
 
 class DecodeState:
-    # most rows per step for which the norms and the SwiGLU product are folded into the projections
-    max_fused_rows = 8
+    # most rows per step for which the norms and the SwiGLU product are folded into the projections, for
+    # models of up to 2048 and of more columns
+    max_fused_rows = (8, 2)
 
     def __init__(self, wts: DecoderWeights, head: ScoringHead, gate_layer: int, pf: PrefillResult,
                  max_new_tokens: int, prune_below_gate: bool = False, graph: bool = False, fused: bool = True):
@@ -139,7 +140,8 @@ class DecodeState:
         dev = tokens.device
         x = torch.nn.functional.embedding(tokens, w.embed)
         # rows beyond max_fused_rows take the separate norm / SwiGLU launches
-        fused = self.fused and B <= self.max_fused_rows and s.d_model % 512 == 0 and s.d_ff % 512 == 0
+        wide = s.d_model > 2048
+        fused = self.fused and B <= self.max_fused_rows[wide] and s.d_model % 512 == 0 and s.d_ff % 512 == 0
         res = None if fused else x.clone()
         normed = torch.empty_like(x)
         hid = torch.empty_like(x)
@@ -150,8 +152,8 @@ class DecodeState:
         rope, r_dec = decode_begin(self.next_pos, w.inv_freq, self.used, self.slots)
         scale = 1.0 / math.sqrt(s.head_dim)
         if fused:
-            # each norm is folded into the projection after it, and the SwiGLU product into the
-            # gate|up projection; the residual stream alternates between two buffers (a fused norm reads one
+            # each norm is folded into the projection after it, and the SwiGLU product into the gate|up
+            # projection (wide models: into the down projection); the residual stream alternates between two buffers (a fused norm reads one
             # and writes the other)
             rbuf = [torch.empty_like(x), torch.empty_like(x)]
             cur = 0
@@ -176,9 +178,14 @@ class DecodeState:
                              r_dec if (r_dec is not None and g) else None, out=att)
             linear_rows(att.view(B, -1), lw.w_o, out=hid)
             if fused:
-                act = linear_rows_norm_act(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur], residual_out=rbuf[1 - cur])
+                if wide:
+                    gu = linear_rows_norm(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur], residual_out=rbuf[1 - cur])
+                    linear_rows_swiglu(gu, lw.w_down, out=hid)
+                else:
+                    act = linear_rows_norm_act(hid, lw.ln2, s.rms_eps, lw.w_gu, residual=rbuf[cur],
+                                               residual_out=rbuf[1 - cur])
+                    linear_rows(act, lw.w_down, out=hid)
                 cur = 1 - cur
-                linear_rows(act, lw.w_down, out=hid)
             else:
                 rmsnorm(hid, lw.ln2, s.rms_eps, residual=res, residual_out=res, out=normed)
                 act = silu_mul(linear_rows(normed, lw.w_gu))

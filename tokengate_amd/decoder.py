@@ -521,7 +521,7 @@ def linear_rows_norm_act(h: torch.Tensor, norm_w: torch.Tensor, eps: float, weig
                          residual: Optional[torch.Tensor] = None, residual_out: Optional[torch.Tensor] = None,
                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """silu(g) * u of F.linear(RMSNorm(h + residual), weight) = [g | u] for up to 8 rows in one launch
-    (tg_linear_rows_norm_act); residual_out as in linear_rows_norm."""
+    (tg_linear_rows_norm_act; dim up to 2048); residual_out as in linear_rows_norm."""
     n, d = h.shape
     inter = weight.shape[0] // 2
     if not (1 <= n <= 8 and d % 512 == 0 and _rows_ok(h, residual, residual_out) and weight.stride(1) == 1
