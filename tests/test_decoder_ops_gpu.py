@@ -269,6 +269,27 @@ def test_argmax_rows(cuda, rows, V):
     assert int(got[0]) == V // 3
 
 
+@pytest.mark.parametrize("V", [1, 3, 4, 4095, 4096, 4100, 32768, 32772, 40961])
+def test_argmax_rows_sizes(cuda, V):
+    """Sizes around the scan's strides; ties, infinities of both signs, negative zeros and a row whose
+    maximum is its last element, against torch.argmax."""
+    from tokengate_amd import decoder as dec
+    g = torch.Generator(device=cuda).manual_seed(V)
+    x = torch.randn(8, V + 4 - V % 4, generator=g, device=cuda)[:, :V]
+    x[0] = x[0].round()                          # many ties
+    x[1] = -x[1].abs() - 1.0
+    x[1, V - 1] = -0.5
+    x[2, V // 2:] = float("inf")
+    x[3] = -float("inf")
+    x[3, V // 3] = -1e30
+    x[4] = 0.0
+    x[4, : V // 2] = -0.0
+    x[5, V - 1] = float("nan")
+    x[6] = 7.25                                  # all equal
+    got = dec.argmax_rows(x)
+    assert torch.equal(got, x.argmax(-1)), (got, x.argmax(-1))
+
+
 def test_decoder_op_errors(cuda):
     from tokengate_amd import decoder as dec
     x = torch.zeros(4, 2050, dtype=torch.bfloat16, device=cuda)
