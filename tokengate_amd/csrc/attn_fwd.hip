@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
     rank = a.n_heavy + (VARLEN ? r2 % n_light : r2 / a.batch);
   }
   int qt = a.n_qtiles - 1 - rank;
-  if constexpr (VARLEN) {
+  if constexpr (VARLEN && !DEC) {
     if (a.level_order) {
       const LevelTile lt = level_tile<BM>(a.cu_seqlens, a.batch, a.sq, bid / per_q, lane);
       if (lt.seq < 0) return;   // workgroup-uniform: past the last tile
@@ -360,25 +360,24 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
   if constexpr (DEC) {
     if (chunk >= 0 && t_lo == t_hi && (n_tiles > 0 || chunk > 0)) return;   // workgroup-uniform
   }
-  // decode: 16 threads per row, HP query rows, then the new k and v rows (the last tile's workgroup)
-  [[maybe_unused]] const int drow = tid >> 4, dj = tid & 15;
+  // decode: a wave forms one row, 8 elements per lane (16 lanes, the four groups alike): the waves with a
+  // query their head's q, waves 1 and 3 the new k and v of the last tile's workgroup
+  [[maybe_unused]] const int dj = lane & 15, dwave = __builtin_amdgcn_readfirstlane(wave);
   [[maybe_unused]] const bool has_new = t_hi == n_tiles && n_tiles > 0;
-  [[maybe_unused]] const bool dwork = DEC && (drow < HP || (has_new && drow < HP + 2));
+  [[maybe_unused]] const bool is_k = DEC && has_new && dwave == 1, is_v = DEC && has_new && dwave == 3;
   [[maybe_unused]] u32x4 draw = {0u, 0u, 0u, 0u}, dnw = draw;
   [[maybe_unused]] f32x4 dcs[4];
   [[maybe_unused]] float dscale = 1.f;
-  if constexpr (DEC) {   // requested before the first tile: loads complete in issue order
-    if (dwork) {
-      const int head = drow < HP ? h0 + drow : drow == HP ? a.h + kh : a.h + a.hkv + kh;
+  if constexpr (DEC) {   // requested before the first tiles: loads complete in issue order
+    if (wave_has_rows || is_k || is_v) {
+      const int head = wave_has_rows ? h0 + hw : is_k ? a.h + kh : a.h + a.hkv + kh;
       draw = ld16(dec.qkv + b * dec.qkv_rs + (int64_t)head * kHeadDim + 8 * dj);
-      if (drow <= HP) {
-        dnw = ld16((drow < HP ? dec.qw : dec.kw) + 8 * dj);
-        const f32x4 *rp = reinterpret_cast<const f32x4 *>(dec.rope + b * (kHeadDim / 2) + 8 * (dj & 7));
+      dnw = ld16((wave_has_rows ? dec.qw : dec.kw) + 8 * dj);
+      const f32x4 *rp = reinterpret_cast<const f32x4 *>(dec.rope + b * (kHeadDim / 2) + 8 * (dj & 7));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dcs[i] = rp[i];
-      }
-      if (drow < HP)
-        dscale = (float)(__bf16)((dec.q_head_scale ? dec.q_head_scale[h0 + drow] : 1.f) *
+      for (int i = 0; i < 4; ++i) dcs[i] = rp[i];
+      if (wave_has_rows)
+        dscale = (float)(__bf16)((dec.q_head_scale ? dec.q_head_scale[h0 + hw] : 1.f) *
                                  (dec.q_row_scale ? dec.q_row_scale[b] : 1.f));
     }
   }
@@ -456,13 +455,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
     ring_barrier();
     if constexpr (DEC) {
       if (t == n_tiles - 1) {   // the new key's rows replace what the cache held there
-        const int key = (sk - 1) & 63;
-        if (drow == HP) {
-          const int lr = kperm_inv(key);
-          *reinterpret_cast<u32x4 *>(kslot(buf_c) + lr * kKRowBytes + 16 * (dj ^ (lr & 15))) = draw;
-        } else if (drow == HP + 1) {
-          *reinterpret_cast<u32x4 *>(vslot(buf_c) + key * kKRowBytes + 16 * (dj ^ vswz(key))) = draw;
-        }
+        const int key = (sk - 1) & 63, lr = kperm_inv(key);
+        if ((is_k || is_v) && lane < 16)
+          *reinterpret_cast<u32x4 *>(is_k ? kslot(buf_c) + lr * kKRowBytes + 16 * (dj ^ (lr & 15))
+                                          : vslot(buf_c) + key * kKRowBytes + 16 * (dj ^ vswz(key))) = draw;
         ring_barrier();
       }
     }
@@ -611,8 +607,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
   };
   if (t_lo < t_hi) issue_tile(t_lo, std::integral_constant<int, 0>());
   if constexpr (DEC) {
-    __shared__ __attribute__((aligned(16))) bf16_t qs[HP][kHeadDim];
-    if (dwork && drow <= HP) {
+    if (wave_has_rows || is_k) {
       float x[8], wf[8], y[8], cs[8][2];
       unpack8(draw, x);
       unpack8(dnw, wf);
@@ -623,24 +618,26 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
       }
       norm_rope8(x, wf, dec.eps, cs, dj, dscale, y);
       draw = pack8(y);
-      if (drow < HP) *reinterpret_cast<u32x4 *>(&qs[drow][8 * dj]) = draw;
     }
     // the new rows go to the cache, from one of the head groups that read this KV head
-    if (dwork && drow >= HP && hg == 0 && a.used_k[b] <= a.sk) {
+    if ((is_k || is_v) && lane < 16 && hg == 0 && a.used_k[b] <= a.sk) {
       const int64_t crow = krow0 + sk - 1;
-      bf16_t *dst = drow == HP ? dec.k_cache + crow * a.k_rs + (int64_t)kh * a.k_hs
-                               : dec.v_cache + crow * a.v_rs + (int64_t)kh * a.v_hs;
+      bf16_t *dst = is_k ? dec.k_cache + crow * a.k_rs + (int64_t)kh * a.k_hs
+                         : dec.v_cache + crow * a.v_rs + (int64_t)kh * a.v_hs;
       st16(dst + 8 * dj, draw);
     }
-    ring_barrier();
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
+    for (int ks = 0; ks < 4; ++ks) {   // lane 16 G of column block 0: elements 32 ks + 8 G .. + 7
+      u32x4 v;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(&qs[hw][32 * ks + 8 * G]);
-        qf[cb][ks] = __builtin_bit_cast(bf16x8, qvalid[cb] ? v : zero);
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t own = draw[e];
+        v[e] = __shfl(own, 4 * ks + G);
       }
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+      qf[0][ks] = __builtin_bit_cast(bf16x8, qvalid[0] ? v : zero);
+      qf[1][ks] = __builtin_bit_cast(bf16x8, zero);
+    }
   }
   int t = t_lo;
   for (; t + 1 < t_hi; t += 2) {
@@ -732,19 +729,23 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void keybias_fwd_kernel(FwdArgs a,
         constexpr int kR = 4;   // chunks in flight
         for (int c0 = cg; c0 < a.ns; c0 += kR * CG) {
           uint64_t ml[kR], w0[kR], w1[kR];
+          // (every load is made, a chunk past the end the last: loads under a condition would be waited for
+          // one by one)
+#pragma unroll
+          for (int r = 0; r < kR; ++r) {
+            const int64_t at = (unit * a.ns + min(c0 + r * CG, a.ns - 1)) * HP + hl;
+            ml[r] = ld_agent(dec.ml + at);
+            w0[r] = ld_agent(dec.po + at * 32 + 2 * piece);
+            w1[r] = ld_agent(dec.po + at * 32 + 2 * piece + 1);
+          }
 #pragma unroll
           for (int r = 0; r < kR; ++r) {
             const int c = c0 + r * CG;
             const bool there = c < a.ns && (int)((int64_t)n_tiles * c / a.ns) < (int)((int64_t)n_tiles * (c + 1) / a.ns);
-            const int64_t at = (unit * a.ns + c) * HP + hl;
-            ml[r] = there ? ld_agent(dec.ml + at) : 0u;
-            w0[r] = there ? ld_agent(dec.po + at * 32 + 2 * piece) : 0u;
-            w1[r] = there ? ld_agent(dec.po + at * 32 + 2 * piece + 1) : 0u;
-          }
-#pragma unroll
-          for (int r = 0; r < kR; ++r) {
             const u32x2 a0 = __builtin_bit_cast(u32x2, w0[r]), a1 = __builtin_bit_cast(u32x2, w1[r]);
-            fold_chunk(f, __builtin_bit_cast(float2, ml[r]), u32x4{a0[0], a0[1], a1[0], a1[1]});
+            float2 mc = __builtin_bit_cast(float2, ml[r]);
+            mc.y = there ? mc.y : 0.f;
+            fold_chunk(f, mc, u32x4{a0[0], a0[1], a1[0], a1[1]});
           }
         }
         if (cg > 0) store_fold(f, &part[cg - 1][0][item], kItems);
