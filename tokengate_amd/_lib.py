@@ -75,6 +75,8 @@ def lib_path(site: str = None) -> str:
 def load(site: str = None):
     """Load (once) and return the ctypes library with argtypes set."""
     global _lib
+    if site is None and _lib is not None:   # set once, when every signature is in place
+        return _lib
     with _lock:
         if _lib is not None and site is None:
             return _lib
@@ -101,6 +103,12 @@ def fwd_workspace(size_fn: str, device, *size_args):
     import torch
     ws = torch.empty(n, dtype=torch.uint8, device=device)
     return ws, ws.data_ptr(), n
+
+
+def stream_of(t) -> int:
+    """The current stream of the tensor's device, as the handle the library takes."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 SELECT_PACK_ERROR_OFFSET = 8   # byte offset of tg_gate_select_pack's wait-timeout flag (global word 2)

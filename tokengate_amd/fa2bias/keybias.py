@@ -56,8 +56,7 @@ def require_varlen() -> None:
 @torch.library.custom_op("recursive_kvs::fa2_keybias_fwd", mutates_args=())
 def _fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias_raw: torch.Tensor,
          scale: float, causal: bool) -> tuple[torch.Tensor, torch.Tensor]:
-    out, lse, _, _ = ext().fwd(q, k, v, None, bias_raw, 0.0, scale, causal, -1, -1, 0.0, False, None)
-    return out, lse
+    return ext().forward(q, k, v, bias_raw, scale, causal)
 
 
 @_fwd.register_fake
@@ -83,12 +82,15 @@ def _setup_context(ctx, inputs, output):
     q, k, v, bias_raw, scale, causal = inputs
     out, lse = output
     ctx.save_for_backward(q, k, v, out, lse, bias_raw)
+    ctx.set_materialize_grads(False)   # lse's gradient is not used: no zeros for it
     ctx.scale = scale
     ctx.causal = causal
 
 
 def _backward(ctx, dout, dlse):
     q, k, v, out, lse, bias_raw = ctx.saved_tensors
+    if dout is None:
+        dout = torch.zeros_like(out)
     if dout.stride(-1) != 1:
         dout = dout.contiguous()
     dq, dk, dv, dbias = torch.ops.recursive_kvs.fa2_keybias_bwd(dout, q, k, v, out, lse, bias_raw,
@@ -107,9 +109,7 @@ def flash_attn_key_bias(q, k, v, key_bias, softmax_scale, causal=True):
 @torch.library.custom_op("recursive_kvs::fa2_keybias_varlen_fwd", mutates_args=())
 def _vfwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias_raw: torch.Tensor, cu_seqlens: torch.Tensor,
           max_seqlen: int, scale: float, causal: bool) -> tuple[torch.Tensor, torch.Tensor]:
-    out, lse, _, _ = ext().varlen_fwd(q, k, v, None, cu_seqlens, cu_seqlens, None, None, None, bias_raw,
-                                      max_seqlen, max_seqlen, 0.0, scale, False, causal, -1, -1, 0.0, False, None)
-    return out, lse
+    return ext().varlen_forward(q, k, v, bias_raw, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, scale, causal)
 
 
 @_vfwd.register_fake
@@ -136,6 +136,7 @@ def _vsetup_context(ctx, inputs, output):
     q, k, v, bias_raw, cu_seqlens, max_seqlen, scale, causal = inputs
     out, lse = output
     ctx.save_for_backward(q, k, v, out, lse, bias_raw, cu_seqlens)
+    ctx.set_materialize_grads(False)   # lse's gradient is not used: no zeros for it
     ctx.max_seqlen = max_seqlen
     ctx.scale = scale
     ctx.causal = causal
@@ -143,6 +144,8 @@ def _vsetup_context(ctx, inputs, output):
 
 def _vbackward(ctx, dout, dlse):
     q, k, v, out, lse, bias_raw, cu_seqlens = ctx.saved_tensors
+    if dout is None:
+        dout = torch.zeros_like(out)
     if dout.stride(-1) != 1:
         dout = dout.contiguous()
     dq, dk, dv, dbias = torch.ops.recursive_kvs.fa2_keybias_varlen_bwd(

@@ -20,8 +20,7 @@ def _check(cond, msg):
         raise RuntimeError(msg)
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+_stream = _lib.stream_of
 
 
 def _check_qkv(q, k, v):
@@ -58,12 +57,17 @@ class KeyBiasExt:
             window_size_left, window_size_right, softcap, return_softmax, gen_):
         _check_qkv(q, k, v)
         _check_unsupported(p_dropout, window_size_left, window_size_right, softcap, return_softmax)
+        out, lse = self.forward(q, k, v, alibi_slopes_, softmax_scale, is_causal, out_)
+        return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
+
+    def forward(self, q, k, v, bias, softmax_scale, is_causal, out_=None):
+        """fwd's out and lse alone, for callers that use no more of it."""
+        _check_qkv(q, k, v)
         _check(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q, k, v must be (batch, seqlen, heads, head_dim)")
         B, Sq, H, D = q.shape
         Sk, Hkv = k.shape[1], k.shape[2]
         _check(tuple(k.shape) == (B, Sk, Hkv, D) and tuple(v.shape) == (B, Sk, Hkv, D), "k and v shape mismatch")
         _check(H % Hkv == 0, "Number of heads in key/value must divide number of heads in query")
-        bias = alibi_slopes_
         if bias is not None:
             _check_bias(bias, B, H, Sk)
         if out_ is not None:
@@ -79,11 +83,10 @@ class KeyBiasExt:
             _lib.call("tg_keybias_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(),
                       bias.data_ptr() if bias is not None else None, out.data_ptr(), lse.data_ptr(),
                       B, Sq, Sk, H, Hkv, D,
-                      q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-                      v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1), out.stride(2),
-                      bias.stride(0) if bias is not None else 0, bias.stride(1) if bias is not None else 0,
+                      *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3],
+                      *(bias.stride()[:2] if bias is not None else (0, 0)),
                       float(softmax_scale), int(bool(is_causal)), ws_ptr, ws_bytes, _stream(q))
-        return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
+        return out, lse
 
     def varlen_fwd(self, q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table_,
                    alibi_slopes_, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale, zero_tensors,
@@ -92,6 +95,14 @@ class KeyBiasExt:
         _check_unsupported(p_dropout, window_size_left, window_size_right, softcap, return_softmax)
         _check(seqused_k is None and leftpad_k is None and block_table_ is None,
                "seqused_k, leftpad_k and block_table are not supported")
+        out, lse = self.varlen_forward(q, k, v, alibi_slopes_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
+                                       softmax_scale, is_causal, out_, zero_tensors)
+        return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
+
+    def varlen_forward(self, q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
+                       is_causal, out_=None, zero_tensors=False):
+        """varlen_fwd's out and lse alone, for callers that use no more of it."""
+        _check_qkv(q, k, v)
         _check(cu_seqlens_q.data_ptr() == cu_seqlens_k.data_ptr() and max_seqlen_q == max_seqlen_k,
                "this library runs self-attention over one cu_seqlens (q and k must share it)")
         _check(cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.is_cuda and cu_seqlens_q.is_contiguous(),
@@ -102,7 +113,6 @@ class KeyBiasExt:
         _check(k.shape[0] == total and tuple(v.shape) == tuple(k.shape), "k and v shape mismatch")
         _check(H % Hkv == 0, "Number of heads in key/value must divide number of heads in query")
         nseq = cu_seqlens_q.numel() - 1
-        bias = alibi_slopes_
         if bias is not None:
             _check_bias(bias, nseq, H, max_seqlen_k, "key bias (num_seqs, num_heads, max_seqlen_k)")
         out = out_ if out_ is not None else torch.empty_like(q)
@@ -115,11 +125,10 @@ class KeyBiasExt:
             _lib.call("tg_keybias_varlen_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(),
                       bias.data_ptr() if bias is not None else None, out.data_ptr(), lse.data_ptr(),
                       cu_seqlens_q.data_ptr(), nseq, int(max_seqlen_q), total, H, Hkv, D,
-                      q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                      out.stride(0), out.stride(1),
-                      bias.stride(0) if bias is not None else 0, bias.stride(1) if bias is not None else 0,
+                      *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2],
+                      *(bias.stride()[:2] if bias is not None else (0, 0)),
                       float(softmax_scale), int(bool(is_causal)), ws_ptr, ws_bytes, _stream(q))
-        return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
+        return out, lse
 
     def bwd(self, dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, alibi_slopes_, p_dropout, softmax_scale,
             is_causal, window_size_left, window_size_right, softcap, deterministic, gen_, rng_state):
@@ -144,9 +153,9 @@ class KeyBiasExt:
         dbias = torch.empty((B, H, Sk), dtype=torch.float32, device=q.device) if bias is not None else None
         strides = []
         for t in (q, k, v, out, dout, dq, dk, dv):
-            strides += [t.stride(0), t.stride(1), t.stride(2)]
-        strides += [bias.stride(0), bias.stride(1)] if bias is not None else [0, 0]
-        strides += [dbias.stride(0), dbias.stride(1)] if dbias is not None else [0, 0]
+            strides += t.stride()[:3]
+        strides += bias.stride()[:2] if bias is not None else (0, 0)
+        strides += dbias.stride()[:2] if dbias is not None else (0, 0)
         arr = (ctypes.c_int64 * len(strides))(*strides)
         if B and Sq and Sk:
             _lib.call("tg_keybias_bwd", dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -187,9 +196,9 @@ class KeyBiasExt:
         dbias = torch.zeros((nseq, H, max_seqlen_k), dtype=torch.float32, device=q.device) if bias is not None else None
         strides = []
         for t in (q, k, v, out, dout, dq, dk, dv):
-            strides += [t.stride(0), t.stride(1)]
-        strides += [bias.stride(0), bias.stride(1)] if bias is not None else [0, 0]
-        strides += [dbias.stride(0), dbias.stride(1)] if dbias is not None else [0, 0]
+            strides += t.stride()[:2]
+        strides += bias.stride()[:2] if bias is not None else (0, 0)
+        strides += dbias.stride()[:2] if dbias is not None else (0, 0)
         arr = (ctypes.c_int64 * len(strides))(*strides)
         if nseq > 0 and total > 0 and max_seqlen_q > 0:
             _lib.call("tg_keybias_varlen_bwd", dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),

@@ -32,8 +32,7 @@ class PackStream(ctypes.Structure):
                 ("chunk_bytes", ctypes.c_int32), ("n_chunks", ctypes.c_int32), ("dst_seq_gap", ctypes.c_int64)]
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+_stream = _lib.stream_of
 
 
 def k_clamped(K: int, n_art: int) -> int:
@@ -333,19 +332,35 @@ def _row_stream(src: torch.Tensor, dst: torch.Tensor, gap: int = 0) -> PackStrea
     if src.dtype != dst.dtype:
         raise RuntimeError("pack: source and destination dtypes differ")
     es = src.element_size()
-    if src.dim() == 3 and not src[0].is_contiguous():
-        if src.stride(2) != 1:
+    shape, stride = src.shape, src.stride()
+    if shape[0] == 0 or dst.shape[0] == 0:
+        raise IndexError("pack: a source and its destination need at least one row")
+    row = _row_elems(shape, stride)
+    if len(shape) == 3 and row < 0:
+        if stride[2] != 1:
             raise RuntimeError("pack: the innermost source axis must be contiguous")
-        n_chunks, chunk = src.shape[1], src.shape[2] * es
-        chunk_stride = src.stride(1) * es
+        n_chunks, chunk = shape[1], shape[2] * es
+        chunk_stride = stride[1] * es
     else:
-        if not src[0].is_contiguous():
+        if row < 0:
             raise RuntimeError("pack: source rows must be contiguous (or (rows, chunks, elems))")
-        n_chunks, chunk, chunk_stride = 1, src[0].numel() * es, 0
-    if not dst[0].is_contiguous() or dst[0].numel() * dst.element_size() != n_chunks * chunk:
+        n_chunks, chunk, chunk_stride = 1, row * es, 0
+    dst_stride = dst.stride()
+    if _row_elems(dst.shape, dst_stride) * es != n_chunks * chunk:
         raise RuntimeError("pack: destination rows must be contiguous and as long as a source row")
-    return PackStream(src.data_ptr(), dst.data_ptr(), src.stride(0) * es, dst.stride(0) * es, chunk_stride,
+    return PackStream(src.data_ptr(), dst.data_ptr(), stride[0] * es, dst_stride[0] * es, chunk_stride,
                       chunk, n_chunks, gap)
+
+
+def _row_elems(shape, stride) -> int:
+    """Elements of t[0] for a tensor of this shape and stride if t[0] is contiguous, else -1 (what
+    t[0].is_contiguous() and t[0].numel() say, without making the view: its price, twice per stream, was
+    half of a call's host time)."""
+    n, ok = 1, True
+    for i in range(len(shape) - 1, 0, -1):
+        ok = ok and (shape[i] == 1 or stride[i] == n)
+        n *= shape[i]
+    return n if ok or n == 0 else -1
 
 
 def pack(keep: torch.Tensor, p: KeepPlan, pairs: Sequence[tuple],
