@@ -242,25 +242,53 @@ template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
-// Butterfly sum over the 64 lanes (x += x[l ^ 1], ^ 2, ^ 4, ... ^ 32) without the LDS crossbar: pairs
-// inside a quad, then mirrored halves of 8 and 16 lanes (whose quads / octets already agree), then the
-// row swaps.  Same additions, so the same bits as wave_sum.
-__device__ __forceinline__ float wave_sum_dpp(float x) {
+// Butterfly sum over the 16 lanes of a row (x += x[l ^ 1], ^ 2, ^ 4, ^ 8) without the LDS crossbar: pairs
+// inside a quad, then mirrored halves of 8 and 16 lanes, whose quads / octets already agree.
+__device__ __forceinline__ float row_sum_dpp(float x) {
   x += dpp<0xB1>(x);    // quad_perm 1 0 3 2
   x += dpp<0x4E>(x);    // quad_perm 2 3 0 1
   x += dpp<0x141>(x);   // row_half_mirror
   x += dpp<0x140>(x);   // row_mirror
-  {
-    const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
-                                                     false, false);
-    const uint32_t lo = sw[0], hi = sw[1];
-    x = u32_as_f32(lo) + u32_as_f32(hi);
-  }
-  const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+  return x;
+}
+// a[l] + a[l ^ 16] in rows 0 and 2, b's in rows 1 and 3
+__device__ __forceinline__ float swap16_add(float a, float b) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
                                                    false, false);
   const uint32_t lo = sw[0], hi = sw[1];
   return u32_as_f32(lo) + u32_as_f32(hi);
 }
+// a[l] + a[l ^ 32] in the lower half, b's in the upper
+__device__ __forceinline__ float swap32_add(float a, float b) {
+  const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                   false, false);
+  const uint32_t lo = sw[0], hi = sw[1];
+  return u32_as_f32(lo) + u32_as_f32(hi);
+}
+// The additions of wave_sum, so its bits
+__device__ __forceinline__ float wave_sum_dpp(float x) {
+  x = row_sum_dpp(x);
+  x = swap16_add(x, x);
+  return swap32_add(x, x);
+}
+// wave_sum of N values at once: the row swaps take two values each and leave value 4 k + r in row r of
+// register k, so a value costs 4 + 1 + 1/2 additions instead of six and no select per value.  Lane l gets
+// value wave_sums_index(l) (of N, if it is less).
+template <int N>
+__device__ __forceinline__ float wave_sums(const float (&v)[N], int lane) {
+  constexpr int K = (N + 3) / 4;
+  float y = 0.f;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    float x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = 4 * k + i < N ? row_sum_dpp(v[4 * k + i < N ? 4 * k + i : 0]) : 0.f;
+    const float t = swap32_add(swap16_add(x[0], x[1]), swap16_add(x[2], x[3]));
+    y = (lane & 15) == k ? t : y;
+  }
+  return y;
+}
+__device__ __forceinline__ int wave_sums_index(int lane) { return 4 * (lane & 15) + (lane >> 4); }
 // acc[r][b] += the 8 columns of weight row r times those of input row b
 template <int RW>
 __device__ __forceinline__ void lin_dot8(const u32x4 (&wv)[RW], u32x4 xv, float (&acc)[RW]) {
@@ -404,27 +432,23 @@ __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t
         for (int b = 0; b < NR; ++b) lin_dot8(wf[0], xrow(b, ch), acc[b]);
       }
     }
-    // lane b OW + o stores output o of input row b
-    float mine = 0.f, up = 0.f;
+    // value b OW + o: output o of input row b
+    float sums[NR * OW], ups[ACT ? NR * OW : 1];
 #pragma unroll
     for (int b = 0; b < NR; ++b)
 #pragma unroll
       for (int o = 0; o < OW; ++o) {
-        const float t = wave_sum_dpp(acc[b][o]);
-        mine = lane == b * OW + o ? t : mine;
-        if constexpr (ACT) {
-          const float u = wave_sum_dpp(acc[b][OW + o]);
-          up = lane == b * OW + o ? u : up;
-        }
+        sums[b * OW + o] = acc[b][o];
+        if constexpr (ACT) ups[b * OW + o] = acc[b][OW + o];
       }
-    const int64_t v = v0 + lane % OW;
-    if (lane < NR * OW && v < n_out) {
-      if constexpr (ACT) {
-        const float g = (float)(__bf16)mine, u = (float)(__bf16)up;
-        mine = g / (1.f + __expf(-g)) * u;
-      }
-      lin_store(out + (lane / OW) * out_rs + v, mine);
+    float mine = wave_sums(sums, lane);
+    if constexpr (ACT) {
+      const float g = (float)(__bf16)mine, u = (float)(__bf16)wave_sums(ups, lane);
+      mine = g / (1.f + __expf(-g)) * u;
     }
+    const int vi = wave_sums_index(lane);
+    const int64_t v = v0 + vi % OW;
+    if (vi < NR * OW && v < n_out) lin_store(out + (vi / OW) * out_rs + v, mine);
     v0 += step;
   } while (WALK && v0 < n_out);
 }
@@ -504,15 +528,14 @@ __global__ __launch_bounds__(256) void linear_rows_splitk_kernel(LinIn in, const
       for (int b = 0; b < NR; ++b) lin_dot8(wf[0], lin_input<PRE>(in, b, c + 8 * lane, rinv[b]), acc[b]);
     }
   }
-  float mine = 0.f;
+  float sums[NR * R];
 #pragma unroll
   for (int b = 0; b < NR; ++b)
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const float t = wave_sum_dpp(acc[b][r]);
-      mine = lane == R * b + r ? t : mine;
-    }
-  if (lane < R * NR) part[wv][lane / R][lane % R] = mine;
+    for (int r = 0; r < R; ++r) sums[b * R + r] = acc[b][r];
+  const float mine = wave_sums(sums, lane);
+  const int vi = wave_sums_index(lane);
+  if (vi < NR * R) part[wv][vi / R][vi % R] = mine;
   __syncthreads();
   const int t = threadIdx.x;
   if (t < R * NR && v0 + t % R < n_out) {
