@@ -321,18 +321,29 @@ template <int NR, int RW, int NC, typename OutT, int PRE, bool ACT, bool WALK>
 __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
                                                           int dim, OutT *__restrict__ out, int64_t out_rs) {
   static_assert(!WALK || NC > 0, "the next round's weights are held in registers");
-  constexpr int kXsRow = 2048, OW = ACT ? RW / 2 : RW, NCR = NC > 0 ? NC : 1, kIn = (NR + 1) / 2;
+  constexpr int kXsRow = 2048, OW = ACT ? RW / 2 : RW, NCR = NC > 0 ? NC : 1;
+  constexpr bool kRowWave = PRE == kPreNorm && NR >= 5 && RW <= 2;
+  constexpr int kIn = kRowWave ? 4 : (NR + 1) / 2;   // rows of at most 2048
   __shared__ __attribute__((aligned(16))) bf16_t xs[NR * kXsRow];
   __shared__ float rinv_s[8];
   const int lane = threadIdx.x & 63, wv = wave_id();
-  const int groups = NC > 0 ? 64 * NC : dim / 8;   // 16-byte pieces of a row
+  // The thread's 16-byte pieces of the input rows.  kRowWave: wave b forms row b, lane l its pieces l,
+  // l + 64, ..., so that the norm needs neither LDS nor a barrier; with fewer rows, or four weight rows
+  // per wave (whose registers leave no room), the pieces are dealt over all waves instead (4096 / 12288 x
+  // 2048 with the norm, us, dealt and row per wave: 4.8 / 10.4 and 5.2 / 11.0 at one row, 6.5 / 11.3 and
+  // 5.7 / 11.8 at four, 7.8 / 13.2 and 7.5 / 13.2 at eight; 151936 rows, eight rows: 115 and 131).
   u32x4 xin[kIn], rin[kIn], nwv[kIn];
   int row[kIn], col[kIn];
 #pragma unroll
   for (int i = 0; i < kIn; ++i) {
-    const int idx = threadIdx.x + 512 * i;
-    row[i] = idx / groups;
-    col[i] = 8 * (idx - row[i] * groups);
+    if constexpr (kRowWave) {
+      col[i] = 8 * lane + 512 * i;
+      row[i] = NC > 0 || col[i] < dim ? wv : NR;
+    } else {
+      const int groups = NC > 0 ? 64 * NC : dim / 8, idx = threadIdx.x + 512 * i;
+      row[i] = idx / groups;
+      col[i] = 8 * (idx - row[i] * groups);
+    }
     if (row[i] < NR) {
       xin[i] = ld16(in.x + row[i] * in.x_rs + col[i]);
       if constexpr (PRE == kPreNorm) {
@@ -361,48 +372,60 @@ __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t
 #pragma unroll
     for (int ch = 0; ch < NC; ++ch) load(wf[ch], ch);
   // ---- input stage ----
+  auto to_lds = [&](int i) { *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = xin[i]; };
   if constexpr (PRE == kPreNorm) {
-    // s = bf16(h + res) to LDS (block 0 also writes res_out), wave b the sum of row b's squares in the
-    // RMSNorm kernel's order (lane l its pieces l, l + 64, ... element by element, then the butterfly),
-    // then every thread scales its own pieces in place
+    // s = bf16(h + res) (block 0 also writes res_out); the sum of a row's squares is a lane's pieces element
+    // by element, then the butterfly, as in the RMSNorm kernel
     const bool writer = blockIdx.x == 0 && in.res_out != nullptr;
 #pragma unroll
     for (int i = 0; i < kIn; ++i)
       if (row[i] < NR) {
-        float v[8];
-        unpack8(xin[i], v);
         if (in.res) {
-          float r[8];
+          float v[8], r[8];
+          unpack8(xin[i], v);
           unpack8(rin[i], r);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
+          xin[i] = pack8(v);
         }
-        xin[i] = pack8(v);
         if (writer) st16(in.res_out + row[i] * in.ro_rs + col[i], xin[i]);
-        *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = xin[i];
+        if constexpr (!kRowWave) to_lds(i);
       }
-    ring_barrier();
-    if (wv < NR) {
-      float ss = 0.f;
-      for (int c = 8 * lane; c < dim; c += 512) {
-        float v[8];
-        unpack8(*reinterpret_cast<const u32x4 *>(xs + wv * kXsRow + c), v);
+    float ss = 0.f;
+    auto squares = [&](u32x4 x) {
+      float v[8];
+      unpack8(x, v);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-      }
-      ss = wave_sum_dpp(ss);
-      if (lane == 0) rinv_s[wv] = rsqrtf(ss / (float)dim + in.eps);
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+    };
+    if constexpr (kRowWave) {
+#pragma unroll
+      for (int i = 0; i < kIn; ++i)
+        if (row[i] < NR) squares(xin[i]);
+    } else {
+      ring_barrier();
+      if (wv < NR)
+        for (int c = 8 * lane; c < dim; c += 512) squares(*reinterpret_cast<const u32x4 *>(xs + wv * kXsRow + c));
     }
-    ring_barrier();
+    float rinv = rsqrtf(wave_sum_dpp(ss) / (float)dim + in.eps);
+    if constexpr (!kRowWave) {
+      if (wv < NR && lane == 0) rinv_s[wv] = rinv;
+      ring_barrier();
+    }
 #pragma unroll
     for (int i = 0; i < kIn; ++i)
-      if (row[i] < NR) *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = norm8(xin[i], nwv[i], rinv_s[row[i]]);
-  } else {
+      if (row[i] < NR) {
+        if constexpr (!kRowWave) rinv = rinv_s[row[i]];
+        xin[i] = norm8(xin[i], nwv[i], rinv);
+      }
+  } else if constexpr (PRE == kPreSwiGLU) {
 #pragma unroll
     for (int i = 0; i < kIn; ++i)
-      if (row[i] < NR)
-        *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = PRE == kPreSwiGLU ? swiglu8(xin[i], rin[i]) : xin[i];
+      if (row[i] < NR) xin[i] = swiglu8(xin[i], rin[i]);
   }
+#pragma unroll
+  for (int i = 0; i < kIn; ++i)
+    if (row[i] < NR) to_lds(i);
   ring_barrier();
   // ---- rounds ----
   auto xrow = [&](int b, int ch) { return *reinterpret_cast<const u32x4 *>(xs + b * kXsRow + 512 * ch + 8 * lane); };
