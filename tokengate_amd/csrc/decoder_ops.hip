@@ -313,10 +313,10 @@ __device__ __forceinline__ void lin_store(OutT *p, float sum) {
 // runs while the weights stream in).  Before, workgroups of 16 rows formed them (or every wave read them
 // for 4 rows: twice the weight's bytes at 8 input rows) and each of the 4 NR sums took six steps through
 // the LDS crossbar.  Before -> now, weights from HBM, at 1 / 8 input rows (us): 4096 x 2048 with the norm
-// 6.9 / 14.5 -> 4.9 / 8.4, 2048 x 2048 4.3 / 8.3 -> 3.3 / 4.6, 12288 x 2048 with the norm 12.4 / 28.6 ->
-// 10.6 / 14.5 (and with the SwiGLU product 10.4 / 14.1), 151936 x 2048 with the norm 109 / 250 -> 104 /
-// 123 (6.0 / 5.1 TB/s).  WALK: fewer workgroups than blocks, which walk them with the
-// next round's weights in flight, so that the input stage is paid once for more of the weight.
+// 6.9 / 14.5 -> 4.8 / 7.5, 2048 x 2048 4.3 / 8.3 -> 3.3 / 4.3, 12288 x 2048 with the norm 12.4 / 28.6 ->
+// 10.5 / 13.4 (and with the SwiGLU product 10.4 / 13.2), 151936 x 2048 with the norm 109 / 250 -> 105 /
+// 117 (5.9 / 5.3 TB/s).  WALK: fewer workgroups than blocks, which walk them with the next round's weights
+// in flight, so that the input stage is paid once for more of the weight.
 template <int NR, int RW, int NC, typename OutT, int PRE, bool ACT, bool WALK>
 __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
                                                           int dim, OutT *__restrict__ out, int64_t out_rs) {
@@ -479,8 +479,8 @@ __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t
 // Rows of more than 2048 inputs (the down projection, 6144): four waves per 4 weight rows, wave wv the
 // 512-column chunks wv, wv + 4, wv + 8, ... of them, their partial sums added in wave order through LDS.
 // When dim is 2048 * NJ (NJ = 3: 6144) a wave's inputs and then all its weights are requested at once;
-// other multiples of 512 go chunk by chunk (NJ = 0).  2048 x 6144 at 1 / 8 input rows: 6.3 / 12.1 -> 6.1 /
-// 9.7 us (the weights used to come first, so that the inputs' way was paid after theirs).
+// other multiples of 512 go chunk by chunk (NJ = 0).  2048 x 6144 at 1 / 8 input rows: 6.3 / 12.1 -> 6.0 /
+// 8.8 us (the weights used to come first, so that the inputs' way was paid after theirs).
 template <int NR, typename OutT, int PRE, int NJ>
 __global__ __launch_bounds__(256) void linear_rows_splitk_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
                                                                  int dim, OutT *__restrict__ out, int64_t out_rs) {
@@ -787,7 +787,8 @@ namespace tg {
 namespace {
 
 // n_out: stored outputs (ACT: weight holds 2 n_out rows, [gate; up]).
-// Weight rows per wave and round (RW) and workgroups, us at 1 / 8 input rows, weights from HBM:
+// Weight rows per wave and round (RW) and workgroups, us at 1 / 8 input rows, weights from HBM (before the
+// lane sums shared their swaps, which took 0.3 to 1 us off every eight-row figure):
 //   * under 4096 weight rows one each, for enough workgroups (2048 x 2048: RW 1 / 2 / 4 3.3 / 3.6 / 4.7 and
 //     4.6 / 5.7 / 8.2);
 //   * from 65536 (the LM head) four, half as many workgroups that form the input (151936 rows with the
