@@ -129,6 +129,21 @@ def test_backward_forms(cuda, B, Sq, Sk, H, Hkv, causal, has_bias):
                 assert_close_grad(f"{what} {b}", to_np(x), r.cpu().numpy())
 
 
+@pytest.mark.parametrize("n,H,Hkv", [(1, 16, 8), (33, 2, 2), (517, 16, 8), (2049, 6, 2), (4096, 16, 8)])
+def test_backward_row_sums_keep_their_order(cuda, n, H, Hkv):
+    """A dense backward forms D = rowsum(dO * O) inside the dQ kernel, a packed one in a launch of its own:
+    the same products added in the same order, so the same bits."""
+    from tokengate_amd.fa2bias.keybias import ext
+    g = torch.Generator(device=cuda).manual_seed(n + H)
+    q, k, v, dout = (torch.randn(1, n, h, 128, generator=g, device=cuda).to(torch.bfloat16) for h in (H, Hkv, Hkv, H))
+    out, lse, _, _ = ext().fwd(q, k, v, None, None, 0.0, 0.1, True, -1, -1, 0.0, False, None)
+    dense = ext().bwd(dout, q, k, v, out, lse, None, None, None, None, 0.0, 0.1, True, -1, -1, 0.0, False, None, None)[3]
+    cu = torch.tensor([0, n], dtype=torch.int32, device=cuda)
+    packed = ext().varlen_bwd(dout[0], q[0], k[0], v[0], out[0], lse[0].contiguous(), None, None, None, cu, cu, None, n, n,
+                              0.0, 0.1, False, True, -1, -1, 0.0, False, None, None)[3]
+    assert torch.equal(dense[0], packed)
+
+
 RAGGED = {
     "nine": [0, 1, 63, 64, 65, 300, 0, 129, 700],
     "equal": [512, 512, 512],

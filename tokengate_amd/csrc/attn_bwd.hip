@@ -241,24 +241,27 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   }
   // D = rowsum(dO * O) of this workgroup's rows (dense: every row belongs to one workgroup, which also
   // writes it for the dK/dV kernel; varlen rows outside every sequence have none, so there the
-  // preprocess kernel forms it)
+  // preprocess kernel forms it).  The order of the sum is the preprocess kernel's, so its bits: each
+  // 16-byte piece (4 ks4 + G there) element by element, then neighbouring pieces pairwise.
   if constexpr (!VARLEN) {
     const int64_t ob = (int64_t)b * a.o_bs;
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      float d = 0.f;
+      float d[4];
 #pragma unroll
       for (int ks4 = 0; ks4 < 4; ++ks4) {
         const u32x4 ov = gload16(a.o + ob + (int64_t)qrow[cb] * a.o_rs + (int64_t)hh[cb] * a.o_hs + 32 * ks4 + 8 * G,
                                  qvalid[cb]);
         const u32x4 dv = __builtin_bit_cast(u32x4, df[cb][ks4]);
+        float acc = 0.f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          d += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
-          d += bf16_to_f32((bf16_t)(ov[w] >> 16)) * bf16_to_f32((bf16_t)(dv[w] >> 16));
+          acc += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
+          acc += bf16_to_f32((bf16_t)(ov[w] >> 16)) * bf16_to_f32((bf16_t)(dv[w] >> 16));
         }
+        d[ks4] = quad_sum(acc);
       }
-      dsum[cb] = quad_sum(d);
+      dsum[cb] = (d[0] + d[1]) + (d[2] + d[3]);
       if (qvalid[cb] && G == 0 && kg == 0) a.softmax_d[((int64_t)b * a.h + hh[cb]) * sq + qrow[cb]] = dsum[cb];
     }
   }
