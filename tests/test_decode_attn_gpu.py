@@ -75,6 +75,23 @@ def test_decode_attention(cuda, used, gap, H, Hkv, bias, scaled):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+def test_decode_attention_shared_workspace(cuda):
+    """Launches of different batch sizes, head counts and key counts share one workspace: the counters stay
+    apart from every launch's partials and are zero again after each."""
+    from tokengate_amd import decoder as dec
+    sizes = [([3000] * 4, 16, 8), ([2500] * 12, 16, 8), ([900] * 40, 12, 4), ([20000], 16, 8), ([700] * 30, 16, 8)]
+    cases = [_case(cuda, used, 3, H, Hkv, 40 + len(used), True, False) for used, H, Hkv in sizes]
+    ws = max((dec.decode_attention_workspace(len(c[7]), c[0], c[9], cuda) for c in cases), key=lambda t: t.numel())
+    for i in (0, 1, 2, 0, 4, 3, 1, 2, 4):
+        shape, lw, qkv, pos, inv, k0, v0, start, n, max_k, kb, qs, rs = cases[i]
+        rope, _ = dec.decode_begin(pos.clone(), inv)
+        k, v = k0.clone(), v0.clone()
+        out = torch.full((len(n), shape.n_heads, 128), float("nan"), dtype=torch.bfloat16, device=cuda)
+        dec.decode_attention(qkv, rope, lw, shape, k, v, start, n, max_k, 128 ** -0.5, ws, kb, out=out)
+        torch.cuda.synchronize()
+        _check(cases[i], out, k, v)
+
+
 def test_decode_attention_masked_keys(cuda):
     """Bias of -inf hides a key; a head that sees no key at all gets zeros."""
     from tokengate_amd import decoder as dec

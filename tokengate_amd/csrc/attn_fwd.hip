@@ -1351,6 +1351,9 @@ struct DecLayout {
   int64_t units, ml, po, bytes;   // byte offsets; the counters come first
   FwdPlan plan;
 };
+// The counters' region is the same for every launch, so that launches of other sizes that share a workspace
+// never write partials where one of them counts: a split has units * ns <= 2 CUs slots and ns >= 2.
+int64_t decode_counter_bytes() { return ((int64_t)device_cus() * 4 + 255) / 256 * 256; }
 DecLayout decode_layout(int64_t num_seqs, int num_heads, int num_heads_k, int max_k) {
   DecLayout w{};
   w.hp = (num_heads / num_heads_k) % 2 == 0 ? 2 : 1;
@@ -1360,7 +1363,7 @@ DecLayout decode_layout(int64_t num_seqs, int num_heads, int num_heads_k, int ma
   w.plan.n_qtiles = 1;
   w.plan.split = plan_split(kForms[1], t, w.units);
   const int64_t parts = w.plan.split.heavy_units * w.plan.split.ns * w.hp;
-  w.ml = (w.units * 4 + 255) / 256 * 256;
+  w.ml = decode_counter_bytes();
   w.po = w.ml + (parts * 8 + 255) / 256 * 256;
   w.bytes = w.plan.split.ns > 1 ? w.po + parts * 256 : 0;
   return w;
