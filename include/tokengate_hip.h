@@ -390,7 +390,8 @@ int tg_decode_begin(int64_t *positions, int32_t num_seqs, const float *inv_freq,
  * head over the cache rows kv_start[b] .. kv_start[b] + kv_used[b] - 1 (the new row included), logits
  * softmax_scale * (q . k_j + bias_raw[b, h, j]), fp32 weights.  kv_used[b] is at least 1 and at most
  * max_seqlen_k (FormDecodeState.step, qwen3_flex_attention.py:1017-1117).
- * out: bf16 rows (num_heads * 128).  workspace: tg_decode_attention_workspace_size bytes, zeroed once
+ * out: bf16 rows (num_heads * 128); tensors 16-byte aligned, row strides multiples of 8 elements.  The scales
+ * are dense fp32: q_head_scale[num_heads], q_row_scale[num_seqs].  workspace: tg_decode_attention_workspace_size bytes, zeroed once
  * when it is allocated; every launch leaves the words it counts in at zero, so launches of one stream
  * share it (launches that may overlap need one each). */
 int64_t tg_decode_attention_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_heads_k,

@@ -105,6 +105,41 @@ def test_lm_head_rejects_bad_arguments_without_touching_the_gpu():
         assert rc != 0 and msg in lib.tg_last_error(), ("linear_rows", args, lib.tg_last_error())
 
 
+def test_decode_attention_rejects_bad_arguments_without_touching_the_gpu():
+    from tokengate_amd import _lib
+    lib = _lib.load()
+
+    def call(**kw):
+        a = dict(qkv=16, qkv_rs=4096, rope=16, nseq=2, H=16, Hkv=8, D=128, qw=16, kw=16, eps=1e-6, qh=None, qr=None,
+                 k=16, k_rs=1024, v=16, v_rs=1024, start=16, used=16, max_k=8, bias=None, bias_bs=0, bias_hs=0, scale=0.1,
+                 out=16, out_rs=2048, ws=None, ws_bytes=0, stream=None)
+        assert set(kw) <= set(a)
+        a.update(kw)
+        return lib.tg_decode_attention(*a.values()), lib.tg_last_error()
+
+    for kw, msg in ((dict(out=8), b"aligned"), (dict(out_rs=2052), b"stride"), (dict(out_rs=2040), b"stride"),
+                    (dict(out=None), b"null"), (dict(k=24), b"aligned"), (dict(qkv_rs=4100), b"stride"),
+                    (dict(D=64), b"head_dim"), (dict(scale=0.0), b"softmax_scale"), (dict(nseq=-1), b"negative"),
+                    (dict(max_k=1 << 21), b"4 GiB")):
+        rc, err = call(**kw)
+        assert rc != 0 and msg in err, (kw, err)
+
+
+def test_decode_attention_wrapper_rejects_bad_scales():
+    from tokengate_amd import decoder as dec
+    shape = dec.DecoderShape(n_layers=1, n_heads=4, n_kv_heads=2, d_model=512)
+    bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    lw = dec.LayerWeights(None, None, bf(128), bf(128), None, None, None, None)
+    i32 = torch.ones(3, dtype=torch.int32)
+    args = (bf(3, 8 * 128), torch.zeros(3, 64, 2), lw, shape, bf(9, 2, 128), bf(9, 2, 128), i32, i32, 8, 0.1,
+            torch.zeros(16, dtype=torch.uint8))
+    for kw, what in ((dict(q_head_scale=torch.ones(3)), "q_head_scale"), (dict(q_head_scale=torch.ones(8)[::2]), "q_head_scale"),
+                     (dict(q_head_scale=torch.ones(4).half()), "q_head_scale"), (dict(q_row_scale=torch.ones(2)), "q_row_scale"),
+                     (dict(q_row_scale=torch.ones(6)[::2]), "q_row_scale"), (dict(q_row_scale=torch.ones(3).double()), "q_row_scale")):
+        with pytest.raises(RuntimeError, match=what):
+            dec.decode_attention(*args, **kw)
+
+
 def test_argmax_rows_rejects_bad_arguments_without_touching_the_gpu():
     from tokengate_amd import _lib
     lib = _lib.load()

@@ -1393,13 +1393,13 @@ extern "C" int tg_decode_attention(const void *qkv, int64_t qkv_row_stride, cons
   TG_CHECK(num_heads > 0 && num_heads_k > 0 && num_heads <= 256 && num_heads % num_heads_k == 0,
            "decode_attention: heads must be in 1..256 and a multiple of the KV heads");
   TG_CHECK(num_seqs >= 0 && max_seqlen_k >= 0, "decode_attention: negative size");
-  TG_CHECK(qkv_row_stride % 8 == 0 && k_row_stride % 8 == 0 && v_row_stride % 8 == 0 &&
+  TG_CHECK(qkv_row_stride % 8 == 0 && k_row_stride % 8 == 0 && v_row_stride % 8 == 0 && out_row_stride % 8 == 0 &&
                qkv_row_stride >= (int64_t)(num_heads + 2 * num_heads_k) * kHeadDim &&
                k_row_stride >= (int64_t)num_heads_k * kHeadDim && v_row_stride >= (int64_t)num_heads_k * kHeadDim &&
                out_row_stride >= (int64_t)num_heads * kHeadDim,
            "decode_attention: row strides must be multiples of 8 elements that hold every head");
   TG_CHECK(aligned16(qkv) && aligned16(k_cache) && aligned16(v_cache) && aligned16(q_norm_weight) &&
-               aligned16(k_norm_weight) && aligned16(rope) && aligned16(workspace),
+               aligned16(k_norm_weight) && aligned16(rope) && aligned16(out) && aligned16(workspace),
            "decode_attention: pointers must be 16-byte aligned");
   TG_CHECK(softmax_scale > 0.f, "decode_attention: softmax_scale must be positive");
   if (num_seqs == 0) return 0;

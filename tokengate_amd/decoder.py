@@ -270,8 +270,10 @@ def decode_attention(qkv: torch.Tensor, rope: torch.Tensor, lw: LayerWeights, sh
             raise RuntimeError("decode_attention: cache rows must hold the heads back to back")
     if out.stride(-1) != 1 or out.stride(-2) != D or qkv.stride(1) != 1:
         raise RuntimeError("decode_attention: qkv and out rows must be contiguous")
-    if q_row_scale is not None and (q_row_scale.dtype != torch.float32 or q_row_scale.numel() < B):
-        raise RuntimeError("decode_attention: q_row_scale must be fp32 with one entry per sequence")
+    for t, n, what in ((q_head_scale, H, "q_head_scale must be contiguous fp32 with one entry per head"),
+                       (q_row_scale, B, "q_row_scale must be contiguous fp32 with one entry per sequence")):
+        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.numel() < n):
+            raise RuntimeError("decode_attention: " + what)
     if bias_raw is not None and (bias_raw.dtype != torch.float32 or bias_raw.stride(-1) != 1
                                  or bias_raw.shape[-1] < max_k):
         raise RuntimeError("decode_attention: bias must be fp32 with a contiguous key axis of >= max_k")
