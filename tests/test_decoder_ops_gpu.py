@@ -285,9 +285,39 @@ def test_argmax_rows_sizes(cuda, V):
     x[4] = 0.0
     x[4, : V // 2] = -0.0
     x[5, V - 1] = float("nan")
+    x[5, V // 2] = float("nan")                  # the first of several wins, also inside a 16-byte piece
+    x[5, V // 2 + 1:V // 2 + 3] = float("inf")
     x[6] = 7.25                                  # all equal
+    x[7] = -float("inf")                         # nothing but masked columns
     got = dec.argmax_rows(x)
     assert torch.equal(got, x.argmax(-1)), (got, x.argmax(-1))
+
+
+def test_argmax_rows_time_does_not_depend_on_the_values(cuda):
+    """A row with masked (-inf) columns takes the time of a finite row and one with a NaN 1.6 times that
+    (general scans after the short one took 3.8 times as long), and gives torch's index."""
+    from tokengate_amd import decoder as dec
+    x = torch.randn(1, 151936, device=cuda)
+    masked = torch.where(torch.arange(151936, device=cuda) % 2 == 0, x, -float("inf"))
+    nan = x.clone()
+    nan[0, 70001:70007] = float("nan")
+
+    def us(t):
+        best = 1e9
+        for _ in range(10):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(50):
+                dec.argmax_rows(t)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 20)
+        return best
+    us(x)
+    for t in (masked, nan):
+        assert torch.equal(dec.argmax_rows(t), t.argmax(-1))
+        assert us(t) < 2.5 * us(x)
 
 
 def test_decoder_op_errors(cuda):
