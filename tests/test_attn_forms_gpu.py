@@ -182,3 +182,42 @@ def test_varlen_tile_order(cuda, name, H, Hkv):
         for what, got, ref in zip(("dq", "dk", "dv", "db"), (dq[s], dk[s], dv[s], db[b, :, :n]),
                                   _grads(q[s], k[s], v[s], bias[b, :, :n], dout[s], scale)):
             assert_close_grad(f"{what} {b}", to_np(got), ref.cpu().numpy())
+
+
+@pytest.mark.parametrize("rows", [100, 500])
+def test_varlen_tile_order_costs_little(cuda, rows):
+    """64 short sequences, which run in level order, take little longer than 65, which run sequence after
+    sequence (finding a workgroup's tile by walking over the sequences made the backward 2.6 times and the
+    forward 1.5 times as slow)."""
+    from tokengate_amd.fa2bias.keybias import ext
+    g = torch.Generator(device=cuda).manual_seed(rows)
+
+    def us(nseq):
+        q, k, v, dout = (torch.randn(nseq * rows, 8, 128, generator=g, device=cuda).to(torch.bfloat16) for _ in range(4))
+        cu = torch.arange(nseq + 1, dtype=torch.int32, device=cuda) * rows
+        fw = lambda: ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, None, rows, rows, 0.0, 0.1, False, True,
+                                      -1, -1, 0.0, False, None)
+        out, lse, _, _ = fw()
+        bw = lambda: ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, None, rows, rows, 0.0, 0.1, False,
+                                      True, -1, -1, 0.0, False, None, None)
+        best = []
+        for f in (fw, bw):
+            graph = torch.cuda.CUDAGraph()
+            f()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graph):
+                for _ in range(5):
+                    f()
+            t = 1e9
+            for _ in range(10):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                a.record()
+                graph.replay()
+                b.record()
+                b.synchronize()
+                t = min(t, a.elapsed_time(b) * 200)
+            best.append(t)
+        return best
+    level, major = us(64), us(65)
+    print(f"64 / 65 sequences of {rows}: forward {level[0]:.1f} / {major[0]:.1f} us, backward {level[1]:.1f} / {major[1]:.1f}")
+    assert level[0] < 1.3 * major[0] and level[1] < 1.3 * major[1]

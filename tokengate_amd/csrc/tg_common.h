@@ -210,12 +210,28 @@ __device__ __forceinline__ void wait_vm_outstanding(int n) {
 #undef TG_VMCNT
 }
 
+// Sum over the 64 lanes, in every lane, without the LDS crossbar.
+__device__ __forceinline__ int wave_sum_int(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true);    // quad_perm 1 0 3 2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true);    // quad_perm 2 3 0 1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true);   // row_half_mirror
+  x += __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, true);   // row_mirror
+  const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  const uint32_t y = r[0] + r[1];
+  const auto h = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  return (int)(h[0] + h[1]);
+}
+
 // Level order of the tiles of n <= 64 packed sequences: the longest sequence's last tile first, then
-// level by level down, at each level (tile index) one tile of every sequence that has it, longest
-// first.  Only tiles that exist are counted: workgroups are handed to an XCD's shader engines in strict
-// rotation, so workgroups that leave at once between those that stay would unbalance the engines (six
-// packed sequences of 260 to 4021 tokens, forward, profiled: sequence-major 185 us, heaviest first with
-// the shorter sequences' missing tiles in between 205, in level order 178).  Tile i of the order, for every lane of the wave alike; seq < 0 past the end.
+// level by level down, at each level (tile index) one tile of every sequence that has it.  Only tiles that
+// exist are counted: workgroups are handed to an XCD's shader engines in strict rotation, so workgroups
+// that leave at once between those that stay would unbalance the engines (six packed sequences of 260 to
+// 4021 tokens, forward, profiled: sequence-major 185 us, heaviest first with the shorter sequences'
+// missing tiles in between 205, in level order 178).  Tile i of the order, for every lane of the wave
+// alike; seq < 0 past the end.  Every workgroup pays for it before its first load, so the level is found by
+// bisection over the tiles from a level up, a sum over the lanes per step: 64 sequences of 500 tokens, 16 / 8
+// heads, forward / backward, sequence-major 169 / 573 us, in level order found by a walk over the sequences
+// 232 / 672 (6 us per workgroup), now 148 / 482; 64 of 100 tokens, 8 / 8 heads, backward 55, 145, 60.
 struct LevelTile {
   int seq, level, n_tiles;   // n_tiles: of that sequence
 };
@@ -223,25 +239,25 @@ template <int ROWS>
 __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int max_len, int i, int lane) {
   const int len = lane < n ? max(0, min(cu[lane + 1] - cu[lane], max_len)) : 0;
   const int nt = (len + ROWS - 1) / ROWS;
-  int rank = 0;   // by tiles, ties by index
-  for (int j = 0; j < n; ++j) {
-    const int tj = __builtin_amdgcn_readlane(nt, j);
-    rank += (tj > nt || (tj == nt && j < lane)) ? 1 : 0;
-  }
-  rank = lane < n ? rank : 64;
-  auto lane_of = [&](int r) { return (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == r)); };
-  int hi = __builtin_amdgcn_readlane(nt, lane_of(0));
-  for (int m = 1; m <= n; ++m) {   // levels that exactly m sequences have
-    const int lo = m < n ? __builtin_amdgcn_readlane(nt, lane_of(m)) : 0;
-    const int c = (hi - lo) * m;
-    if (i < c) {
-      const int seq = lane_of(i % m);
-      return LevelTile{seq, hi - 1 - i / m, __builtin_amdgcn_readlane(nt, seq)};
+  // tiles at level l and above
+  auto from = [&](int l) { return __builtin_amdgcn_readfirstlane(wave_sum_int(max(0, nt - l))); };
+  if (i >= from(0)) return LevelTile{-1, 0, 0};
+  int lo = 0, hi = (max_len + ROWS - 1) / ROWS, above = 0;   // from(lo) > i >= above = from(hi)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, t = from(mid);
+    if (t > i) {
+      lo = mid;
+    } else {
+      hi = mid;
+      above = t;
     }
-    i -= c;
-    hi = lo;
   }
-  return LevelTile{-1, 0, 0};
+  // tile i - above of level lo: that sequence in order among those that have it
+  const bool has = nt > lo;
+  const uint64_t m = __builtin_amdgcn_ballot_w64(has);
+  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+  const int seq = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(has && before == i - above));
+  return LevelTile{seq, lo, __builtin_amdgcn_readlane(nt, seq)};
 }
 
 // Index of this wave in its workgroup, held in a scalar register.  The compiler cannot prove that
