@@ -184,40 +184,50 @@ def test_varlen_tile_order(cuda, name, H, Hkv):
             assert_close_grad(f"{what} {b}", to_np(got), ref.cpu().numpy())
 
 
+def _times(lens, heads, causal, device):
+    """Time of a packed forward and backward in us, best of ten replays of five launches each."""
+    from tokengate_amd.fa2bias.keybias import ext
+    g = torch.Generator(device=device).manual_seed(sum(lens))
+    q, k, v, dout = (torch.randn(sum(lens), heads, 128, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
+    cu, mx = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=device), max(lens)
+    fw = lambda: ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, None, mx, mx, 0.0, 0.1, False, causal,
+                                  -1, -1, 0.0, False, None)
+    out, lse, _, _ = fw()
+    bw = lambda: ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, None, mx, mx, 0.0, 0.1, False,
+                                  causal, -1, -1, 0.0, False, None, None)
+    best = []
+    for f in (fw, bw):
+        graph = torch.cuda.CUDAGraph()
+        f()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            for _ in range(5):
+                f()
+        t = 1e9
+        for _ in range(10):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            t = min(t, a.elapsed_time(b) * 200)
+        best.append(t)
+    return best
+
+
 @pytest.mark.parametrize("rows", [100, 500])
 def test_varlen_tile_order_costs_little(cuda, rows):
     """64 short sequences, which run in level order, take little longer than 65, which run sequence after
     sequence (finding a workgroup's tile by walking over the sequences made the backward 2.6 times and the
     forward 1.5 times as slow)."""
-    from tokengate_amd.fa2bias.keybias import ext
-    g = torch.Generator(device=cuda).manual_seed(rows)
-
-    def us(nseq):
-        q, k, v, dout = (torch.randn(nseq * rows, 8, 128, generator=g, device=cuda).to(torch.bfloat16) for _ in range(4))
-        cu = torch.arange(nseq + 1, dtype=torch.int32, device=cuda) * rows
-        fw = lambda: ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, None, rows, rows, 0.0, 0.1, False, True,
-                                      -1, -1, 0.0, False, None)
-        out, lse, _, _ = fw()
-        bw = lambda: ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, None, rows, rows, 0.0, 0.1, False,
-                                      True, -1, -1, 0.0, False, None, None)
-        best = []
-        for f in (fw, bw):
-            graph = torch.cuda.CUDAGraph()
-            f()
-            torch.cuda.synchronize()
-            with torch.cuda.graph(graph):
-                for _ in range(5):
-                    f()
-            t = 1e9
-            for _ in range(10):
-                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-                a.record()
-                graph.replay()
-                b.record()
-                b.synchronize()
-                t = min(t, a.elapsed_time(b) * 200)
-            best.append(t)
-        return best
-    level, major = us(64), us(65)
+    level, major = _times([rows] * 64, 8, True, cuda), _times([rows] * 65, 8, True, cuda)
     print(f"64 / 65 sequences of {rows}: forward {level[0]:.1f} / {major[0]:.1f} us, backward {level[1]:.1f} / {major[1]:.1f}")
     assert level[0] < 1.3 * major[0] and level[1] < 1.3 * major[1]
+
+
+def test_varlen_non_causal_runs_sequence_after_sequence(cuda):
+    """Without the causal mask the level order gains nothing and interleaves the sequences' K/V, so 64
+    sequences take the time of 65, which never ran in level order (there 64 took 1.35 times as long)."""
+    short, major = _times([6000, 4000] + [64] * 62, 8, False, cuda), _times([6000, 4000] + [64] * 63, 8, False, cuda)
+    print(f"non-causal, 64 / 65 sequences: forward {short[0]:.1f} / {major[0]:.1f} us, backward {short[1]:.1f} / {major[1]:.1f}")
+    assert short[0] < 1.1 * major[0] and short[1] < 1.1 * major[1]

@@ -840,7 +840,7 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
     hipLaunchKernelGGL(bwd_preprocess_kernel, dim3((unsigned)((nrows * 16 + 255) / 256)), dim3(256), 0, st, a, nrows);
   const int hp = (a.group % 2 == 0) ? 2 : 1;
   // a batch that runs sequence-major fills the chip with one group
-  a.level_order = VARLEN && varlen_level_order(a.batch, a.lse_total, a.hkv);
+  a.level_order = VARLEN && varlen_level_order(causal, a.batch, a.lse_total, a.hkv);
   if (VARLEN && a.batch > 1 && !a.level_order) groups = false;
   const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
   const int bmq = dq_bm(ks, hp);

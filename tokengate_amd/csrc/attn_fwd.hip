@@ -1281,7 +1281,8 @@ int keybias_fwd_varlen(const void *q, const void *k, const void *v, const float 
   const FwdPlan plan = plan_varlen(hp, max_seqlen_q, max_seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0);
   int64_t nblocks = apply_plan(a, plan, units, workspace);
   a.level_order = a.n_heavy == 0 && a.n_qtiles > 1 &&
-                  varlen_level_order(num_seqs, cu_k != nullptr ? (int64_t)num_seqs * max_seqlen_k : total_q, num_heads_k);
+                  varlen_level_order(causal != 0, num_seqs, cu_k != nullptr ? (int64_t)num_seqs * max_seqlen_k : total_q,
+                                     num_heads_k);
   if (a.level_order) nblocks = level_tiles(num_seqs, total_q, plan.nw * 32 / hp) * (num_heads / hp);
   TG_CHECK(nblocks < (1ll << 31), "grid too large");
   dispatch_fwd<true>(a, plan.nw, plan.ks, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
