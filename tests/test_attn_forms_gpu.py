@@ -231,3 +231,11 @@ def test_varlen_non_causal_runs_sequence_after_sequence(cuda):
     short, major = _times([6000, 4000] + [64] * 62, 8, False, cuda), _times([6000, 4000] + [64] * 63, 8, False, cuda)
     print(f"non-causal, 64 / 65 sequences: forward {short[0]:.1f} / {major[0]:.1f} us, backward {short[1]:.1f} / {major[1]:.1f}")
     assert short[0] < 1.1 * major[0] and short[1] < 1.1 * major[1]
+
+
+def test_varlen_short_rows_keep_one_group(cuda):
+    """The backward of short packed sequences takes one group per workgroup, as 65 sequences always do: the
+    estimate behind the choice counted a part of a tile as none, and so took four (1.3 to 1.8 times the time)."""
+    few, major = _times([91] + [40] * 61, 8, True, cuda), _times([91] + [40] * 64, 8, True, cuda)
+    print(f"62 / 65 short sequences: backward {few[1]:.1f} / {major[1]:.1f} us")
+    assert few[1] < 1.12 * major[1]

@@ -772,8 +772,11 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
 // ---- host dispatch ---------------------------------------------------------------------------
 // Groups per workgroup (KS of the dQ kernel, KQ of the dK/dV kernel): the form with the least
 // grid_cost.  A step is 64 keys (dQ) or queries of one head (dK/dV) with one group and 128 with more;
-// its cost and a workgroup's are fitted to launches of 128 to 8192 rows timed in each form, and the form
-// they pick is the fastest, or within 6 % of it, at every one.  Where the forms differ most (16 / 8 heads,
+// its cost and a workgroup's (start, merge, stores) are fitted to 219 launches timed in each form (dense of
+// 33 to 12000 rows, packed of 2 to 64 sequences of 20 to 6000).  More than one group has to promise 5 %, and
+// for packed rows 20 %, since their lengths behind max_seqlen are not known here: so no launch of the 219 is
+// more than 2 % slower than with one group, and on average the backward is 23 % faster (dense; 24 with the
+// best form of each) and 8 % (packed; 9).  Where the forms differ most (16 / 8 heads,
 // causal, with bias, us with 1 / 2 / 4 groups): dQ at 1024 rows 45 / 31 / 23, 2048 81 / 52 / 46, 4096
 // 152 / 108 / 140, 8192 356 / 378 / 460; dK/dV 64 / 44 / 29, 122 / 82 / 62, 239 / 172 / 205, 569 / 639 / 740,
 // and at 5000 rows of 8 / 2 heads 547 / 345 / 212.
@@ -781,12 +784,12 @@ struct GroupForm {
   int groups;
   float wg, solo, full;
 };
-constexpr GroupForm kDqForms[] = {{1, 8.f, 2.2f, 2.55f}, {2, 8.f, 2.45f, 2.75f}, {4, 8.f, 1.65f, 1.7f}};
-constexpr GroupForm kDkvForms[] = {{1, 6.f, 1.82f, 2.05f}, {2, 6.f, 2.45f, 2.45f}, {4, 6.f, 1.5f, 1.45f}};
+constexpr GroupForm kDqForms[] = {{1, 8.f, 2.2f, 2.55f}, {2, 11.f, 2.45f, 2.75f}, {4, 10.f, 1.65f, 1.7f}};
+constexpr GroupForm kDkvForms[] = {{1, 6.f, 1.82f, 2.05f}, {2, 9.f, 2.45f, 2.45f}, {4, 6.f, 1.5f, 1.45f}};
 template <typename Cost>
-int cheapest(const GroupForm (&forms)[3], Cost cost) {
+int cheapest(const GroupForm (&forms)[3], bool varlen, Cost cost) {
   int best = 1;
-  float c0 = cost(forms[0]);
+  float c0 = cost(forms[0]) * (varlen ? 0.8f : 0.95f);
   for (int i = 1; i < 3; ++i) {
     const float c = cost(forms[i]);
     if (c < c0) { c0 = c; best = forms[i].groups; }
@@ -795,7 +798,7 @@ int cheapest(const GroupForm (&forms)[3], Cost cost) {
 }
 // The r-th heaviest tile's level (tiles before it in dQ's order of work, after it in dK/dV's) among the
 // launch's sequences: dense, n tiles of each; packed, one sequence of n tiles and the others of `rest` on
-// average (their lengths are on the device).
+// average (their lengths are on the device), a part of a tile counted as one.
 struct Levels {
   int n, rest, others;
   int count() const { return n + rest * others; }
@@ -805,12 +808,13 @@ Levels levels_of(const BwdArgs &a, bool varlen, int len, int tile) {
   Levels v{(len + tile - 1) / tile, 0, 0};
   if (varlen && a.batch > 1) {
     v.others = a.batch - 1;
-    v.rest = (int)std::min<int64_t>(v.n, std::max<int64_t>(0, (a.lse_total - len) / v.others) / tile);
+    const int64_t rows = std::max<int64_t>(0, (a.lse_total - len + v.others - 1) / v.others);
+    v.rest = (int)std::min<int64_t>(v.n, (rows + tile - 1) / tile);
   }
   return v;
 }
 int dq_groups(const BwdArgs &a, int hp, bool causal, bool varlen) {
-  return cheapest(kDqForms, [&](const GroupForm &f) {
+  return cheapest(kDqForms, varlen, [&](const GroupForm &f) {
     const int bm = dq_bm(f.groups, hp), step = f.groups == 1 ? 64 : 128;
     const Levels v = levels_of(a, varlen, a.sq, bm);
     return grid_cost(v.count(), (int64_t)(varlen ? 1 : a.batch) * (a.h / hp), device_cus(), f.wg, f.solo, f.full, [&](int r) {
@@ -820,7 +824,7 @@ int dq_groups(const BwdArgs &a, int hp, bool causal, bool varlen) {
   });
 }
 int dkv_groups(const BwdArgs &a, bool causal, bool varlen) {
-  return cheapest(kDkvForms, [&](const GroupForm &f) {
+  return cheapest(kDkvForms, varlen, [&](const GroupForm &f) {
     const int keys = dkv_keys(f.groups), slot = f.groups == 1 ? 64 : 128;
     const Levels v = levels_of(a, varlen, a.sk, keys);
     return grid_cost(v.count(), (int64_t)(varlen ? 1 : a.batch) * a.hkv, device_cus(), f.wg, f.solo, f.full, [&](int r) {
@@ -840,11 +844,12 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
     hipLaunchKernelGGL(bwd_preprocess_kernel, dim3((unsigned)((nrows * 16 + 255) / 256)), dim3(256), 0, st, a, nrows);
   const int hp = (a.group % 2 == 0) ? 2 : 1;
   // a batch that runs sequence-major fills the chip with one group
-  a.level_order = VARLEN && varlen_level_order(causal, a.batch, a.lse_total, a.hkv);
-  if (VARLEN && a.batch > 1 && !a.level_order) groups = false;
+  const bool level_order = VARLEN && varlen_level_order(causal, a.batch, a.lse_total, a.hkv);
+  if (VARLEN && a.batch > 1 && !level_order) groups = false;
   const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
   const int bmq = dq_bm(ks, hp);
   a.n_tiles = (a.sq + bmq - 1) / bmq;
+  a.level_order = level_order && a.n_tiles > 1;   // one tile each: sequence after sequence is the same order
   const unsigned nq = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, bmq) : (int64_t)a.n_tiles * a.batch) *
                                  (a.h / hp));
 #define TG_DQ(K, HPV, C, B)                                                                            \
@@ -859,6 +864,7 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
   const int kq = groups ? dkv_groups(a, causal, VARLEN) : 1;
   const int keys = dkv_keys(kq);
   a.n_tiles = (a.sk + keys - 1) / keys;
+  a.level_order = level_order && a.n_tiles > 1;
   const unsigned nk = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, keys) : (int64_t)a.n_tiles * a.batch) *
                                  a.hkv);
 #define TG_DKV(K, C, B)                                                                                \
