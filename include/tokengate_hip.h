@@ -64,6 +64,12 @@ int tg_keybias_fwd(const void *q, const void *k, const void *v, const float *bia
 int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
                                       int32_t num_heads, int32_t num_heads_k, int32_t causal);
 
+/* The form tg_keybias_fwd takes for these sizes and this workspace on the current device, without a launch:
+ * plan[0] waves per workgroup, [1] key groups among them, [2] chunks that a split query tile's keys are cut
+ * into (1: no split), [3] query tiles that are split, [4] query tiles. */
+int tg_keybias_fwd_plan(int32_t batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads, int32_t num_heads_k,
+                        int32_t causal, int64_t workspace_bytes, int32_t plan[5]);
+
 /* tg_keybias_fwd for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference, whose
  * mha_fwd allocates its split-KV accumulators itself.  Same arguments and results as

@@ -1,0 +1,33 @@
+"""The form that a dense forward takes (tg_keybias_fwd_plan; without a device the plan is that of 256 compute
+units): waves per workgroup, key groups, chunks of a split tile.  The shapes are those where the choice was
+wrong or is close; the comments give the times in us that speak for it."""
+import pytest
+
+from tokengate_amd import _lib
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,form", [
+    # the forms without key groups: other choices were slower
+    (1, 3000, 32768, 16, 8, True, (4, 1, 2)),     # 760; unsplit 827
+    (1, 3072, 4096, 16, 8, False, (4, 1, 2)),     # 108; unsplit 116
+    (1, 3072, 3072, 16, 8, False, (4, 1, 2)),     # 87; unsplit 93
+    (8, 1024, 1024, 16, 8, True, (8, 1, 1)),      # 46; four waves 49
+    (16, 512, 512, 16, 8, True, (8, 1, 1)),       # 36; four waves 37.4
+    (3, 1700, 1700, 12, 4, True, (4, 1, 1)),      # 42; two key groups 44.5
+    (16, 225, 225, 8, 2, True, (4, 1, 1)),        # two key groups 1.15 times
+    (1, 6000, 6000, 16, 8, True, (4, 1, 1)),      # 145; two key groups 162
+    (1, 8192, 8192, 16, 8, True, (8, 1, 1)), (1, 32768, 32768, 16, 8, True, (8, 1, 1)),
+    # key groups
+    (1, 1024, 1024, 16, 8, True, (8, 4, 1)),      # 18; four waves, split 24
+    (1, 2048, 2048, 16, 8, True, (8, 4, 1)),      # 34; 42
+    (1, 4096, 4096, 16, 8, True, (8, 2, 1)),      # 76; unsplit 91
+    (1, 2320, 2320, 12, 4, True, (8, 4, 1)),      # 35; 41
+])
+def test_form(B, Sq, Sk, H, Hkv, causal, form):
+    assert _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, 1 << 40)[:3] == form
+
+
+def test_plan_rejects_bad_sizes():
+    for a in ((0, 8, 8, 2, 1, 1, 0), (1, 0, 8, 2, 1, 1, 0), (1, 8, -1, 2, 1, 1, 0), (1, 8, 8, 3, 2, 1, 0), (1, 8, 8, 2, 1, 1, -1)):
+        with pytest.raises(RuntimeError, match="bad sizes"):
+            _lib.fwd_plan(*a)

@@ -24,6 +24,7 @@ SIGNATURES = {
                        i64, i64, i64, i64, i64, i64, i64, i64, i64, i64, i64, i64,
                        i64, i64, f32, i32, vp, i64, vp],
     "tg_keybias_fwd_workspace_size": [i32, i32, i32, i32, i32, i32],
+    "tg_keybias_fwd_plan": [i32, i32, i32, i32, i32, i32, i64, vp],
     "tg_keybias_fwd_noalloc": [vp, vp, vp, vp, vp, vp,
                                i32, i32, i32, i32, i32, i32,
                                i64, i64, i64, i64, i64, i64, i64, i64, i64, i64, i64, i64,
@@ -109,6 +110,13 @@ def stream_of(t) -> int:
     """The current stream of the tensor's device, as the handle the library takes."""
     import torch
     return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+def fwd_plan(B, Sq, Sk, H, Hkv, causal, workspace_bytes):
+    """(waves, key groups, chunks, split tiles, tiles) of a dense forward (tg_keybias_fwd_plan)."""
+    plan = (C.c_int32 * 5)()
+    call("tg_keybias_fwd_plan", B, Sq, Sk, H, Hkv, int(causal), int(workspace_bytes), plan)
+    return tuple(plan)
 
 
 SELECT_PACK_ERROR_OFFSET = 8   # byte offset of tg_gate_select_pack's wait-timeout flag (global word 2)

@@ -989,23 +989,32 @@ SplitPlan plan_split(const Form &f, const Tiles &t, int64_t units) {
 
 // Estimated time of a launch, in microseconds: grid_cost with the form's workgroup cost (start, first
 // loads, merge of the key groups, stores) and its costs per key step; `combine` is the split's second
-// launch.  The constants are fitted to launches of 1 to 16384 rows (8 to 16 heads, batches of 1 to 8)
-// timed in each form; the form they pick is within 5 % of the fastest at all of those, and where the
-// forms differ most: 4 waves / 8 waves / 8 waves with 2 / with 4 key groups take, at 1024 rows 22.6 /
-// 25.0 / 20.8 / 16.0 us, at 2048 40.5 / 40.2 / 36.6 / 32.9, at 4096 88.9 / 107.4 / 76.6 / 98.4, at 6001
-// 142 / 158 / 160 / 194, at 8192 266 / 239 / 268 / 339 (16 / 8 heads, causal, with bias).
+// launch.  Two workgroups of four waves that share a CU both take `full` per step until the shorter ends.
+// The constants are fitted to launches of 1 to 16384 rows (8 to 16 heads, batches of 1 to 8) timed in each
+// form.  Where the forms differ most: 4 waves / 8 waves / 8 waves with 2 / with 4 key groups take, at 1024
+// rows 22.6 / 25.0 / 20.8 / 16.0 us, at 2048 40.5 / 40.2 / 36.6 / 32.9, at 4096 88.9 / 107.4 / 76.6 / 98.4, at
+// 6001 142 / 158 / 160 / 194, at 8192 266 / 239 / 268 / 339 (16 / 8 heads, causal, with bias).
 constexpr Form kForms[] = {{8, 1, 3.5f, 1.6f, 1.77f, 6.f},
                            {4, 1, 2.4f, 1.3f, 1.95f, 6.f},
                            {8, 2, 4.0f, 1.75f, 1.88f, 10.f},
                            {8, 4, 4.2f, 1.2f, 1.25f, 6.f}};
 float launch_cost(const Form &f, const Tiles &t, int64_t units, const SplitPlan &p) {
-  if (p.ns > 1) {   // one round; two workgroups of four waves share each CU throughout
+  const int64_t cus = device_cus();
+  if (p.ns > 1) {   // one round
     const int chunk = (t.steps(t.n_qtiles - 1) + p.ns - 1) / p.ns;
     const int light = p.n_heavy < t.n_qtiles ? t.steps(t.n_qtiles - 1 - p.n_heavy) : 0;
-    return (f.nw == 4 ? f.full : f.solo) * std::max(chunk, light) + f.group + f.combine;
+    const int longest = std::max(chunk, light);
+    if (f.nw == 8) return f.solo * longest + f.group + f.combine;
+    const int64_t n_longest = chunk > light ? p.heavy_units * p.ns : (t.n_qtiles - p.n_heavy) * units;
+    const int partner = n_longest > cus ? longest : std::min(chunk, light);
+    return f.solo * longest + (f.full - f.solo) * partner + f.group + f.combine;
   }
-  return grid_cost(t.n_qtiles, units, (int64_t)device_cus() * (8 / f.nw), f.group, f.solo, f.full,
-                   [&](int r) { return t.steps(t.n_qtiles - 1 - r); });
+  const float cost = grid_cost(t.n_qtiles, units, cus * (8 / f.nw), f.group, f.solo, f.full,
+                               [&](int r) { return t.steps(t.n_qtiles - 1 - r); });
+  if (f.nw == 8 || t.n_qtiles * units <= cus) return cost;
+  // the heaviest workgroup's partner is the (CUs + 1)-th, but about half of its time falls elsewhere
+  const int partner = t.steps(t.n_qtiles - 1 - (int)(cus / units));
+  return std::max(cost, f.solo * t.steps(t.n_qtiles - 1) + 0.6f * (f.full - f.solo) * partner + f.group);
 }
 
 struct FwdPlan {
@@ -1013,27 +1022,43 @@ struct FwdPlan {
   SplitPlan split;
 };
 
-// A dense launch's form and split: the cheapest of the four forms, each with and without its split
-// where it has one and the workspace holds it.  key_groups: whether ks > 1 may be taken (its last
-// step's LDS DMA offsets reach up to 127 rows past sk and must not wrap at 4 GiB).
+// A dense launch's form and split.  Without key groups: eight waves where the grid gives at least two
+// workgroups per CU, else four, with the split where they have one and the workspace holds it.  Another
+// form, with or without its split, takes their place where the estimate promises 10 % (against a
+// split launch) or 20 %, about what it is off by between forms: of 151 launches timed in each form (33 to
+// 12000 rows, up to 32768 keys) no choice is then more than 2 % slower than the first rule's, and on
+// average they take 6.2 % less (7.3 with the best form of each).  With no margin 17 were slower, by up to
+// 15 %: 3000 rows over 32768 keys 760 -> 830 us, 3072 x 4096 without the mask 108 -> 117.
+// key_groups: whether ks > 1 may be taken (its last step's LDS DMA offsets reach up to 127 rows past sk and
+// must not wrap at 4 GiB).
 FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, int64_t workspace_bytes, bool key_groups) {
   FwdPlan best;
   float best_cost = INFINITY;
+  // the form with its split if wanted, and if it has one that the workspace holds
+  auto consider = [&](const Form &f, bool split) {
+    const Tiles t(f, hp, sq, sk, causal);
+    SplitPlan p;
+    if (split) {
+      p = plan_split(f, t, units);
+      if (p.ns == 1 || p.bytes > workspace_bytes) return false;
+    }
+    const float cost = launch_cost(f, t, units, p);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best.nw = f.nw;
+      best.ks = f.ks;
+      best.n_qtiles = t.n_qtiles;
+      best.split = p;
+    }
+    return true;
+  };
+  const Form &first = kForms[Tiles(kForms[0], hp, sq, sk, causal).n_qtiles * units >= 2 * device_cus() ? 0 : 1];
+  if (!consider(first, true)) consider(first, false);
+  best_cost *= best.split.ns > 1 ? 0.9f : 0.8f;
   for (const Form &f : kForms) {
     if (f.ks > 1 && !key_groups) continue;
-    const Tiles t(f, hp, sq, sk, causal);
-    const SplitPlan s = plan_split(f, t, units);
-    for (int with = s.ns > 1 && s.bytes <= workspace_bytes ? 1 : 0; with >= 0; --with) {
-      const SplitPlan p = with ? s : SplitPlan{};
-      const float cost = launch_cost(f, t, units, p);
-      if (cost < best_cost) {
-        best_cost = cost;
-        best.nw = f.nw;
-        best.ks = f.ks;
-        best.n_qtiles = t.n_qtiles;
-        best.split = p;
-      }
-    }
+    consider(f, true);
+    consider(f, false);
   }
   return best;
 }
@@ -1337,6 +1362,20 @@ extern "C" int64_t tg_keybias_varlen_kv_fwd_workspace_size(int32_t num_seqs, int
 extern "C" int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
                                                   int32_t num_heads, int32_t num_heads_k, int32_t causal) {
   return fwd_workspace_size(false, batch, seqlen_q, seqlen_k, num_heads, num_heads_k, causal);
+}
+
+extern "C" int tg_keybias_fwd_plan(int32_t batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads,
+                                   int32_t num_heads_k, int32_t causal, int64_t workspace_bytes, int32_t *plan) {
+  clear_error();
+  TG_CHECK(plan != nullptr, "fwd_plan: null plan");
+  TG_CHECK(batch > 0 && seqlen_q > 0 && seqlen_k >= 0 && num_heads > 0 && num_heads_k > 0 && workspace_bytes >= 0 &&
+               num_heads % num_heads_k == 0,
+           "fwd_plan: bad sizes");
+  const int hp = (num_heads / num_heads_k) % 2 == 0 ? 2 : 1;
+  const FwdPlan p = plan_dense(hp, seqlen_q, seqlen_k, (int64_t)batch * (num_heads / hp), causal != 0, workspace_bytes, true);
+  const int32_t v[5] = {p.nw, p.ks, p.split.ns, p.split.n_heavy, p.n_qtiles};
+  std::copy(v, v + 5, plan);
+  return 0;
 }
 
 extern "C" int64_t tg_keybias_varlen_fwd_workspace_size(int32_t num_seqs, int32_t max_seqlen, int32_t num_heads,
