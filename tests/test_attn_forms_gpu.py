@@ -148,6 +148,7 @@ RAGGED = {
     "nine": [0, 1, 63, 64, 65, 300, 0, 129, 700],
     "equal": [512, 512, 512],
     "sixty_four": [17 * (i % 7) for i in range(64)],
+    "long": [4500, 0, 333, 2100],                 # more than 64 levels of 32 and of 64 rows
     "sixty_five": [40 + (i % 3) for i in range(65)],
 }
 

@@ -228,36 +228,57 @@ __device__ __forceinline__ int wave_sum_int(int x) {
 // that leave at once between those that stay would unbalance the engines (six packed sequences of 260 to
 // 4021 tokens, forward, profiled: sequence-major 185 us, heaviest first with the shorter sequences'
 // missing tiles in between 205, in level order 178).  Tile i of the order, for every lane of the wave
-// alike; seq < 0 past the end.  Every workgroup pays for it before its first load, so the level is found by
-// bisection over the tiles from a level up, a sum over the lanes per step: 64 sequences of 500 tokens, 16 / 8
-// heads, forward / backward, sequence-major 169 / 573 us, in level order found by a walk over the sequences
-// 232 / 672 (6 us per workgroup), now 148 / 482; 64 of 100 tokens, 8 / 8 heads, backward 55, 145, 60.
+// alike; seq < 0 past the end.  Every workgroup pays for it before its first load.  Up to 16 sequences: each lane
+// adds up the tiles from a level of its own on, by a walk over the sequences; more: bisection over the levels,
+// a sum over the lanes per step.  64 sequences of 500 tokens, 16 / 8 heads, forward / backward: sequence-major
+// 169 / 573 us, in level order with a walk over sequences and levels 232 / 672 (6 us per workgroup),
+// bisection 148 / 482; 64 of 100 tokens, 8 / 8 heads, backward 55, 145, 60.  The six sequences above, forward +
+// backward: bisection 683 us, with the longest first at a level (whose places in the order then do not move
+// when others join) 681, lane by level 677.
 struct LevelTile {
   int seq, level, n_tiles;   // n_tiles: of that sequence
 };
 template <int ROWS>
 __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int max_len, int i, int lane) {
   const int len = lane < n ? max(0, min(cu[lane + 1] - cu[lane], max_len)) : 0;
-  const int nt = (len + ROWS - 1) / ROWS;
-  // tiles at level l and above
-  auto from = [&](int l) { return __builtin_amdgcn_readfirstlane(wave_sum_int(max(0, nt - l))); };
-  if (i >= from(0)) return LevelTile{-1, 0, 0};
-  int lo = 0, hi = (max_len + ROWS - 1) / ROWS, above = 0;   // from(lo) > i >= above = from(hi)
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1, t = from(mid);
-    if (t > i) {
-      lo = mid;
-    } else {
-      hi = mid;
-      above = t;
+  const int nt = (len + ROWS - 1) / ROWS, levels = (max_len + ROWS - 1) / ROWS;
+  int level = 0, above = 0;   // the tile's level and the tiles above it
+  int place = 0;              // of this lane's sequence among those that reach the level
+  if (n <= 16) {
+    int s = (levels + 63) >> 6;
+    while (true) {
+      const int l = level + s * lane;
+      int t = 0;   // tiles at level l and above, falling from lane to lane
+      for (int j = 0; j < n; ++j) t += max(0, __builtin_amdgcn_readlane(nt, j) - l);
+      const int k = __builtin_popcountll(__builtin_amdgcn_ballot_w64(t > i));
+      if (k == 0) return LevelTile{-1, 0, 0};
+      level += s * (k - 1);
+      above = k < 64 ? __builtin_amdgcn_readlane(t, k) : above;
+      if (s == 1) break;
+      s = (s + 63) >> 6;
     }
+    for (int j = 0; j < n; ++j) {   // by tiles, ties by index
+      const int tj = __builtin_amdgcn_readlane(nt, j);
+      place += (tj > nt || (tj == nt && j < lane)) ? 1 : 0;
+    }
+  } else {
+    auto from = [&](int l) { return __builtin_amdgcn_readfirstlane(wave_sum_int(max(0, nt - l))); };
+    if (i >= from(0)) return LevelTile{-1, 0, 0};
+    int hi = levels;   // from(level) > i >= above = from(hi)
+    while (hi - level > 1) {
+      const int mid = (level + hi) >> 1, t = from(mid);
+      if (t > i) {
+        level = mid;
+      } else {
+        hi = mid;
+        above = t;
+      }
+    }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(nt > level);
+    place = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
   }
-  // tile i - above of level lo: that sequence in order among those that have it
-  const bool has = nt > lo;
-  const uint64_t m = __builtin_amdgcn_ballot_w64(has);
-  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-  const int seq = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(has && before == i - above));
-  return LevelTile{seq, lo, __builtin_amdgcn_readlane(nt, seq)};
+  const int seq = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(nt > level && place == i - above));
+  return LevelTile{seq, level, __builtin_amdgcn_readlane(nt, seq)};
 }
 
 // Index of this wave in its workgroup, held in a scalar register.  The compiler cannot prove that
