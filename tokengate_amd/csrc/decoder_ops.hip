@@ -307,7 +307,7 @@ __device__ __forceinline__ void lin_store(OutT *p, float sum) {
   if constexpr (std::is_same<OutT, float>::value) *p = (float)y;
   else *p = __builtin_bit_cast(bf16_t, y);
 }
-// Rows of at most 2048 inputs (512 NC; NC = 0: any multiple of 512).  A workgroup of 8 waves, each wave
+// Rows of at most 2048 inputs (512 NC; NC = 0: 512, 1024 or 1536).  A workgroup of 8 waves, each wave
 // RW weight rows (ACT: RW / 2 outputs, their gate and up rows) per round.  The NR input rows are formed
 // once per workgroup in LDS, requested before the weights (loads complete in issue order, so the stage
 // runs while the weights stream in).  Before, workgroups of 16 rows formed them (or every wave read them
@@ -316,12 +316,17 @@ __device__ __forceinline__ void lin_store(OutT *p, float sum) {
 // 6.9 / 14.5 -> 4.8 / 7.5, 2048 x 2048 4.3 / 8.3 -> 3.3 / 4.3, 12288 x 2048 with the norm 12.4 / 28.6 ->
 // 10.5 / 13.4 (and with the SwiGLU product 10.4 / 13.2), 151936 x 2048 with the norm 109 / 250 -> 105 /
 // 117 (5.9 / 5.3 TB/s).  WALK: fewer workgroups than blocks, which walk them with the next round's weights
-// in flight, so that the input stage is paid once for more of the weight.
+// in flight, so that the input stage is paid once for more of the weight.  NC = 0 requests its chunks one by
+// one after the stage (more of them in flight cost eight rows up to 18 %, in registers), except for one input
+// row (kAhead), whose chunks are requested before it: 4096 x 1024 4.0 -> 3.8 us, 4096 x 1536 4.95 -> 4.5 (with
+// the norm and two weight rows the stage hides it: 6144 x 1024 5.1 against 5.2).
 template <int NR, int RW, int NC, typename OutT, int PRE, bool ACT, bool WALK>
 __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t *__restrict__ w, int64_t n_out,
                                                           int dim, OutT *__restrict__ out, int64_t out_rs) {
   static_assert(!WALK || NC > 0, "the next round's weights are held in registers");
-  constexpr int kXsRow = 2048, OW = ACT ? RW / 2 : RW, NCR = NC > 0 ? NC : 1;
+  constexpr int kXsRow = 2048, OW = ACT ? RW / 2 : RW;
+  constexpr bool kAhead = NC > 0 || (NR == 1 && (RW != 2 || PRE != kPreNorm));
+  constexpr int NCR = NC > 0 ? NC : kAhead ? 3 : 1;
   constexpr bool kRowWave = PRE == kPreNorm && NR >= 5 && RW <= 2;
   constexpr int kIn = kRowWave ? 4 : (NR + 1) / 2;   // rows of at most 2048
   __shared__ __attribute__((aligned(16))) bf16_t xs[NR * kXsRow];
@@ -368,9 +373,10 @@ __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t
   };
   rows_from(v0);
   u32x4 wf[NCR][RW];
-  if constexpr (NC > 0)
+  if constexpr (kAhead)
 #pragma unroll
-    for (int ch = 0; ch < NC; ++ch) load(wf[ch], ch);
+    for (int ch = 0; ch < NCR; ++ch)
+      if (NC > 0 || 512 * ch < dim) load(wf[ch], ch);
   // ---- input stage ----
   auto to_lds = [&](int i) { *reinterpret_cast<u32x4 *>(xs + row[i] * kXsRow + col[i]) = xin[i]; };
   if constexpr (PRE == kPreNorm) {
@@ -449,10 +455,18 @@ __global__ __launch_bounds__(512) void linear_rows_kernel(LinIn in, const bf16_t
 #pragma unroll
           for (int r = 0; r < RW; ++r) wf[ch][r] = wn[ch][r];
     } else {
-      for (int ch = 0; 512 * ch < dim; ++ch) {
-        load(wf[0], ch);
+      if constexpr (kAhead) {
 #pragma unroll
-        for (int b = 0; b < NR; ++b) lin_dot8(wf[0], xrow(b, ch), acc[b]);
+        for (int ch = 0; ch < NCR; ++ch)
+          if (512 * ch < dim)
+#pragma unroll
+            for (int b = 0; b < NR; ++b) lin_dot8(wf[ch], xrow(b, ch), acc[b]);
+      } else {
+        for (int ch = 0; 512 * ch < dim; ++ch) {
+          load(wf[0], ch);
+#pragma unroll
+          for (int b = 0; b < NR; ++b) lin_dot8(wf[0], xrow(b, ch), acc[b]);
+        }
       }
     }
     // value b OW + o: output o of input row b
@@ -823,6 +837,7 @@ namespace {
 //     4.6 / 5.7 / 8.2);
 //   * from 65536 (the LM head) four, half as many workgroups that form the input (151936 rows with the
 //     norm: RW 2 / 4 110 / 104 and 143 / 123; walked, RW 2, 112 and 123);
+//     With one or two plain rows of 1024 or 1536 inputs two (151936 x 1024 56.7 -> 54.3);
 //   * between them two (4096 rows with the norm: RW 1 / 2 / 4 5.0 / 4.9 / 5.5 and 8.9 / 8.4 / 10.8); with two
 //     blocks per CU and more, one workgroup per CU walks them (12288 rows with norm and SwiGLU: 10.4
 //     against 10.3 and 14.1 against 16.9; two workgroups per CU 10.5 and 17.5).
@@ -860,7 +875,8 @@ void launch_linear_rows_nr(const LinIn &in, const bf16_t *w, int64_t n_out, int3
   const int64_t w_rows = ACT ? 2 * n_out : n_out;
   if constexpr (!ACT)
     if (w_rows < 4096) return with_rows(std::integral_constant<int, 1>());
-  if (w_rows < 65536) return with_rows(std::integral_constant<int, 2>());
+  if (w_rows < 65536 || (PRE == kPrePlain && NR <= 2 && dim > 512 && dim < 2048))
+    return with_rows(std::integral_constant<int, 2>());
   with_rows(std::integral_constant<int, 4>());
 }
 template <typename OutT, int PRE, bool ACT = false>
