@@ -207,13 +207,17 @@ __device__ __forceinline__ u32x4 swiglu8(u32x4 gv, u32x4 uv) {
   for (int e = 0; e < 8; ++e) y[e] = g[e] / (1.f + __expf(-g[e])) * u[e];
   return pack8(y);
 }
-__device__ __forceinline__ u32x4 norm8(u32x4 sv, u32x4 nwv, float rinv) {
-  float v[8], wf[8], y[8];
-  unpack8(sv, v);
+__device__ __forceinline__ u32x4 norm8(const float (&v)[8], u32x4 nwv, float rinv) {
+  float wf[8], y[8];
   unpack8(nwv, wf);
 #pragma unroll
   for (int e = 0; e < 8; ++e) y[e] = wf[e] * (v[e] * rinv);
   return pack8(y);
+}
+__device__ __forceinline__ u32x4 norm8(u32x4 sv, u32x4 nwv, float rinv) {
+  float v[8];
+  unpack8(sv, v);
+  return norm8(v, nwv, rinv);
 }
 // Eight inputs of input row b from column c on (rinv: the row's normaliser, norm stage only)
 template <int PRE>
@@ -231,7 +235,7 @@ __device__ __forceinline__ u32x4 lin_input(const LinIn &in, int b, int c, float 
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (float)(__bf16)(v[e] + r[e]);
     }
-    return norm8(pack8(v), ld16(in.nw + c), rinv);   // (v is exact in bf16)
+    return norm8(v, ld16(in.nw + c), rinv);
   }
 }
 // The order of every sum is fixed: lane l of a wave takes columns 8 l .. 8 l + 7 of each 512-column chunk,
