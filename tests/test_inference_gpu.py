@@ -146,6 +146,27 @@ def test_decode_fused_projections_match_unfused(cuda):
         assert torch.equal(plain.last_logits, fused.last_logits), f"step {i}: logits differ"
 
 
+def test_decode_fused_row_limit_is_a_number(cuda):
+    """max_fused_rows is the number of rows up to which a step folds its norms: two sequences with a limit of
+    one run the separate launches (fused=False's bits), with the default and with two the folded ones."""
+    from tokengate_amd import inference as I
+    from tokengate_amd.decode import DecodeState
+    m = _model(cuda, seed=12, ssmax=False)
+    split = [I.split_state_span(p) for p in _prompts([260, 300], [(12, 250), (0, 280)], 5)]
+    logits = []
+    for limit in (None, 0, 1, 2):
+        pf = m.prefill(split, [30, 40], decode_headroom=2)
+        d = DecodeState(m.weights, m.gate, m.gate_layer, pf, 2)
+        assert d.max_fused_rows == 8 and m.weights.shape.d_model <= 2048
+        if limit is not None:
+            d.max_fused_rows = limit
+        d.step(pf.first_tokens)
+        logits.append(d.last_logits)
+    torch.cuda.synchronize()
+    for x in logits[1:]:
+        assert torch.equal(x, logits[0])
+
+
 def test_decode_graph_replays_match_eager(cuda):
     """Every replay of the captured decode step equals the eager step bit for bit (tokens and
     logits), with eager work and host synchronisations between the replays; the two decodes

@@ -54,14 +54,16 @@ def _relayout(kv: LayerKV, cu: List[int], gap: int) -> LayerKV:
 
 
 class DecodeState:
-    # most rows per step for which the norms and the SwiGLU product are folded into the projections, for
-    # models of up to 2048 and of more columns
-    max_fused_rows = (8, 2)
+    # most rows per step for which the norms and the SwiGLU product are folded into the projections (a number
+    # set here or on a state holds for every model; else a state takes 8 up to 2048 columns and 2 beyond)
+    max_fused_rows: Optional[int] = None
 
     def __init__(self, wts: DecoderWeights, head: ScoringHead, gate_layer: int, pf: PrefillResult,
                  max_new_tokens: int, prune_below_gate: bool = False, graph: bool = False, fused: bool = True):
         shape = wts.shape
         self.wts, self.shape = wts, shape
+        if self.max_fused_rows is None:
+            self.max_fused_rows = 8 if shape.d_model <= 2048 else 2
         dev = wts.device
         B = len(pf.n_kept)
         self.B = B
@@ -141,7 +143,7 @@ class DecodeState:
         x = torch.nn.functional.embedding(tokens, w.embed)
         # rows beyond max_fused_rows take the separate norm / SwiGLU launches
         wide = s.d_model > 2048
-        fused = self.fused and B <= self.max_fused_rows[wide] and s.d_model % 512 == 0 and s.d_ff % 512 == 0
+        fused = self.fused and B <= self.max_fused_rows and s.d_model % 512 == 0 and s.d_ff % 512 == 0
         res = None if fused else x.clone()
         normed = torch.empty_like(x)
         hid = torch.empty_like(x)
@@ -153,8 +155,8 @@ class DecodeState:
         scale = 1.0 / math.sqrt(s.head_dim)
         if fused:
             # each norm is folded into the projection after it, and the SwiGLU product into the gate|up
-            # projection (wide models: into the down projection); the residual stream alternates between two buffers (a fused norm reads one
-            # and writes the other)
+            # projection (wide models: into the down projection); the residual stream alternates between two
+            # buffers (a fused norm reads one and writes the other)
             rbuf = [torch.empty_like(x), torch.empty_like(x)]
             cur = 0
         for l in range(s.n_layers):
