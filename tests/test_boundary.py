@@ -152,6 +152,24 @@ def test_argmax_rows_rejects_bad_arguments_without_touching_the_gpu():
         assert rc != 0 and msg in lib.tg_last_error(), (args, lib.tg_last_error())
 
 
+@pytest.mark.parametrize("varlen", [False, True])
+def test_forward_checks_its_inputs_once(monkeypatch, varlen):
+    from tokengate_amd.fa2bias import native
+    seen = []
+    monkeypatch.setattr(native, "_check_qkv", lambda q, k, v: seen.append(1))
+    q, cu = torch.zeros(2, 128), torch.zeros(2, dtype=torch.int32)
+    e = native.KeyBiasExt()
+    with pytest.raises(RuntimeError):        # too few dimensions, or not on the device: the checks after it
+        if varlen:
+            e.varlen_fwd(q, q, q, None, cu, cu, None, None, None, None, 1, 1, 0.0, 0.1, False, True, -1, -1, 0.0, False, None)
+        else:
+            e.fwd(q, q, q, None, None, 0.0, 0.1, True, -1, -1, 0.0, False, None)
+    assert len(seen) == 1
+    with pytest.raises(RuntimeError):
+        e.varlen_forward(q, q, q, None, cu, cu, 1, 1, 0.1, True) if varlen else e.forward(q, q, q, None, 0.1, True)
+    assert len(seen) == 2
+
+
 def test_select_pack_layout_and_keys_per_thread():
     """gate.plan's chunking for tg_gate_select_pack: 4 keys per thread (chunks of 2048 scores) for
     small batches (every span at most 32768 scores, at most 64 chunks in all), else the smallest of

@@ -57,12 +57,15 @@ class KeyBiasExt:
             window_size_left, window_size_right, softcap, return_softmax, gen_):
         _check_qkv(q, k, v)
         _check_unsupported(p_dropout, window_size_left, window_size_right, softcap, return_softmax)
-        out, lse = self.forward(q, k, v, alibi_slopes_, softmax_scale, is_causal, out_)
+        out, lse = self._forward(q, k, v, alibi_slopes_, softmax_scale, is_causal, out_)
         return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
 
     def forward(self, q, k, v, bias, softmax_scale, is_causal, out_=None):
         """fwd's out and lse alone, for callers that use no more of it."""
         _check_qkv(q, k, v)
+        return self._forward(q, k, v, bias, softmax_scale, is_causal, out_)
+
+    def _forward(self, q, k, v, bias, softmax_scale, is_causal, out_):
         _check(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q, k, v must be (batch, seqlen, heads, head_dim)")
         B, Sq, H, D = q.shape
         Sk, Hkv = k.shape[1], k.shape[2]
@@ -95,14 +98,19 @@ class KeyBiasExt:
         _check_unsupported(p_dropout, window_size_left, window_size_right, softcap, return_softmax)
         _check(seqused_k is None and leftpad_k is None and block_table_ is None,
                "seqused_k, leftpad_k and block_table are not supported")
-        out, lse = self.varlen_forward(q, k, v, alibi_slopes_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-                                       softmax_scale, is_causal, out_, zero_tensors)
+        out, lse = self._varlen_forward(q, k, v, alibi_slopes_, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
+                                        softmax_scale, is_causal, out_, zero_tensors)
         return [out, lse, torch.empty(0, device=q.device), torch.empty(0, device=q.device)]
 
     def varlen_forward(self, q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
                        is_causal, out_=None, zero_tensors=False):
         """varlen_fwd's out and lse alone, for callers that use no more of it."""
         _check_qkv(q, k, v)
+        return self._varlen_forward(q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
+                                    is_causal, out_, zero_tensors)
+
+    def _varlen_forward(self, q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
+                        is_causal, out_, zero_tensors):
         _check(cu_seqlens_q.data_ptr() == cu_seqlens_k.data_ptr() and max_seqlen_q == max_seqlen_k,
                "this library runs self-attention over one cu_seqlens (q and k must share it)")
         _check(cu_seqlens_q.dtype == torch.int32 and cu_seqlens_q.is_cuda and cu_seqlens_q.is_contiguous(),
