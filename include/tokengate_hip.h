@@ -60,7 +60,7 @@ int tg_keybias_fwd(const void *q, const void *k, const void *v, const float *bia
                    float softmax_scale, int32_t causal,
                    void *workspace, int64_t workspace_bytes, hipStream_t stream);
 
-/* Workspace bytes tg_keybias_fwd uses for these sizes on the current device (0: no split). */
+/* Workspace bytes tg_keybias_fwd uses for these sizes on the current device (0: it does not split). */
 int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
                                       int32_t num_heads, int32_t num_heads_k, int32_t causal);
 

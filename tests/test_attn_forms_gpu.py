@@ -42,6 +42,7 @@ SHAPES = [
     (1, 161, 417, 16, 8, True, True), (1, 300, 140, 16, 8, True, True), (1, 257, 129, 16, 8, False, True),
     (1, 777, 777, 16, 8, False, True), (1, 1025, 1025, 16, 8, True, True), (1, 1000, 1000, 3, 1, True, True),
     (3, 999, 999, 4, 4, True, False), (1, 2049, 2049, 16, 8, True, True), (1, 2320, 2320, 12, 4, True, True),
+    (1, 2320, 2320, 16, 8, True, True), (2, 1500, 1500, 6, 2, True, True), (1, 2048, 2048, 16, 8, False, True),
     (1, 3071, 3071, 16, 8, True, True), (1, 4097, 4097, 16, 8, True, False), (1, 4096, 4096, 8, 8, True, True),
 ]
 

@@ -27,6 +27,25 @@ def test_form(B, Sq, Sk, H, Hkv, causal, form):
     assert _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, 1 << 40)[:3] == form
 
 
+def test_workspace_is_what_the_plan_needs():
+    """tg_keybias_fwd_workspace_size is 0 exactly where the launch does not split, and with any fewer bytes the
+    launch is the one without a workspace."""
+    size = _lib.load().tg_keybias_fwd_workspace_size
+    split = set()
+    for Sq in (1, 3, 64, 200, 700, 1024, 1500, 2320, 3000, 4096):
+        for Sk in (Sq, 3000, 9000, 32768, 131072):
+            for H, Hkv in ((16, 8), (8, 8), (6, 2), (1, 1)):
+                for causal in (True, False):
+                    s = (1, Sq, Sk, H, Hkv, causal)
+                    n, full, none = size(*s[:5], int(causal)), _lib.fwd_plan(*s, 1 << 40), _lib.fwd_plan(*s, 0)
+                    assert (n > 0) == (full[2] > 1) and none[2] == 1, s
+                    assert _lib.fwd_plan(*s, n) == full
+                    if n > 0:
+                        split.add(full[:2])
+                        assert _lib.fwd_plan(*s, n - 1) == _lib.fwd_plan(*s, 16) == none
+    assert split == {(4, 1), (8, 1), (8, 2), (8, 4)}       # every form has launches that split
+
+
 def test_plan_rejects_bad_sizes():
     for a in ((0, 8, 8, 2, 1, 1, 0), (1, 0, 8, 2, 1, 1, 0), (1, 8, -1, 2, 1, 1, 0), (1, 8, 8, 3, 2, 1, 0), (1, 8, 8, 2, 1, 1, -1)):
         with pytest.raises(RuntimeError, match="bad sizes"):

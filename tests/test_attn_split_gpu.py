@@ -46,25 +46,30 @@ def _rows(Sq):
 
 
 CASES = [
-    # B, Sq, Sk, H, Hkv, causal, bias
-    (1, 2320, 2320, 16, 8, True, True),      # Phase 2 at K=2000
-    (2, 1500, 1500, 6, 2, True, True),       # odd GQA group (one head per MFMA column block)
-    (1, 2048, 2048, 16, 8, False, True),     # non-causal: every tile split
-    (1, 700, 3000, 16, 8, True, False),      # Sq < Sk, no bias
-    (1, 1, 20000, 16, 8, True, True),        # one decode row over a long cache
-    (2, 3, 9000, 16, 8, True, True),         # a few rows per sequence
+    # B, Sq, Sk, H, Hkv, causal, bias, and the form that is split: waves, key groups
+    (1, 1500, 1500, 6, 2, True, True, (4, 1)),       # odd GQA group (one head per MFMA column block)
+    (1, 1200, 1200, 6, 2, False, True, (4, 1)),      # non-causal: every tile as heavy as the last
+    (1, 700, 3000, 16, 8, True, False, (4, 1)),      # Sq < Sk, no bias
+    (1, 1, 3000, 16, 8, True, True, (4, 1)),         # one decode row
+    (1, 200, 20000, 16, 8, True, True, (8, 1)),      # a chunk of a prompt over a long cache
+    (1, 64, 131072, 16, 8, True, True, (8, 2)),      # the key groups' partials: over a very long cache,
+    (1, 1, 20000, 16, 8, True, True, (8, 4)),        # one row over a long one,
+    (2, 3, 9000, 16, 8, True, True, (8, 4)),         # a few rows per sequence
+    (1, 300, 4000, 3, 1, False, False, (8, 4)),      # odd group, more than one tile, no bias
 ]
+IDS = ["odd_group", "noncausal", "sq_lt_sk", "decode_row", "chunk", "two_groups", "long_row", "few_rows", "four_groups"]
 
 
-@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,has_bias", CASES,
-                         ids=["2320", "odd_group", "noncausal", "sq_lt_sk", "decode_row", "few_rows"])
-def test_split_matches_oracle_and_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_bias):
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,has_bias,form", CASES, ids=IDS)
+def test_split_matches_oracle_and_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_bias, form):
     g = torch.Generator(device=cuda).manual_seed(Sq * 7 + Sk + H)
     q, k, v = qkv(B, Sq, Sk, H, Hkv, g, cuda)
     scale = 128 ** -0.5
     bias_raw = (torch.randn(B, H, Sk, device=cuda, generator=g) * 2.0 / scale).contiguous() if has_bias else None
     out_s, lse_s, n = _dense(q, k, v, bias_raw, scale, causal, "planned")
-    assert n > 0, "this shape is expected to be split"
+    plan = _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, n)
+    assert n > 0 and plan[:2] == form and plan[2] > 1, "this shape is expected to be split in this form"
+    assert _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, 0)[2] == 1
     out_u, lse_u, _ = _dense(q, k, v, bias_raw, scale, causal, "none")
     rows = _rows(Sq)
     ro, rl = ora.keybias_fwd(to_np(q), to_np(k), to_np(v), None if bias_raw is None else to_np(bias_raw),
@@ -81,15 +86,20 @@ def test_split_matches_oracle_and_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_b
     assert_close("split vs unsplit lse", to_np(lse_s), to_np(lse_u))
 
 
-def test_short_workspace_runs_unsplit(cuda):
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,has_bias,form", [CASES[0], CASES[5], CASES[7]],
+                         ids=[IDS[0], IDS[5], IDS[7]])
+def test_short_workspace_runs_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_bias, form):
+    """One byte less than planned: not the split's bits (its partials are rounded) but the unsplit launch's."""
     g = torch.Generator(device=cuda).manual_seed(5)
-    q, k, v = qkv(1, 2320, 2320, 16, 8, g, cuda)
+    q, k, v = qkv(B, Sq, Sk, H, Hkv, g, cuda)
     scale = 128 ** -0.5
-    bias_raw = (torch.randn(1, 16, 2320, device=cuda, generator=g) / scale).contiguous()
-    out_short, lse_short, n = _dense(q, k, v, bias_raw, scale, True, "short")
-    out_none, lse_none, _ = _dense(q, k, v, bias_raw, scale, True, "none")
-    assert n > 0
+    bias_raw = (torch.randn(B, H, Sk, device=cuda, generator=g) / scale).contiguous()
+    out_short, lse_short, n = _dense(q, k, v, bias_raw, scale, causal, "short")
+    out_none, lse_none, _ = _dense(q, k, v, bias_raw, scale, causal, "none")
+    out_split, _, _ = _dense(q, k, v, bias_raw, scale, causal, "planned")
+    assert n > 0 and _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, n - 1)[2] == 1
     assert torch.equal(out_short, out_none) and torch.equal(lse_short, lse_none)
+    assert not torch.equal(out_split, out_none)
 
 
 @pytest.mark.parametrize("lens,causal,has_bias", [([2320], True, True), ([1000, 0, 600], True, True),

@@ -54,12 +54,15 @@ def test_noalloc_matches_workspace_entry_point(cuda):
     # then grids of more than half the resident slots (a few thousand rows over a long cache, and a
     # non-causal one), whose split plans once needed more than the static scratch
     shapes = [(2, 3, 9000, 16, 8, True), (1, 1, 3000, 16, 8, True), (1, 3072, 32768, 16, 8, True),
-              (1, 3000, 32768, 16, 8, True), (1, 3072, 4096, 16, 8, False)]
+              (1, 3000, 32768, 16, 8, True), (1, 3072, 4096, 16, 8, False),
+              # and splits of the forms with two and four key groups, and of eight waves
+              (1, 64, 131072, 16, 8, True), (1, 1, 20000, 16, 8, True), (1, 200, 20000, 16, 8, True)]
     for i, (B, Sq, Sk, H, Hkv, causal) in enumerate(shapes):
         print(f"[noalloc] call {i}: B{B} Sq{Sq} Sk{Sk} H{H}/{Hkv}", flush=True)
         q, k, v, b, scale = _inputs(B, Sq, Sk, H, Hkv, 40 + i, cuda)
         n, (o1, l1), (o2, l2) = _both(q, k, v, b, scale, causal)
-        assert n > 0, "this launch is meant to use the key-range split (and so the scratch)"
+        assert n > 0 and _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, n)[2] > 1, \
+            "this launch is meant to use the key-range split (and so the scratch)"
         assert torch.equal(o1, o2) and torch.equal(l1, l2), f"call {i}: noalloc differs from tg_keybias_fwd"
 
 

@@ -1023,7 +1023,7 @@ struct FwdPlan {
 };
 
 // A dense launch's form and split.  Without key groups: eight waves where the grid gives at least two
-// workgroups per CU, else four, with the split where they have one and the workspace holds it.  Another
+// workgroups per CU, else four, with the split where they have one (splits).  Another
 // form, with or without its split, takes their place where the estimate promises 10 % (against a
 // split launch) or 20 %, about what it is off by between forms: of 151 launches timed in each form (33 to
 // 12000 rows, up to 32768 keys) no choice is then more than 2 % slower than the first rule's, and on
@@ -1031,16 +1031,16 @@ struct FwdPlan {
 // 15 %: 3000 rows over 32768 keys 760 -> 830 us, 3072 x 4096 without the mask 108 -> 117.
 // key_groups: whether ks > 1 may be taken (its last step's LDS DMA offsets reach up to 127 rows past sk and
 // must not wrap at 4 GiB).
-FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, int64_t workspace_bytes, bool key_groups) {
+FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool splits, bool key_groups) {
   FwdPlan best;
   float best_cost = INFINITY;
-  // the form with its split if wanted, and if it has one that the workspace holds
+  // the form with its split if wanted, and if it has one
   auto consider = [&](const Form &f, bool split) {
     const Tiles t(f, hp, sq, sk, causal);
     SplitPlan p;
     if (split) {
-      p = plan_split(f, t, units);
-      if (p.ns == 1 || p.bytes > workspace_bytes) return false;
+      if (splits) p = plan_split(f, t, units);
+      if (p.ns == 1) return false;
     }
     const float cost = launch_cost(f, t, units, p);
     if (cost < best_cost) {
@@ -1061,6 +1061,11 @@ FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, int64_t w
     consider(f, false);
   }
   return best;
+}
+// The same with a workspace of so many bytes: without a split where they do not hold the plan's.
+FwdPlan plan_dense_in(int hp, int sq, int sk, int64_t units, bool causal, int64_t workspace_bytes, bool key_groups) {
+  const FwdPlan p = plan_dense(hp, sq, sk, units, causal, true, key_groups);
+  return p.split.bytes <= workspace_bytes ? p : plan_dense(hp, sq, sk, units, causal, false, key_groups);
 }
 
 // A varlen launch (prefill and decode over packed rows): 8-wave workgroups when the grid gives at
@@ -1160,8 +1165,8 @@ int keybias_fwd_dense(const void *q, const void *k, const void *v, const float *
   const int hp = (a.group % 2 == 0) ? 2 : 1;
   const int64_t units = (int64_t)batch * (num_heads / hp);
   TG_CHECK(workspace == nullptr || aligned16(workspace), "workspace must be 16-byte aligned");
-  const FwdPlan plan = plan_dense(hp, seqlen_q, seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0,
-                                span_ok(seqlen_k + 128ll, k_row_stride) && span_ok(seqlen_k + 128ll, v_row_stride));
+  const FwdPlan plan = plan_dense_in(hp, seqlen_q, seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0,
+                                   span_ok(seqlen_k + 128ll, k_row_stride) && span_ok(seqlen_k + 128ll, v_row_stride));
   const int64_t nblocks = apply_plan(a, plan, units, workspace);
   TG_CHECK(nblocks < (1ll << 31), "grid too large");
   dispatch_fwd<false>(a, plan.nw, plan.ks, hp, causal != 0, bias_raw != nullptr, (int)nblocks, stream);
@@ -1169,7 +1174,8 @@ int keybias_fwd_dense(const void *q, const void *k, const void *v, const float *
   return 0;
 }
 
-// Workspace of a dense launch (the largest split that any form of it has) or of a varlen one.
+// Workspace of a dense or varlen launch's split (a dense one whose key groups are refused for the size of its
+// k or v, see plan_dense, may have another plan, and then runs without a split if that needs more).
 int64_t fwd_workspace_size(bool varlen, int32_t units_batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads,
                            int32_t num_heads_k, int32_t causal) {
   if (units_batch <= 0 || seqlen_q <= 0 || seqlen_k <= 0 || num_heads <= 0 || num_heads_k <= 0 ||
@@ -1177,11 +1183,9 @@ int64_t fwd_workspace_size(bool varlen, int32_t units_batch, int32_t seqlen_q, i
     return 0;
   const int hp = ((num_heads / num_heads_k) % 2 == 0) ? 2 : 1;
   const int64_t units = (int64_t)units_batch * (num_heads / hp);
-  if (varlen) return plan_varlen(hp, seqlen_q, seqlen_k, units, causal != 0, INT64_MAX).split.bytes;
-  int64_t bytes = 0;
-  for (const Form &f : kForms)
-    bytes = std::max(bytes, plan_split(f, Tiles(f, hp, seqlen_q, seqlen_k, causal != 0), units).bytes);
-  return bytes;
+  return (varlen ? plan_varlen(hp, seqlen_q, seqlen_k, units, causal != 0, INT64_MAX)
+                 : plan_dense(hp, seqlen_q, seqlen_k, units, causal != 0, true, true))
+      .split.bytes;
 }
 
 // Device scratch of tg_keybias_fwd_noalloc: the key-range split's partial results.  plan_split
@@ -1372,7 +1376,8 @@ extern "C" int tg_keybias_fwd_plan(int32_t batch, int32_t seqlen_q, int32_t seql
                num_heads % num_heads_k == 0,
            "fwd_plan: bad sizes");
   const int hp = (num_heads / num_heads_k) % 2 == 0 ? 2 : 1;
-  const FwdPlan p = plan_dense(hp, seqlen_q, seqlen_k, (int64_t)batch * (num_heads / hp), causal != 0, workspace_bytes, true);
+  const FwdPlan p = plan_dense_in(hp, seqlen_q, seqlen_k, (int64_t)batch * (num_heads / hp), causal != 0, workspace_bytes,
+                                  true);
   const int32_t v[5] = {p.nw, p.ks, p.split.ns, p.split.n_heavy, p.n_qtiles};
   std::copy(v, v + 5, plan);
   return 0;
