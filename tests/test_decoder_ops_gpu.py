@@ -156,8 +156,12 @@ def test_lm_head(cuda, rows, vocab, dim):
     assert torch.equal(got.argmax(-1)[clear], tl.argmax(-1)[clear])
 
 
+# (the last two lines: walked blocks with a partial last round, 514 and 769 of 16 rows on 256 compute units;
+# one row of narrower inputs, whose weights are requested ahead, in one, two and many weight rows)
 @pytest.mark.parametrize("rows,n_out,dim", [(1, 4096, 2048), (3, 2048, 6144), (8, 12288, 2048), (2, 2048, 1024),
-                                          (2, 1000, 4096), (1, 517, 2560)])
+                                          (2, 1000, 4096), (1, 517, 2560),
+                                          (1, 8209, 2048), (5, 12301, 2048), (8, 8209, 2048),
+                                          (1, 1027, 512), (1, 4099, 1024), (1, 2051, 1536), (2, 65539, 1024), (1, 65541, 512)])
 def test_linear_rows(cuda, rows, n_out, dim):
     """The decode-step projection GEMV (tg_linear_rows, bf16 out) against the float64 product of
     the same bf16 inputs rounded to bf16 (F.linear on bf16 tensors): within one bf16 ulp
@@ -180,7 +184,9 @@ def test_linear_rows(cuda, rows, n_out, dim):
 
 
 @pytest.mark.parametrize("rows,n_out,dim", [(1, 4096, 2048), (5, 2048, 1024), (8, 12288, 2048), (2, 1000, 4096),
-                                          (3, 517, 2560), (7, 333, 512)])
+                                          (3, 517, 2560), (7, 333, 512),
+                                          (1, 8209, 2048), (5, 12301, 2048), (8, 12301, 2048),   # partial last rounds
+                                          (1, 4099, 1024), (1, 1027, 1536), (1, 65541, 1536)])
 @pytest.mark.parametrize("with_res", [False, True])
 def test_linear_rows_norm_and_swiglu(cuda, rows, n_out, dim, with_res):
     """The fused-input projections equal their two-launch forms bit for bit: RMSNorm (tg_rmsnorm,
@@ -223,7 +229,8 @@ def test_linear_rows_swiglu_long_rows(cuda, rows, n_out, inter):
     assert torch.equal(got, ref)
 
 
-@pytest.mark.parametrize("rows,inter,dim", [(1, 6144, 2048), (8, 6144, 2048), (2, 1027, 512), (3, 5, 1536), (7, 40000, 2048)])
+@pytest.mark.parametrize("rows,inter,dim", [(1, 6144, 2048), (8, 6144, 2048), (2, 1027, 512), (3, 5, 1536), (7, 40000, 2048),
+                                            (1, 6145, 2048), (5, 6151, 2048), (8, 6145, 2048), (1, 515, 1024)])
 def test_linear_rows_norm_act(cuda, rows, inter, dim):
     """The gate|up projection with the SwiGLU product formed on the way out equals the norm-fused
     projection followed by silu_mul bit for bit (the SwiGLU kernel reads rows of whole 16-byte

@@ -15,7 +15,7 @@ and attention over its segment's used rows are ONE launch (tg_decode_attention).
 prefill without enough headroom is re-laid out once (one copy per layer) into that layout.
 The per-step counters live on the device, so nothing in a step synchronises with the host, and
 every step launches the same kernels with the same arguments: with graph=True the second and
-later steps replay one captured HIP graph of the whole step (146 launches for 28 layers), whose inputs
+later steps replay one captured HIP graph of the whole step (144 launches for 28 layers), whose inputs
 and outputs are static device buffers; the first step runs eagerly and warms every kernel and
 library handle the capture records.
 """
