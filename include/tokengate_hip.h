@@ -46,8 +46,8 @@ const char *tg_last_error(void);
  * workspace: caller-allocated device memory of tg_keybias_fwd_workspace_size() bytes (16-byte
  * aligned) for the key-range split of launches too small to fill the GPU, like the split-KV
  * accumulators the reference's mha_fwd allocates for itself (softmax_lse_accum / out_accum in
- * flash-attn's set_params_splitkv); NULL, or fewer bytes, runs without the split.  Contents need
- * no initialisation; calls that share one workspace must be stream-ordered. */
+ * flash-attn's set_params_splitkv); with NULL, or fewer bytes than its split needs, the launch runs
+ * without one, in the form that is best then.  Contents need no initialisation; calls that share one workspace must be stream-ordered. */
 int tg_keybias_fwd(const void *q, const void *k, const void *v, const float *bias_raw,
                    void *out, float *lse,
                    int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
@@ -60,7 +60,8 @@ int tg_keybias_fwd(const void *q, const void *k, const void *v, const float *bia
                    float softmax_scale, int32_t causal,
                    void *workspace, int64_t workspace_bytes, hipStream_t stream);
 
-/* Workspace bytes tg_keybias_fwd uses for these sizes on the current device (0: it does not split). */
+/* Workspace bytes that hold the key-range split of whichever form tg_keybias_fwd takes for these sizes on the
+ * current device (0: none of them has one; tg_keybias_fwd_plan tells whether the form it takes is split). */
 int64_t tg_keybias_fwd_workspace_size(int32_t batch, int32_t seqlen_q, int32_t seqlen_k,
                                       int32_t num_heads, int32_t num_heads_k, int32_t causal);
 

@@ -27,9 +27,20 @@ def test_form(B, Sq, Sk, H, Hkv, causal, form):
     assert _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, 1 << 40)[:3] == form
 
 
-def test_workspace_is_what_the_plan_needs():
-    """tg_keybias_fwd_workspace_size is 0 exactly where the launch does not split, and with any fewer bytes the
-    launch is the one without a workspace."""
+def split_bytes(s):
+    """Fewest workspace bytes with which a launch that splits does (found by bisection), else 0."""
+    full, lo, hi = _lib.fwd_plan(*s, 1 << 40), 0, 1 << 30
+    if full[2] == 1:
+        return 0
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if _lib.fwd_plan(*s, mid) == full else (mid, hi)
+    return hi
+
+
+def test_a_launch_splits_as_planned_or_not_at_all():
+    """tg_keybias_fwd_workspace_size holds the split of the launch's plan, and with fewer bytes than that split
+    needs the launch is the one without a workspace, never the split of another form."""
     size = _lib.load().tg_keybias_fwd_workspace_size
     split = set()
     for Sq in (1, 3, 64, 200, 700, 1024, 1500, 2320, 3000, 4096):
@@ -38,11 +49,12 @@ def test_workspace_is_what_the_plan_needs():
                 for causal in (True, False):
                     s = (1, Sq, Sk, H, Hkv, causal)
                     n, full, none = size(*s[:5], int(causal)), _lib.fwd_plan(*s, 1 << 40), _lib.fwd_plan(*s, 0)
-                    assert (n > 0) == (full[2] > 1) and none[2] == 1, s
-                    assert _lib.fwd_plan(*s, n) == full
-                    if n > 0:
+                    need = split_bytes(s)
+                    assert n >= need and none[2] == 1 and _lib.fwd_plan(*s, n) == full, s
+                    if need > 0:
                         split.add(full[:2])
-                        assert _lib.fwd_plan(*s, n - 1) == _lib.fwd_plan(*s, 16) == none
+                        for w in (need - 1, need // 2, 16):
+                            assert _lib.fwd_plan(*s, w) == none, (s, w)
     assert split == {(4, 1), (8, 1), (8, 2), (8, 4)}       # every form has launches that split
 
 

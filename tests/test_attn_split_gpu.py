@@ -12,6 +12,7 @@ import torch
 
 from oracle import attention as ora
 from tests.attn_util import assert_close, qkv, to_np
+from tests.test_attn_plan_cpu import split_bytes
 from tokengate_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -19,7 +20,7 @@ pytestmark = pytest.mark.gpu
 
 def _dense(q, k, v, bias_raw, scale, causal, ws_mode="planned"):
     """tg_keybias_fwd with ws_mode 'planned' (the size the library asks for), 'none' or 'short'
-    (one byte less than planned).  Returns out, lse and the planned workspace size."""
+    (one byte less than the launch's split needs).  Returns out, lse and the workspace size asked for."""
     B, Sq, H, D = q.shape
     Sk, Hkv = k.shape[1], k.shape[2]
     out = torch.empty_like(q)
@@ -27,7 +28,8 @@ def _dense(q, k, v, bias_raw, scale, causal, ws_mode="planned"):
     n = int(_lib.load().tg_keybias_fwd_workspace_size(B, Sq, Sk, H, Hkv, int(causal)))
     ws = None
     if ws_mode != "none" and n > 0:
-        ws = torch.full((n if ws_mode == "planned" else n - 1,), 0xFF, dtype=torch.uint8, device=q.device)
+        size = n if ws_mode == "planned" else split_bytes((B, Sq, Sk, H, Hkv, causal)) - 1
+        ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=q.device)
     _lib.call("tg_keybias_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(),
               bias_raw.data_ptr() if bias_raw is not None else None, out.data_ptr(), lse.data_ptr(),
               B, Sq, Sk, H, Hkv, D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
@@ -89,7 +91,7 @@ def test_split_matches_oracle_and_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_b
 @pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,has_bias,form", [CASES[0], CASES[5], CASES[7]],
                          ids=[IDS[0], IDS[5], IDS[7]])
 def test_short_workspace_runs_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_bias, form):
-    """One byte less than planned: not the split's bits (its partials are rounded) but the unsplit launch's."""
+    """One byte less than the split needs: not its bits (its partials are rounded) but the unsplit launch's."""
     g = torch.Generator(device=cuda).manual_seed(5)
     q, k, v = qkv(B, Sq, Sk, H, Hkv, g, cuda)
     scale = 128 ** -0.5
@@ -97,7 +99,7 @@ def test_short_workspace_runs_unsplit(cuda, B, Sq, Sk, H, Hkv, causal, has_bias,
     out_short, lse_short, n = _dense(q, k, v, bias_raw, scale, causal, "short")
     out_none, lse_none, _ = _dense(q, k, v, bias_raw, scale, causal, "none")
     out_split, _, _ = _dense(q, k, v, bias_raw, scale, causal, "planned")
-    assert n > 0 and _lib.fwd_plan(B, Sq, Sk, H, Hkv, causal, n - 1)[2] == 1
+    assert n >= split_bytes((B, Sq, Sk, H, Hkv, causal)) > 0
     assert torch.equal(out_short, out_none) and torch.equal(lse_short, lse_none)
     assert not torch.equal(out_split, out_none)
 

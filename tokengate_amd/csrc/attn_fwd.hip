@@ -1174,8 +1174,8 @@ int keybias_fwd_dense(const void *q, const void *k, const void *v, const float *
   return 0;
 }
 
-// Workspace of a dense or varlen launch's split (a dense one whose key groups are refused for the size of its
-// k or v, see plan_dense, may have another plan, and then runs without a split if that needs more).
+// Workspace of a dense launch (the largest split that any form of it has, so that it holds whatever plan the
+// launch takes) or of a varlen one.
 int64_t fwd_workspace_size(bool varlen, int32_t units_batch, int32_t seqlen_q, int32_t seqlen_k, int32_t num_heads,
                            int32_t num_heads_k, int32_t causal) {
   if (units_batch <= 0 || seqlen_q <= 0 || seqlen_k <= 0 || num_heads <= 0 || num_heads_k <= 0 ||
@@ -1183,9 +1183,11 @@ int64_t fwd_workspace_size(bool varlen, int32_t units_batch, int32_t seqlen_q, i
     return 0;
   const int hp = ((num_heads / num_heads_k) % 2 == 0) ? 2 : 1;
   const int64_t units = (int64_t)units_batch * (num_heads / hp);
-  return (varlen ? plan_varlen(hp, seqlen_q, seqlen_k, units, causal != 0, INT64_MAX)
-                 : plan_dense(hp, seqlen_q, seqlen_k, units, causal != 0, true, true))
-      .split.bytes;
+  if (varlen) return plan_varlen(hp, seqlen_q, seqlen_k, units, causal != 0, INT64_MAX).split.bytes;
+  int64_t bytes = 0;
+  for (const Form &f : kForms)
+    bytes = std::max(bytes, plan_split(f, Tiles(f, hp, seqlen_q, seqlen_k, causal != 0), units).bytes);
+  return bytes;
 }
 
 // Device scratch of tg_keybias_fwd_noalloc: the key-range split's partial results.  plan_split
