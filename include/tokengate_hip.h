@@ -393,22 +393,25 @@ int tg_decode_begin(int64_t *positions, int32_t num_seqs, const float *inv_freq,
 
 /* Attention of one decode step, one query row per sequence, from the raw q|k|v projection rows to the
  * attention output in one launch: q/k RMSNorm, rotary embedding (rope: tg_decode_begin's table) and query
- * scale as tg_qk_norm_rope (same roundings); the new k / v rows written to cache row kv_start[b] + kv_used[b] - 1; then every
- * head over the cache rows kv_start[b] .. kv_start[b] + kv_used[b] - 1 (the new row included), logits
- * softmax_scale * (q . k_j + bias_raw[b, h, j]), fp32 weights.  kv_used[b] is at least 1 and at most
+ * scale as tg_qk_norm_rope (same roundings); the new k / v rows written to cache row
+ * kv_start[b] + kv_used[b] - 1; then every head over the cache rows kv_start[b] .. kv_start[b] + kv_used[b] - 1
+ * (the new row included), logits softmax_scale * (q . k_j + bias_raw[b, h, j]).  The arithmetic and its
+ * roundings are tg_keybias_varlen_kv_fwd's, and so are the bits: weights in bf16, fp32 sums, and where the keys
+ * are split among workgroups each part's normalised result in bf16.  kv_used[b] is at least 1 and at most
  * max_seqlen_k (FormDecodeState.step, qwen3_flex_attention.py:1017-1117).
  * out: bf16 rows (num_heads * 128); tensors 16-byte aligned, row strides multiples of 8 elements.  The scales
- * are dense fp32: q_head_scale[num_heads], q_row_scale[num_seqs].  workspace: tg_decode_attention_workspace_size bytes, zeroed once
- * when it is allocated; every launch leaves the words it counts in at zero, so launches of one stream
- * share it (launches that may overlap need one each). */
+ * are dense fp32: q_head_scale[num_heads], q_row_scale[num_seqs].  workspace:
+ * tg_decode_attention_workspace_size bytes, zeroed once when it is allocated; every launch leaves the words it
+ * counts in at zero, so launches of one stream, of any sizes that it holds, share it (launches that may overlap
+ * need one each). */
 int64_t tg_decode_attention_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_heads_k,
                                            int32_t max_seqlen_k);
 int tg_decode_attention(const void *qkv, int64_t qkv_row_stride, const float *rope, int32_t num_seqs,
                         int32_t num_heads, int32_t num_heads_k, int32_t head_dim, const void *q_norm_weight,
                         const void *k_norm_weight, float eps, const float *q_head_scale, const float *q_row_scale,
                         void *k_cache, int64_t k_row_stride, void *v_cache, int64_t v_row_stride,
-                        const int32_t *kv_start, const int32_t *kv_used, int32_t max_seqlen_k, const float *bias_raw, int64_t bias_seq_stride,
-                        int64_t bias_head_stride, float softmax_scale, void *out, int64_t out_row_stride,
+                        const int32_t *kv_start, const int32_t *kv_used, int32_t max_seqlen_k, const float *bias_raw,
+                        int64_t bias_seq_stride, int64_t bias_head_stride, float softmax_scale, void *out, int64_t out_row_stride,
                         void *workspace, int64_t workspace_bytes, hipStream_t stream);
 
 /* Greedy next token: out[b] = argmax_v x[b, v] (int64) with torch.argmax's rules (a NaN wins, ties

@@ -203,8 +203,8 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
       raw_rsrc(bbase, (HAS_BIAS && sk > 0) ? (uint32_t)(((int64_t)(HP - 1) * a.bias_hs + sk) * 4) : 0u);
 
   // this wave's 32 columns: 32 query positions of one head (HP = 2: the first half of a group's column
-  // waves the first head of the pair, the others the second), block cb (0, 1) = positions 16 cb .. 16 cb + 15, lane l holding column
-  // l % 16 of each block; one head per wave means one bias row per wave
+  // waves the first head of the pair, the others the second), block cb (0, 1) = positions 16 cb ..
+  // 16 cb + 15, lane l holding column l % 16 of each block; one head per wave means one bias row per wave
   const int cw = KS == 1 ? wave : wave % CW, kg = KS == 1 ? 0 : wave / CW;
   const int hw = HP == 2 ? cw / (CW / 2) : 0;
   const int qw0 = q0 + QW * (HP == 2 ? cw % (CW / 2) : cw);

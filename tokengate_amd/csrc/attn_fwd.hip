@@ -1427,8 +1427,9 @@ extern "C" int64_t tg_decode_attention_workspace_size(int32_t num_seqs, int32_t 
 extern "C" int tg_decode_attention(const void *qkv, int64_t qkv_row_stride, const float *rope, int32_t num_seqs,
                                    int32_t num_heads, int32_t num_heads_k, int32_t head_dim, const void *q_norm_weight,
                                    const void *k_norm_weight, float eps, const float *q_head_scale,
-                                   const float *q_row_scale, void *k_cache, int64_t k_row_stride, void *v_cache, int64_t v_row_stride, const int32_t *kv_start,
-                                   const int32_t *kv_used, int32_t max_seqlen_k, const float *bias_raw,
+                                   const float *q_row_scale, void *k_cache, int64_t k_row_stride, void *v_cache,
+                                   int64_t v_row_stride, const int32_t *kv_start, const int32_t *kv_used,
+                                   int32_t max_seqlen_k, const float *bias_raw,
                                    int64_t bias_seq_stride, int64_t bias_head_stride, float softmax_scale, void *out,
                                    int64_t out_row_stride, void *workspace, int64_t workspace_bytes,
                                    hipStream_t stream) {

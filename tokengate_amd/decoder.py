@@ -242,21 +242,22 @@ def decode_begin(positions: torch.Tensor, inv_freq: torch.Tensor, kv_used: Optio
         raise RuntimeError("decode_begin: slots must be contiguous fp32 (B,)")
     rope = torch.empty(B, 64, 2, dtype=torch.float32, device=positions.device)
     ratio = torch.empty(B, dtype=torch.float32, device=positions.device) if slots is not None else None
+    groups = kv_used.numel() // B if kv_used is not None and B else 0
     _lib.call("tg_decode_begin", positions.data_ptr(), B, inv_freq.data_ptr(), rope.data_ptr(),
-              kv_used.data_ptr() if kv_used is not None else None, kv_used.numel() // B if kv_used is not None and B else 0,
+              kv_used.data_ptr() if kv_used is not None else None, groups,
               slots.data_ptr() if slots is not None else None, ratio.data_ptr() if ratio is not None else None,
               _stream(positions))
     return rope, ratio
 
 
-def decode_attention(qkv: torch.Tensor, rope: torch.Tensor, lw: LayerWeights, shape: DecoderShape, k: torch.Tensor, v: torch.Tensor, kv_start: torch.Tensor,
-                     kv_used: torch.Tensor, max_k: int, scale: float, workspace: torch.Tensor,
-                     bias_raw: Optional[torch.Tensor] = None, q_head_scale: Optional[torch.Tensor] = None,
+def decode_attention(qkv: torch.Tensor, rope: torch.Tensor, lw: LayerWeights, shape: DecoderShape, k: torch.Tensor,
+                     v: torch.Tensor, kv_start: torch.Tensor, kv_used: torch.Tensor, max_k: int, scale: float,
+                     workspace: torch.Tensor, bias_raw: Optional[torch.Tensor] = None, q_head_scale: Optional[torch.Tensor] = None,
                      q_row_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """qk_norm_rope and varlen_kv_attention of one row per sequence in one launch (tg_decode_attention), at
-    the positions of decode_begin's rotary table:
-    the new key of sequence b goes to cache row kv_start[b] + kv_used[b] - 1 and its query attends over
-    rows kv_start[b] .. kv_start[b] + kv_used[b] - 1; bias_raw (nseq, H, >= max_k) as varlen_kv_attention."""
+    the positions of decode_begin's rotary table: the new key of sequence b goes to cache row
+    kv_start[b] + kv_used[b] - 1 and its query attends over rows kv_start[b] .. kv_start[b] + kv_used[b] - 1;
+    bias_raw (nseq, H, >= max_k) as varlen_kv_attention."""
     B = qkv.shape[0]
     H, Hkv, D = shape.n_heads, shape.n_kv_heads, shape.head_dim
     out = torch.empty(B, H, D, dtype=qkv.dtype, device=qkv.device) if out is None else out
