@@ -47,7 +47,8 @@ const char *tg_last_error(void);
  * aligned) for the key-range split of launches too small to fill the GPU, like the split-KV
  * accumulators the reference's mha_fwd allocates for itself (softmax_lse_accum / out_accum in
  * flash-attn's set_params_splitkv); with NULL, or fewer bytes than its split needs, the launch runs
- * without one, in the form that is best then.  Contents need no initialisation; calls that share one workspace must be stream-ordered. */
+ * without one, in the form that is best then.  Contents need no initialisation; calls that share one
+ * workspace must be stream-ordered. */
 int tg_keybias_fwd(const void *q, const void *k, const void *v, const float *bias_raw,
                    void *out, float *lse,
                    int32_t batch, int32_t seqlen_q, int32_t seqlen_k,

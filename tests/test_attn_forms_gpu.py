@@ -186,6 +186,29 @@ def test_varlen_tile_order(cuda, name, H, Hkv):
             assert_close_grad(f"{what} {b}", to_np(got), ref.cpu().numpy())
 
 
+def test_varlen_backward_with_a_far_larger_max_seqlen(cuda):
+    """max_seqlen may be any bound on the lengths: the gradients are those of the exact one, and the host does
+    not walk over tiles that cannot exist (half a million of them per estimate)."""
+    import time
+    from tokengate_amd.fa2bias.keybias import ext
+    lens = [300, 77, 1200]
+    g = torch.Generator(device=cuda).manual_seed(6)
+    q, k, v, dout = (torch.randn(sum(lens), h, 128, generator=g, device=cuda).to(torch.bfloat16) for h in (4, 2, 2, 4))
+    cu = torch.tensor([0, 300, 377, 1577], dtype=torch.int32, device=cuda)
+    out, lse, _, _ = ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, None, 1200, 1200, 0.0, 0.1, False, True,
+                                      -1, -1, 0.0, False, None)
+    got, host = [], []
+    for mx in (1200, 1 << 24):
+        t = time.perf_counter()
+        got.append(ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, None, mx, mx, 0.0, 0.1, False, True,
+                                    -1, -1, 0.0, False, None, None)[:3])
+        host.append(time.perf_counter() - t)
+    torch.cuda.synchronize()
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+    assert host[1] < 0.1
+
+
 def _times(lens, heads, causal, device):
     """Time of a packed forward and backward in us, best of ten replays of five launches each."""
     from tokengate_amd.fa2bias.keybias import ext

@@ -805,6 +805,7 @@ struct Levels {
   int level(int r) const { return r < n - rest ? n - 1 - r : rest - 1 - (r - (n - rest)) / (1 + others); }
 };
 Levels levels_of(const BwdArgs &a, bool varlen, int len, int tile) {
+  if (varlen) len = (int)std::min<int64_t>(len, a.lse_total);   // max_seqlen may be far above any length
   Levels v{(len + tile - 1) / tile, 0, 0};
   if (varlen && a.batch > 1) {
     v.others = a.batch - 1;

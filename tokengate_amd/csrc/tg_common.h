@@ -241,7 +241,7 @@ struct LevelTile {
 template <int ROWS>
 __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int max_len, int i, int lane) {
   const int len = lane < n ? max(0, min(cu[lane + 1] - cu[lane], max_len)) : 0;
-  const int nt = (len + ROWS - 1) / ROWS, levels = (max_len + ROWS - 1) / ROWS;
+  const int nt = (len + ROWS - 1) / ROWS, levels = (int)(((uint32_t)max(1, max_len) + (ROWS - 1)) / ROWS);   // >= 1
   int level = 0, above = 0;   // the tile's level and the tiles above it
   int place = 0;              // of this lane's sequence among those that reach the level
   if (n <= 16) {

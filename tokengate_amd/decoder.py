@@ -252,8 +252,9 @@ def decode_begin(positions: torch.Tensor, inv_freq: torch.Tensor, kv_used: Optio
 
 def decode_attention(qkv: torch.Tensor, rope: torch.Tensor, lw: LayerWeights, shape: DecoderShape, k: torch.Tensor,
                      v: torch.Tensor, kv_start: torch.Tensor, kv_used: torch.Tensor, max_k: int, scale: float,
-                     workspace: torch.Tensor, bias_raw: Optional[torch.Tensor] = None, q_head_scale: Optional[torch.Tensor] = None,
-                     q_row_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     workspace: torch.Tensor, bias_raw: Optional[torch.Tensor] = None,
+                     q_head_scale: Optional[torch.Tensor] = None, q_row_scale: Optional[torch.Tensor] = None,
+                     out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """qk_norm_rope and varlen_kv_attention of one row per sequence in one launch (tg_decode_attention), at
     the positions of decode_begin's rotary table: the new key of sequence b goes to cache row
     kv_start[b] + kv_used[b] - 1 and its query attends over rows kv_start[b] .. kv_start[b] + kv_used[b] - 1;
