@@ -209,11 +209,12 @@ def test_varlen_backward_with_a_far_larger_max_seqlen(cuda):
     assert host[1] < 0.1
 
 
-def _times(lens, heads, causal, device):
+def _times(lens, heads, causal, device, heads_k=None):
     """Time of a packed forward and backward in us, best of ten replays of five launches each."""
     from tokengate_amd.fa2bias.keybias import ext
     g = torch.Generator(device=device).manual_seed(sum(lens))
-    q, k, v, dout = (torch.randn(sum(lens), heads, 128, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
+    q, k, v, dout = (torch.randn(sum(lens), h, 128, generator=g, device=device).to(torch.bfloat16)
+                     for h in (heads, heads_k or heads, heads_k or heads, heads))
     cu, mx = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=device), max(lens)
     fw = lambda: ext().varlen_fwd(q, k, v, None, cu, cu, None, None, None, None, mx, mx, 0.0, 0.1, False, causal,
                                   -1, -1, 0.0, False, None)
@@ -256,6 +257,17 @@ def test_varlen_non_causal_runs_sequence_after_sequence(cuda):
     short, major = _times([6000, 4000] + [64] * 62, 8, False, cuda), _times([6000, 4000] + [64] * 63, 8, False, cuda)
     print(f"non-causal, 64 / 65 sequences: forward {short[0]:.1f} / {major[0]:.1f} us, backward {short[1]:.1f} / {major[1]:.1f}")
     assert short[0] < 1.1 * major[0] and short[1] < 1.1 * major[1]
+
+
+def test_varlen_forward_level_order_only_where_it_balances(cuda):
+    """Where every query tile has a place from the start the forward runs sequence after sequence, so the causal
+    mask makes no such batch slower (level order, which only causal launches take: 1.15 times).  So do sequences
+    of one length with up to three tiles: 64 take the time of 65, which never run in level order (1.1 times)."""
+    lens = list(range(21, 81, 4)) + [80]
+    causal, full = _times(lens, 16, True, cuda, 8)[0], _times(lens, 16, False, cuda, 8)[0]
+    few, major = _times([354] * 64, 16, True, cuda, 8)[0], _times([354] * 65, 16, True, cuda, 8)[0]
+    print(f"one round, causal / full: {causal:.1f} / {full:.1f} us, 64 / 65 sequences: {few:.1f} / {major:.1f} us")
+    assert causal < 1.02 * full and few < 1.08 * major
 
 
 def test_varlen_short_rows_keep_one_group(cuda):

@@ -174,15 +174,16 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
   // varlen: level order, or sequence-major (resident workgroups share one sequence's K/V in L2 / MALL)
   int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
   int qt = a.n_tiles - 1 - (VARLEN ? rest % a.n_tiles : rest / a.batch);
-  if constexpr (VARLEN) {
-    if (a.level_order) {
-      const LevelTile lt = level_tile<BM>(a.cu_seqlens, a.batch, a.sq, rest, lane);
-      if (lt.seq < 0) return;
-      b = lt.seq;
-      qt = lt.level;
-    }
+  Seq sq_;
+  if (VARLEN && a.level_order) {
+    const LevelTile lt = level_tile<BM>(a.cu_seqlens, a.batch, a.sq, rest, lane);
+    if (lt.seq < 0) return;
+    b = lt.seq;
+    qt = lt.level;
+    sq_ = Seq{lt.row0, lt.len, lt.len};
+  } else {
+    sq_ = seq_of<VARLEN>(a, b);
   }
-  const Seq sq_ = seq_of<VARLEN>(a, b);
   const int sq = sq_.sq, sk = sq_.sk;
   const int64_t row0 = sq_.row0;
   const int q0 = qt * BM;
@@ -510,15 +511,16 @@ __global__ __launch_bounds__(kK16Threads, 1) void bwd_dkdv16_kernel(BwdArgs a) {
   const int rest = blockIdx.x / a.hkv;
   int b = VARLEN ? rest / a.n_tiles : rest % a.batch;
   int kt = VARLEN ? rest % a.n_tiles : rest / a.batch;
-  if constexpr (VARLEN) {
-    if (a.level_order) {   // a key tile's causal work is the query tiles after it
-      const LevelTile lt = level_tile<kKBlock>(a.cu_seqlens, a.batch, a.sq, rest, lane);
-      if (lt.seq < 0) return;
-      b = lt.seq;
-      kt = lt.n_tiles - 1 - lt.level;
-    }
+  Seq sq_;
+  if (VARLEN && a.level_order) {   // a key tile's causal work is the query tiles after it
+    const LevelTile lt = level_tile<kKBlock>(a.cu_seqlens, a.batch, a.sq, rest, lane);
+    if (lt.seq < 0) return;
+    b = lt.seq;
+    kt = lt.n_tiles - 1 - lt.level;
+    sq_ = Seq{lt.row0, lt.len, lt.len};
+  } else {
+    sq_ = seq_of<VARLEN>(a, b);
   }
-  const Seq sq_ = seq_of<VARLEN>(a, b);
   const int sq = sq_.sq, sk = sq_.sk;
   const int64_t row0 = sq_.row0;
   const int n0 = kt * kKBlock;
@@ -850,9 +852,11 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
   const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
   const int bmq = dq_bm(ks, hp);
   a.n_tiles = (a.sq + bmq - 1) / bmq;
-  a.level_order = level_order && a.n_tiles > 1;   // one tile each: sequence after sequence is the same order
-  const unsigned nq = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, bmq) : (int64_t)a.n_tiles * a.batch) *
-                                 (a.h / hp));
+  // (with one tile each, sequence after sequence is the same order; where all have a place from the start, the
+  // order decides nothing)
+  const int64_t level_q = level_tiles(a.batch, a.lse_total, bmq) * (a.h / hp);
+  a.level_order = level_order && a.n_tiles > 1 && level_q > device_cus();
+  const unsigned nq = (unsigned)(a.level_order ? level_q : (int64_t)a.n_tiles * a.batch * (a.h / hp));
 #define TG_DQ(K, HPV, C, B)                                                                            \
   if (ks == K && hp == HPV && causal == C && has_bias == B)                                            \
     hipLaunchKernelGGL((bwd_dq_kernel<K, HPV, C, B, VARLEN>), dim3(nq), dim3(kQThreads), 0, st, a);
@@ -865,9 +869,9 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
   const int kq = groups ? dkv_groups(a, causal, VARLEN) : 1;
   const int keys = dkv_keys(kq);
   a.n_tiles = (a.sk + keys - 1) / keys;
-  a.level_order = level_order && a.n_tiles > 1;
-  const unsigned nk = (unsigned)((a.level_order ? level_tiles(a.batch, a.lse_total, keys) : (int64_t)a.n_tiles * a.batch) *
-                                 a.hkv);
+  const int64_t level_k = level_tiles(a.batch, a.lse_total, keys) * a.hkv;
+  a.level_order = level_order && a.n_tiles > 1 && level_k > device_cus();
+  const unsigned nk = (unsigned)(a.level_order ? level_k : (int64_t)a.n_tiles * a.batch * a.hkv);
 #define TG_DKV(K, C, B)                                                                                \
   if (kq == K && causal == C && has_bias == B)                                                         \
     hipLaunchKernelGGL((bwd_dkdv16_kernel<K, C, B, VARLEN>), dim3(nk), dim3(kK16Threads), 0, st, a);

@@ -236,11 +236,12 @@ __device__ __forceinline__ int wave_sum_int(int x) {
 // backward: bisection 683 us, with the longest first at a level (whose places in the order then do not move
 // when others join) 681, lane by level 677.
 struct LevelTile {
-  int seq, level, n_tiles;   // n_tiles: of that sequence
+  int seq, level;
+  int n_tiles, row0, len;   // of that sequence: the lanes hold them, a load by its index would wait once more
 };
 template <int ROWS>
 __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int max_len, int i, int lane) {
-  const int len = lane < n ? max(0, min(cu[lane + 1] - cu[lane], max_len)) : 0;
+  const int row0 = lane < n ? cu[lane] : 0, len = lane < n ? max(0, min(cu[lane + 1] - row0, max_len)) : 0;
   const int nt = (len + ROWS - 1) / ROWS, levels = (int)(((uint32_t)max(1, max_len) + (ROWS - 1)) / ROWS);   // >= 1
   int level = 0, above = 0;   // the tile's level and the tiles above it
   int place = 0;              // of this lane's sequence among those that reach the level
@@ -251,7 +252,7 @@ __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int ma
       int t = 0;   // tiles at level l and above, falling from lane to lane
       for (int j = 0; j < n; ++j) t += max(0, __builtin_amdgcn_readlane(nt, j) - l);
       const int k = __builtin_popcountll(__builtin_amdgcn_ballot_w64(t > i));
-      if (k == 0) return LevelTile{-1, 0, 0};
+      if (k == 0) return LevelTile{-1, 0, 0, 0, 0};
       level += s * (k - 1);
       above = k < 64 ? __builtin_amdgcn_readlane(t, k) : above;
       if (s == 1) break;
@@ -263,7 +264,7 @@ __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int ma
     }
   } else {
     auto from = [&](int l) { return __builtin_amdgcn_readfirstlane(wave_sum_int(max(0, nt - l))); };
-    if (i >= from(0)) return LevelTile{-1, 0, 0};
+    if (i >= from(0)) return LevelTile{-1, 0, 0, 0, 0};
     int hi = levels;   // from(level) > i >= above = from(hi)
     while (hi - level > 1) {
       const int mid = (level + hi) >> 1, t = from(mid);
@@ -278,7 +279,8 @@ __device__ __forceinline__ LevelTile level_tile(const int32_t *cu, int n, int ma
     place = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
   }
   const int seq = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(nt > level && place == i - above));
-  return LevelTile{seq, level, __builtin_amdgcn_readlane(nt, seq)};
+  return LevelTile{seq, level, __builtin_amdgcn_readlane(nt, seq), __builtin_amdgcn_readlane(row0, seq),
+                   __builtin_amdgcn_readlane(len, seq)};
 }
 
 // Index of this wave in its workgroup, held in a scalar register.  The compiler cannot prove that
