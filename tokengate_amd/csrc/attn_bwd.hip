@@ -240,34 +240,15 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
       if constexpr (VARLEN) dsum[cb] = a.softmax_d[li];
     }
   }
-  // D = rowsum(dO * O) of this workgroup's rows (dense: every row belongs to one workgroup, which also
-  // writes it for the dK/dV kernel; varlen rows outside every sequence have none, so there the
-  // preprocess kernel forms it).  The order of the sum is the preprocess kernel's, so its bits: each
-  // 16-byte piece (4 ks4 + G there) element by element, then neighbouring pieces pairwise.
-  if constexpr (!VARLEN) {
-    const int64_t ob = (int64_t)b * a.o_bs;
+  // dense: O as well, for D below
+  u32x4 of[2][4];
+  if constexpr (!VARLEN)
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      float d[4];
+    for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-      for (int ks4 = 0; ks4 < 4; ++ks4) {
-        const u32x4 ov = gload16(a.o + ob + (int64_t)qrow[cb] * a.o_rs + (int64_t)hh[cb] * a.o_hs + 32 * ks4 + 8 * G,
-                                 qvalid[cb]);
-        const u32x4 dv = __builtin_bit_cast(u32x4, df[cb][ks4]);
-        float acc = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          acc += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
-          acc += bf16_to_f32((bf16_t)(ov[w] >> 16)) * bf16_to_f32((bf16_t)(dv[w] >> 16));
-        }
-        d[ks4] = quad_sum(acc);
-      }
-      dsum[cb] = (d[0] + d[1]) + (d[2] + d[3]);
-      if (qvalid[cb] && G == 0 && kg == 0) a.softmax_d[((int64_t)b * a.h + hh[cb]) * sq + qrow[cb]] = dsum[cb];
-    }
-  }
-
-  const f32x4 nd4[2] = {f32x4{-dsum[0], -dsum[0], -dsum[0], -dsum[0]}, f32x4{-dsum[1], -dsum[1], -dsum[1], -dsum[1]}};
+      for (int ks4 = 0; ks4 < 4; ++ks4)
+        of[cb][ks4] = gload16(a.o + (int64_t)b * a.o_bs + (int64_t)qrow[cb] * a.o_rs + (int64_t)hh[cb] * a.o_hs +
+                                  32 * ks4 + 8 * G, qvalid[cb]);
   int kv_end = sk;
   if constexpr (CAUSAL) kv_end = min(sk, q0 + BM + off);
   const int n_tiles = kv_end > 0 ? (kv_end + SK - 1) / SK : 0;
@@ -340,6 +321,32 @@ __global__ __launch_bounds__(kQThreads, 1) void bwd_dq_kernel(BwdArgs a) {
     for (int d = 0; d < 8; ++d) dqacc[cb][d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   if (n_tiles > 0) issue_tile(0, 0);
+  // D = rowsum(dO * O) of this workgroup's rows (dense: every row belongs to one workgroup, which also
+  // writes it for the dK/dV kernel; varlen rows outside every sequence have none, so there the
+  // preprocess kernel forms it).  The order of the sum is the preprocess kernel's, so its bits: each
+  // 16-byte piece (4 ks4 + G there) element by element, then neighbouring pieces pairwise.  Formed while the
+  // first tile is on its way: ahead of it, a row of tiles waited for O first and then for K and V (48 rows,
+  // whole backward 18.2 us, now 17.5).
+  if constexpr (!VARLEN) {
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      float d[4];
+#pragma unroll
+      for (int ks4 = 0; ks4 < 4; ++ks4) {
+        const u32x4 ov = of[cb][ks4], dv = __builtin_bit_cast(u32x4, df[cb][ks4]);
+        float acc = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          acc += bf16_to_f32((bf16_t)(ov[w] & 0xffff)) * bf16_to_f32((bf16_t)(dv[w] & 0xffff));
+          acc += bf16_to_f32((bf16_t)(ov[w] >> 16)) * bf16_to_f32((bf16_t)(dv[w] >> 16));
+        }
+        d[ks4] = quad_sum(acc);
+      }
+      dsum[cb] = (d[0] + d[1]) + (d[2] + d[3]);
+      if (qvalid[cb] && G == 0 && kg == 0) a.softmax_d[((int64_t)b * a.h + hh[cb]) * sq + qrow[cb]] = dsum[cb];
+    }
+  }
+  const f32x4 nd4[2] = {f32x4{-dsum[0], -dsum[0], -dsum[0], -dsum[0]}, f32x4{-dsum[1], -dsum[1], -dsum[1], -dsum[1]}};
   for (int t = 0; t < n_tiles; ++t) {
     const int buf = t & 1;
     const int n0 = t * SK + KN * kg;   // this wave's first key of the step
