@@ -209,8 +209,27 @@ def test_varlen_backward_with_a_far_larger_max_seqlen(cuda):
     assert host[1] < 0.1
 
 
+def _best(f):
+    """Time of f in us, best of ten replays of five launches each."""
+    graph = torch.cuda.CUDAGraph()
+    f()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        for _ in range(5):
+            f()
+    t = 1e9
+    for _ in range(10):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        graph.replay()
+        b.record()
+        b.synchronize()
+        t = min(t, a.elapsed_time(b) * 200)
+    return t
+
+
 def _times(lens, heads, causal, device, heads_k=None):
-    """Time of a packed forward and backward in us, best of ten replays of five launches each."""
+    """Times of a packed forward and backward in us."""
     from tokengate_amd.fa2bias.keybias import ext
     g = torch.Generator(device=device).manual_seed(sum(lens))
     q, k, v, dout = (torch.randn(sum(lens), h, 128, generator=g, device=device).to(torch.bfloat16)
@@ -221,24 +240,7 @@ def _times(lens, heads, causal, device, heads_k=None):
     out, lse, _, _ = fw()
     bw = lambda: ext().varlen_bwd(dout, q, k, v, out, lse, None, None, None, cu, cu, None, mx, mx, 0.0, 0.1, False,
                                   causal, -1, -1, 0.0, False, None, None)
-    best = []
-    for f in (fw, bw):
-        graph = torch.cuda.CUDAGraph()
-        f()
-        torch.cuda.synchronize()
-        with torch.cuda.graph(graph):
-            for _ in range(5):
-                f()
-        t = 1e9
-        for _ in range(10):
-            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            a.record()
-            graph.replay()
-            b.record()
-            b.synchronize()
-            t = min(t, a.elapsed_time(b) * 200)
-        best.append(t)
-    return best
+    return [_best(fw), _best(bw)]
 
 
 @pytest.mark.parametrize("rows", [100, 500])
@@ -276,3 +278,18 @@ def test_varlen_short_rows_keep_one_group(cuda):
     few, major = _times([91] + [40] * 61, 8, True, cuda), _times([91] + [40] * 64, 8, True, cuda)
     print(f"62 / 65 short sequences: backward {few[1]:.1f} / {major[1]:.1f} us")
     assert few[1] < 1.12 * major[1]
+
+
+@pytest.mark.parametrize("rows", [16, 32, 48])
+def test_few_rows_keep_one_group(cuda, rows):
+    """The dense backward of up to 64 rows takes one group, as the packed one does, and so is faster than that by
+    the packed one's third launch (four groups, three of them idle, took as long as the packed one)."""
+    from tokengate_amd.fa2bias.keybias import ext
+    g = torch.Generator(device=cuda).manual_seed(rows)
+    q, k, v, dout = (torch.randn(1, rows, h, 128, generator=g, device=cuda).to(torch.bfloat16) for h in (16, 8, 8, 16))
+    out, lse, _, _ = ext().fwd(q, k, v, None, None, 0.0, 0.1, True, -1, -1, 0.0, False, None)
+    dense = _best(lambda: ext().bwd(dout, q, k, v, out, lse, None, None, None, None, 0.0, 0.1, True, -1, -1, 0.0, False,
+                                    None, None))
+    packed = _times([rows], 16, True, cuda, 8)[1]
+    print(f"{rows} rows: backward dense {dense:.1f}, packed {packed:.1f} us")
+    assert dense < 0.96 * packed

@@ -834,6 +834,10 @@ int dq_groups(const BwdArgs &a, int hp, bool causal, bool varlen) {
   });
 }
 int dkv_groups(const BwdArgs &a, bool causal, bool varlen) {
+  // One step of one group holds every query, and half a workgroup every key: most of more groups would idle (16
+  // rows, whole backward 13.3 us with one, 15.9 with four; 48 rows 15.8 / 17.7).  From about 80 keys on the larger
+  // number of workgroups pays (64 queries x 80 keys 20.2 / 21.1, 64 x 128 23.1 / 21.1, 16 x 256 20.4 / 19.5).
+  if (a.sq <= 64 && a.sk <= 64) return 1;
   return cheapest(kDkvForms, varlen, [&](const GroupForm &f) {
     const int keys = dkv_keys(f.groups), slot = f.groups == 1 ? 64 : 128;
     const Levels v = levels_of(a, varlen, a.sk, keys);
