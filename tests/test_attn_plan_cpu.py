@@ -15,8 +15,14 @@ from tokengate_amd import _lib
     (16, 512, 512, 16, 8, True, (8, 1, 1)),       # 36; four waves 37.4
     (3, 1700, 1700, 12, 4, True, (4, 1, 1)),      # 42; two key groups 44.5
     (16, 225, 225, 8, 2, True, (4, 1, 1)),        # two key groups 1.15 times
+    (1, 3510, 5394, 4, 4, True, (4, 1, 4)),       # 43; eight waves 48
     (1, 6000, 6000, 16, 8, True, (4, 1, 1)),      # 145; two key groups 162
     (1, 8192, 8192, 16, 8, True, (8, 1, 1)), (1, 32768, 32768, 16, 8, True, (8, 1, 1)),
+    # eight against four waves in two rounds and over
+    (16, 1074, 1074, 8, 8, True, (4, 1, 1)),      # 56; eight waves 64
+    (64, 287, 446, 12, 4, True, (4, 1, 1)),       # 76; 95
+    (64, 112, 112, 8, 8, False, (4, 1, 1)),       # 17; 19
+    (1, 8040, 8040, 16, 8, True, (8, 1, 1)),      # 231; four waves 258
     # key groups
     (1, 1024, 1024, 16, 8, True, (8, 4, 1)),      # 18; four waves, split 24
     (1, 2048, 2048, 16, 8, True, (8, 4, 1)),      # 34; 42

@@ -52,7 +52,7 @@ CASES = [
     (1, 1500, 1500, 6, 2, True, True, (4, 1)),       # odd GQA group (one head per MFMA column block)
     (1, 1200, 1200, 6, 2, False, True, (4, 1)),      # non-causal: every tile as heavy as the last
     (1, 700, 3000, 16, 8, True, False, (4, 1)),      # Sq < Sk, no bias
-    (1, 1, 3000, 16, 8, True, True, (4, 1)),         # one decode row
+    (1, 1, 3000, 16, 8, True, True, (8, 4)),         # one decode row
     (1, 200, 20000, 16, 8, True, True, (8, 1)),      # a chunk of a prompt over a long cache
     (1, 64, 131072, 16, 8, True, True, (8, 2)),      # the key groups' partials: over a very long cache,
     (1, 1, 20000, 16, 8, True, True, (8, 4)),        # one row over a long one,

@@ -1010,8 +1010,14 @@ float launch_cost(const Form &f, const Tiles &t, int64_t units, const SplitPlan 
     const int light = p.n_heavy < t.n_qtiles ? t.steps(t.n_qtiles - 1 - p.n_heavy) : 0;
     const int longest = std::max(chunk, light);
     if (f.nw == 8) return f.solo * longest + f.group + f.combine;
-    const int64_t n_longest = chunk > light ? p.heavy_units * p.ns : (t.n_qtiles - p.n_heavy) * units;
-    const int partner = n_longest > cus ? longest : std::min(chunk, light);
+    // the heaviest workgroup's partner on its CU is the (CUs + 1)-th by length
+    int partner = std::min(chunk, light);
+    if (chunk > light) {
+      const int r = (int)(cus / (units * p.ns));   // of that tile
+      if (r < p.n_heavy) partner = (t.steps(t.n_qtiles - 1 - r) + p.ns - 1) / p.ns;
+    } else if ((t.n_qtiles - p.n_heavy) * units > cus) {
+      partner = longest;
+    }
     return f.solo * longest + (f.full - f.solo) * partner + f.group + f.combine;
   }
   const float cost = grid_cost(t.n_qtiles, units, cus * (8 / f.nw), f.group, f.solo, f.full,
@@ -1028,19 +1034,22 @@ struct FwdPlan {
 };
 
 // A dense launch's form and split.  Without key groups: eight waves where the grid gives at least two
-// workgroups per CU, else four, with the split where they have one (splits).  Another
-// form, with or without its split, takes their place where the estimate promises 10 % (against a
-// split launch) or 20 %, about what it is off by between forms: of 151 launches timed in each form (33 to
-// 12000 rows, up to 32768 keys) no choice is then more than 2 % slower than the first rule's, and on
-// average they take 6.2 % less (7.3 with the best form of each).  With no margin 17 were slower, by up to
+// workgroups per CU, else four, with the split where they have one (splits).  Another form, with or without
+// its split, takes their place where the estimate promises about what it is off by: against a split launch
+// 10 %, with key groups anything; against an unsplit one 20 %, and without any split 10 % from eight waves
+// to four and 6 % from four to eight.  Of 151 launches timed in each form (33 to 12000 rows, up to 32768 keys) and
+// 82 more of two rounds and over, none is then more than 2 % slower than the first rule's, and on average they
+// take 6.4 % and 4.4 % less.
+// Eight against four waves: 16 x 1074 rows of 8 / 8 heads 64 / 56 us, 64 x 287 x 446 of 12 / 4 95 / 76, 8040 of
+// 16 / 8 231 / 258, where the grid just misses two per CU.  With no margin 17 of the 151 were slower, by up to
 // 15 %: 3000 rows over 32768 keys 760 -> 830 us, 3072 x 4096 without the mask 108 -> 117.
 // key_groups: whether ks > 1 may be taken (its last step's LDS DMA offsets reach up to 127 rows past sk and
 // must not wrap at 4 GiB).
 FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool splits, bool key_groups) {
   FwdPlan best;
   float best_cost = INFINITY;
-  // the form with its split if wanted, and if it has one
-  auto consider = [&](const Form &f, bool split) {
+  // the form with its split if wanted, and if it has one, where it costs less than the best so far and `limit`
+  auto consider = [&](const Form &f, bool split, float limit) {
     const Tiles t(f, hp, sq, sk, causal);
     SplitPlan p;
     if (split) {
@@ -1048,7 +1057,7 @@ FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool spli
       if (p.ns == 1) return false;
     }
     const float cost = launch_cost(f, t, units, p);
-    if (cost < best_cost) {
+    if (cost < std::min(best_cost, limit)) {
       best_cost = cost;
       best.nw = f.nw;
       best.ks = f.ks;
@@ -1058,12 +1067,14 @@ FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool spli
     return true;
   };
   const Form &first = kForms[Tiles(kForms[0], hp, sq, sk, causal).n_qtiles * units >= 2 * device_cus() ? 0 : 1];
-  if (!consider(first, true)) consider(first, false);
-  best_cost *= best.split.ns > 1 ? 0.9f : 0.8f;
+  if (!consider(first, true, INFINITY)) consider(first, false, INFINITY);
+  const float first_cost = best_cost;
+  const bool first_split = best.split.ns > 1;
   for (const Form &f : kForms) {
     if (f.ks > 1 && !key_groups) continue;
-    consider(f, true);
-    consider(f, false);
+    const float margin = !first_split ? 0.8f : f.ks > 1 ? 1.f : 0.9f;
+    consider(f, true, margin * first_cost);
+    consider(f, false, (first_split || f.ks > 1 ? margin : f.nw == 4 ? 0.9f : 0.94f) * first_cost);
   }
   return best;
 }
