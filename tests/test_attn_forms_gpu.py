@@ -293,3 +293,13 @@ def test_few_rows_keep_one_group(cuda, rows):
     packed = _times([rows], 16, True, cuda, 8)[1]
     print(f"{rows} rows: backward dense {dense:.1f}, packed {packed:.1f} us")
     assert dense < 0.96 * packed
+
+
+def test_packed_non_causal_backward_takes_groups(cuda):
+    """Groups are chosen by the batch's size and lengths, not by the order of its tiles: a small batch with one
+    long sequence takes them without the mask as well, and so runs faster than 65 sequences, which never do
+    (with one group it took as long as they)."""
+    lens = [1227] + [44] * 5
+    few, many = (_times(x, 32, False, cuda, 8)[1] for x in (lens, lens + [1] * 59))
+    print(f"non-causal, 6 / 65 sequences: backward {few:.1f} / {many:.1f} us")
+    assert few < 0.85 * many

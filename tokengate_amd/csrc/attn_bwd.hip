@@ -838,6 +838,9 @@ int dkv_groups(const BwdArgs &a, bool causal, bool varlen) {
   // rows, whole backward 13.3 us with one, 15.9 with four; 48 rows 15.8 / 17.7).  From about 80 keys on the larger
   // number of workgroups pays (64 queries x 80 keys 20.2 / 21.1, 64 x 128 23.1 / 21.1, 16 x 256 20.4 / 19.5).
   if (a.sq <= 64 && a.sk <= 64) return 1;
+  // nor do packed sequences of up to one tile of one group gain without the mask, which leaves no long tiles to
+  // shorten (9 of up to 100 tokens, 8 / 8 heads, 1.11 times as long with four, 59 of up to 107, 8 / 2, 1.05)
+  if (varlen && !causal && a.sk <= dkv_keys(1)) return 1;
   return cheapest(kDkvForms, varlen, [&](const GroupForm &f) {
     const int keys = dkv_keys(f.groups), slot = f.groups == 1 ? 64 : 128;
     const Levels v = levels_of(a, varlen, a.sk, keys);
@@ -857,9 +860,9 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
   if constexpr (VARLEN)
     hipLaunchKernelGGL(bwd_preprocess_kernel, dim3((unsigned)((nrows * 16 + 255) / 256)), dim3(256), 0, st, a, nrows);
   const int hp = (a.group % 2 == 0) ? 2 : 1;
-  // a batch that runs sequence-major fills the chip with one group
   const bool level_order = VARLEN && varlen_level_order(causal, a.batch, a.lse_total, a.hkv);
-  if (VARLEN && a.batch > 1 && !level_order) groups = false;
+  // a large batch fills the chip with one group
+  if (VARLEN && a.batch > 1 && !varlen_small(a.batch, a.lse_total, a.hkv)) groups = false;
   const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
   const int bmq = dq_bm(ks, hp);
   a.n_tiles = (a.sq + bmq - 1) / bmq;

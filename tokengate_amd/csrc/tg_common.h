@@ -382,16 +382,20 @@ float grid_cost(int n, int64_t units, int64_t slots, float wg, float solo, float
   return cost;
 }
 
+// Whether a varlen attention launch is small: up to 64 sequences (as many as one wave orders) and K/V of at most
+// half the 256 MB last-level cache.
+inline bool varlen_small(int num_seqs, int64_t key_rows, int num_heads_k) {
+  return num_seqs <= 64 && key_rows * num_heads_k * 512 <= (128ll << 20);
+}
 // Whether a varlen attention launch takes its tiles in level order, which packs the CUs best but streams
-// every sequence's K/V at once: causal launches (without the mask a tile's work does not depend on its
+// every sequence's K/V at once: small causal launches (without the mask a tile's work does not depend on its
 // level, and the short sequences' tiles only come between those that share a long one's K/V: 8192 and 4096
-// tokens, 8 / 8 heads, forward 329 us sequence-major, 411 in level order; backward 1121 and 1245), up to 64
-// sequences (one wave orders them) and K/V of at most half the 256 MB last-level cache.  Six packed
+// tokens, 8 / 8 heads, forward 329 us sequence-major, 411 in level order; backward 1121 and 1245).  Six packed
 // sequences of 260 to 4021 tokens (48 MB): forward + backward 761 -> 674 us against sequence-major, four of
 // 2048 forward 106 -> 74; eight prompts of 16k to 128k (2.9 GB) ran at 682 TFLOP/s heaviest first and 996
 // sequence-major.
 inline bool varlen_level_order(bool causal, int num_seqs, int64_t key_rows, int num_heads_k) {
-  return causal && num_seqs > 1 && num_seqs <= 64 && key_rows * num_heads_k * 512 <= (128ll << 20);
+  return causal && num_seqs > 1 && varlen_small(num_seqs, key_rows, num_heads_k);
 }
 // At most this many tiles of `rows` rows exist among total_rows rows of num_seqs sequences.
 inline int64_t level_tiles(int num_seqs, int64_t total_rows, int rows) { return total_rows / rows + num_seqs; }
