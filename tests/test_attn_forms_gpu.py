@@ -262,14 +262,19 @@ def test_varlen_non_causal_runs_sequence_after_sequence(cuda):
 
 
 def test_varlen_forward_level_order_only_where_it_balances(cuda):
-    """Where every query tile has a place from the start the forward runs sequence after sequence, so the causal
+    """Where every query tile has a CU of its own the forward runs sequence after sequence, so the causal
     mask makes no such batch slower (level order, which only causal launches take: 1.15 times).  So do sequences
-    of one length with up to three tiles: 64 take the time of 65, which never run in level order (1.1 times)."""
+    of one length with up to three tiles: 64 take the time of 65, which never run in level order (1.1 times).
+    Where two tiles share a CU, uneven sequences do run in level order (17.8 us without, 14.1 with)."""
     lens = list(range(21, 81, 4)) + [80]
     causal, full = _times(lens, 16, True, cuda, 8)[0], _times(lens, 16, False, cuda, 8)[0]
     few, major = _times([354] * 64, 16, True, cuda, 8)[0], _times([354] * 65, 16, True, cuda, 8)[0]
-    print(f"one round, causal / full: {causal:.1f} / {full:.1f} us, 64 / 65 sequences: {few:.1f} / {major:.1f} us")
+    print(f"own CUs, causal / full: {causal:.1f} / {full:.1f} us, 64 / 65 sequences: {few:.1f} / {major:.1f} us")
     assert causal < 1.02 * full and few < 1.08 * major
+    lens = [115, 42, 175, 106, 191, 119, 149, 83, 65, 83, 141, 91, 42, 160, 96, 21, 94, 166, 200, 99]
+    causal, full = (_times(lens, 16, c, cuda, 8)[0] for c in (True, False))
+    print(f"two to a CU, causal / full: {causal:.1f} / {full:.1f} us")
+    assert causal < 0.8 * full
 
 
 def test_varlen_short_rows_keep_one_group(cuda):

@@ -866,7 +866,7 @@ void launch_bwd(const BwdArgs &a0, bool causal, bool has_bias, int64_t nrows, bo
   const int ks = groups ? dq_groups(a, hp, causal, VARLEN) : 1;
   const int bmq = dq_bm(ks, hp);
   a.n_tiles = (a.sq + bmq - 1) / bmq;
-  // (with one tile each, sequence after sequence is the same order; where all have a place from the start, the
+  // (with one tile each, sequence after sequence is the same order; where all have a CU of their own, the
   // order decides nothing)
   const int64_t level_q = level_tiles(a.batch, a.lse_total, bmq) * (a.h / hp);
   a.level_order = level_order && a.n_tiles > 1 && level_q > device_cus();

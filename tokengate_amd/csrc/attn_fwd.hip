@@ -1327,16 +1327,18 @@ int keybias_fwd_varlen(const void *q, const void *k, const void *v, const float 
   TG_CHECK(workspace == nullptr || aligned16(workspace), "workspace must be 16-byte aligned");
   const FwdPlan plan = plan_varlen(hp, max_seqlen_q, max_seqlen_k, units, causal != 0, workspace ? workspace_bytes : 0);
   int64_t nblocks = apply_plan(a, plan, units, workspace);
-  // Sequence-major where level order has nothing to give.  Where every tile has a place from the start the order
-  // decides nothing (16 sequences of 21 to 80 tokens: 8.7 us, in level order 10.1).  Sequences of one length finish
+  // Sequence-major where level order has nothing to give.  Where every tile has a CU of its own the order decides
+  // nothing (16 sequences of 21 to 80 tokens: 8.7 us, in level order 10.1); it does where two four-wave workgroups
+  // share one (level / sequence-major, us: 20 of up to 200, 16 / 8 heads, 13.8 / 17.3, 23 of up to 370, 8 / 8, 15.7 /
+  // 16.9, 60 of up to 90, 8 / 2, 9.8 / 12.1; 8 of up to 150, 32 / 8, 9.3 / 8.5).  Sequences of one length finish
   // evenly by themselves; with up to three tiles each, level order then parts the few workgroups that share a
   // sequence's keys and mends no tail (level / sequence-major, 14 shapes of 8 to 32 heads: 22 x 360 tokens 1.17,
   // 54 x 378 1.13, 18 x 367 1.10, in the mean 1.05), with more there are long tiles to put first (64 x 500 with 16
   // heads 0.88, 8 x 2048 0.86, 30 x 1000 0.92; 52 x 609 1.08; in the mean of 19 0.99).
   const int64_t level_blocks = level_tiles(num_seqs, total_q, plan.nw * 32 / hp) * (num_heads / hp);
-  const bool one_round = level_blocks <= (int64_t)device_cus() * (8 / plan.nw);
+  const bool own_cu = level_blocks <= device_cus();
   const bool few_even_tiles = a.n_qtiles < 4 && total_q == (int64_t)num_seqs * max_seqlen_q;
-  a.level_order = a.n_heavy == 0 && a.n_qtiles > 1 && !one_round && !few_even_tiles &&
+  a.level_order = a.n_heavy == 0 && a.n_qtiles > 1 && !own_cu && !few_even_tiles &&
                   varlen_level_order(causal != 0, num_seqs, cu_k != nullptr ? (int64_t)num_seqs * max_seqlen_k : total_q,
                                      num_heads_k);
   if (a.level_order) nblocks = level_blocks;
