@@ -20,6 +20,8 @@ from tokengate_amd import _lib
     (1, 8192, 8192, 16, 8, True, (8, 1, 1)), (1, 32768, 32768, 16, 8, True, (8, 1, 1)),
     # eight against four waves in two rounds and over
     (16, 1074, 1074, 8, 8, True, (4, 1, 1)),      # 56; eight waves 64
+    (16, 626, 626, 12, 4, True, (4, 1, 1)),       # 38; 47
+    (4, 3944, 3944, 12, 4, True, (4, 1, 1)),      # 0.89 times
     (64, 287, 446, 12, 4, True, (4, 1, 1)),       # 76; 95
     (64, 112, 112, 8, 8, False, (4, 1, 1)),       # 17; 19
     (1, 8040, 8040, 16, 8, True, (8, 1, 1)),      # 231; four waves 258

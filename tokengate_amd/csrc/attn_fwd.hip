@@ -1036,10 +1036,10 @@ struct FwdPlan {
 // A dense launch's form and split.  Without key groups: eight waves where the grid gives at least two
 // workgroups per CU, else four, with the split where they have one (splits).  Another form, with or without
 // its split, takes their place where the estimate promises about what it is off by: against a split launch
-// 10 %, with key groups anything; against an unsplit one 20 %, and without any split 10 % from eight waves
-// to four and 6 % from four to eight.  Of 151 launches timed in each form (33 to 12000 rows, up to 32768 keys) and
-// 82 more of two rounds and over, none is then more than 2 % slower than the first rule's, and on average they
-// take 6.4 % and 4.4 % less.
+// 10 %, with key groups anything; against an unsplit one 20 %, and without any split 6 % from four waves to
+// eight and from eight to four 10 % in two even rounds (8 x 1024 46 / 48 us), past them anything.  Of 151
+// launches timed in each form (33 to 12000 rows, up to 32768 keys) and 82 more of two rounds and over, none is
+// then more than 2 % slower than the first rule's, and on average they take 6.6 % and 5.2 % less.
 // Eight against four waves: 16 x 1074 rows of 8 / 8 heads 64 / 56 us, 64 x 287 x 446 of 12 / 4 95 / 76, 8040 of
 // 16 / 8 231 / 258, where the grid just misses two per CU.  With no margin 17 of the 151 were slower, by up to
 // 15 %: 3000 rows over 32768 keys 760 -> 830 us, 3072 x 4096 without the mask 108 -> 117.
@@ -1066,7 +1066,8 @@ FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool spli
     }
     return true;
   };
-  const Form &first = kForms[Tiles(kForms[0], hp, sq, sk, causal).n_qtiles * units >= 2 * device_cus() ? 0 : 1];
+  const int64_t wide = Tiles(kForms[0], hp, sq, sk, causal).n_qtiles * units, two_rounds = 2 * device_cus();
+  const Form &first = kForms[wide >= two_rounds ? 0 : 1];
   if (!consider(first, true, INFINITY)) consider(first, false, INFINITY);
   const float first_cost = best_cost;
   const bool first_split = best.split.ns > 1;
@@ -1074,7 +1075,7 @@ FwdPlan plan_dense(int hp, int sq, int sk, int64_t units, bool causal, bool spli
     if (f.ks > 1 && !key_groups) continue;
     const float margin = !first_split ? 0.8f : f.ks > 1 ? 1.f : 0.9f;
     consider(f, true, margin * first_cost);
-    consider(f, false, (first_split || f.ks > 1 ? margin : f.nw == 4 ? 0.9f : 0.94f) * first_cost);
+    consider(f, false, (first_split || f.ks > 1 ? margin : f.nw == 8 ? 0.94f : wide > two_rounds ? 1.f : 0.9f) * first_cost);
   }
   return best;
 }
